@@ -160,3 +160,32 @@ def test_trained_network_against_heuristic_and_plain(fc, orc):
             f"learned vs heuristic {ms['heuristic'] / ms['learned']:.3f}x")
         assert ms["learned"] * 1.05 < ms["plain"]
         assert ms["learned"] < 1.10 * ms["heuristic"]
+
+
+@pytest.mark.parametrize("n", [1, 3, 15, 16, 17, 63, 64, 65, 255, 256, 257, 287, 288, 511, 513, 3001])
+def test_gradient_at_the_edges_of_the_row_tiles(fc, n):
+    """Row counts around the 16-row blocks of the forward/backward pass and
+    the 256-row tiles (and 32-row steps) of the parameter sums. The bound is
+    the one of a recursive FP32 sum, (terms + 1) * 2^-24 * sum |term|, for
+    the n rows and the at most 117 FMAs behind each term."""
+    w, X, T = _data(40 + n, n)
+    wr = np.random.default_rng(n).uniform(0.0, 4.0, n).astype(np.float32)
+    wr[0] = 1.0
+    lo, go = mlp.loss_grad(w, X, T, wr)
+    aw = np.abs(w.astype(np.float64))
+    W1, b1 = aw[:384].reshape(32, 12), aw[384:416]
+    W2, b2 = aw[416:1440].reshape(32, 32), aw[1440:1472]
+    W3, b3 = aw[1472:1760].reshape(9, 32), aw[1760:]
+    h1 = np.abs(X).astype(np.float64) @ W1.T + b1
+    h2 = h1 @ W2.T + b2
+    dy = (h2 @ W3.T + b3 + np.abs(T)) * (wr / wr.astype(np.float64).sum())[:, None]
+    d2 = dy @ W3
+    d1 = d2 @ W2
+    size = np.concatenate([x.reshape(-1) for x in (d1.T @ np.abs(X), d1.sum(0), d2.T @ h1, d2.sum(0), dy.T @ h2,
+                                                   dy.sum(0))])
+    with fc.Graph(fc.gen_grid(8, 8, 0.0, 1)) as g:
+        g.sched_set_params(w)
+        say(f"sched gradient n={n}")
+        loss, grad = g.sched_gradient(X, T, wr)
+        assert np.all(np.abs(grad - go) <= (n + 118) * 2.0 ** -24 * size)
+        assert abs(loss - lo) <= (n + 118) * 2.0 ** -24 * float((dy * (h2 @ W3.T + b3 + np.abs(T))).sum())
