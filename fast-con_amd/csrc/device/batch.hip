@@ -16,8 +16,16 @@
 // A query is not connected when an expanded side gains no new vertex for it.
 // These verdicts and distances equal the plain visit's (and the host BFS's).
 //
-// Execution follows the visit engine: one launch per phase, the last block
-// to finish decides the next phase, the host replays captured launches.
+// Two engines run the same phases. batch_team_kernel answers a whole batch in
+// one launch: every XCD's blocks form one or two wave machines that step from
+// phase to phase with a barrier inside the XCD (team.hpp). batch_kernel is one
+// launch per phase over all blocks, for traces, directed graphs, graphs whose
+// machines' workspaces would not fit and callers that ask for lanes. In both
+// the last block to finish a phase decides the next one.
+// Measured (R-MAT s22, 1,024 queries; s24, 16,384 of uneven reach): launches
+// on three lanes 2.06 and 83 ms, teams 0.22 and 8.8 ms: no launch between two
+// phases, every wave's state in the L2 of its XCD, narrower waves when there
+// are too few, and hub steps in place of most level-2 expansions.
 // Only the masks a wave touched are cleared afterwards (dirty bitmap), so a
 // wave costs nothing proportional to V beyond the bottom-up steps.
 #include "batch.hpp"
@@ -35,11 +43,13 @@
 #include "engine.hpp"
 #include "hubstage.hpp"
 #include "mlp.hpp"
+#include "team.hpp"
 
 namespace fcd {
 
 using fc::fail;
 
+static_assert(kRCount <= 12 && kRMfS == 4 && kRedSlots == 16, "three rounds of four words; four of them are ORs");
 constexpr uint32_t kBStage = 512;  // staged entries per wave and list
 // The control block's state: the words before the phase log, which the
 // finalising wave copies to LDS.
@@ -99,7 +109,7 @@ struct BShared {
   unsigned long long hedge[2][kWavesPerBlock];  // staged hub edges per side
   uint32_t base[2];
   unsigned long long hbase[2];
-  unsigned long long red[kRCount][kWavesPerBlock];
+  unsigned long long red[12][kWavesPerBlock];
   int last;
 };
 
@@ -112,7 +122,7 @@ __device__ __forceinline__ int64_t bdeg(const BatchParams<OffT>& p, int32_t u) {
 // sum for the rest) into this block's slot; lanes 0..kRCount-1 of wave 0
 // issue one atomic each, skipping zeros.
 __device__ __forceinline__ void block_reduce_slots(const unsigned long long* vals, unsigned long long* red,
-                                                   BShared& sh) {
+                                                   int bid, BShared& sh) {
   const int w = (int)(threadIdx.x >> 6);
 #pragma unroll
   for (int k = 0; k < kRCount; ++k) {
@@ -125,7 +135,7 @@ __device__ __forceinline__ void block_reduce_slots(const unsigned long long* val
     const int k = (int)threadIdx.x;
     unsigned long long a = 0;
     for (int i = 0; i < kWavesPerBlock; ++i) a = k < kRMfS ? (a | sh.red[k][i]) : (a + sh.red[k][i]);
-    unsigned long long* dst = red + (size_t)(blockIdx.x % kRedSlots) * kRedWords + k;
+    unsigned long long* dst = red + (size_t)((uint32_t)bid % kRedSlots) * kRedWords + k;
     if (a) {
       if (k < kRMfS)
         atomicOr(dst, a);
@@ -139,6 +149,41 @@ __device__ __forceinline__ void block_reduce_slots(const unsigned long long* val
 struct RedTot {
   unsigned long long v[kRCount];
 };
+
+// Loads of the workspace, which this launch writes. In a team (TEAM) other
+// blocks may have written the word earlier in the same launch, so the load
+// bypasses the L1; otherwise the launch boundary has ordered it.
+template <bool TEAM, typename T>
+__device__ __forceinline__ T ldw(const T* p) {
+  return TEAM ? ld_team(p) : *p;
+}
+
+// A field of the control block that every lane reads alike. A team's copy is
+// in LDS, from where the compiler would keep it in vector registers and turn
+// every loop over it into one with a lane mask.
+template <bool TEAM, typename T>
+__device__ __forceinline__ T uni(T v) {
+  if (!TEAM) return v;
+  if constexpr (sizeof(T) == 8) {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uint64_t)v);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)((uint64_t)v >> 32));
+    return (T)(((uint64_t)hi << 32) | lo);
+  } else {
+    return (T)__builtin_amdgcn_readfirstlane((int)v);
+  }
+}
+
+// A wave's OR of v into word k of the block's slot (the steps that only look
+// for meets: their registers go to the searches).
+__device__ __forceinline__ void wave_or_slot(unsigned long long* red, int bid, int k, unsigned long long v) {
+  const unsigned long long m = (unsigned long long)wave_reduce_full_nz_u64<kWaveOr>(v);
+  if (m && lane_id() == 0) atomicOr(red + (size_t)((uint32_t)bid % kRedSlots) * kRedWords + k, m);
+}
+
+__device__ __forceinline__ void wave_add_slot(unsigned long long* red, int bid, int k, unsigned long long v) {
+  const unsigned long long t = (unsigned long long)wave_reduce_full_nz_u64<kWaveSum>(v);
+  if (t && lane_id() == 0) atomicAdd(red + (size_t)((uint32_t)bid % kRedSlots) * kRedWords + k, t);
+}
 
 // Per-wave append state of the commit, bottom-up and filter phases: the next
 // frontier lists of both sides (normal vertices and hubs).
@@ -235,14 +280,29 @@ __device__ __forceinline__ void appends_block_flush(const BatchParams<OffT>& p, 
 // belongs to that side.
 template <typename OffT>
 __device__ __forceinline__ unsigned long long* rec_of(const BatchParams<OffT>& p, int x, int64_t u) {
-  return p.rec + 2 * (int64_t)p.V * x + 2 * u;
+  return (unsigned long long*)p.rec + 2 * (int64_t)p.V * x + 2 * u;
 }
 
-template <typename OffT>
+// The pair as one 16-byte load. A team's goes through a buffer descriptor
+// of the side's records, whose loads take the cache policy that bypasses the
+// L1 (there is no 16-byte atomic load); 16 * V < 2^32 (kTeamMaxV).
+template <bool TEAM, typename OffT>
+__device__ __forceinline__ ulonglong2 rec_load(const BatchParams<OffT>& p, int x, int64_t u) {
+  if (!TEAM) return *reinterpret_cast<const ulonglong2*>(rec_of(p, x, u));
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  constexpr int kSc1 = 16, kRawDword = 0x00027000;
+  const __amdgpu_buffer_rsrc_t rs =
+      __builtin_amdgcn_make_buffer_rsrc(rec_of(p, x, 0), 0, (int)((uint32_t)p.V * 16u), kRawDword);
+  const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)((uint32_t)u * 16u), 0, kSc1);
+  return make_ulonglong2(((unsigned long long)v.y << 32) | v.x, ((unsigned long long)v.w << 32) | v.z);
+}
+constexpr int64_t kTeamMaxV = (1ll << 28) - 1;
+
+template <bool TEAM, typename OffT>
 __device__ __forceinline__ ulonglong2 probe_load(const BatchParams<OffT>& p, int x, unsigned long long fm, int32_t u,
                                                  bool act) {
   ulonglong2 vn = make_ulonglong2(~0ull, 0ull);
-  if (act && fm) vn = *reinterpret_cast<const ulonglong2*>(rec_of(p, x, u));  // {visited, next}
+  if (act && fm) vn = rec_load<TEAM>(p, x, u);  // {visited, next}
   return vn;
 }
 
@@ -252,17 +312,22 @@ __device__ __forceinline__ void probe_apply(const BatchParams<OffT>& p, int x, u
   const unsigned long long m = fm & ~vn.x;
   if (m & ~vn.y) {
     __hip_atomic_fetch_or(rec_of(p, x, u) + 1, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (vn.y == 0) p.tm[u >> 5] = 1;
+    if (vn.y == 0) p.tm[group_pos((uint32_t)u / kGroup, p.gk)] = 1;
   }
 }
 
-template <typename OffT, int VW>
-__device__ __forceinline__ void expand_normal(const BatchParams<OffT>& p, int x, int par, uint32_t n,
-                                              unsigned long long act, int gwave, int nwaves,
+// The width is a run-time value and both sides run the same code: five
+// widths and two sides inlined made the kernel 110 KB, more than the 64 KB of
+// instruction cache that two CUs share, and every phase of a small wave
+// waited for its instructions (14-20 us where 5 us of work were left).
+template <bool TEAM, typename OffT>
+__device__ __forceinline__ void expand_normal(const BatchParams<OffT>& p, int x, int par, int vw,
+                                              uint32_t n, unsigned long long act, int gwave, int nwaves,
                                               unsigned long long& a_cnt, unsigned long long& e_cnt) {
-  constexpr int G = kWave / VW;
   const int lane = lane_id();
-  const int grp = lane / VW, sub = lane % VW;
+  const int sh = 31 - __builtin_clz((uint32_t)vw);  // vw is a power of two in [4, 64]
+  const int grp = lane >> sh, sub = lane & (vw - 1);
+  const uint32_t G = (uint32_t)kWave >> sh;
   const int32_t* list = p.fl[x][par];
   unsigned long long* F = p.F[x][par];
   if (n > (uint32_t)p.V) n = (uint32_t)p.V;
@@ -272,9 +337,9 @@ __device__ __forceinline__ void expand_normal(const BatchParams<OffT>& p, int x,
     OffT b = 0, e = 0;
     unsigned long long fm = 0;
     if (i < n) {
-      v = list[i];
+      v = ldw<TEAM>(list + i);
       if ((uint32_t)v < (uint32_t)p.V) {
-        fm = F[v] & act;
+        fm = ldw<TEAM>(F + v) & act;
         b = p.off[v] + (OffT)sub;
         e = p.off[v + 1];
         if (sub == 0 && fm) {
@@ -291,14 +356,14 @@ __device__ __forceinline__ void expand_normal(const BatchParams<OffT>& p, int x,
     if (v >= 0 && sub == 0) F[v] = 0ull;
     if (!fm) e = b;
     while (ballot(b < e)) {
-      const bool a0 = b < e, a1 = b + VW < e;
+      const bool a0 = b < e, a1 = b + vw < e;
       const int32_t u0 = a0 ? p.col[b] : 0;
-      const int32_t u1 = a1 ? p.col[b + VW] : 0;
-      const ulonglong2 r0 = probe_load(p, x, fm, u0, a0);
-      const ulonglong2 r1 = probe_load(p, x, fm, u1, a1);
+      const int32_t u1 = a1 ? p.col[b + vw] : 0;
+      const ulonglong2 r0 = probe_load<TEAM>(p, x, fm, u0, a0);
+      const ulonglong2 r1 = probe_load<TEAM>(p, x, fm, u1, a1);
       if (a0) probe_apply(p, x, fm, u0, r0);
       if (a1) probe_apply(p, x, fm, u1, r1);
-      b += 2 * VW;
+      b += 2 * vw;
     }
   }
 }
@@ -311,7 +376,7 @@ __device__ __forceinline__ void expand_normal(const BatchParams<OffT>& p, int x,
 // more waves: a wave's chain of dependent loads per pass, not the edge
 // count, then sets the phase's time (the roots' expansion at the start of a
 // wave has a few thousand hub edges).
-template <typename OffT>
+template <bool TEAM, typename OffT>
 __device__ __forceinline__ void expand_hubs(const BatchParams<OffT>& p, int x, int par, unsigned long long hubpk,
                                             unsigned long long act, int tile, int gwave, int nwaves,
                                             unsigned long long& a_cnt, unsigned long long& e_cnt) {
@@ -336,7 +401,7 @@ __device__ __forceinline__ void expand_hubs(const BatchParams<OffT>& p, int x, i
       const uint32_t span = hi - lo;
       const uint32_t step = (span + 63u) / 64u;
       const uint32_t pr = lo + (uint32_t)lane * step;
-      const bool le = pr < hi && (uint64_t)hb[pr] <= cb;
+      const bool le = pr < hi && (uint64_t)ldw<TEAM>(hb + pr) <= cb;
       const uint64_t m = ballot(le);
       const uint32_t k = 63u - (uint32_t)__builtin_clzll((unsigned long long)m);
       lo = lo + k * step;
@@ -355,16 +420,16 @@ __device__ __forceinline__ void expand_hubs(const BatchParams<OffT>& p, int x, i
         fm[j] = 0;
         pos[j] = 0;
         if (ae[j]) {
-          while (s + 1 < nh && (uint64_t)hb[s + 1] <= g) ++s;
-          const int32_t v = hl[s];
-          const uint64_t b0 = (uint64_t)hb[s];
+          while (s + 1 < nh && (uint64_t)ldw<TEAM>(hb + s + 1) <= g) ++s;
+          const int32_t v = ldw<TEAM>(hl + s);
+          const uint64_t b0 = (uint64_t)ldw<TEAM>(hb + s);
           bool good = (uint32_t)v < (uint32_t)p.V && b0 <= g;
           if (good) {
             pos[j] = p.off[v] + (OffT)(g - b0);
             good = pos[j] < p.off[v + 1];
           }
           if (good) {
-            fm[j] = F[v] & act;
+            fm[j] = ldw<TEAM>(F + v) & act;
             if (fm[j]) {
               e_cnt += 1;
               if (b0 == g) a_cnt += 1;  // first edge of a hub with live queries
@@ -380,7 +445,7 @@ __device__ __forceinline__ void expand_hubs(const BatchParams<OffT>& p, int x, i
       for (int j = 0; j < R; ++j) u[j] = (ae[j] && fm[j]) ? p.col[pos[j]] : 0;
       ulonglong2 r[R];
 #pragma unroll
-      for (int j = 0; j < R; ++j) r[j] = probe_load(p, x, fm[j], u[j], ae[j]);
+      for (int j = 0; j < R; ++j) r[j] = probe_load<TEAM>(p, x, fm[j], u[j], ae[j]);
 #pragma unroll
       for (int j = 0; j < R; ++j)
         if (ae[j] && fm[j]) probe_apply(p, x, fm[j], u[j], r[j]);
@@ -388,125 +453,149 @@ __device__ __forceinline__ void expand_hubs(const BatchParams<OffT>& p, int x, i
   }
 }
 
-template <typename OffT>
-__device__ __forceinline__ void expand_side(const BatchParams<OffT>& p, int x, int vw, int chunk,
+// rc: the launch's (a team: the phase's) copy of the control block.
+template <bool TEAM, typename OffT>
+__device__ __forceinline__ void expand_side(const BatchParams<OffT>& p, const BatchCtl* rc, int x, int vw, int chunk,
                                             unsigned long long act, int gwave, int nwaves,
                                             unsigned long long& a_cnt, unsigned long long& e_cnt) {
-  const BatchCtl* ctl = p.ctl;
-  const int par = ctl->cur[x];
-  const uint32_t n = ctl->fl_n[x][par];
-  switch (vw) {
-    case 4: expand_normal<OffT, 4>(p, x, par, n, act, gwave, nwaves, a_cnt, e_cnt); break;
-    case 8: expand_normal<OffT, 8>(p, x, par, n, act, gwave, nwaves, a_cnt, e_cnt); break;
-    case 16: expand_normal<OffT, 16>(p, x, par, n, act, gwave, nwaves, a_cnt, e_cnt); break;
-    case 32: expand_normal<OffT, 32>(p, x, par, n, act, gwave, nwaves, a_cnt, e_cnt); break;
-    default: expand_normal<OffT, 64>(p, x, par, n, act, gwave, nwaves, a_cnt, e_cnt); break;
-  }
-  expand_hubs(p, x, par, ctl->hub[x][par], act, chunk, gwave, nwaves, a_cnt, e_cnt);
-}
-
-// Groups of 32 vertices are dealt to the waves of a launch round-robin:
-// wave w owns groups w, w + nwaves, w + 2 nwaves, ... With vertices
-// numbered by decreasing degree the touched groups crowd at low ids, and
-// this spreads them over every wave. A wave reads the marks of 64 of its
-// groups at a time; slot k of such a read is group (jb + k) * nwaves + w.
-struct GroupDeal {
-  int64_t jb;
-  int nwaves, gwave;
-  __device__ __forceinline__ int64_t operator()(int k) const { return (jb + k) * (int64_t)nwaves + gwave; }
-};
-
-// Number of groups owned by wave gwave (groups = ceil(V / 32) < 2^27, so
-// a 32-bit division does).
-__device__ __forceinline__ int64_t owned_groups(int64_t groups, int gwave, int nwaves) {
-  return groups > gwave ? (int64_t)(((uint32_t)groups - (uint32_t)gwave + (uint32_t)nwaves - 1u) / (uint32_t)nwaves)
-                        : 0;
+  const int par = uni<TEAM>(rc->cur[x]);
+  const uint32_t n = uni<TEAM>(rc->fl_n[x][par]);
+  expand_normal<TEAM>(p, x, par, vw, n, act, gwave, nwaves, a_cnt, e_cnt);
+  expand_hubs<TEAM>(p, x, par, uni<TEAM>(rc->hub[x][par]), act, chunk, gwave, nwaves, a_cnt, e_cnt);
 }
 
 // Mark dirty vertices (visited words became non-zero this wave) in the dirty
-// bitmap, for a pass whose lanes 0..31 / 32..63 hold the 32 vertices of
-// groups g0 / g1 (each group owned by this wave in this launch). dbw is the
-// group's dirty word as loaded with the pass's records, so that the update
+// bitmap, for a pass whose lanes 8k .. 8k + 7 hold the vertices of the group
+// at position pos (each group owned by this wave in this launch). dbw is the
+// group's dirty byte as loaded with the pass's records, so that the update
 // waits for no load of its own.
 template <typename OffT>
-__device__ __forceinline__ void mark_dirty(const BatchParams<OffT>& p, bool dirty, int64_t g0, int64_t g1,
-                                           uint32_t dbw) {
-  const uint64_t dm = ballot(dirty);
+__device__ __forceinline__ void mark_dirty(const BatchParams<OffT>& p, bool dirty, uint32_t pos, uint8_t dbw) {
   const int lane = lane_id();
-  if (lane == 0 && (uint32_t)dm) p.db[g0] = dbw | (uint32_t)dm;
-  if (lane == 32 && (dm >> 32) && g1 >= 0) p.db[g1] = dbw | (uint32_t)(dm >> 32);
+  const uint8_t mine = (uint8_t)(ballot(dirty) >> (lane & ~(int)(kGroup - 1)));
+  if (mine && (lane & (int)(kGroup - 1)) == 0) p.db[pos] = dbw | mine;
 }
 
 // Commit: every vertex of a touched group folds its N words into its visited
-// words, and newly reached vertices join the next frontiers. The wave reads
-// the marks of 64 of its groups (dealt round-robin), then handles the marked
-// groups two at a time (lanes 0..31 and 32..63, each half-wave reading and
-// writing one group's records in address order); the records and
-// offsets of the next pair are loaded before the current pair is processed,
+// words, and newly reached vertices join the next frontiers. A wave takes a
+// run of positions of the marks (MarkWalk),
+// lists the marked ones in LDS and handles them eight at a time (eight lanes
+// reading and writing one group's records in address order); the records and
+// offsets of the next eight are loaded before the current ones are processed,
 // so each pass costs about one memory round trip. Each group belongs to one
-// wave of the launch, which therefore updates its dirty-bitmap word without
-// an atomic.
+// wave of the launch, which therefore updates its dirty byte without an
+// atomic. The marks had been dealt
+// group by group round-robin, a cache line per mark: a team of 256 waves
+// would have read 524,288 lines per commit at R-MAT s24, 16 us of its L2.
+constexpr uint32_t kMarkChunk = 2048;
+
+// A wave's walk over the bytes of a group array (marks, dirty bits), which it
+// clears: chunks of up to kMarkChunk positions (down to 64, until every wave
+// has one), eight positions a lane and load, all loads of a chunk in flight
+// together (at R-MAT s24 a team's wave walks 8,192 positions, and one load
+// after another took a memory round trip per 512).
+struct MarkWalk {
+  uint8_t* bytes;
+  uint32_t P, chunk, step, at;
+  __device__ __forceinline__ MarkWalk(uint8_t* b, uint32_t P_, int gwave, int nwaves) : bytes(b), P(P_) {
+    chunk = kMarkChunk;
+    while (chunk > kWave && P < chunk * (uint32_t)nwaves) chunk >>= 1;
+    at = (uint32_t)gwave * chunk;
+    step = (uint32_t)nwaves * chunk;
+  }
+  // List the next chunk's non-zero bytes: put(k, position, byte) for k = 0 ..
+  // cnt - 1. False at the end of the walk.
+  template <bool TEAM, typename Put>
+  __device__ __forceinline__ bool next(uint32_t& cnt, Put put) {
+    if (at >= P) return false;
+    constexpr int N = kMarkChunk / (8 * kWave);
+    const uint32_t lane8 = 8u * (uint32_t)lane_id();
+    unsigned long long w[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      const uint32_t o = (uint32_t)k * 8 * kWave + lane8;
+      w[k] = 0;
+      if (o < chunk) {
+        unsigned long long* q = reinterpret_cast<unsigned long long*>(bytes + at + o);
+        w[k] = ldw<TEAM>(q);
+        if (w[k]) *q = 0ull;
+      }
+    }
+    cnt = 0;
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      if (!ballot(w[k] != 0)) continue;
+#pragma unroll 1
+      for (int b = 0; b < 8; ++b) {
+        const uint8_t v = (uint8_t)(w[k] >> (8 * b));
+        const uint64_t m = ballot(v != 0);
+        if (v) put(cnt + lane_rank(m), at + (uint32_t)k * 8 * kWave + lane8 + (uint32_t)b, v);
+        cnt += (uint32_t)__popcll(m);
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+    at += step;
+    return true;
+  }
+};
+
 template <typename OffT>
 struct CommitLoad {
   ulonglong2 a, b;  // {visS, NS}, {visT, NT}
   OffT o0, o1;
   int32_t u;
-  uint32_t dbw;     // the dirty-bitmap word of the lane's group
+  uint32_t pos;     // the position of the lane's group
+  uint8_t dbw;      // its dirty byte
   bool valid;
 };
 
-template <typename OffT>
-__device__ __forceinline__ CommitLoad<OffT> commit_load(const BatchParams<OffT>& p, const GroupDeal& gd, int k0,
-                                                        int k1) {
+template <bool TEAM, typename OffT>
+__device__ __forceinline__ CommitLoad<OffT> commit_load(const BatchParams<OffT>& p, const uint16_t* list,
+                                                        uint32_t at, uint32_t i, uint32_t cnt) {
   const int lane = lane_id();
-  const int mine = lane < 32 ? k0 : k1;
+  const uint32_t k = i + (uint32_t)lane / kGroup;
   CommitLoad<OffT> c;
-  const int64_t u = gd(mine < 0 ? 0 : mine) * 32 + (lane & 31);
-  c.u = (int32_t)u;
-  c.valid = mine >= 0 && u < p.V;
+  c.valid = false;
   c.a = c.b = make_ulonglong2(0ull, 0ull);
   c.o0 = c.o1 = 0;
-  c.dbw = mine >= 0 ? p.db[gd(mine)] : 0u;
-  if (c.valid) {
-    c.a = *reinterpret_cast<const ulonglong2*>(rec_of(p, 0, u));
-    c.b = *reinterpret_cast<const ulonglong2*>(rec_of(p, 1, u));
-    c.o0 = p.off[u];
-    c.o1 = p.off[u + 1];
+  c.dbw = 0;
+  c.pos = 0;
+  c.u = 0;
+  if (k < cnt) {
+    const uint32_t pos = at + list[k];
+    const int64_t u = (int64_t)group_at(pos, p.gk) * kGroup + (lane & (int)(kGroup - 1));
+    c.pos = pos;
+    c.u = (int32_t)u;
+    c.valid = u < p.V;
+    c.dbw = ldw<TEAM>(p.db + pos);
+    if (c.valid) {
+      c.a = rec_load<TEAM>(p, 0, u);
+      c.b = rec_load<TEAM>(p, 1, u);
+      c.o0 = p.off[u];
+      c.o1 = p.off[u + 1];
+    }
   }
   return c;
 }
 
-__device__ __forceinline__ bool take_pair(uint64_t& nz, int& k0, int& k1) {
-  if (!nz) return false;
-  k0 = __builtin_ctzll(nz);
-  nz &= nz - 1;
-  k1 = -1;
-  if (nz) {
-    k1 = __builtin_ctzll(nz);
-    nz &= nz - 1;
-  }
-  return true;
-}
-
-template <typename OffT>
+// s_list: kMarkChunk entries of this wave's LDS.
+template <bool TEAM, typename OffT>
 __device__ __forceinline__ void commit_pass(const BatchParams<OffT>& p, Appends& ap, unsigned long long act,
-                                            const int* nxt, int gwave, int nwaves, unsigned long long* red) {
+                                            const int* nxt, int gwave, int nwaves, uint16_t* s_list,
+                                            unsigned long long* red) {
   const int lane = lane_id();
-  const int64_t per = owned_groups(((int64_t)p.V + 31) / 32, gwave, nwaves);
-  for (int64_t jb = 0; jb < per; jb += kWave) {
-    const GroupDeal gd{jb, nwaves, gwave};
-    const int64_t gi = gd(lane);
-    const bool marked = jb + lane < per && p.tm[gi] != 0;
-    if (marked) p.tm[gi] = 0;
-    uint64_t nz = ballot(marked);
-    int k0, k1;
-    if (!take_pair(nz, k0, k1)) continue;
-    CommitLoad<OffT> cur = commit_load(p, gd, k0, k1);
-    for (;;) {
-      int n0 = -1, n1 = -1;
-      const bool more = take_pair(nz, n0, n1);
+  MarkWalk mw(p.tm, kGroupClasses * (uint32_t)p.gk, gwave, nwaves);
+  uint32_t cnt;
+  for (;;) {
+    const uint32_t at = mw.at;
+    if (!mw.next<TEAM>(cnt, [&](uint32_t k, uint32_t pos, uint8_t) { s_list[k] = (uint16_t)(pos - at); })) break;
+    if (!cnt) continue;
+    CommitLoad<OffT> cur = commit_load<TEAM>(p, s_list, at, 0, cnt);
+    constexpr uint32_t kStep = kWave / kGroup;
+    for (uint32_t i = 0; i < cnt; i += kStep) {
       CommitLoad<OffT> nx;
-      if (more) nx = commit_load(p, gd, n0, n1);
+      if (i + kStep < cnt) nx = commit_load<TEAM>(p, s_list, at, i + kStep, cnt);
       unsigned long long nS = 0, nT = 0, vS = 0, vT = 0;
       int64_t deg = 0;
       const int32_t u = cur.u;
@@ -532,27 +621,23 @@ __device__ __forceinline__ void commit_pass(const BatchParams<OffT>& p, Appends&
       }
       push_frontier(p, ap, 0, nxt[0], nS != 0, u, deg);
       push_frontier(p, ap, 1, nxt[1], nT != 0, u, deg);
-      mark_dirty(p, ((vS | vT) == 0) && ((nS | nT) != 0), gd(k0), k1 >= 0 ? gd(k1) : (int64_t)-1, cur.dbw);
-      if (!more) break;
-      cur = nx;
-      k0 = n0;
-      k1 = n1;
+      mark_dirty(p, ((vS | vT) == 0) && ((nS | nT) != 0), cur.pos, cur.dbw);
+      if (i + kStep < cnt) cur = nx;
     }
   }
 }
 
-// Bottom-up step for the sides in SIDES (bit x = side x): every vertex still
+// Bottom-up step for the given sides (bit x = side x): every vertex still
 // needed by some live query ORs the current frontier masks of its
 // neighbours, stopping once it has every bit it needs. Both sides share one
 // scan of the adjacency list.
-template <typename OffT, int SIDES>
-__device__ __forceinline__ void bottom_up(const BatchParams<OffT>& p, Appends& ap, unsigned long long act,
+template <bool TEAM, typename OffT>
+__device__ __forceinline__ void bottom_up(const BatchParams<OffT>& p, const BatchCtl* rc, int sides, Appends& ap, unsigned long long act,
                                           int gwave, int nwaves, unsigned long long* red) {
-  const BatchCtl* ctl = p.ctl;
-  constexpr bool DS = (SIDES & 1) != 0, DT = (SIDES & 2) != 0;
-  const int nxt[2] = {ctl->cur[0] ^ 1, ctl->cur[1] ^ 1};
-  const unsigned long long* FS = p.F[0][ctl->cur[0]];
-  const unsigned long long* FT = p.F[1][ctl->cur[1]];
+  const bool DS = (sides & 1) != 0, DT = (sides & 2) != 0;
+  const int nxt[2] = {uni<TEAM>(rc->cur[0]) ^ 1, uni<TEAM>(rc->cur[1]) ^ 1};
+  const unsigned long long* FS = p.F[0][uni<TEAM>(rc->cur[0])];
+  const unsigned long long* FT = p.F[1][uni<TEAM>(rc->cur[1])];
   const int lane = lane_id();
   const int64_t nthr = (int64_t)nwaves * kWave;
   // isolated vertices (the tail of a degree-ordered numbering) gain no bit
@@ -560,11 +645,11 @@ __device__ __forceinline__ void bottom_up(const BatchParams<OffT>& p, Appends& a
     const int32_t u = (int32_t)(base + lane);
     unsigned long long accS = 0, accT = 0, needS = 0, needT = 0, vS = 0, vT = 0;
     OffT b = 0, e = 0;
-    // this lane's group's dirty word (lanes 0..31: base / 32, 32..63: the next)
-    const uint32_t dbw = base + (lane & 32) < p.V ? p.db[(base >> 5) + (lane >> 5)] : 0u;
+    const uint32_t dpos = group_pos((uint32_t)u / kGroup, p.gk);
+    const uint8_t dbw = u < p.V ? ldw<TEAM>((const uint8_t*)p.db + dpos) : (uint8_t)0;
     if (u < p.V) {
-      vS = rec_of(p, 0, u)[0];
-      vT = rec_of(p, 1, u)[0];
+      vS = ldw<TEAM>(rec_of(p, 0, u));
+      vT = ldw<TEAM>(rec_of(p, 1, u));
       if (DS) needS = act & ~vS;
       if (DT) needT = act & ~vT;
       if (needS | needT) {
@@ -583,8 +668,8 @@ __device__ __forceinline__ void bottom_up(const BatchParams<OffT>& p, Appends& a
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
           if (c[k] < 0) continue;
-          if (DS) accS |= FS[c[k]];
-          if (DT) accT |= FT[c[k]];
+          if (DS) accS |= ldw<TEAM>(FS + c[k]);
+          if (DT) accT |= ldw<TEAM>(FT + c[k]);
         }
         red[kRActE] += (unsigned long long)((j + 4 <= e) ? 4 : (e - j));
         if ((accS & needS) == needS && (accT & needT) == needT) break;
@@ -610,7 +695,7 @@ __device__ __forceinline__ void bottom_up(const BatchParams<OffT>& p, Appends& a
     if (DS) push_frontier(p, ap, 0, nxt[0], nS != 0, u, deg);
     if (DT) push_frontier(p, ap, 1, nxt[1], nT != 0, u, deg);
     // vertices base .. base+63 are this wave's alone in this launch
-    mark_dirty(p, (nS | nT) != 0 && (vS | vT) == 0, base >> 5, (base >> 5) + 1, dbw);
+    mark_dirty(p, (nS | nT) != 0 && (vS | vT) == 0, dpos, dbw);
   }
 }
 
@@ -618,36 +703,45 @@ __device__ __forceinline__ void bottom_up(const BatchParams<OffT>& p, Appends& a
 // queries resolved since they were built. Keep each vertex's mask restricted
 // to the live queries in the other parity, clear the old mask, and rebuild
 // the lists (and the hub edge bases) from the survivors only.
-template <typename OffT, int x>
-__device__ __forceinline__ void filter_side(const BatchParams<OffT>& p, Appends& ap, unsigned long long act,
-                                            int gwave, int nwaves, unsigned long long* red) {
-  const BatchCtl* ctl = p.ctl;
-  const int c = ctl->cur[x], nx = c ^ 1;
+template <bool TEAM, typename OffT>
+__device__ __forceinline__ void filter_sides(const BatchParams<OffT>& p, const BatchCtl* rc, int sides, Appends& ap,
+                                             unsigned long long act, int gwave, int nwaves, unsigned long long* red) {
   const int lane = lane_id();
-  unsigned long long* Fc = p.F[x][c];
-  unsigned long long* Fn = p.F[x][nx];
-  uint32_t n = ctl->fl_n[x][c];
-  if (n > (uint32_t)p.V) n = (uint32_t)p.V;
-  uint32_t nh = (uint32_t)(ctl->hub[x][c] >> kHubEdgeBits);
-  if (nh > p.hcap) nh = p.hcap;
-  const uint32_t tot = n + nh;
-  for (uint32_t base = (uint32_t)gwave * kWave; base < tot; base += (uint32_t)nwaves * kWave) {
-    const uint32_t i = base + (uint32_t)lane;
-    int32_t v = -1;
-    if (i < tot) v = i < n ? p.fl[x][c][i] : p.hl[x][c][i - n];
-    unsigned long long keep = 0;
-    int64_t deg = 0;
-    if ((uint32_t)v < (uint32_t)p.V) {
-      const unsigned long long fm = Fc[v];
-      Fc[v] = 0ull;
-      keep = fm & act;
-      if (keep) {
-        Fn[v] = keep;
-        deg = bdeg(p, v);
-        red[kRMfS + x] += (unsigned long long)deg;
+#pragma unroll 1
+  for (int x = 0; x < 2; ++x) {
+    if (!(sides & (1 << x))) continue;
+    const int c = uni<TEAM>(rc->cur[x]), nx = c ^ 1;
+    unsigned long long* Fc = p.F[x][c];
+    unsigned long long* Fn = p.F[x][nx];
+    uint32_t n = uni<TEAM>(rc->fl_n[x][c]);
+    if (n > (uint32_t)p.V) n = (uint32_t)p.V;
+    uint32_t nh = (uint32_t)(uni<TEAM>(rc->hub[x][c]) >> kHubEdgeBits);
+    if (nh > p.hcap) nh = p.hcap;
+    const uint32_t tot = n + nh;
+    unsigned long long mf = 0;
+    for (uint32_t base = (uint32_t)gwave * kWave; base < tot; base += (uint32_t)nwaves * kWave) {
+      const uint32_t i = base + (uint32_t)lane;
+      int32_t v = -1;
+      if (i < tot) v = ldw<TEAM>(i < n ? p.fl[x][c] + i : p.hl[x][c] + (i - n));
+      unsigned long long keep = 0;
+      int64_t deg = 0;
+      if ((uint32_t)v < (uint32_t)p.V) {
+        const unsigned long long fm = ldw<TEAM>(Fc + v);
+        Fc[v] = 0ull;
+        keep = fm & act;
+        if (keep) {
+          Fn[v] = keep;
+          deg = bdeg(p, v);
+          mf += (unsigned long long)deg;
+        }
       }
+      // one of the two, with its own stages (constant indices keep them in
+      // registers)
+      push_frontier(p, ap, 0, nx, x == 0 && keep != 0, v, deg);
+      push_frontier(p, ap, 1, nx, x == 1 && keep != 0, v, deg);
     }
-    push_frontier(p, ap, x, nx, keep != 0, v, deg);
+    red[kRMfS] += x == 0 ? mf : 0ull;
+    red[kRMfT] += x == 1 ? mf : 0ull;
   }
 }
 
@@ -664,11 +758,11 @@ __device__ __forceinline__ void filter_side(const BatchParams<OffT>& p, Appends&
 // at distance 3, and the level-1 hubs that the next expansion would scan
 // (millions of edges) belong almost only to them: the queries that survive
 // a bridge carry about 5% of those edges. A pair left untested only leaves
-// its queries to the expansion, which finds the same distance, so each wave
-// tests at most kBridgeMaxTests pairs and the step's time stays bounded.
+// its queries to the expansion, which finds the same distance, so a step
+// tests at most about kBridgeMaxTests pairs and its time stays bounded.
 constexpr uint32_t kBridgeQueue = 256;             // pairs queued per wave (16 bytes each, 4 KB)
 constexpr uint64_t kBridgeMaxPairs = 1ull << 26;   // list-entry pairs a bridge step may enumerate
-constexpr uint32_t kBridgeMaxTests = 1024;         // pairs a wave tests (16 rounds of 64 searches)
+constexpr uint32_t kBridgeMaxTests = 1u << 21;      // pairs a step tests, shared evenly by its waves
 constexpr uint64_t kBridgeMinEdges = 1ull << 20;   // live frontier edges of the cheaper side (default)
 static_assert(kBridgeQueue * 16 * kWavesPerBlock <= 2 * kWavesPerBlock * kBStage * sizeof(int32_t),
               "bridge queues fit the appends' stage");
@@ -760,26 +854,31 @@ __device__ __forceinline__ void bridge_flush(const BatchParams<OffT>& p, const i
   __builtin_amdgcn_wave_barrier();
 }
 
-template <typename OffT>
-__device__ __forceinline__ void bridge_pass(const BatchParams<OffT>& p, unsigned long long act, int gwave,
-                                            int nwaves, unsigned char* lds, unsigned long long& meets) {
-  const BatchCtl* ctl = p.ctl;
+template <bool TEAM, typename OffT>
+__device__ __forceinline__ void bridge_pass(const BatchParams<OffT>& p, const BatchCtl* rc, unsigned long long act,
+                                            int gwave, int nwaves, unsigned char* lds, unsigned long long& meets,
+                                            unsigned long long& untested) {
   const int lane = lane_id(), w = (int)(threadIdx.x >> 6);
   int32_t* qa = reinterpret_cast<int32_t*>(lds + (size_t)w * kBridgeQueue * 16);
   int32_t* qb = qa + kBridgeQueue;
   unsigned long long* qm = reinterpret_cast<unsigned long long*>(qb + kBridgeQueue);
-  const int c0 = ctl->cur[0], c1 = ctl->cur[1];
+  const int c0 = uni<TEAM>(rc->cur[0]), c1 = uni<TEAM>(rc->cur[1]);
   const uint32_t V = (uint32_t)p.V;
-  const uint32_t n0 = ctl->fl_n[0][c0] < V ? ctl->fl_n[0][c0] : V;
-  const uint32_t n1 = ctl->fl_n[1][c1] < V ? ctl->fl_n[1][c1] : V;
-  uint32_t h0 = (uint32_t)(ctl->hub[0][c0] >> kHubEdgeBits), h1 = (uint32_t)(ctl->hub[1][c1] >> kHubEdgeBits);
+  const uint32_t n0 = uni<TEAM>(rc->fl_n[0][c0]) < V ? uni<TEAM>(rc->fl_n[0][c0]) : V;
+  const uint32_t n1 = uni<TEAM>(rc->fl_n[1][c1]) < V ? uni<TEAM>(rc->fl_n[1][c1]) : V;
+  uint32_t h0 = (uint32_t)(uni<TEAM>(rc->hub[0][c0]) >> kHubEdgeBits), h1 = (uint32_t)(uni<TEAM>(rc->hub[1][c1]) >> kHubEdgeBits);
   h0 = h0 < p.hcap ? h0 : p.hcap;
   h1 = h1 < p.hcap ? h1 : p.hcap;
   const uint32_t nS = n0 + h0, nT = n1 + h1;
   const uint32_t ct = (nT + kWave - 1) / kWave;
   const uint64_t tiles = (uint64_t)((nS + kWave - 1) / kWave) * ct;
   uint32_t cnt = 0, tested = 0;
-  for (uint64_t tile = (uint64_t)gwave; tile < tiles && tested < kBridgeMaxTests; tile += (uint64_t)nwaves) {
+  const uint32_t max_tests = kBridgeMaxTests / (uint32_t)nwaves;
+  for (uint64_t tile = (uint64_t)gwave; tile < tiles; tile += (uint64_t)nwaves) {
+    if (tested >= max_tests) {
+      untested = 1;
+      break;
+    }
     // tiles < 2^32: a bridge step runs only when the lists' product is at
     // most kBridgeMaxPairs
     const uint32_t ti = (uint32_t)tile / ct;
@@ -788,16 +887,16 @@ __device__ __forceinline__ void bridge_pass(const BatchParams<OffT>& p, unsigned
     int32_t a = -1, b = -1;
     unsigned long long fa = 0, fb = 0;
     if (i < nS) {
-      a = i < n0 ? p.fl[0][c0][i] : p.hl[0][c0][i - n0];
+      a = ldw<TEAM>(i < n0 ? p.fl[0][c0] + i : p.hl[0][c0] + (i - n0));
       if ((uint32_t)a < V)
-        fa = p.F[0][c0][a] & act;
+        fa = ldw<TEAM>(p.F[0][c0] + a) & act;
       else
         atomicOr(&p.ctl->err, 2u);
     }
     if (j < nT) {
-      b = j < n1 ? p.fl[1][c1][j] : p.hl[1][c1][j - n1];
+      b = ldw<TEAM>(j < n1 ? p.fl[1][c1] + j : p.hl[1][c1] + (j - n1));
       if ((uint32_t)b < V)
-        fb = p.F[1][c1][b] & act;
+        fb = ldw<TEAM>(p.F[1][c1] + b) & act;
       else
         atomicOr(&p.ctl->err, 2u);
     }
@@ -815,7 +914,10 @@ __device__ __forceinline__ void bridge_pass(const BatchParams<OffT>& p, unsigned
         bridge_flush(p, qa, qb, qm, cnt, meets);
         tested += cnt;
         cnt = 0;
-        if (tested >= kBridgeMaxTests) break;
+        if (tested >= max_tests) {
+          untested = 1;
+          break;
+        }
       }
       if (hit) {
         const uint32_t pos = cnt + lane_rank(hm);
@@ -827,6 +929,129 @@ __device__ __forceinline__ void bridge_pass(const BatchParams<OffT>& p, unsigned
     }
   }
   if (cnt) bridge_flush(p, qa, qb, qm, cnt, meets);
+}
+
+// Hub step (teams): meets at the top vertices, those of the highest degrees
+// (device ids below hub_tab under the degree numbering), which on a skewed
+// graph lie in almost every small ball. A list in id order holds its top
+// neighbours first, so only the head of each frontier vertex's list is read,
+// and the top vertices' masks fit LDS, so nothing is claimed with atomics.
+// Two kinds of meets, at levels (i, j) of a query still live, whose distance
+// is therefore > i + j:
+//  * a top neighbour of one side's frontier vertex that lies in the other
+//    side's ball: a path of at most i + 1 + j edges, so the distance is
+//    i + j + 1 (odd);
+//  * a top vertex next to both sides' frontiers: a path of i + j + 2 edges.
+//    That is the distance once a complete bridge step has excluded
+//    i + j + 1, so the bridge step at the same levels settles these.
+// A meet that is missed only leaves its query to the later steps, which find
+// the same distance. At R-MAT s22 the level-1 frontiers' expansion and its
+// commit took 400 us of a wave's 680 on one XCD, bound by atomics (3.4 G/s
+// per XCD) and by reading all groups of records; the queries that a hub and
+// a bridge step leave carry a few per cent of its edges.
+constexpr int kHubTab = 512;
+static_assert(4 * kHubTab * sizeof(unsigned long long) <= 2 * kWavesPerBlock * kBStage * sizeof(int32_t),
+              "hub tables fit the appends' stage");
+
+template <typename OffT>
+__device__ __forceinline__ void hub_pass(const BatchParams<OffT>& p, const BatchCtl* rc, unsigned long long act,
+                                         int bid, int gwave, int nwaves, unsigned long long* tab,
+                                         unsigned long long& odd) {
+  // tab: visited masks of sides s and t, then the masks of their frontiers' neighbours
+  const int K = p.hub_tab;
+  for (int u = (int)threadIdx.x; u < K; u += kBlock) {
+    tab[u] = ld_team(rec_of(p, 0, u));
+    tab[kHubTab + u] = ld_team(rec_of(p, 1, u));
+    tab[2 * kHubTab + u] = 0ull;
+    tab[3 * kHubTab + u] = 0ull;
+  }
+  __syncthreads();
+  // Four lanes take a vertex of the normal list, a whole wave one of the hub
+  // list, with four columns a lane in flight; the entry of the round after
+  // next and the mask and offsets of the next round are loaded while a
+  // round's columns are read.
+  constexpr int R = 4;
+  const int lane = lane_id();
+#pragma unroll 1
+  for (int x = 0; x < 2; ++x) {
+    const unsigned long long* other = tab + (x ^ 1) * kHubTab;
+    unsigned long long* next = tab + (2 + x) * kHubTab;
+    const int c = uni<true>(rc->cur[x]);
+    uint32_t n = uni<true>(rc->fl_n[x][c]);
+    if (n > (uint32_t)p.V) n = (uint32_t)p.V;
+    uint32_t nh = (uint32_t)(uni<true>(rc->hub[x][c]) >> kHubEdgeBits);
+    if (nh > p.hcap) nh = p.hcap;
+#pragma unroll 1
+    for (int hubs = 0; hubs < 2; ++hubs) {
+      const uint32_t tot = hubs ? nh : n;
+      const int32_t* list = hubs ? p.hl[x][c] : p.fl[x][c];
+      const int vw = hubs ? kWave : 4, grp = hubs ? 0 : lane >> 2, sub = hubs ? lane : lane & 3;
+      const uint32_t per = hubs ? 1u : (uint32_t)kWave / 4u, stride = (uint32_t)nwaves * per;
+      auto entry = [&](uint32_t i) { return i < tot ? ld_team(list + i) : -1; };
+      struct Head {
+        OffT b;
+        int32_t len;  // a degree is at most V <= kTeamMaxV
+        unsigned long long fm;
+      };
+      auto head = [&](int32_t v) {
+        Head h{0, 0, 0ull};
+        if ((uint32_t)v < (uint32_t)p.V) {
+          h.fm = ld_team(p.F[x][c] + v) & act;
+          h.b = p.off[v];
+          h.len = (int32_t)(p.off[v + 1] - h.b);
+        }
+        return h;
+      };
+      const uint32_t first = (uint32_t)gwave * per;
+      Head cur = head(entry(first + (uint32_t)grp));
+      int32_t v1 = entry(first + stride + (uint32_t)grp);
+      for (uint32_t base = first; base < tot; base += stride) {
+        const int32_t v2 = entry(base + 2 * stride + (uint32_t)grp);
+        const Head nx = head(v1);
+        const unsigned long long fm = cur.fm;
+        int32_t len = fm ? cur.len : 0;
+        for (int32_t r = sub; ballot(r < len);) {
+          int32_t u[R];
+#pragma unroll
+          for (int k = 0; k < R; ++k) u[k] = r + k * vw < len ? p.col[cur.b + (OffT)(r + k * vw)] : K;
+          r += R * vw;
+#pragma unroll
+          for (int k = 0; k < R; ++k) {
+            if (u[k] >= K) continue;
+            odd |= fm & other[u[k]];
+            if (fm & ~next[u[k]]) atomicOr(next + u[k], fm);
+          }
+          if (u[R - 1] >= K) len = 0;  // the rest of the list has larger ids
+        }
+        cur = nx;
+        v1 = v2;
+      }
+    }
+  }
+  __syncthreads();
+  for (int u = (int)threadIdx.x; u < 2 * K; u += kBlock) {
+    const int x = u >= K ? 1 : 0;
+    p.ht[(size_t)(2 * bid + x) * kHubTab + (u - x * K)] = tab[(2 + x) * kHubTab + (u - x * K)];
+  }
+}
+
+// The queries with a top vertex next to both sides' frontiers, from the
+// blocks' tables: a wave takes a top vertex, its lanes the blocks. Part of
+// the bridge step that follows, where all blocks share it (in the hub step's
+// finalising block alone it took 60 us).
+template <typename OffT>
+__device__ __forceinline__ unsigned long long hub_even(const BatchParams<OffT>& p, int nb, int gwave, int nwaves) {
+  unsigned long long ev = 0;
+  for (int u = gwave; u < p.hub_tab; u += nwaves) {
+    unsigned long long a = 0, b = 0;
+    for (int k = lane_id(); k < nb; k += kWave) {
+      a |= ld_team(p.ht + (size_t)(2 * k) * kHubTab + u);
+      b |= ld_team(p.ht + (size_t)(2 * k + 1) * kHubTab + u);
+    }
+    ev |= (unsigned long long)wave_reduce_full_nz_u64<kWaveOr>(a) &
+          (unsigned long long)wave_reduce_full_nz_u64<kWaveOr>(b);
+  }
+  return ev;
 }
 
 // Whether a bridge step runs before the pending step decision (lane 0 of the
@@ -936,6 +1161,35 @@ __device__ __forceinline__ bool bridge_due(const BatchParams<OffT>& p, const Bat
   return (m0 < m1 ? m0 : m1) >= ctl->bridge_min_e;
 }
 
+// Teams: whether a hub step runs before the pending decision: once per pair
+// of levels, on frontiers large enough to be worth a phase.
+template <typename OffT>
+__device__ __forceinline__ bool hub_due(const BatchParams<OffT>& p, const BatchCtl* ctl) {
+  if (ctl->policy == 0 || !p.hub_tab || !ctl->act) return false;
+  if (ctl->hub_lv == (((ctl->lvl[0] + 1) << 16) | (ctl->lvl[1] + 1))) return false;
+  return live_mf(ctl, 0) + live_mf(ctl, 1) >= ctl->hub_min_e;
+}
+
+// The sides (bit x) whose lists carry enough resolved queries for a filter to
+// pay.
+__device__ __forceinline__ int filter_due(const BatchCtl* ctl, int sides) {
+  int filt = 0;
+  for (int x = 0; x < 2; ++x) {
+    if (!(sides & (1 << x))) continue;
+    const int c = ctl->cur[x];
+    // expected work saved: the share dead / built of the list's queries
+    // resolved since it was built (integer products: the lane-0 decision
+    // sits on every decision launch's critical path, and double-precision
+    // divisions there are slow)
+    const uint64_t built = (uint64_t)__popcll(ctl->lact[x]);
+    const uint64_t dead = (uint64_t)__popcll(ctl->lact[x] & ~ctl->act);
+    if (!dead || !built) continue;
+    const uint64_t size = (uint64_t)ctl->fl_n[x][c] + (ctl->hub[x][c] >> kHubEdgeBits);
+    if (size * dead >= ctl->filt_min_v * built || ctl->fl_mf[x][c] * dead >= ctl->filt_min_e * built) filt |= 1 << x;
+  }
+  return filt;
+}
+
 // Heuristic (or plain) action for the pending step; also fills the feature
 // vector f when the learned policy or a trace needs it (double-precision
 // logarithms on one lane: not worth computing otherwise). One lane of the
@@ -985,23 +1239,7 @@ __device__ __forceinline__ void batch_apply(BatchCtl* ctl, int a, bool allow_fil
   if (ctl->vw_fixed > 0) d.vw = ctl->vw_fixed;
   if (a / 3 == 1) d.vw = 64;  // the wide top-down actions
   ctl->dec = d;
-  int filt = 0;
-  if (allow_filter) {
-    for (int x = 0; x < 2; ++x) {
-      if (!(d.sides & (1 << x))) continue;
-      const int c = ctl->cur[x];
-      // expected work saved: the share dead / built of the list's queries
-      // resolved since it was built (integer products: the lane-0 decision
-      // sits on every decision launch's critical path, and double-precision
-      // divisions there are slow)
-      const uint64_t built = (uint64_t)__popcll(ctl->lact[x]);
-      const uint64_t dead = (uint64_t)__popcll(ctl->lact[x] & ~ctl->act);
-      if (!dead || !built) continue;
-      const uint64_t size = (uint64_t)ctl->fl_n[x][c] + (ctl->hub[x][c] >> kHubEdgeBits);
-      if (size * dead >= ctl->filt_min_v * built || ctl->fl_mf[x][c] * dead >= ctl->filt_min_e * built)
-        filt |= 1 << x;
-    }
-  }
+  const int filt = allow_filter ? filter_due(ctl, d.sides) : 0;
   if (filt) {
     ctl->filt = filt;
     ctl->phase = kBFilter;
@@ -1079,7 +1317,7 @@ __device__ __forceinline__ int batch_finalize(const BatchParams<OffT>& p, BatchC
       ctl->lvl[0] = ctl->lvl[1] = 0;
       ctl->live0 = __popcll(act);
       ctl->vis_pairs[0] = ctl->vis_pairs[1] = ctl->live0;
-      ctl->bridge_lv = 0;
+      ctl->bridge_lv = ctl->hub_lv = 0;
       for (int x = 0; x < 2; ++x) {
         ctl->fl_n[x][0] = ln[x];
         ctl->hub[x][0] = lh[x];
@@ -1132,10 +1370,22 @@ __device__ __forceinline__ int batch_finalize(const BatchParams<OffT>& p, BatchC
     case kBBridge: {
       const unsigned long long act = ctl->act;
       const unsigned long long hit = r.v[kROdd] & act;
-      fd = FinDist{hit, 0ull, 0ull, ctl->lvl[0] + ctl->lvl[1]};
-      ctl->act = act & ~hit;
+      // when every pair was tested, the rest are further apart than
+      // lvl[0] + lvl[1] + 1, and a hub step's candidates are settled
+      const bool settled = r.v[kREven] == 0 && ctl->hub_lv == ctl->bridge_lv;
+      const unsigned long long even = settled ? r.v[kRAnyS] & act & ~hit : 0ull;
+      fd = FinDist{hit, even, 0ull, ctl->lvl[0] + ctl->lvl[1]};
+      ctl->act = act & ~(hit | even);
       ctl->bridges++;
       ctl->bridged += __popcll(hit);
+      return batch_next(ctl, true);
+    }
+    case kBHub: {
+      const unsigned long long act = ctl->act;
+      const unsigned long long hit = r.v[kROdd] & act;
+      fd = FinDist{hit, 0ull, 0ull, ctl->lvl[0] + ctl->lvl[1]};
+      ctl->act = act & ~hit;
+      ctl->hub_steps++;
       return batch_next(ctl, true);
     }
     case kBClearF: {
@@ -1197,13 +1447,13 @@ __device__ __forceinline__ int batch_finalize(const BatchParams<OffT>& p, BatchC
 // stores suffice; repeated roots within a side are merged in LDS first. The
 // counters are written with agent-scope stores for the finalising block.
 template <typename OffT>
-__device__ __forceinline__ void init_wave(const BatchParams<OffT>& p, int32_t* s_root) {
+__device__ __forceinline__ void init_wave(const BatchParams<OffT>& p, int wave, int qw, int nq, int32_t* s_root) {
   BatchCtl* ctl = p.ctl;
   const int q = lane_id(), x = (int)(threadIdx.x >> 6);
-  const int qi = ctl->wave * 64 + q;
+  const int qi = wave * qw + q;
   bool live = false;
   int32_t s = 0, t = 0;
-  if (qi < ctl->nq) {
+  if (q < qw && qi < nq) {
     s = p.qs[qi];
     t = p.qt[qi];
     live = s != t && (uint32_t)s < (uint32_t)p.V && (uint32_t)t < (uint32_t)p.V;
@@ -1231,7 +1481,8 @@ __device__ __forceinline__ void init_wave(const BatchParams<OffT>& p, int32_t* s
   if (owner) {
     rec_of(p, x, u)[0] = mask;
     p.F[x][0][u] = mask;
-    atomicOr(&p.db[u >> 5], 1u << (u & 31));
+    const uint32_t pos = group_pos((uint32_t)u / kGroup, p.gk);
+    atomicOr((uint32_t*)(uint8_t*)p.db + (pos >> 2), 1u << (8u * (pos & 3u) + ((uint32_t)u & (kGroup - 1))));
     deg = bdeg(p, u);
   }
   const bool hub = owner && deg >= p.hub_threshold;
@@ -1258,99 +1509,121 @@ __device__ __forceinline__ void init_wave(const BatchParams<OffT>& p, int32_t* s
   }
 }
 
-template <typename OffT>
-__global__ __launch_bounds__(kBlock, 4) void batch_kernel(BatchParams<OffT> p) {
-  BatchCtl* ctl = p.ctl;
-  const int phase = ctl->phase;
-  if (phase == kBIdle || phase == kBPause) return;
-  const uint32_t nb = gridDim.x;
-  const int gwave = (int)(blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6));
-  const int nwaves = (int)(nb * kWavesPerBlock);
-  const int64_t gtid = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+// LDS of a block of the batch kernels.
+struct BatchLds {
+  int32_t stage[2][kWavesPerBlock * kBStage];
+  int32_t hub[2][2][kWavesPerBlock * kHubStage];
+  uint16_t list[kWavesPerBlock * kMarkChunk];
+  BShared sh;
+  alignas(16) unsigned long long ctl[kCtlHotWords];  // a copy of the control block's state
+};
+
+// One phase of the wave machine as block bid of nb runs it. rc: the control
+// block (a team: this block's copy of its state). A team commits an expansion
+// in the same phase, after a barrier (bar, bars: team_barrier's) that decides
+// nothing; false when that barrier failed.
+template <bool TEAM, typename OffT>
+__device__ __forceinline__ bool batch_phase(const BatchParams<OffT>& p, const BatchCtl* rc, int phase, int bid, int nb,
+                                            BatchLds& lds, TeamBar* bar, uint32_t& bars) {
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int gwave = bid * kWavesPerBlock + w;
+  const int nwaves = nb * kWavesPerBlock;
+  const int64_t gtid = (int64_t)bid * kBlock + threadIdx.x;
   const int64_t nthr = (int64_t)nb * kBlock;
-  __shared__ int32_t s_stage[2][kWavesPerBlock * kBStage];
-  __shared__ int32_t s_hub[2][2][kWavesPerBlock * kHubStage];
-  __shared__ BShared sh;
-  const BatchDecision d = ctl->dec;
-  const unsigned long long act = ctl->act;
-  const int w = (int)(threadIdx.x >> 6);
-  const int nxt[2] = {ctl->cur[0] ^ 1, ctl->cur[1] ^ 1};
-  Appends ap{{{&s_stage[0][w * kBStage], 0u}, {&s_stage[1][w * kBStage], 0u}},
-             {{&s_hub[0][0][w * kHubStage], &s_hub[0][1][w * kHubStage], 0u},
-              {&s_hub[1][0][w * kHubStage], &s_hub[1][1][w * kHubStage], 0u}}};
+  const int sides = uni<TEAM>(rc->dec.sides), vw = uni<TEAM>(rc->dec.vw);
+  const unsigned long long act = uni<TEAM>(rc->act);
+  const int nxt[2] = {uni<TEAM>(rc->cur[0]) ^ 1, uni<TEAM>(rc->cur[1]) ^ 1};
+  Appends ap{{{&lds.stage[0][w * kBStage], 0u}, {&lds.stage[1][w * kBStage], 0u}},
+             {{&lds.hub[0][0][w * kHubStage], &lds.hub[0][1][w * kHubStage], 0u},
+              {&lds.hub[1][0][w * kHubStage], &lds.hub[1][1][w * kHubStage], 0u}}};
   unsigned long long red[kRCount];
 #pragma unroll
   for (int k = 0; k < kRCount; ++k) red[k] = 0;
+  // zero the side-x frontier masks of parity c through its lists
+  auto clear_masks = [&](int x, int c, bool normal) {
+    if (normal) {
+      const uint32_t n = uni<TEAM>(rc->fl_n[x][c]) < (uint32_t)p.V ? uni<TEAM>(rc->fl_n[x][c]) : (uint32_t)p.V;
+      for (int64_t i = gtid; i < n; i += nthr) {
+        const int32_t v = ldw<TEAM>(p.fl[x][c] + i);
+        if ((uint32_t)v < (uint32_t)p.V) p.F[x][c][v] = 0ull;
+      }
+    }
+    uint32_t nh = (uint32_t)(uni<TEAM>(rc->hub[x][c]) >> kHubEdgeBits);
+    if (nh > p.hcap) nh = p.hcap;
+    for (int64_t i = gtid; i < nh; i += nthr) {
+      const int32_t v = ldw<TEAM>(p.hl[x][c] + i);
+      if ((uint32_t)v < (uint32_t)p.V) p.F[x][c][v] = 0ull;
+    }
+  };
 
+  // One call site each for the block-wide publication and reduction keeps
+  // the code small.
+  bool publish = false, reduce = true;
   switch (phase) {
     case kBInit: {
-      if (blockIdx.x == 0 && threadIdx.x < 128) init_wave(p, &s_stage[0][0]);
+      if (bid == 0 && threadIdx.x < 128) init_wave(p, uni<TEAM>(rc->wave), uni<TEAM>(rc->qw), uni<TEAM>(rc->nq),
+                                                 &lds.stage[0][0]);
+      reduce = false;
       break;
     }
     case kBExpand: {
-      const int chunk = ctl->tile > 0 ? ctl->tile : 256;
-#pragma unroll
+      const int tile = uni<TEAM>(rc->tile);
+#pragma unroll 1
       for (int x = 0; x < 2; ++x)
-        if (d.sides & (1 << x)) expand_side(p, x, d.vw, chunk, act, gwave, nwaves, red[kRActV], red[kRActE]);
-      block_reduce_slots(red, p.red, sh);
-      break;
+        if (sides & (1 << x))
+          expand_side<TEAM>(p, rc, x, vw, tile > 0 ? tile : 256, act, gwave, nwaves, red[kRActV], red[kRActE]);
+      if (!TEAM) break;
+      wave_add_slot(p.red, bid, kRActV, red[kRActV]);
+      wave_add_slot(p.red, bid, kRActE, red[kRActE]);
+      red[kRActV] = red[kRActE] = 0;
+      if (!team_barrier(bar, (uint32_t)nb, bars, &lds.sh.last)) return false;
     }
+      [[fallthrough]];
     case kBCommit: {
       // hub frontier masks are cleared here: every expand wave is done
-      for (int x = 0; x < 2; ++x) {
-        if (!(d.sides & (1 << x))) continue;
-        const int c = ctl->cur[x];
-        uint32_t nh = (uint32_t)(ctl->hub[x][c] >> kHubEdgeBits);
-        if (nh > p.hcap) nh = p.hcap;
-        for (int64_t i = gtid; i < nh; i += nthr) {
-          const int32_t v = p.hl[x][c][i];
-          if ((uint32_t)v < (uint32_t)p.V) p.F[x][c][v] = 0ull;
-        }
-      }
-      commit_pass(p, ap, act, nxt, gwave, nwaves, red);
-      appends_block_flush(p, ap, nxt, sh);
-      block_reduce_slots(red, p.red, sh);
+#pragma unroll 1
+      for (int x = 0; x < 2; ++x)
+        if (sides & (1 << x)) clear_masks(x, uni<TEAM>(rc->cur[x]), false);
+      commit_pass<TEAM>(p, ap, act, nxt, gwave, nwaves, &lds.list[w * kMarkChunk], red);
+      publish = true;
       break;
     }
     case kBBottomUp: {
-      if (d.sides == kSideS)
-        bottom_up<OffT, 1>(p, ap, act, gwave, nwaves, red);
-      else if (d.sides == kSideT)
-        bottom_up<OffT, 2>(p, ap, act, gwave, nwaves, red);
-      else
-        bottom_up<OffT, 3>(p, ap, act, gwave, nwaves, red);
-      appends_block_flush(p, ap, nxt, sh);
-      block_reduce_slots(red, p.red, sh);
+      bottom_up<TEAM>(p, rc, sides, ap, act, gwave, nwaves, red);
+      publish = true;
       break;
     }
     case kBFilter: {
-      if (ctl->filt & 1) filter_side<OffT, 0>(p, ap, act, gwave, nwaves, red);
-      if (ctl->filt & 2) filter_side<OffT, 1>(p, ap, act, gwave, nwaves, red);
-      appends_block_flush(p, ap, nxt, sh);
-      block_reduce_slots(red, p.red, sh);
+      filter_sides<TEAM>(p, rc, uni<TEAM>(rc->filt), ap, act, gwave, nwaves, red);
+      publish = true;
       break;
     }
     case kBBridge: {
-      bridge_pass(p, act, gwave, nwaves, reinterpret_cast<unsigned char*>(&s_stage[0][0]), red[kROdd]);
-      block_reduce_slots(red, p.red, sh);
+      unsigned long long meets = 0, untested = 0;
+      if (TEAM && uni<TEAM>(rc->hub_lv) == uni<TEAM>(rc->bridge_lv))
+        wave_or_slot(p.red, bid, kRAnyS, hub_even(p, nb, gwave, nwaves));
+      bridge_pass<TEAM>(p, rc, act, gwave, nwaves, reinterpret_cast<unsigned char*>(&lds.stage[0][0]), meets,
+                        untested);
+      wave_or_slot(p.red, bid, kROdd, meets);
+      wave_or_slot(p.red, bid, kREven, untested);
+      reduce = false;
+      break;
+    }
+    case kBHub: {
+      if (TEAM) {
+        unsigned long long meets = 0;
+        hub_pass(p, rc, act, bid, gwave, nwaves, reinterpret_cast<unsigned long long*>(&lds.stage[0][0]), meets);
+        wave_or_slot(p.red, bid, kROdd, meets);
+      }
+      reduce = false;
       break;
     }
     case kBClearF: {
-      for (int x = 0; x < 2; ++x) {
-        if (!(ctl->bu_sides & (1 << x))) continue;
-        const int c = ctl->cur[x] ^ 1;  // the parity consumed by the bottom-up step
-        const uint32_t n = ctl->fl_n[x][c] < (uint32_t)p.V ? ctl->fl_n[x][c] : (uint32_t)p.V;
-        for (int64_t i = gtid; i < n; i += nthr) {
-          const int32_t v = p.fl[x][c][i];
-          if ((uint32_t)v < (uint32_t)p.V) p.F[x][c][v] = 0ull;
-        }
-        uint32_t nh = (uint32_t)(ctl->hub[x][c] >> kHubEdgeBits);
-        if (nh > p.hcap) nh = p.hcap;
-        for (int64_t i = gtid; i < nh; i += nthr) {
-          const int32_t v = p.hl[x][c][i];
-          if ((uint32_t)v < (uint32_t)p.V) p.F[x][c][v] = 0ull;
-        }
-      }
+      // the parity that the bottom-up step consumed
+#pragma unroll 1
+      for (int x = 0; x < 2; ++x)
+        if (uni<TEAM>(rc->bu_sides) & (1 << x)) clear_masks(x, uni<TEAM>(rc->cur[x]) ^ 1, true);
+      reduce = false;
       break;
     }
     case kBCleanup: {
@@ -1358,82 +1631,92 @@ __global__ __launch_bounds__(kBlock, 4) void batch_kernel(BatchParams<OffT> p) {
       // lists (an expansion clears the masks it reads, a commit its hub
       // masks, a filter and kBClearF the lists they consume): clear them
       // through the lists. Every vertex with a non-zero record is dirty:
-      // clear the records of the dirty vertices in address order.
-      for (int x = 0; x < 2; ++x) {
-        const int c = ctl->cur[x];
-        const uint32_t n = ctl->fl_n[x][c] < (uint32_t)p.V ? ctl->fl_n[x][c] : (uint32_t)p.V;
-        for (int64_t i = gtid; i < n; i += nthr) {
-          const int32_t v = p.fl[x][c][i];
-          if ((uint32_t)v < (uint32_t)p.V) p.F[x][c][v] = 0ull;
-        }
-        uint32_t nh = (uint32_t)(ctl->hub[x][c] >> kHubEdgeBits);
-        if (nh > p.hcap) nh = p.hcap;
-        for (int64_t i = gtid; i < nh; i += nthr) {
-          const int32_t v = p.hl[x][c][i];
-          if ((uint32_t)v < (uint32_t)p.V) p.F[x][c][v] = 0ull;
-        }
-      }
+      // clear the records of the dirty vertices, the dirty bytes read as the
+      // commit reads its marks, eight groups at a time.
+#pragma unroll 1
+      for (int x = 0; x < 2; ++x) clear_masks(x, uni<TEAM>(rc->cur[x]), true);
+      reduce = false;
       const int lane = lane_id();
-      const int64_t per = owned_groups(((int64_t)p.V + 31) / 32, gwave, nwaves);
-      for (int64_t jb = 0; jb < per; jb += kWave) {
-        const GroupDeal gd{jb, nwaves, gwave};
-        const int64_t wi = gd(lane);
-        const uint32_t word = jb + lane < per ? p.db[wi] : 0u;
-        if (word) p.db[wi] = 0u;
-        uint64_t nz = ballot(word != 0);
-        while (nz) {
-          const int k0 = __builtin_ctzll(nz);
-          nz &= nz - 1;
-          int k1 = -1;
-          if (nz) {
-            k1 = __builtin_ctzll(nz);
-            nz &= nz - 1;
-          }
-          const int mine = lane < 32 ? k0 : k1;
-          const uint32_t wv = (uint32_t)__shfl((int)word, mine < 0 ? 0 : mine);
-          const int64_t u = gd(mine < 0 ? 0 : mine) * 32 + (lane & 31);
-          if (mine >= 0 && ((wv >> (lane & 31)) & 1u) && u < p.V) {
+      // the wave's bytes and positions go to its share of the appends' stage
+      // and of the lists
+      uint16_t* s_list = &lds.list[w * kMarkChunk];
+      uint8_t* s_byte = reinterpret_cast<uint8_t*>(&lds.stage[0][0]) + w * kMarkChunk;
+      static_assert(kWavesPerBlock * kMarkChunk <= sizeof(lds.stage), "bytes fit the stage");
+      MarkWalk mw(p.db, kGroupClasses * (uint32_t)p.gk, gwave, nwaves);
+      uint32_t cnt;
+      for (;;) {
+        const uint32_t at = mw.at;
+        if (!mw.next<TEAM>(cnt, [&](uint32_t k, uint32_t pos, uint8_t v) {
+              s_list[k] = (uint16_t)(pos - at);
+              s_byte[k] = v;
+            }))
+          break;
+        for (uint32_t i = (uint32_t)lane / kGroup; i < cnt; i += kWave / kGroup) {
+          const int sub = lane & (int)(kGroup - 1);
+          const int64_t u = (int64_t)group_at(at + s_list[i], p.gk) * kGroup + sub;
+          if (((s_byte[i] >> sub) & 1u) && u < p.V) {
             *reinterpret_cast<ulonglong2*>(rec_of(p, 0, u)) = make_ulonglong2(0ull, 0ull);
             *reinterpret_cast<ulonglong2*>(rec_of(p, 1, u)) = make_ulonglong2(0ull, 0ull);
           }
         }
+        __builtin_amdgcn_wave_barrier();
       }
       break;
     }
     default:
+      reduce = false;
       break;
   }
+  if (publish) appends_block_flush(p, ap, nxt, lds.sh);
+  if (reduce) block_reduce_slots(red, p.red, bid, lds.sh);
+  return true;
+}
 
+// The end of a phase in one block: every store is out, and the block votes.
+// Returns (to all threads) whether it is the last one.
+template <typename OffT>
+__device__ __forceinline__ bool batch_vote(const BatchParams<OffT>& p, int bid, int nb, BShared& sh) {
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   if (threadIdx.x == 0) {
     // Two-level ticket: the blocks of group b % kRedSlots count on their own
     // word, and the last block of each group counts on the launch ticket, so
     // no single address takes an atomic from every block.
-    const uint32_t k = blockIdx.x % kRedSlots;
-    const uint32_t gsize = (nb - k + kRedSlots - 1) / kRedSlots;
+    const uint32_t k = (uint32_t)bid % kRedSlots;
+    const uint32_t gsize = ((uint32_t)nb - k + kRedSlots - 1) / kRedSlots;
     unsigned long long* sub = p.red + (size_t)(kRedSlots + k) * kRedWords;
     const unsigned long long t1 = __hip_atomic_fetch_add(sub, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     bool last = false;
     if (t1 == gsize - 1) {
       __hip_atomic_store(sub, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const uint32_t groups = nb < (uint32_t)kRedSlots ? nb : (uint32_t)kRedSlots;
-      const uint32_t t2 = __hip_atomic_fetch_add(&ctl->ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const uint32_t groups = nb < kRedSlots ? (uint32_t)nb : (uint32_t)kRedSlots;
+      const uint32_t t2 = __hip_atomic_fetch_add(&p.ctl->ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       last = t2 == groups - 1;
     }
     sh.last = last;
   }
   __syncthreads();
-  if (!sh.last || threadIdx.x >= kWave) return;
-  // Wave 0 of the last block finalises: slot sums, the state update (lane
-  // 0), and, when a step must be chosen, the decision (the learned policy
-  // evaluates its network across the wave). The network's weights are
-  // copied from global memory straight into LDS (the appends' stage is free
-  // now) first, so that the copy overlaps the finalisation.
+  return sh.last;
+}
+
+// Finalise a phase: wave 0 of the last block. Slot sums, the state update
+// (lane 0), and, when a step must be chosen, the decision (the learned
+// policy evaluates its network across the wave).
+// LEARN: the learned policy may be asked for (its features and network are
+// code that the other schedules need not fetch).
+template <bool TEAM, bool LEARN, typename OffT>
+__device__ __forceinline__ void batch_finish(const BatchParams<OffT>& p, const BatchCtl* rc, int phase,
+                                             BatchLds& lds) {
+  BatchCtl* ctl = p.ctl;
+  const BatchDecision d = rc->dec;
+  const int nxt[2] = {rc->cur[0] ^ 1, rc->cur[1] ^ 1};
+  // The network's weights are copied from global memory straight into LDS
+  // (the appends' stage is free now) first, so that the copy overlaps the
+  // finalisation.
   constexpr int kPer = (kMlpParams + kWave - 1) / kWave;
-  static_assert(kPer * kWave * sizeof(float) <= sizeof(s_stage), "network does not fit the LDS stage");
-  const bool mlp_on = ctl->policy == 2 && p.mlp != nullptr;
-  float* s_mlp = reinterpret_cast<float*>(&s_stage[0][0]);
+  static_assert(kPer * kWave * sizeof(float) <= sizeof(lds.stage), "network does not fit the LDS stage");
+  const bool mlp_on = LEARN && rc->policy == 2 && p.mlp != nullptr;
+  float* s_mlp = reinterpret_cast<float*>(&lds.stage[0][0]);
   if (mlp_on) {
     typedef __attribute__((address_space(1))) void* gptr;
     typedef __attribute__((address_space(3))) void* lptr;
@@ -1454,7 +1737,7 @@ __global__ __launch_bounds__(kBlock, 4) void batch_kernel(BatchParams<OffT> p) {
   // Every other block has voted, so no one else writes these words now.
   // The state words and the launch's reduction slots are loaded together,
   // in one round trip.
-  __shared__ __align__(16) unsigned long long s_ctl[kCtlHotWords];
+  unsigned long long* s_ctl = lds.ctl;
   // A cleanup claims the machine's next wave now, so that the counter's
   // round trip overlaps the state loads.
   uint32_t next_wave = 0;
@@ -1466,40 +1749,56 @@ __global__ __launch_bounds__(kBlock, 4) void batch_kernel(BatchParams<OffT> p) {
     unsigned long long c0 = 0, c1 = 0;
     if (lane < (int)kCtlHotWords) c0 = ld_agent(gw + lane);
     if (lane + kWave < (int)kCtlHotWords) c1 = ld_agent(gw + lane + kWave);
-    unsigned long long* row = p.red + (size_t)(lane < kRedSlots ? lane : 0) * kRedWords;
-    unsigned long long v[kRCount];
+    // Row j of 16 lanes takes word 4 t + j of the 16 slots in round t; the
+    // first four words are ORs, the others sums.
+    unsigned long long* word = p.red + (size_t)(lane & 15) * kRedWords + (lane >> 4);
+    unsigned long long v[3];
 #pragma unroll
-    for (int k = 0; k < kRCount; ++k) v[k] = lane < kRedSlots ? ld_agent(row + k) : 0ull;
+    for (int t = 0; t < 3; ++t) v[t] = ld_agent(word + 4 * t);
     if (lane < (int)kCtlHotWords) s_ctl[lane] = c0;
     if (lane + kWave < (int)kCtlHotWords) s_ctl[lane + kWave] = c1;
 #pragma unroll
-    for (int k = 0; k < kRCount; ++k) {
-      if (v[k]) row[k] = 0ull;
-      tot.v[k] = k < kRMfS ? (unsigned long long)wave_reduce_full_nz_u64<kWaveOr>(v[k])
-                           : (unsigned long long)wave_reduce_full_nz_u64<kWaveSum>(v[k]);
+    for (int t = 0; t < 3; ++t) {
+      if (v[t]) word[4 * t] = 0ull;
+      v[t] = t == 0 ? (unsigned long long)row_reduce_u64<kWaveOr>(v[t])
+                    : (unsigned long long)row_reduce_u64<kWaveSum>(v[t]);
+      if ((lane & 15) == 15) lds.sh.red[4 * t + (lane >> 4)][0] = v[t];
     }
   }
   __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int k = 0; k < kRCount; ++k) tot.v[k] = lds.sh.red[k][0];
   BatchCtl* lc = reinterpret_cast<BatchCtl*>(s_ctl);
   int need = kFinDone;
   {
     FinPre pre = fin_prefetch(lc, phase, nxt);
     pre.next_wave = next_wave;
-    const int wave0 = lc->wave * 64;
+    const int wave0 = lc->wave * lc->qw;
     FinDist fd{0ull, 0ull, 0ull, 0};
     if (threadIdx.x == 0) {
       const int64_t ph = lc->phases;
-      if (ph < kPhaseLog) {
+      if (!TEAM && ph < kPhaseLog) {
         ctl->plog[ph] = (int8_t)(phase * 16 + (phase == kBExpand || phase == kBBottomUp ? d.sides : 0));
         ctl->ptime[ph] = (int64_t)wall_clock64();
         ctl->pwork[ph] = (int64_t)(phase == kBCommit ? tot.v[kRTouched] : tot.v[kRActE]);
       }
-      lc->phases = ph + 1;
-      if (phase == kBDecide) {
+      lc->phases = ph + (TEAM && phase == kBCommit ? 2 : 1);  // a team's commit follows its expansion
+      if (!TEAM && phase == kBDecide) {
         need = lc->pause_filter ? kFinDecideFilter : kFinDecide;
       } else {
         need = batch_finalize(p, lc, phase, d, tot, pre, fd);
-        if (need != kFinDone && bridge_due(p, lc)) {
+        // A team filters before it looks for meets: the bridge's pairs are the
+        // product of the two lists' lengths.
+        const int filt = TEAM && need == kFinDecideFilter && lc->policy != 0 ? filter_due(lc, kSideBoth) : 0;
+        if (filt) {
+          lc->filt = filt;
+          lc->phase = kBFilter;
+          need = kFinDone;
+        } else if (TEAM && need != kFinDone && hub_due(p, lc)) {
+          lc->hub_lv = ((lc->lvl[0] + 1) << 16) | (lc->lvl[1] + 1);
+          lc->phase = kBHub;
+          need = kFinDone;
+        } else if (need != kFinDone && bridge_due(p, lc)) {
           lc->bridge_lv = ((lc->lvl[0] + 1) << 16) | (lc->lvl[1] + 1);
           lc->phase = kBBridge;
           need = kFinDone;
@@ -1519,10 +1818,11 @@ __global__ __launch_bounds__(kBlock, 4) void batch_kernel(BatchParams<OffT> p) {
   if (need != kFinDone) {
     float f[12] = {};
     int a = 0;
-    if (threadIdx.x == 0) a = batch_heuristic(lc, p.V, p.E, f, mlp_on || lc->trace);
+    if (threadIdx.x == 0) a = batch_heuristic(lc, p.V, p.E, f, mlp_on || (!TEAM && lc->trace));
     a = __shfl(a, 0);
-    const bool forced = phase == kBDecide && lc->force_action >= 0;
-    const bool pause = phase != kBDecide && lc->trace &&
+    // traces pause and force decisions; they run on the launch engine
+    const bool forced = !TEAM && phase == kBDecide && lc->force_action >= 0;
+    const bool pause = !TEAM && phase != kBDecide && lc->trace &&
                        lc->decisions % (lc->trace_every > 0 ? lc->trace_every : 1) == 0;
     if (!forced && !pause && mlp_on) {
       __builtin_amdgcn_s_waitcnt(0);  // the weights are in LDS
@@ -1541,7 +1841,7 @@ __global__ __launch_bounds__(kBlock, 4) void batch_kernel(BatchParams<OffT> p) {
         batch_apply(lc, a, need == kFinDecideFilter);
         lc->decisions++;
       }
-      if (phase == kBDecide) lc->t_decide = (int64_t)wall_clock64();
+      if (!TEAM && phase == kBDecide) lc->t_decide = (int64_t)wall_clock64();
     }
   }
   // no copy into LDS may still be in flight when the wave ends
@@ -1556,6 +1856,122 @@ __global__ __launch_bounds__(kBlock, 4) void batch_kernel(BatchParams<OffT> p) {
 }
 
 template <typename OffT>
+__global__ __launch_bounds__(kBlock, 4) void batch_kernel(BatchParams<OffT> p) {
+  const int phase = p.ctl->phase;
+  if (phase == kBIdle || phase == kBPause) return;
+  __shared__ BatchLds lds;
+  uint32_t none = 0;
+  batch_phase<false>(p, p.ctl, phase, (int)blockIdx.x, (int)gridDim.x, lds, nullptr, none);
+  if (!batch_vote(p, (int)blockIdx.x, (int)gridDim.x, lds.sh) || threadIdx.x >= kWave) return;
+  batch_finish<false, true>(p, p.ctl, phase, lds);
+}
+
+// A batch in one launch: every team (team.hpp) is a wave machine of its own,
+// with its own workspace (stride bytes apart), that claims waves of 64
+// queries until none is left and runs their phases with a team barrier
+// between them. Eight or sixteen waves are in flight, each in the L2 of its
+// XCD, where the launch engine's three lanes took 10-20 us from one phase's
+// launch to the next's.
+struct TeamRun {
+  TeamSync* sync;          // [kXcds]
+  TeamWord* gen;           // [kXcds * teams] phases finished
+  TeamBar* bar;            // [kXcds * teams] team_barrier's words
+  const unsigned long long* init;  // kCtlHotWords: the machines' initial state
+  unsigned long long* out;         // [kXcds * teams][kTeamOutWords] final states
+  uint32_t* err;
+  uint32_t* ticket;        // next unclaimed wave
+  const void* params;      // BatchParams of each machine
+  int32_t teams;           // per XCD
+  uint32_t expected;       // blocks per XCD
+};
+constexpr uint32_t kTeamOutWords = 64;
+static_assert(kCtlHotWords <= kTeamOutWords, "final state fits");
+
+template <typename OffT, bool LEARN>
+__global__ __launch_bounds__(kBlock, 4) void batch_team_kernel(TeamRun tr) {
+  // Constant address space: the parameters are read with scalar loads (the
+  // launch does not write them).
+  typedef __attribute__((address_space(4))) const BatchParams<OffT>* params_ptr;
+  const params_ptr all = (params_ptr)(uintptr_t)tr.params;
+  __shared__ BatchLds lds;
+  __shared__ int s_num, s_size;
+  TeamSync* ts = tr.sync + xcc_id();
+  if (threadIdx.x == 0) {
+    uint32_t members = 0;
+    s_num = team_register(ts, tr.expected, &members);
+    s_size = (int)members;
+  }
+  __syncthreads();
+  const int num = __builtin_amdgcn_readfirstlane(s_num);
+  if (num < 0) return;
+  BatchCtl* lc = reinterpret_cast<BatchCtl*>(lds.ctl);
+  if (num == 0) {
+    // the XCD's first block writes its teams' control blocks
+    if (threadIdx.x < kWave) {
+      const int lane = lane_id();
+      for (int t = 0; t < tr.teams; ++t) {
+        if (lane < (int)kCtlHotWords) lds.ctl[lane] = tr.init[lane];
+        __builtin_amdgcn_wave_barrier();
+        if (lane == 0) {
+          const uint32_t wave = t < s_size ? atomicAdd(tr.ticket, 1u) : 0x7fffffffu;
+          lc->wave = (int32_t)wave;
+          lc->phase = wave < (uint32_t)lc->nwaves ? kBInit : kBIdle;
+        }
+        __builtin_amdgcn_wave_barrier();
+        const params_ptr pt = all + (xcc_id() * tr.teams + t);
+        unsigned long long* gw = (unsigned long long*)(BatchCtl*)pt->ctl;
+        if (lane < (int)kCtlHotWords) gw[lane] = lds.ctl[lane];
+        __builtin_amdgcn_wave_barrier();
+      }
+      __builtin_amdgcn_s_waitcnt(0);
+      if (lane == 0) st_agent(&ts->size.v, (uint32_t)s_size);
+    }
+  } else if (threadIdx.x == 0) {
+    s_size = team_wait(&ts->size.v, 1u) ? (int)ld_agent(&ts->size.v) : 0;
+    if (!s_size) st_agent(tr.err, 1u);
+  }
+  __syncthreads();
+  const int size = __builtin_amdgcn_readfirstlane(s_size);
+  if (size == 0) return;
+  const int team = num % tr.teams, bid = num / tr.teams;
+  const int nb = (size - team + tr.teams - 1) / tr.teams;
+  const int machine = xcc_id() * tr.teams + team;
+  uintptr_t mine = (uintptr_t)(all + machine);
+  uint32_t bars = 0;
+  for (uint32_t round = 1;; ++round) {
+    // The parameters are loaded where a phase needs them: kept in registers
+    // across the loop, as loop invariants, they would not fit.
+    asm volatile("" : "+s"(mine));
+    const BatchParams<OffT>& p = *(const BatchParams<OffT>*)(params_ptr)mine;
+    const unsigned long long* gw = (const unsigned long long*)(const BatchCtl*)p.ctl;
+    // this phase's state, read from the L2 by every block
+    if (threadIdx.x < kCtlHotWords) lds.ctl[threadIdx.x] = ld_team(gw + threadIdx.x);
+    __syncthreads();
+    int phase = __builtin_amdgcn_readfirstlane(lc->phase);
+    if (phase == kBIdle) break;
+    if (!batch_phase<true>(p, lc, phase, bid, nb, lds, &tr.bar[machine], bars)) {
+      if (threadIdx.x == 0) st_agent(tr.err, 1u);
+      return;
+    }
+    if (phase == kBExpand) phase = kBCommit;
+    const bool last = batch_vote(p, bid, nb, lds.sh);
+    if (last) {
+      if (threadIdx.x < kWave) {
+        batch_finish<true, LEARN>(p, lc, phase, lds);
+        __builtin_amdgcn_s_waitcnt(0);
+        if (threadIdx.x == 0) st_agent(&tr.gen[machine].v, round);
+      }
+    } else if (threadIdx.x == 0) {
+      s_size = team_wait(&tr.gen[machine].v, round);
+      if (!s_size) st_agent(tr.err, 1u);
+    }
+    __syncthreads();
+    if (!last && !__builtin_amdgcn_readfirstlane(s_size)) return;
+  }
+  if (bid == 0 && threadIdx.x < kCtlHotWords) tr.out[(size_t)machine * kTeamOutWords + threadIdx.x] = lds.ctl[threadIdx.x];
+}
+
+template <typename OffT>
 hipError_t launch_batch_phase(const BatchParams<OffT>& p, int blocks, hipStream_t s) {
   hipLaunchKernelGGL(batch_kernel<OffT>, dim3(blocks), dim3(kBlock), 0, s, p);
   return hipGetLastError();
@@ -1565,6 +1981,13 @@ template <typename OffT>
 int batch_occupancy() {
   int nb = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, batch_kernel<OffT>, kBlock, 0) != hipSuccess) return 0;
+  return nb;
+}
+
+template <typename OffT>
+static int team_occupancy() {
+  int nb = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, batch_team_kernel<OffT, true>, kBlock, 0) != hipSuccess) return 0;
   return nb;
 }
 
@@ -1583,10 +2006,11 @@ struct BatchWorkspace {
   unsigned long long* F[2][2] = {};
   uint8_t* tm = nullptr;
   unsigned long long* red = nullptr;
+  unsigned long long* ht = nullptr;
   int32_t* fl[2][2] = {};
   int32_t* hl[2][2] = {};
   int64_t* hb[2][2] = {};
-  uint32_t* db = nullptr;
+  uint8_t* db = nullptr;
   BatchCtl* ctl = nullptr;
   int32_t* qs = nullptr;
   int32_t* qt = nullptr;
@@ -1638,52 +2062,70 @@ void batch_free(BatchWorkspace* b) {
   delete b;
 }
 
+// Pieces of one wave machine's workspace, as offsets from its start.
+struct BatchLayout {
+  size_t ht, rec, F, F1, tm, red, fl, fl1, hl, hl1, hb, hb1, db, ctl, wt, bytes;  // F1, fl1, ...: from one array to the next
+};
+
+// ht_blocks: blocks of a team (0: a launch-driven machine).
+static BatchLayout batch_layout(int64_t V64, size_t hcap, int ht_blocks = 0) {
+  auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
+  const size_t V = (size_t)V64, P = (size_t)kGroupClasses * (size_t)group_class_len(V64);
+  BatchLayout l;
+  size_t o = 0;
+  auto take = [&](size_t bytes) {
+    const size_t at = o;
+    o += al(bytes);
+    return at;
+  };
+  l.rec = take(32 * V);
+  l.F1 = al(8 * V);
+  l.F = take(4 * l.F1);
+  l.tm = take(P);
+  l.red = take(sizeof(unsigned long long) * 2 * kRedSlots * kRedWords);  // slots, then group tickets
+  l.fl1 = al(4 * V);
+  l.fl = take(4 * l.fl1);
+  l.hl1 = al(4 * hcap);
+  l.hl = take(4 * l.hl1);
+  l.hb1 = al(8 * hcap);
+  l.hb = take(4 * l.hb1);
+  l.db = take(P);
+  l.ht = take(sizeof(unsigned long long) * 2 * kHubTab * (size_t)ht_blocks);
+  l.ctl = take(sizeof(BatchCtl));
+  l.wt = take(sizeof(uint32_t));
+  l.bytes = o;
+  return l;
+}
+
+static void batch_pieces(BatchWorkspace* b, char* mem, const BatchLayout& l) {
+  b->rec = (unsigned long long*)(mem + l.rec);
+  for (int x = 0; x < 2; ++x) {
+    for (int c = 0; c < 2; ++c) {
+      const size_t k = (size_t)(x * 2 + c);
+      b->F[x][c] = (unsigned long long*)(mem + l.F + k * l.F1);
+      b->fl[x][c] = (int32_t*)(mem + l.fl + k * l.fl1);
+      b->hl[x][c] = (int32_t*)(mem + l.hl + k * l.hl1);
+      b->hb[x][c] = (int64_t*)(mem + l.hb + k * l.hb1);
+    }
+  }
+  b->tm = (uint8_t*)(mem + l.tm);
+  b->red = (unsigned long long*)(mem + l.red);
+  b->ht = (unsigned long long*)(mem + l.ht);
+  b->db = (uint8_t*)(mem + l.db);
+  b->ctl = (BatchCtl*)(mem + l.ctl);
+  b->wticket = (uint32_t*)(mem + l.wt);
+}
+
 static fc_status batch_alloc_lane(fc_graph* g, BatchWorkspace** out, bool own_stream) {
   BatchWorkspace* b = new BatchWorkspace();
-  const size_t V = (size_t)g->V;
-  const size_t hcap = g->hcap;
-  auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
-  size_t o = 0;
-  const size_t o_rec = o;
-  o += al(32 * V);
-  const size_t o_F = o;
-  o += 4 * al(8 * V);
-  const size_t o_tm = o;
-  o += al((V + 31) / 32 + 64);
-  const size_t o_red = o;
-  o += al(sizeof(unsigned long long) * 2 * kRedSlots * kRedWords);  // slots, then group tickets
-  const size_t o_fl = o;
-  o += 4 * al(4 * V);
-  const size_t o_hl = o;
-  o += 4 * al(4 * hcap);
-  const size_t o_hb = o;
-  o += 4 * al(8 * hcap);
-  const size_t o_db = o;
-  o += al(4 * ((V + 63) / 32));
-  const size_t o_ctl = o;
-  o += al(sizeof(BatchCtl));
-  const size_t o_wt = o;
-  o += al(sizeof(uint32_t));
-  b->bytes = o;
+  const BatchLayout l = batch_layout(g->V, g->hcap);
+  b->bytes = l.bytes;
   hipError_t e = hipMalloc((void**)&b->mem, b->bytes);
   if (e != hipSuccess) {
     delete b;
     return hip_fail(e, "batch workspace allocation");
   }
-  b->rec = (unsigned long long*)(b->mem + o_rec);
-  for (int x = 0; x < 2; ++x) {
-    for (int c = 0; c < 2; ++c) {
-      b->F[x][c] = (unsigned long long*)(b->mem + o_F + (size_t)(x * 2 + c) * al(8 * V));
-      b->fl[x][c] = (int32_t*)(b->mem + o_fl + (size_t)(x * 2 + c) * al(4 * V));
-      b->hl[x][c] = (int32_t*)(b->mem + o_hl + (size_t)(x * 2 + c) * al(4 * hcap));
-      b->hb[x][c] = (int64_t*)(b->mem + o_hb + (size_t)(x * 2 + c) * al(8 * hcap));
-    }
-  }
-  b->tm = (uint8_t*)(b->mem + o_tm);
-  b->red = (unsigned long long*)(b->mem + o_red);
-  b->db = (uint32_t*)(b->mem + o_db);
-  b->ctl = (BatchCtl*)(b->mem + o_ctl);
-  b->wticket = (uint32_t*)(b->mem + o_wt);
+  batch_pieces(b, b->mem, l);
   int occ = g->off64 ? batch_occupancy<int64_t>() : batch_occupancy<int32_t>();
   if (occ < 1) {
     batch_free(b);
@@ -1774,33 +2216,36 @@ template <typename OffT>
 static BatchParams<OffT> batch_params(fc_graph* g, BatchWorkspace* b) {
   BatchParams<OffT> p;
   std::memset(&p, 0, sizeof(p));
-  p.off = (const OffT*)g->d_off;
-  p.col = g->d_col;
+  set_param(p.off, (const OffT*)g->d_off);
+  set_param(p.col, g->d_col);
   p.V = (int32_t)g->V;
   p.hub_threshold = g->hub_threshold;
   p.E = g->E;
-  p.rec = b->rec;
+  set_param(p.rec, b->rec);
   for (int x = 0; x < 2; ++x) {
     for (int c = 0; c < 2; ++c) {
-      p.F[x][c] = b->F[x][c];
-      p.fl[x][c] = b->fl[x][c];
-      p.hl[x][c] = b->hl[x][c];
-      p.hb[x][c] = b->hb[x][c];
+      set_param(p.F[x][c], b->F[x][c]);
+      set_param(p.fl[x][c], b->fl[x][c]);
+      set_param(p.hl[x][c], b->hl[x][c]);
+      set_param(p.hb[x][c], b->hb[x][c]);
     }
   }
   p.hcap = g->hcap;
-  p.tm = b->tm;
-  p.red = b->red;
-  p.db = b->db;
-  p.ctl = b->ctl;
-  p.qs = b->run_qs;
-  p.qt = b->run_qt;
-  p.dist = b->run_dist;
-  p.wave_ticket = b->run_ticket;
-  p.perm = g->relabeled ? g->d_perm : nullptr;
+  set_param(p.tm, b->tm);
+  set_param(p.red, b->red);
+  set_param(p.ht, b->ht);
+  set_param(p.db, b->db);
+  p.gk = group_class_len(g->V);
+  set_param(p.ctl, b->ctl);
+  set_param(p.qs, b->run_qs);
+  set_param(p.qt, b->run_qt);
+  set_param(p.dist, b->run_dist);
+  set_param(p.wave_ticket, b->run_ticket);
+  set_param(p.perm, g->relabeled ? g->d_perm : nullptr);
   p.v_active = (int32_t)g->v_active;
   p.sorted_lists = g->lists_sorted ? 1 : 0;
-  p.mlp = g->d_mlp + kMlpParams;  // the copy in mlp_t_index order
+  p.hub_tab = g->lists_sorted && g->hub_steps ? (int32_t)std::min<int64_t>(kHubTab, g->V) : 0;
+  set_param(p.mlp, g->d_mlp + kMlpParams);  // the copy in mlp_t_index order
   return p;
 }
 
@@ -1837,13 +2282,22 @@ static fc_status batch_graph(fc_graph* g, BatchWorkspace* b) {
   return FC_OK;
 }
 
-// Prepare the control block for a batch of n queries (already on the device).
-fc_status batch_begin(fc_graph* g, BatchWorkspace* b, int32_t n, int policy, int vw, int tile, int trace, int every,
-                      float margin, int32_t first_wave) {
-  BatchCtl init;
+// A threshold of the schedule, which an environment variable overrides.
+// Capped at 2^56 (beyond any graph's counts), so that the decision's products
+// with query counts (at most 64) cannot overflow.
+static uint64_t batch_threshold(const char* name, uint64_t dflt) {
+  const char* v = std::getenv(name);
+  const uint64_t x = v && std::strtoull(v, nullptr, 10) > 0 ? (uint64_t)std::strtoull(v, nullptr, 10) : dflt;
+  return std::min<uint64_t>(x, 1ull << 56);
+}
+
+// A control block for a batch of n queries.
+static void batch_init(fc_graph* g, BatchCtl& init, int32_t n, int policy, int vw, int tile, int trace, int every,
+                       float margin, int32_t first_wave) {
   std::memset(&init, 0, sizeof(init));
   init.phase = kBInit;
   init.wave = first_wave;
+  init.qw = 64;
   init.nwaves = (n + 63) / 64;
   init.nq = n;
   init.policy = policy;
@@ -1855,17 +2309,17 @@ fc_status batch_begin(fc_graph* g, BatchWorkspace* b, int32_t n, int policy, int
   init.trace_every = every;
   init.learn_margin_milli = (int32_t)std::lround((margin < 0.f ? kDefaultLearnMargin : margin) * 1000.f);
   init.f_branch = g->f_branch;
-  // Thresholds are capped at 2^56 (beyond any graph's counts), so that the
-  // decision's products with query counts (at most 64) cannot overflow.
-  auto env_u64 = [](const char* name, uint64_t dflt) {
-    const char* v = std::getenv(name);
-    const uint64_t x = v && std::strtoull(v, nullptr, 10) > 0 ? (uint64_t)std::strtoull(v, nullptr, 10) : dflt;
-    return std::min<uint64_t>(x, 1ull << 56);
-  };
-  init.filt_min_v = env_u64("FASTCON_FILTER_MIN_VERTICES", kFilterMinVertices);
-  init.filt_min_e = env_u64("FASTCON_FILTER_MIN_EDGES", kFilterMinEdges);
-  init.both_max_e = env_u64("FASTCON_BOTH_MAX_EDGES", kBothMaxEdges);
-  init.bridge_min_e = env_u64("FASTCON_BRIDGE_MIN_EDGES", kBridgeMinEdges);
+  init.filt_min_v = batch_threshold("FASTCON_FILTER_MIN_VERTICES", kFilterMinVertices);
+  init.filt_min_e = batch_threshold("FASTCON_FILTER_MIN_EDGES", kFilterMinEdges);
+  init.both_max_e = batch_threshold("FASTCON_BOTH_MAX_EDGES", kBothMaxEdges);
+  init.bridge_min_e = batch_threshold("FASTCON_BRIDGE_MIN_EDGES", kBridgeMinEdges);
+}
+
+// Prepare the control block for a batch of n queries (already on the device).
+fc_status batch_begin(fc_graph* g, BatchWorkspace* b, int32_t n, int policy, int vw, int tile, int trace, int every,
+                      float margin, int32_t first_wave) {
+  BatchCtl init;
+  batch_init(g, init, n, policy, vw, tile, trace, every, margin, first_wave);
   FC_HIP(hipMemcpyAsync(b->ctl, &init, sizeof(init), hipMemcpyHostToDevice, b->stream));
   // the reduction slots are cleared by every finalisation; clear them here
   // too in case an earlier batch stopped on an error
@@ -2015,9 +2469,9 @@ static fc_status batch_run(fc_graph* g, const int32_t* s, const int32_t* t, int3
   }
   if (std::getenv("FASTCON_BATCH_LOG")) {
     // phase sequence of lane 0: I=init E=expand(s/t/b sides) C=commit U=bottom-up X=clear F=filter Z=cleanup
-    // D=traced decision B=bridge
+    // D=traced decision B=bridge H=hub step
     const BatchCtl& c = cs[0];
-    const char* nm = "?IECUXZFPDB?????";
+    const char* nm = "?IECUXZFPDBH????";
     const int64_t np = std::min<int64_t>(c.phases, kPhaseLog);
     for (int64_t i = 0; i < np; ++i) {
       const int ph = (uint8_t)c.plog[i] >> 4, sd = c.plog[i] & 15;
@@ -2027,6 +2481,202 @@ static fc_status batch_run(fc_graph* g, const int32_t* s, const int32_t* t, int3
       std::fputc(ph == kBCleanup ? '\n' : ' ', stderr);
     }
   }
+  return FC_OK;
+}
+
+// ---------------------------------------------------------------------------
+// Team engine: one launch per batch (batch_team_kernel).
+// ---------------------------------------------------------------------------
+// Machines per XCD. Two overlap one machine's barriers and round trips with
+// the other's work: R-MAT s22, 1,024 queries, 0.39 ms with one, 0.26 with two,
+// 0.32 with four; s24, 16,384 queries, 12.7, 10.8 and 10.8 ms.
+constexpr int kMaxTeams = 2;
+// Thresholds of the schedule where a phase costs 5 us of barriers and an edge
+// eight times a launch's: each was swept with the others as they are. Both
+// sides at once: 2^15 and 2^19 edges gave a wave on a random graph of 2M
+// vertices 0.28 and 0.33 ms, s22 0.267 and 0.456; 2^16 costs a grid 5% against
+// 2^18. Bridges from 2^14 edges: s22, 200 queries, 0.16 ms against 0.31 from
+// 2^16 and 0.47 from 2^18, but 0.57 against 0.33 on the random graph, so
+// graphs without hub steps keep the launch engine's 2^20. Filters: s22 0.271
+// at 2^11 and 2^16, 0.255 at 2^13 and 2^18, where s24 loses 2%.
+constexpr uint64_t kTeamFilterMinVertices = 1u << 12;
+constexpr uint64_t kTeamFilterMinEdges = 1u << 17;
+constexpr uint64_t kTeamBothMaxEdges = 1u << 16;
+constexpr uint64_t kTeamBridgeMinEdges = 1u << 14;
+constexpr uint64_t kTeamHubMinEdges = 1u << 15;
+constexpr int kTeamTile = 256;  // hub chunk when the caller gives none
+// The machines' workspaces take at most this share of the device's memory
+// (16 machines at R-MAT s24: 22 GB); larger graphs run the launch engine.
+constexpr size_t kTeamMemShare = 8;
+
+struct TeamWorkspace {
+  char* mem = nullptr;
+  BatchLayout layout;
+  size_t stride = 0;
+  int teams = 0;    // per XCD that the memory holds
+  int blocks = 0;
+  char* d_io = nullptr;  // what a run uploads and reads back, and its pinned copy
+  char* h_io = nullptr;
+  size_t io_bytes = 0;
+  bool off = false;  // not available for this graph
+};
+
+void team_free(TeamWorkspace* w) {
+  if (!w) return;
+  (void)hipFree(w->mem);
+  (void)hipFree(w->d_io);
+  if (w->h_io) (void)hipHostFree(w->h_io);
+  delete w;
+}
+
+static fc_status team_alloc(fc_graph* g) {
+  if (!g->team) g->team = new TeamWorkspace();
+  TeamWorkspace* w = g->team;
+  if (w->mem || w->off) return FC_OK;
+  hipDeviceProp_t prop;
+  FC_HIP(hipGetDeviceProperties(&prop, g->device));
+  const int occ = g->off64 ? team_occupancy<int64_t>() : team_occupancy<int32_t>();
+  const int blocks = std::min(occ, 4) * g->cus;
+  const BatchLayout l = batch_layout(g->V, g->hcap, blocks / kXcds);
+  const size_t stride = l.bytes, budget = prop.totalGlobalMem / kTeamMemShare;
+  int teams = kMaxTeams;
+  while (teams > 0 && (size_t)(kXcds * teams) * stride > budget) --teams;
+  if (teams < 1 || occ < 1 || g->V > kTeamMaxV || g->cus % kXcds != 0 || !g->symmetric) {
+    w->off = true;
+    return FC_OK;
+  }
+  if (hipMalloc((void**)&w->mem, (size_t)(kXcds * teams) * stride) != hipSuccess) {
+    (void)hipGetLastError();
+    w->mem = nullptr;
+    w->off = true;
+    return FC_OK;
+  }
+  w->stride = stride;
+  w->layout = l;
+  w->teams = teams;
+  w->blocks = blocks;
+  FC_HIP(hipMemsetAsync(w->mem, 0, (size_t)(kXcds * teams) * stride, g->stream));
+  return FC_OK;
+}
+
+// Answer n queries with the team engine; *ran is false when it is not
+// available for this graph. Distances land in *dist (pinned, valid until the
+// next run).
+static fc_status team_run(fc_graph* g, const int32_t* s, const int32_t* t, int32_t n, int policy, int vw, int tile,
+                          float margin, float* ms, BatchCtl* ctl_out, const int32_t** dist, bool* ran) {
+  *ran = false;
+  const char* env = std::getenv("FASTCON_BATCH_TEAMS");
+  if ((env && std::atoi(env) == 0 && env[0]) || std::getenv("FASTCON_BATCH_LOG")) return FC_OK;
+  fc_status st = team_alloc(g);
+  if (st != FC_OK) return st;
+  TeamWorkspace* w = g->team;
+  if (w->off) return FC_OK;
+  // As many machines as there are full waves, up to what the memory holds
+  // (one per XCD, with all its CUs, for up to eight). A batch that does not
+  // fill them gets narrower waves, one for every machine: bit-parallelism
+  // shares little beyond the hubs' lists, so eight waves of 8 queries take
+  // about an eighth of one wave of 64 each. Not under the plain schedule,
+  // whose waves of 64 the counters are defined on.
+  const int64_t full = (n + 63) / 64;
+  int teams = full <= kXcds ? 1 : w->teams;
+  if (env && std::atoi(env) > 0) teams = std::min(std::atoi(env), w->teams);
+  const int machines = kXcds * teams;
+  const int32_t qw = policy == FC_POLICY_PLAIN ? 64 : std::min(64, (n + machines - 1) / machines);
+  const int32_t nw = (n + qw - 1) / qw;
+  auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
+  const size_t o_gen = al(kXcds * sizeof(TeamSync)), o_bar = o_gen + al(kXcds * kMaxTeams * sizeof(TeamWord));
+  const size_t o_tick = o_bar + al(kXcds * kMaxTeams * sizeof(TeamBar));
+  static_assert(sizeof(BatchParams<int32_t>) == sizeof(BatchParams<int64_t>), "one size of parameters");
+  const size_t o_init = o_tick + 256, o_par = o_init + al(8 * kTeamOutWords);
+  const size_t o_qs = o_par + al(sizeof(BatchParams<int64_t>) * kXcds * kMaxTeams), o_qt = o_qs + al(4 * (size_t)n);
+  const size_t o_err = o_qt + al(4 * (size_t)n), o_out = o_err + 256;
+  const size_t o_dist = o_out + al(8 * kTeamOutWords * kXcds * kMaxTeams), bytes = o_dist + al(4 * (size_t)n);
+  if (bytes > w->io_bytes) {
+    (void)hipFree(w->d_io);
+    if (w->h_io) (void)hipHostFree(w->h_io);
+    w->d_io = w->h_io = nullptr;
+    w->io_bytes = 0;
+    const size_t cap = std::max<size_t>(bytes, 1u << 17);
+    FC_HIP(hipMalloc((void**)&w->d_io, cap));
+    FC_HIP(hipHostMalloc((void**)&w->h_io, cap, hipHostMallocDefault));
+    w->io_bytes = cap;
+  }
+  std::memset(w->h_io, 0, o_qs);
+  std::memset(w->h_io + o_err, 0, o_dist - o_err);
+  BatchCtl init;
+  batch_init(g, init, n, policy, vw, tile, 0, 1, margin, 0);
+  init.qw = qw;
+  init.nwaves = init.stop_wave = nw;
+  init.filt_min_v = batch_threshold("FASTCON_FILTER_MIN_VERTICES", kTeamFilterMinVertices);
+  init.filt_min_e = batch_threshold("FASTCON_FILTER_MIN_EDGES", kTeamFilterMinEdges);
+  init.both_max_e = batch_threshold("FASTCON_BOTH_MAX_EDGES", kTeamBothMaxEdges);
+  init.bridge_min_e = batch_threshold("FASTCON_BRIDGE_MIN_EDGES", g->hub_steps ? kTeamBridgeMinEdges : kBridgeMinEdges);
+  init.hub_min_e = batch_threshold("FASTCON_HUB_MIN_EDGES", kTeamHubMinEdges);
+  std::memcpy(w->h_io + o_init, &init, 8 * kCtlHotWords);
+  std::memcpy(w->h_io + o_qs, s, 4 * (size_t)n);
+  std::memcpy(w->h_io + o_qt, t, 4 * (size_t)n);
+  for (int k = 0; k < machines; ++k) {
+    BatchWorkspace m;
+    batch_pieces(&m, w->mem + (size_t)k * w->stride, w->layout);
+    batch_bind(&m, (int32_t*)(w->d_io + o_qs), (int32_t*)(w->d_io + o_qt), (int32_t*)(w->d_io + o_dist),
+               (uint32_t*)(w->d_io + o_tick));
+    if (g->off64)
+      ((BatchParams<int64_t>*)(w->h_io + o_par))[k] = batch_params<int64_t>(g, &m);
+    else
+      ((BatchParams<int32_t>*)(w->h_io + o_par))[k] = batch_params<int32_t>(g, &m);
+  }
+  TeamRun tr;
+  tr.sync = (TeamSync*)w->d_io;
+  tr.gen = (TeamWord*)(w->d_io + o_gen);
+  tr.bar = (TeamBar*)(w->d_io + o_bar);
+  tr.init = (unsigned long long*)(w->d_io + o_init);
+  tr.out = (unsigned long long*)(w->d_io + o_out);
+  tr.err = (uint32_t*)(w->d_io + o_err);
+  tr.ticket = (uint32_t*)(w->d_io + o_tick);
+  tr.params = w->d_io + o_par;
+  tr.teams = teams;
+  tr.expected = (uint32_t)(w->blocks / kXcds);
+  FC_HIP(hipMemcpyAsync(w->d_io, w->h_io, o_dist, hipMemcpyHostToDevice, g->stream));
+  FC_HIP(hipEventRecord(g->ev0, g->stream));
+  const bool learn = policy == FC_POLICY_LEARNED;
+  auto kernel = g->off64 ? (learn ? batch_team_kernel<int64_t, true> : batch_team_kernel<int64_t, false>)
+                         : (learn ? batch_team_kernel<int32_t, true> : batch_team_kernel<int32_t, false>);
+  hipLaunchKernelGGL(kernel, dim3(w->blocks), dim3(kBlock), 0, g->stream, tr);
+  FC_HIP(hipGetLastError());
+  FC_HIP(hipEventRecord(g->ev1, g->stream));
+  FC_HIP(hipMemcpyAsync(w->h_io + o_err, w->d_io + o_err, bytes - o_err, hipMemcpyDeviceToHost, g->stream));
+  FC_HIP(hipStreamSynchronize(g->stream));
+  FC_HIP(hipEventElapsedTime(ms, g->ev0, g->ev1));
+  std::memset(ctl_out, 0, sizeof(*ctl_out));
+  uint32_t err = 0;
+  int64_t done = 0;
+  for (int k = 0; k < machines; ++k) {
+    BatchCtl c;
+    std::memset(&c, 0, sizeof(c));
+    std::memcpy(&c, w->h_io + o_out + (size_t)k * 8 * kTeamOutWords, 8 * kCtlHotWords);
+    err |= c.err;
+    done += c.waves_done;
+    ctl_out->levels_total += c.levels_total;
+    ctl_out->active_vertices += c.active_vertices;
+    ctl_out->active_edges += c.active_edges;
+    ctl_out->touched_total += c.touched_total;
+    ctl_out->filters += c.filters;
+    ctl_out->phases += c.phases;
+    ctl_out->bridges += c.bridges;
+    ctl_out->bridged += c.bridged;
+  }
+  const bool late = *(const uint32_t*)(w->h_io + o_err) != 0;
+  if (err || late || done != nw) {
+    // the workspaces are in an unknown state: the next run takes new ones
+    team_free(w);
+    g->team = nullptr;
+    if (late) return fail(FC_ERR_TIMEOUT, "batch: a team's wait was given up");
+    if (err) return fail(FC_ERR_CAPACITY, "batch kernel: list guard tripped (err=%u)", err);
+    return fail(FC_ERR_HIP, "batch: %lld of %d waves finished", (long long)done, nw);
+  }
+  ctl_out->nwaves = nw;
+  *dist = (const int32_t*)(w->h_io + o_dist);
+  *ran = true;
   return FC_OK;
 }
 
@@ -2122,33 +2772,47 @@ extern "C" fc_status fc_stcon_batch(fc_graph* g, const int32_t* s, const int32_t
   const int lanes = o.lanes ? o.lanes : fcd::kDefaultLanes;
   if (stats) std::memset(stats, 0, sizeof(*stats));
   if (n == 0) return FC_OK;
-  fc_status st = fcd::batch_alloc(g);
-  if (st != FC_OK) return st;
   g->levels_valid = g->parents_valid = false;
-  fcd::BatchWorkspace* b = g->batch;
   int vw = o.vw, tile = o.tile;
-  if (vw == 0 && tile == 0) {
-    if (b->tuned_vw < 0) {
-      st = fcd::batch_autotune(g, s, t, n, o.policy, lanes);
-      if (st != FC_OK) return st;
-    }
-    vw = b->tuned_vw;
-    tile = b->tuned_tile;
-  }
-  if (tile == 0) tile = 256;
   float ms = 0;
   BatchCtl c;
   int64_t launches = 0;
-  st = fcd::batch_run(g, s, t, n, o.policy, vw, tile, o.use_graph != 0, &ms, &c, &launches, o.learn_margin, lanes);
-  if (st != FC_OK) return st;
+  const int32_t* got = nullptr;
+  fc_status st;
+  // The team engine takes every batch whose lanes the caller leaves open: a
+  // number of lanes asks for that many launch-driven machines.
+  bool ran = false;
+  if (o.lanes == 0) {
+    const int ttile = tile ? tile : fcd::kTeamTile;
+    st = fcd::team_run(g, s, t, n, o.policy, vw, ttile, o.learn_margin, &ms, &c, &got, &ran);
+    if (st != FC_OK) return st;
+    if (ran) tile = ttile, launches = 1;
+  }
+  if (!ran) {
+    st = fcd::batch_alloc(g);
+    if (st != FC_OK) return st;
+    fcd::BatchWorkspace* b = g->batch;
+    if (vw == 0 && tile == 0) {
+      if (b->tuned_vw < 0) {
+        st = fcd::batch_autotune(g, s, t, n, o.policy, lanes);
+        if (st != FC_OK) return st;
+      }
+      vw = b->tuned_vw;
+      tile = b->tuned_tile;
+    }
+    if (tile == 0) tile = 256;
+    st = fcd::batch_run(g, s, t, n, o.policy, vw, tile, o.use_graph != 0, &ms, &c, &launches, o.learn_margin, lanes);
+    if (st != FC_OK) return st;
+    got = b->h_dist;
+  }
   for (int32_t i = 0; i < n; ++i) {
-    const int32_t d = b->h_dist[i];
+    const int32_t d = got[i];
     if (dist) dist[i] = d;
     if (connected) connected[i] = d >= 0 ? 1 : 0;
   }
   if (stats) {
     stats->time_ms = ms;
-    stats->waves = (n + 63) / 64;
+    stats->waves = c.nwaves;
     stats->levels = (int32_t)c.levels_total;
     stats->active_vertices = c.active_vertices;
     stats->active_edges = c.active_edges;

@@ -19,7 +19,8 @@ enum BatchPhase : int32_t {
   kBFilter = 7,    // drop resolved queries from the current frontier lists
   kBPause = 8,     // tracing: stopped at a step decision (launches are no-ops)
   kBDecide = 9,    // tracing: take the pending decision (forced or by policy)
-  kBBridge = 10    // test the edges between the two sides' current frontiers
+  kBBridge = 10,   // test the edges between the two sides' current frontiers
+  kBHub = 11       // teams: meets at the graph's highest-degree vertices
 };
 
 enum BatchSides : int32_t { kSideS = 1, kSideT = 2, kSideBoth = 3 };
@@ -50,6 +51,7 @@ struct BatchCtl {
   int32_t wave;            // current wave index
   int32_t nwaves;
   int32_t nq;              // total queries
+  int32_t qw;              // queries per wave (at most 64)
   int32_t policy;
   int32_t vw_fixed;
   int32_t tile;            // edges per hub chunk
@@ -85,6 +87,9 @@ struct BatchCtl {
   unsigned long long bridge_min_e;  // a bridge step runs before a step whose cheaper side has this many live edges
   int32_t bridge_lv;       // (lvl[0] + 1) << 16 | (lvl[1] + 1) of this wave's last bridge step (0: none)
   int32_t bridges;         // bridge steps (whole batch)
+  int32_t hub_lv;          // as bridge_lv, of the last hub step
+  int32_t hub_steps;       // hub steps (whole batch)
+  unsigned long long hub_min_e;   // a hub step runs when the frontiers have at least this many live edges
   int64_t bridged;         // queries answered by bridge steps (whole batch)
   uint32_t ticket;
   uint32_t err;
@@ -103,8 +108,8 @@ struct BatchCtl {
 
 template <typename OffT>
 struct BatchParams {
-  const OffT* off;
-  const int32_t* col;
+  FC_GLOBAL const OffT* off;
+  FC_GLOBAL const int32_t* col;
   int32_t V;
   int32_t hub_threshold;
   int64_t E;
@@ -112,26 +117,52 @@ struct BatchParams {
   // side-x visited mask of u and rec[2V*x + 2u + 1] = side-x masks ORed in
   // during the current top-down step. One 16-byte load gives a probe both
   // words it needs, and a line holds eight vertices' records of one side.
-  unsigned long long* rec;     // [4*V]
-  unsigned long long* F[2][2]; // frontier masks [side][parity], V entries each
-  uint8_t* tm;                 // touched marks: one byte per 32 vertices whose N words may be non-zero
-  unsigned long long* red;     // [kRedSlots][kRedWords] launch reductions
-  uint32_t* db;                // dirty bitmap: visited words of u non-zero this wave
-  int32_t* fl[2][2];           // frontier lists [side][parity], V entries each
-  int32_t* hl[2][2];           // hub frontier lists (degree >= hub_threshold)
-  int64_t* hb[2][2];           // their edge bases (ascending with slot)
+  FC_GLOBAL unsigned long long* rec;     // [4*V]
+  FC_GLOBAL unsigned long long* F[2][2]; // frontier masks [side][parity], V entries each
+  FC_GLOBAL uint8_t* tm;       // touched marks: one byte per group of kGroup vertices whose N words may be
+                               // non-zero, at group_pos
+  FC_GLOBAL unsigned long long* red;     // [kRedSlots][kRedWords] launch reductions
+  FC_GLOBAL uint8_t* db;       // dirty bitmap: visited words of u non-zero this wave; a group's byte at group_pos
+  int32_t gk;                  // positions of one class of groups (a multiple of 8)
+  FC_GLOBAL int32_t* fl[2][2];           // frontier lists [side][parity], V entries each
+  FC_GLOBAL int32_t* hl[2][2];           // hub frontier lists (degree >= hub_threshold)
+  FC_GLOBAL int64_t* hb[2][2];           // their edge bases (ascending with slot)
   uint32_t hcap;
-  BatchCtl* ctl;
-  const int32_t* qs;           // queries (device), caller ids
-  const int32_t* qt;
-  const int32_t* perm;         // caller id -> device id (null: the same)
-  int32_t* dist;               // results (device), nq entries
-  uint32_t* wave_ticket;       // next unclaimed wave, shared by concurrent machines (null: this
+  FC_GLOBAL BatchCtl* ctl;
+  FC_GLOBAL const int32_t* qs;           // queries (device), caller ids
+  FC_GLOBAL const int32_t* qt;
+  FC_GLOBAL const int32_t* perm;         // caller id -> device id (null: the same)
+  FC_GLOBAL int32_t* dist;               // results (device), nq entries
+  FC_GLOBAL unsigned long long* ht;  // teams: per block the hub step's tables [2][kHubTab]
+  FC_GLOBAL uint32_t* wave_ticket;       // next unclaimed wave, shared by concurrent machines (null: this
                                // machine takes waves wave, wave + 1, ... up to stop_wave)
-  const float* mlp;
+  FC_GLOBAL const float* mlp;
   int32_t v_active;            // vertices [0, v_active) have degree > 0 (the rest are isolated)
+  int32_t hub_tab;             // vertices [0, hub_tab) take part in hub steps (0: none run)
   int32_t sorted_lists;        // every adjacency list is in ascending id order (bridge steps search them)
 };
+
+// Vertices are marked in groups of kGroup, whose records fill one 128-byte
+// line of each side: a commit reads a group's lines whole. (In groups of 32
+// it read 1 KB for the 1.1-2.5 touched vertices of a typical marked group,
+// and at the big commits of a random graph or a grid all records.)
+constexpr uint32_t kGroup = 8;
+// Groups of consecutive vertices are stored by class (group % kGroupClasses):
+// with vertices numbered by decreasing degree the touched groups crowd at low
+// ids, and a wave that reads consecutive positions of the marks, coalesced,
+// still gets groups from all over the range.
+constexpr uint32_t kGroupClasses = 2048;
+__host__ __device__ inline int32_t group_class_len(int64_t V) {
+  const int64_t groups = (V + kGroup - 1) / kGroup;
+  return (int32_t)((((groups + kGroupClasses - 1) / kGroupClasses) + 7) / 8 * 8);
+}
+__host__ __device__ inline uint32_t group_pos(uint32_t g, int32_t gk) {
+  return (g % kGroupClasses) * (uint32_t)gk + g / kGroupClasses;
+}
+__host__ __device__ inline uint32_t group_at(uint32_t pos, int32_t gk) {
+  const uint32_t c = pos / (uint32_t)gk;
+  return (pos - c * (uint32_t)gk) * kGroupClasses + c;
+}
 
 template <typename OffT>
 hipError_t launch_batch_phase(const BatchParams<OffT>& p, int blocks, hipStream_t s);

@@ -14,6 +14,7 @@
 
 namespace fcd {
 struct BatchWorkspace;
+struct TeamWorkspace;
 }
 
 struct fc_graph {
@@ -27,6 +28,8 @@ struct fc_graph {
   int cus = 0;
   int blocks = 0;               // cooperative grid of the visit kernel
   int32_t hub_threshold = 4096;
+  bool symmetric = false;       // every edge is stored in both directions (checked by hash sums)
+  bool hub_steps = false;       // the top vertices are on enough edges for hub steps
   float f_branch = 0.f;         // scheduler feature: log2(1 + sum d^2 / sum d) / 16
   uint32_t hcap = 1;
   uint32_t qcap = 1;
@@ -80,6 +83,7 @@ struct fc_graph {
   std::vector<float> h_mlp;
 
   fcd::BatchWorkspace* batch = nullptr;
+  fcd::TeamWorkspace* team = nullptr;
 };
 
 namespace fcd {
@@ -126,6 +130,7 @@ template <typename OffT>
 int phase_occupancy();
 
 void batch_free(BatchWorkspace* b);
+void team_free(TeamWorkspace* w);
 
 }  // namespace fcd
 

@@ -1,0 +1,111 @@
+// Teams: the blocks of one launch that run on one XCD and work together
+// without ending the launch.
+//
+// MI355X has eight XCDs of 32 CUs with an L2 each. A barrier over the whole
+// grid needs agent-scope fences, which write back and invalidate every L2
+// (16-35 us), so grid-wide steps are separate launches. Blocks of one XCD
+// share its L2, and there a barrier needs neither: it costs an atomic per
+// block and a polled word, 1.2-1.9 us for 32-64 blocks, against 8-20 us from
+// one dependent launch to the next. Measured on this card with data written
+// by plain stores and atomics and read by other CUs of the XCD:
+//  * stores and atomics go through the L1 to the L2 (atomics on to the
+//    memory side, 27 G/s over the chip whatever their scope), and a wave's
+//    are there when its memory counter is zero (s_waitcnt);
+//  * a plain load may hit a line that its own CU's L1 has kept, an
+//    agent-scope load (sc1) never does: it reads the L2 at the same cost as
+//    any L1 miss (90 ns, 250 G/s over the chip). So a team loads whatever
+//    another block may have written in this launch with ld_team, and only
+//    arrays that the launch never writes (the graph, the queries) plainly.
+// An invalidation of the L1 (buffer_inv sc1) at each barrier would allow
+// plain loads, but costs 60 ns a block, one after another.
+//
+// Membership is decided by the hardware: a block reads the XCD it runs on
+// and takes a number there; the first one closes the XCD's registration when
+// the expected blocks are there, or after a short wait when other work holds
+// the CUs. A block that comes later leaves at once. All members are then
+// resident and running, so a team's barriers end whatever else the GPU does;
+// all the same every wait is bounded by the clock.
+#pragma once
+
+#include "wave.hpp"
+
+namespace fcd {
+
+constexpr int kXcds = 8;                   // XCD numbers 0..7
+constexpr uint32_t kTeamClosed = 0x80000000u;
+constexpr uint64_t kTeamJoinTicks = 2000;  // 20 us at 100 MHz: registration closes at the latest
+constexpr uint64_t kTeamWaitTicks = 2000000000ull;  // 20 s: a wait that has failed
+
+// One 128-byte line per word that blocks of a team poll or count on.
+struct alignas(128) TeamWord {
+  uint32_t v;
+  uint32_t pad[31];
+};
+
+// Per XCD; cleared before each launch.
+struct TeamSync {
+  TeamWord reg;     // blocks registered; kTeamClosed once closed
+  TeamWord size;    // members, published when the team's state is ready
+};
+
+// Blocks with blockIdx % kXcds = k run on one XCD; the number is read from
+// the hardware register, so nothing depends on that.
+__device__ __forceinline__ int xcc_id() {
+  constexpr int kHwRegXccId = 20;
+  return (int)__builtin_amdgcn_s_getreg(kHwRegXccId | (3 << 11)) & (kXcds - 1);  // bits 0..3
+}
+
+template <typename T>
+__device__ __forceinline__ T ld_team(const T* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Register with the XCD's team (one thread). Returns this block's number, or
+// -1 when registration is closed. *members is set for number 0 only, which
+// has closed the registration and publishes the size itself (team_publish).
+__device__ __forceinline__ int team_register(TeamSync* ts, uint32_t expected, uint32_t* members) {
+  const uint32_t k = __hip_atomic_fetch_add(&ts->reg.v, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (k & kTeamClosed) return -1;
+  if (k == 0) {
+    const uint64_t t0 = wall_clock64();
+    while (ld_agent(&ts->reg.v) < expected && wall_clock64() - t0 < kTeamJoinTicks) __builtin_amdgcn_s_sleep(1);
+    *members =
+        __hip_atomic_fetch_or(&ts->reg.v, kTeamClosed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & ~kTeamClosed;
+  }
+  return (int)k;
+}
+
+// Wait until the counter *p has reached v (one thread; a difference, so that
+// it may wrap). False when the wait was given up.
+__device__ __forceinline__ bool team_wait(const uint32_t* p, uint32_t v) {
+  const uint64_t t0 = wall_clock64();
+  while ((int32_t)(ld_agent(p) - v) < 0) {
+    if (wall_clock64() - t0 > kTeamWaitTicks) return false;
+    __builtin_amdgcn_s_sleep(1);
+  }
+  return true;
+}
+
+// A team's barrier: every store of the nb blocks is in the L2 when one
+// passes. Blocks count on `arrive` and wait for `gen`, which the last one
+// sets (polling the counter itself would fetch its line from the memory side
+// after every arrival). `passed` counts the barriers. ok: an LDS word of the
+// block. Returns (to all threads) whether the barrier was reached by all.
+struct TeamBar {
+  TeamWord arrive, gen;
+};
+__device__ __forceinline__ bool team_barrier(TeamBar* bar, uint32_t nb, uint32_t& passed, int* ok) {
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  ++passed;
+  if (threadIdx.x == 0) {
+    const uint32_t at =
+        __hip_atomic_fetch_add(&bar->arrive.v, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+    if (at == passed * nb) st_agent(&bar->gen.v, passed);
+    *ok = at == passed * nb || team_wait(&bar->gen.v, passed);
+  }
+  __syncthreads();
+  return __builtin_amdgcn_readfirstlane(*ok) != 0;
+}
+
+}  // namespace fcd

@@ -94,7 +94,18 @@ __device__ __forceinline__ uint64_t wave_reduce_full_u64(uint64_t v) {
   return (uint64_t)bcast64((int64_t)v, 63);
 }
 
-// The same, without any work when every lane holds the identity.
+// Sum or OR over each row of 16 lanes; lane 15 of the row holds the total.
+template <int Op>
+__device__ __forceinline__ uint64_t row_reduce_u64(uint64_t v) {
+  static_assert(Op != kWaveMin, "the identity is 0");
+  constexpr int kRowShr = 0x110;
+  v = wave_apply<Op>(v, dpp_u64<Op, kRowShr + 1, 0xf>(v));
+  v = wave_apply<Op>(v, dpp_u64<Op, kRowShr + 2, 0xf>(v));
+  v = wave_apply<Op>(v, dpp_u64<Op, kRowShr + 4, 0xf>(v));
+  return wave_apply<Op>(v, dpp_u64<Op, kRowShr + 8, 0xf>(v));
+}
+
+// wave_reduce_full_u64 without any work when every lane holds the identity.
 template <int Op>
 __device__ __forceinline__ uint64_t wave_reduce_full_nz_u64(uint64_t v) {
   constexpr uint64_t id = Op == kWaveMin ? ~0ull : 0ull;

@@ -278,7 +278,8 @@ fc_status fc_stcon_sched_many(fc_graph* g, const int32_t* s, const int32_t* t, i
 
 /* Scheduling policy of a visit step. In fc_stcon_batch, the heuristic and
  * learned policies also run bridge steps: before a side whose live frontier
- * has at least 1 M edges (FASTCON_BRIDGE_MIN_EDGES) expands, the edges between
+ * has at least 1 M edges (FASTCON_BRIDGE_MIN_EDGES; 16 K on skewed graphs when
+ * a batch runs in one launch) expands, the edges between
  * the two sides' current frontiers are tested directly, which answers the
  * queries they connect (distance = sum of the two levels + 1). Graphs whose
  * device lists are not id-sorted (FC_GRAPH_KEEP_ORDER, FC_GRAPH_KEEP_IDS)
@@ -294,21 +295,24 @@ typedef struct fc_batch_opts {
   int32_t vw;            /* lanes per vertex for top-down expansion (4..64); 0 = autotuned */
   int32_t tile;          /* hub chunk: edges of the hub lists one wave takes at a time, a
                             multiple of 64 in [64, 65536]; 0 = autotuned */
-  int32_t use_graph;     /* 1: replay captured hipGraphs of 16 phase launches; 0: plain launches */
+  int32_t use_graph;     /* lanes > 0: 1 replays captured hipGraphs of 16 phase launches, 0 launches them one
+                            by one */
   int32_t words;         /* 64-bit query words per vertex: 1 (64 queries per wave) or 0 (the
                             same); other values are FC_ERR_UNSUPPORTED */
   float   learn_margin;  /* learned policy: the network overrides the heuristic's action only
                             when it predicts a log-cost lower by at least this; < 0 = 1.0, the
                             margin chosen on validation graphs for the shipped parameters (at
                             which the network follows the heuristic on held-out graphs) */
-  int32_t lanes;         /* waves run concurrently, each on its own stream and workspace
-                            (1..4); 0 = default (3) */
+  int32_t lanes;         /* 0 (default): one launch per batch, with a wave machine on each XCD of the
+                            GPU or two, each with its own workspace (undirected graphs; see below);
+                            1..4: that many launch-driven wave machines, each on its own stream */
   int32_t reserved;
 } fc_batch_opts;
 
 typedef struct fc_batch_stats {
   double  time_ms;
-  int32_t waves;
+  int32_t waves;               /* waves run; of 64 queries, or narrower where a small batch is spread over
+                                  the machines (lanes 0, heuristic and learned schedules) */
   int32_t levels;              /* sum over waves of visit steps */
   int64_t active_vertices;     /* sum over steps of vertices with a non-zero frontier word */
   int64_t active_edges;        /* sum over steps of their degrees */
@@ -316,15 +320,21 @@ typedef struct fc_batch_stats {
   int32_t vw;                  /* width used */
   int32_t tile;                /* tile schedule used */
   int32_t filters;             /* frontier-list filter passes (resolved queries dropped) */
-  int32_t phases;              /* kernel launches that did work */
-  int64_t launches;            /* kernel launches issued (phases + no-op tail launches) */
+  int32_t phases;              /* phases that did work (lanes > 0: one kernel launch each) */
+  int64_t launches;            /* kernel launches issued (lanes > 0: phases + no-op tail launches) */
   int32_t bridges;             /* bridge steps: edges between the two sides' frontiers tested
                                   directly (heuristic and learned schedules) */
   int32_t bridged;             /* queries a bridge step answered */
 } fc_batch_stats;
 
-/* Batched s–t: queries are run as bit-parallel waves of 64 (one uint64 mask
- * per vertex and side). Verdicts and distances equal fc_stcon's. */
+/* Batched s–t: queries are run as bit-parallel waves of up to 64 (one uint64
+ * mask per vertex and side). Verdicts and distances equal fc_stcon's.
+ * With lanes = 0 a batch runs in one launch when every edge of the graph is
+ * stored in both directions (checked at creation), V < 2^28, and the machines'
+ * workspaces (about 85 bytes per vertex each) take at most an eighth of the
+ * device's memory; otherwise it runs three launch-driven machines. There the
+ * heuristic and learned schedules also run hub steps on skewed graphs: meets
+ * at the 512 vertices of the highest degree, with the same exact distances. */
 fc_status fc_stcon_batch(fc_graph* g, const int32_t* s, const int32_t* t, int32_t n,
                          int32_t* connected, int32_t* dist, const fc_batch_opts* opts,
                          fc_batch_stats* stats);

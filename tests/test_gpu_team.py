@@ -1,0 +1,85 @@
+"""The team engine of fc_stcon_batch (one launch per batch, a wave machine per
+XCD or half of one): distances against the host BFS at the edges of its wave
+and machine counts, with every kind of step forced on small graphs, and the
+graphs it must leave to the launch engine."""
+import numpy as np
+import pytest
+
+from conftest import oracle_pair_dists
+
+pytestmark = pytest.mark.gpu
+
+FORCED = ["FASTCON_HUB_MIN_EDGES", "FASTCON_BRIDGE_MIN_EDGES", "FASTCON_FILTER_MIN_EDGES",
+          "FASTCON_FILTER_MIN_VERTICES"]
+
+
+def _graphs(fc):
+    hub = np.concatenate([[[0, i] for i in range(1, 1500)], [[1, i] for i in range(1400, 2800)],
+                          [[i, i + 1] for i in range(2800, 3000)], [[2799, 2800]]])
+    return {
+        "rmat9": lambda: fc.gen_rmat(9, 16, seed=3),
+        "rmat13": lambda: fc.gen_rmat(13, 16, seed=4),
+        "rmat12-sparse": lambda: fc.gen_rmat(12, 2, a=0.6, b=0.175, c=0.175, seed=5),
+        "two-hubs-and-a-tail": lambda: fc.csr_from_edges(hub, 3100),
+        "er4000": lambda: fc.gen_er(4000, 3.0, 6),
+        "grid60": lambda: fc.gen_grid(60, 61, 0.1, 7),
+        "K300": lambda: fc.csr_from_edges(np.array([[i, j] for i in range(300) for j in range(i)]), 300),
+    }
+
+
+@pytest.mark.parametrize("name", ["rmat9", "rmat13", "rmat12-sparse", "two-hubs-and-a-tail", "er4000", "grid60", "K300"])
+@pytest.mark.parametrize("forced", [False, True])
+def test_team_distances(fc, orc, monkeypatch, name, forced):
+    if forced:  # every level meets the thresholds of every step
+        for v in FORCED:
+            monkeypatch.setenv(v, "1")
+    hg = _graphs(fc)[name]()
+    rng = np.random.default_rng(11)
+    s = rng.integers(0, hg.V, 1100).astype(np.int32)
+    t = rng.integers(0, hg.V, 1100).astype(np.int32)
+    t[5] = s[5]
+    exp = oracle_pair_dists(orc, hg, s, t)
+    for off64, keep_ids in ((False, False), (True, False), (False, True)):
+        with fc.Graph(hg, force64=off64, keep_ids=keep_ids) as g:
+            fc.load_default_sched_params(g)
+            for n in (1, 2, 7, 8, 9, 63, 64, 65, 127, 513, 1100):
+                for pol in (fc.POLICY_HEURISTIC, fc.POLICY_PLAIN, fc.POLICY_LEARNED):
+                    r = g.stcon_batch(s[:n], t[:n], policy=pol, learn_margin=0.0)
+                    assert r.stats["launches"] == 1
+                    assert np.array_equal(r.dist, exp[:n]), (name, off64, keep_ids, n, pol)
+                    assert np.array_equal(r.connected, (exp[:n] >= 0).astype(np.int32))
+
+
+@pytest.mark.parametrize("teams", ["1", "2"])
+def test_team_counts_and_widths(fc, orc, monkeypatch, teams):
+    """One and two machines per XCD, fixed widths and hub chunks, repeated
+    calls on one graph (each leaves its workspace clean)."""
+    monkeypatch.setenv("FASTCON_BATCH_TEAMS", teams)
+    hg = fc.gen_rmat(12, 16, seed=8)
+    rng = np.random.default_rng(12)
+    s = rng.integers(0, hg.V, 700).astype(np.int32)
+    t = rng.integers(0, hg.V, 700).astype(np.int32)
+    exp = oracle_pair_dists(orc, hg, s, t)
+    with fc.Graph(hg) as g:
+        for vw, tile in ((0, 0), (4, 64), (8, 0), (16, 256), (32, 1024), (64, 65536)):
+            for n in (700, 33):
+                assert np.array_equal(g.stcon_batch(s[:n], t[:n], vw=vw, tile=tile).dist, exp[:n]), (vw, tile, n)
+
+
+def test_directed_graphs_keep_the_launch_engine(fc, monkeypatch):
+    """Directed CSRs are accepted as before: their answers depend on the
+    order of the steps, so they stay with the engine whose order they had."""
+    rng = np.random.default_rng(13)
+    e = rng.integers(0, 400, (3000, 2))
+    order = np.argsort(e[:, 0], kind="stable")
+    off = np.zeros(401, np.int64)
+    np.add.at(off, e[:, 0] + 1, 1)
+    hg = fc.HostGraph(np.cumsum(off), e[order, 1].astype(np.int32), directed=True)
+    s = rng.integers(0, 400, 200).astype(np.int32)
+    t = rng.integers(0, 400, 200).astype(np.int32)
+    with fc.Graph(hg) as g:
+        for pol in (fc.POLICY_HEURISTIC, fc.POLICY_PLAIN):
+            a = g.stcon_batch(s, t, policy=pol)
+            b = g.stcon_batch(s, t, policy=pol, lanes=3)
+            assert a.stats["launches"] > 1
+            assert np.array_equal(a.dist, b.dist)
