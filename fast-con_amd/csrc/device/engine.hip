@@ -14,6 +14,7 @@
 // when only a few are needed), reading back the 8-byte phase word between
 // batches to know whether every query has finished.
 #include "engine.hpp"
+#include "team.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -114,12 +115,173 @@ static fc_status ensure_graph(fc_graph* g) {
   return FC_OK;
 }
 
+// ---------------------------------------------------------------------------
+// Plain s–t queries by teams (st_team_kernel): one launch per call.
+// ---------------------------------------------------------------------------
+struct StTeams {
+  char* mem = nullptr;   // kXcds machines' workspaces
+  size_t stride = 0;
+  size_t o_q = 0, q1 = 0, o_hq = 0, hq1 = 0, o_hb = 0, hb1 = 0;  // pieces of one (state words first); x1: one array
+  int blocks = 0;
+  uint32_t epoch_next = 1;
+  char* d_io = nullptr;  // what a run uploads and reads back, and its pinned copy
+  char* h_io = nullptr;
+  size_t io_bytes = 0;
+  bool off = false;      // not available for this graph
+};
+
+void st_teams_free(StTeams* w) {
+  if (!w) return;
+  (void)hipFree(w->mem);
+  (void)hipFree(w->d_io);
+  if (w->h_io) (void)hipHostFree(w->h_io);
+  delete w;
+}
+
+static size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
+
+static fc_status st_teams_alloc(fc_graph* g) {
+  if (!g->st_teams) g->st_teams = new StTeams();
+  StTeams* w = g->st_teams;
+  if (w->mem || w->off) return FC_OK;
+  hipDeviceProp_t prop;
+  FC_HIP(hipGetDeviceProperties(&prop, g->device));
+  const size_t V = (size_t)g->V, hcap = g->hcap;
+  w->q1 = al256(4 * V);
+  w->hq1 = al256(4 * hcap);
+  w->hb1 = al256(8 * hcap);
+  w->o_q = al256(8 * V);
+  w->o_hq = w->o_q + 4 * w->q1;
+  w->o_hb = w->o_hq + 4 * w->hq1;
+  w->stride = w->o_hb + 4 * w->hb1;
+  const int occ = g->off64 ? st_team_occupancy<int64_t>() : st_team_occupancy<int32_t>();
+  // at most an eighth of the device's memory (a 4096^2 grid takes 3.2 GB)
+  if (occ < 1 || g->cus % kXcds != 0 || kXcds * w->stride > prop.totalGlobalMem / 8) {
+    w->off = true;
+    return FC_OK;
+  }
+  if (hipMalloc((void**)&w->mem, kXcds * w->stride) != hipSuccess) {
+    (void)hipGetLastError();
+    w->mem = nullptr;
+    w->off = true;
+    return FC_OK;
+  }
+  // 1,024 queries at s22 took 18.1, 11.9, 10.1 and 9.3 ms with 1 to 4 blocks
+  // per CU, 8 queries on a 4096^2 grid 32.9, 27.1 and 25.4 ms with 1, 2 and 4.
+  w->blocks = std::min(occ, 4) * g->cus;
+  // only the state words are read before they are written
+  for (int k = 0; k < kXcds; ++k) FC_HIP(hipMemsetAsync(w->mem + (size_t)k * w->stride, 0, 8 * V, g->stream));
+  return FC_OK;
+}
+
+// Whether n queries go to the teams: several always (eight are visited at a
+// time: R-MAT s22, 16 queries, 0.42 -> 0.22 ms, two 41 -> 35 us); a single one
+// when one XCD expands its levels as fast as a launch of the whole GPU does
+// (s16, 1.8M edges: 20 us both ways, and 58 against 107 us with the host's
+// share), which is not expected of a skewed graph of more than 2^23 edges.
+static bool st_teams_take(const fc_graph* g, int32_t n) {
+  return g->use_st_teams && (n > 1 || !g->hub_steps || g->E <= (1 << 23));
+}
+
+// Run n plain s–t queries by teams; results in g->h_out. *ran is false when
+// the teams are not available for this graph.
+static fc_status st_teams_run(fc_graph* g, const int32_t* s, const int32_t* t, int32_t n, double* ms, bool* ran) {
+  *ran = false;
+  fc_status st = st_teams_alloc(g);
+  if (st != FC_OK) return st;
+  StTeams* w = g->st_teams;
+  if (w->off) return FC_OK;
+  if ((uint64_t)w->epoch_next + (uint64_t)n >= 0xFFFFFFF0ull) {
+    for (int k = 0; k < kXcds; ++k)
+      FC_HIP(hipMemsetAsync(w->mem + (size_t)k * w->stride, 0, 8 * (size_t)g->V, g->stream));
+    w->epoch_next = 1;
+  }
+  static_assert(sizeof(VisitParams<int32_t>) == sizeof(VisitParams<int64_t>), "one size of parameters");
+  const size_t o_bar = al256(kXcds * sizeof(TeamSync)), o_tick = o_bar + al256(kXcds * sizeof(TeamBar));
+  const size_t o_ctl = o_tick + 256, o_par = o_ctl + al256(kXcds * sizeof(StTeamCtl));
+  const size_t o_qs = o_par + al256(kXcds * sizeof(VisitParams<int64_t>)), o_qt = o_qs + al256(4 * (size_t)n);
+  const size_t o_err = o_qt + al256(4 * (size_t)n), o_out = o_err + 256, bytes = o_out + sizeof(VisitOut) * (size_t)n;
+  if (bytes > w->io_bytes) {
+    (void)hipFree(w->d_io);
+    if (w->h_io) (void)hipHostFree(w->h_io);
+    w->d_io = w->h_io = nullptr;
+    w->io_bytes = 0;
+    const size_t cap = std::max<size_t>(bytes, 1u << 17);
+    FC_HIP(hipMalloc((void**)&w->d_io, cap));
+    FC_HIP(hipHostMalloc((void**)&w->h_io, cap, hipHostMallocDefault));
+    w->io_bytes = cap;
+  }
+  std::memset(w->h_io, 0, o_qs);
+  std::memset(w->h_io + o_err, 0, o_out - o_err);
+  std::memcpy(w->h_io + o_qs, s, 4 * (size_t)n);
+  std::memcpy(w->h_io + o_qt, t, 4 * (size_t)n);
+  StTeamRun tr;
+  tr.sync = (TeamSync*)w->d_io;
+  tr.bar = (TeamBar*)(w->d_io + o_bar);
+  tr.ctl = (StTeamCtl*)(w->d_io + o_ctl);
+  tr.ticket = (uint32_t*)(w->d_io + o_tick);
+  tr.err = (uint32_t*)(w->d_io + o_err);
+  tr.params = w->d_io + o_par;
+  tr.nq = n;
+  tr.epoch0 = w->epoch_next;
+  tr.vw_fixed = g->vw_fixed;
+  tr.expected = (uint32_t)(w->blocks / kXcds);
+  w->epoch_next += (uint32_t)n;
+  auto machine = [&](auto prm, int k) {
+    char* m = w->mem + (size_t)k * w->stride;
+    set_param(prm.sst, (unsigned long long*)m);
+    for (int c = 0; c < 2; ++c)
+      for (int r = 0; r < 2; ++r) {
+        const size_t i = (size_t)(2 * c + r);
+        set_param(prm.q[c][r], (int32_t*)(m + w->o_q + i * w->q1));
+        set_param(prm.hq[c][r], (int32_t*)(m + w->o_hq + i * w->hq1));
+        set_param(prm.hb[c][r], (int64_t*)(m + w->o_hb + i * w->hb1));
+      }
+    set_param(prm.ctl, &tr.ctl[k].v);
+    set_param(prm.qs, (const int32_t*)(w->d_io + o_qs));
+    set_param(prm.qt, (const int32_t*)(w->d_io + o_qt));
+    set_param(prm.out, (VisitOut*)(w->d_io + o_out));
+    std::memcpy(w->h_io + o_par + (size_t)k * sizeof(prm), &prm, sizeof(prm));
+    for (auto& b : ((StTeamCtl*)(w->h_io + o_ctl))[k].best) b = ~0ull;
+  };
+  for (int k = 0; k < kXcds; ++k) {
+    if (g->off64)
+      machine(make_params<int64_t>(g), k);
+    else
+      machine(make_params<int32_t>(g), k);
+  }
+  FC_HIP(hipMemcpyAsync(w->d_io, w->h_io, o_out, hipMemcpyHostToDevice, g->stream));
+  FC_HIP(hipEventRecord(g->ev0, g->stream));
+  FC_HIP(g->off64 ? launch_st_team<int64_t>(tr, w->blocks, g->stream) : launch_st_team<int32_t>(tr, w->blocks, g->stream));
+  FC_HIP(hipEventRecord(g->ev1, g->stream));
+  FC_HIP(hipMemcpyAsync(w->h_io + o_err, w->d_io + o_err, bytes - o_err, hipMemcpyDeviceToHost, g->stream));
+  FC_HIP(hipStreamSynchronize(g->stream));
+  float fms = 0.f;
+  FC_HIP(hipEventElapsedTime(&fms, g->ev0, g->ev1));
+  *ms = fms;
+  if (*(const uint32_t*)(w->h_io + o_err)) {
+    // queues and counters are in an unknown state: the next run takes new ones
+    st_teams_free(w);
+    g->st_teams = nullptr;
+    return fail(FC_ERR_TIMEOUT, "s–t visit: a team's wait was given up");
+  }
+  std::memcpy(g->h_out, w->h_io + o_out, sizeof(VisitOut) * (size_t)n);
+  g->h_out[0].launches = 1;
+  *ran = true;
+  return FC_OK;
+}
+
 fc_status run_visits(fc_graph* g, int mode, const int32_t* s, const int32_t* t, int32_t n, bool parents,
                      double* ms) {
   *ms = 0.0;
   if (n <= 0) return FC_OK;
   fc_status st = ensure_queries(g, n);
   if (st != FC_OK) return st;
+  if (mode == kModePlainSt && !parents && st_teams_take(g, n)) {
+    bool ran = false;
+    st = st_teams_run(g, s, t, n, ms, &ran);
+    if (st != FC_OK || ran) return st;
+  }
   if (g->use_graphs) {
     st = ensure_graph(g);
     if (st != FC_OK) return st;
@@ -278,6 +440,8 @@ static fc_status graph_create(const OffT* off, const int32_t* col, int64_t V, in
   // the same kernel trace normally.
   const char* pg = std::getenv("FASTCON_PLAIN_GRAPHS");
   if (pg && std::strcmp(pg, "0") == 0) g->use_graphs = false;
+  const char* pt = std::getenv("FASTCON_PLAIN_TEAMS");
+  if (pt && std::strcmp(pt, "0") == 0) g->use_st_teams = false;
   int64_t hubs = 0;
   fc_status st = sizeof(OffT) == 8
                      ? fc::validate_csr64((const int64_t*)off, col, V, E, g->hub_threshold, &hubs)
@@ -449,6 +613,7 @@ extern "C" fc_status fc_graph_destroy(fc_graph* g) {
   if (g->stream) (void)hipStreamSynchronize(g->stream);
   fcd::batch_free(g->batch);
   fcd::team_free(g->team);
+  fcd::st_teams_free(g->st_teams);
   if (g->gexec) (void)hipGraphExecDestroy(g->gexec);
   if (g->graph) (void)hipGraphDestroy(g->graph);
   if (g->h_out) (void)hipHostFree(g->h_out);

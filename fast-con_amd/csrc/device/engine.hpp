@@ -15,6 +15,7 @@
 namespace fcd {
 struct BatchWorkspace;
 struct TeamWorkspace;
+struct StTeams;
 }
 
 struct fc_graph {
@@ -84,6 +85,8 @@ struct fc_graph {
 
   fcd::BatchWorkspace* batch = nullptr;
   fcd::TeamWorkspace* team = nullptr;
+  fcd::StTeams* st_teams = nullptr;  // plain s–t queries by teams (allocated on first use)
+  bool use_st_teams = true;          // FASTCON_PLAIN_TEAMS=0: every query through the launches
 };
 
 namespace fcd {
@@ -128,9 +131,14 @@ inline VisitCtl visit_init(const VisitParams<OffT>& prm, int mode, int32_t n, co
 }
 template <typename OffT>
 int phase_occupancy();
+template <typename OffT>
+hipError_t launch_st_team(const StTeamRun& tr, int blocks, hipStream_t s);
+template <typename OffT>
+int st_team_occupancy();
 
 void batch_free(BatchWorkspace* b);
 void team_free(TeamWorkspace* w);
+void st_teams_free(StTeams* w);
 
 }  // namespace fcd
 

@@ -54,6 +54,7 @@
 // proposal appears, and the minimum proposal is the exact distance.
 #include "visit.hpp"
 #include "hubstage.hpp"
+#include "team.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -66,6 +67,13 @@ __device__ __forceinline__ OffT bcast_off(OffT v, int src) {
 
 __device__ __forceinline__ bool test_bit(const uint32_t* bm, int32_t v) {
   return (bm[v >> 5] >> (v & 31)) & 1u;
+}
+
+// Loads of the workspace, which this launch writes: in a team other blocks may
+// have written the word earlier in the same launch (team.hpp).
+template <bool TEAM, typename T>
+__device__ __forceinline__ T ldw(const T* q) {
+  return TEAM ? ld_team(q) : *q;
 }
 
 // Next-frontier appender of one wave. Normal-queue entries are staged in
@@ -250,7 +258,7 @@ struct Probe {
   bool tried;              // the atomic was issued
 };
 
-template <typename OffT>
+template <bool TEAM, typename OffT>
 __device__ __forceinline__ Probe<OffT> probe_look(const Appender<OffT>& a, bool st, int32_t u, bool act) {
   const VisitParams<OffT>& p = *a.p;
   Probe<OffT> r;
@@ -260,9 +268,9 @@ __device__ __forceinline__ Probe<OffT> probe_look(const Appender<OffT>& a, bool 
   r.tried = false;
   if (!act) return r;
   if (!st)
-    r.w = p.visited[u >> 5];
+    r.w = ldw<TEAM>((const uint32_t*)p.visited + (u >> 5));
   else if (u != a.root_own && u != a.root_other)
-    r.w = p.sst[u];
+    r.w = ldw<TEAM>((const unsigned long long*)p.sst + u);
   return r;
 }
 
@@ -336,13 +344,16 @@ __device__ __forceinline__ bool probe_done(Appender<OffT>& a, int32_t* parent, b
   return false;
 }
 
-template <typename OffT, int VW>
-__device__ __forceinline__ void td_normal(Appender<OffT>& a, int32_t* parent, bool st, int lvl, int cur_par,
+// The width is a run-time value: a copy of the code per width had made the
+// kernel 48 KB of the 64 KB of instruction cache that two CUs share.
+template <bool TEAM, typename OffT>
+__device__ __forceinline__ void td_normal(Appender<OffT>& a, int32_t* parent, bool st, int vw, int lvl, int cur_par,
                                           uint32_t n, int gwave, int nwaves) {
   const VisitParams<OffT>& p = *a.p;
-  constexpr int G = kWave / VW;
   const int lane = lane_id();
-  const int grp = lane / VW, sub = lane % VW;
+  const int sh = 31 - __builtin_clz((uint32_t)vw);  // vw is a power of two in [4, 64]
+  const int grp = lane >> sh, sub = lane & (vw - 1);
+  const uint32_t G = (uint32_t)kWave >> sh;
   const int32_t* q = p.q[a.c][cur_par];
   if (n > p.qcap) n = p.qcap;
   for (uint32_t base = (uint32_t)gwave * G; base < n; base += (uint32_t)nwaves * G) {
@@ -350,7 +361,7 @@ __device__ __forceinline__ void td_normal(Appender<OffT>& a, int32_t* parent, bo
     int32_t v = 0;
     OffT b = 0, e = 0;
     if (i < n) {
-      v = q[i];
+      v = ldw<TEAM>(q + i);
       if ((uint32_t)v < (uint32_t)p.V) {
         b = p.off[v] + (OffT)sub;
         e = p.off[v + 1];
@@ -361,10 +372,10 @@ __device__ __forceinline__ void td_normal(Appender<OffT>& a, int32_t* parent, bo
     // two columns per lane per round: both loads are issued before either
     // probe, halving the dependent round trips of long lists
     while (ballot(b < e)) {
-      const bool a0 = b < e, a1 = b + VW < e;
+      const bool a0 = b < e, a1 = b + vw < e;
       const int32_t u0 = a0 ? p.col[b] : 0;
-      const int32_t u1 = a1 ? p.col[b + VW] : 0;
-      Probe<OffT> r0 = probe_look(a, st, u0, a0), r1 = probe_look(a, st, u1, a1);
+      const int32_t u1 = a1 ? p.col[b + vw] : 0;
+      Probe<OffT> r0 = probe_look<TEAM>(a, st, u0, a0), r1 = probe_look<TEAM>(a, st, u1, a1);
       probe_issue(a, st, lvl, u0, a0, r0);
       probe_issue(a, st, lvl, u1, a1, r1);
       int64_t d0, d1;
@@ -372,7 +383,7 @@ __device__ __forceinline__ void td_normal(Appender<OffT>& a, int32_t* parent, bo
       const bool c1 = probe_done(a, parent, st, lvl, v, u1, a1, r1, d1);
       push_next(a, c0, u0, d0, a.bitmaps);
       push_next(a, c1, u1, d1, a.bitmaps);
-      b += 2 * VW;
+      b += 2 * vw;
     }
   }
 }
@@ -386,7 +397,7 @@ __device__ __forceinline__ void td_normal(Appender<OffT>& a, int32_t* parent, bo
 // smaller chunks spread the passes over more waves.
 constexpr int kHubChunkMax = 256;
 
-template <typename OffT>
+template <bool TEAM, typename OffT>
 __device__ __forceinline__ void td_hubs(Appender<OffT>& a, int32_t* parent, bool st, int lvl, int cur_par,
                                         uint64_t hubpk, int gwave, int nwaves) {
   const VisitParams<OffT>& p = *a.p;
@@ -407,7 +418,7 @@ __device__ __forceinline__ void td_hubs(Appender<OffT>& a, int32_t* parent, bool
       const uint32_t span = hi - lo;
       const uint32_t step = (span + 63u) / 64u;
       const uint32_t probe = lo + (uint32_t)lane * step;
-      const bool le = probe < hi && (uint64_t)hb[probe] <= cb;
+      const bool le = probe < hi && (uint64_t)ldw<TEAM>(hb + probe) <= cb;
       const uint64_t m = ballot(le);  // a prefix of lanes (hb ascending); lane 0 always set
       const uint32_t k = 63u - (uint32_t)__builtin_clzll((unsigned long long)m);
       lo = lo + k * step;
@@ -420,12 +431,13 @@ __device__ __forceinline__ void td_hubs(Appender<OffT>& a, int32_t* parent, bool
       int32_t v = -1, u = 0;
       if (act) {
         uint32_t s = lo;
-        while (s + 1 < nh && (uint64_t)hb[s + 1] <= g) ++s;
-        v = hq[s];
-        bool good = (uint32_t)v < (uint32_t)p.V && (uint64_t)hb[s] <= g;
+        while (s + 1 < nh && (uint64_t)ldw<TEAM>(hb + s + 1) <= g) ++s;
+        v = ldw<TEAM>(hq + s);
+        const uint64_t h0 = (uint64_t)ldw<TEAM>(hb + s);
+        bool good = (uint32_t)v < (uint32_t)p.V && h0 <= g;
         OffT k2 = 0;
         if (good) {
-          k2 = p.off[v] + (OffT)(g - (uint64_t)hb[s]);
+          k2 = p.off[v] + (OffT)(g - h0);
           good = k2 < p.off[v + 1];
         }
         if (good) {
@@ -436,7 +448,7 @@ __device__ __forceinline__ void td_hubs(Appender<OffT>& a, int32_t* parent, bool
         }
       }
       const bool ok = act && v >= 0;
-      Probe<OffT> r = probe_look(a, st, u, ok);
+      Probe<OffT> r = probe_look<TEAM>(a, st, u, ok);
       probe_issue(a, st, lvl, u, ok, r);
       int64_t d;
       const bool cl = probe_done(a, parent, st, lvl, v, u, ok, r, d);
@@ -447,7 +459,7 @@ __device__ __forceinline__ void td_hubs(Appender<OffT>& a, int32_t* parent, bool
 
 // Level 0 of an s–t query: the root's adjacency [b, e) cut into 64-edge
 // chunks over the waves of the grid (one edge per lane), whatever its degree.
-template <typename OffT>
+template <bool TEAM, typename OffT>
 __device__ __forceinline__ void td_root(Appender<OffT>& a, int32_t* parent, int32_t r, OffT b, OffT e, int gwave,
                                         int nwaves) {
   const VisitParams<OffT>& p = *a.p;
@@ -455,7 +467,7 @@ __device__ __forceinline__ void td_root(Appender<OffT>& a, int32_t* parent, int3
     const OffT j = k + (OffT)lane_id();
     const bool act = j < e;
     const int32_t u = act ? p.col[j] : 0;
-    Probe<OffT> pr = probe_look(a, true, u, act);
+    Probe<OffT> pr = probe_look<TEAM>(a, true, u, act);
     probe_issue(a, true, 0, u, act, pr);
     int64_t d;
     const bool cl = probe_done(a, parent, true, 0, r, u, act, pr, d);
@@ -608,18 +620,6 @@ __device__ __forceinline__ void bu_step(Appender<OffT>& a, int32_t* parent, int 
   }
 }
 
-template <typename OffT>
-__device__ __forceinline__ void td_dispatch(Appender<OffT>& a, int32_t* parent, bool st, int vw, int lvl, int cur_par,
-                                            uint32_t n, int gwave, int nwaves) {
-  switch (vw) {
-    case 4: td_normal<OffT, 4>(a, parent, st, lvl, cur_par, n, gwave, nwaves); break;
-    case 8: td_normal<OffT, 8>(a, parent, st, lvl, cur_par, n, gwave, nwaves); break;
-    case 16: td_normal<OffT, 16>(a, parent, st, lvl, cur_par, n, gwave, nwaves); break;
-    case 32: td_normal<OffT, 32>(a, parent, st, lvl, cur_par, n, gwave, nwaves); break;
-    default: td_normal<OffT, 64>(a, parent, st, lvl, cur_par, n, gwave, nwaves); break;
-  }
-}
-
 // Width for a top-down level: the smallest power of two >= the average degree
 // of the normal-queue entries, clamped to [4, 64].
 // Every block decides this at launch start: vw < ceil(mf / n) exactly when
@@ -638,6 +638,15 @@ constexpr double kBeta = 24.0;
 __device__ __forceinline__ uint32_t ring_size(const Ring& r) { return r.n + (uint32_t)(r.hub >> kHubEdgeBits); }
 
 __device__ __forceinline__ void zero_ring(Ring* r) { *r = Ring{0u, 0u, 0ull, 0ull}; }
+
+// Waves of colour 0, in proportion to the colours' edges; a colour with edges
+// has at least one.
+__device__ __forceinline__ int colour_split(double e0, double e1, int nwaves) {
+  const int lo = e0 > 0 ? 1 : 0, hi = e1 > 0 ? nwaves - 1 : nwaves;
+  const double f = e0 + e1 > 0 ? e0 / (e0 + e1) : 0.5;
+  const int w0 = (int)((double)nwaves * f + 0.5);
+  return w0 < lo ? lo : (w0 > hi ? hi : w0);
+}
 
 // BFS reset (one launch): clear the bitmaps (and, on the caller's numbering,
 // the levels and parents), and block 0 seeds the root.
@@ -874,15 +883,9 @@ __global__ __launch_bounds__(kBlock) void phase_kernel(VisitCtl* ctl, int parity
   // edges, so that both colours' chains of dependent loads run at the same
   // time; each wave expands one colour and stages into that colour's lists.
   const int cur_par = L & 1;
-  int w0 = nwaves;
-  if (ncol == 2) {
-    const double e0 = start ? (double)(s_root[1] - s_root[0]) : (double)cur[0].mf;
-    const double e1 = start ? (double)(s_root[3] - s_root[2]) : (double)cur[1].mf;
-    const int lo = e0 > 0 ? 1 : 0, hi = e1 > 0 ? nwaves - 1 : nwaves;
-    const double f = e0 + e1 > 0 ? e0 / (e0 + e1) : 0.5;
-    w0 = (int)((double)nwaves * f + 0.5);
-    w0 = w0 < lo ? lo : (w0 > hi ? hi : w0);
-  }
+  const int w0 = ncol == 2 ? colour_split(start ? (double)(s_root[1] - s_root[0]) : (double)cur[0].mf,
+                                          start ? (double)(s_root[3] - s_root[2]) : (double)cur[1].mf, nwaves)
+                           : nwaves;
   const int cw = gwave < w0 ? 0 : 1;  // this wave's colour
   const int lw = cw ? gwave - w0 : gwave, nlw = cw ? nwaves - w0 : w0;
   Appender<OffT> a;
@@ -904,20 +907,205 @@ __global__ __launch_bounds__(kBlock) void phase_kernel(VisitCtl* ctl, int parity
   a.h.d = &s_hub[1][(threadIdx.x >> 6) * kHubStage];
   a.h.cnt = 0;
   if (start) {
-    td_root(a, parent, cw ? dst : src, s_root[2 * cw], s_root[2 * cw + 1], lw, nlw);
+    td_root<false>(a, parent, cw ? dst : src, s_root[2 * cw], s_root[2 * cw + 1], lw, nlw);
   } else if (strat == kTopDown) {
     // selects, not indexing: a local array indexed by a runtime value
     // would live in scratch memory
     const int vwc = cw ? vw1 : vw0;
     const uint32_t nc = cw ? cur[1].n : cur[0].n;
     const uint64_t hc = cw ? cur[1].hub : cur[0].hub;
-    td_dispatch(a, parent, st, vwc, L, cur_par, nc, lw, nlw);
-    td_hubs(a, parent, st, L, cur_par, hc, lw, nlw);
+    td_normal<false>(a, parent, st, vwc, L, cur_par, nc, lw, nlw);
+    td_hubs<false>(a, parent, st, L, cur_par, hc, lw, nlw);
   } else {
     bu_step(a, parent, L, p.fbm[cw][L % 3], lw, nlw);
   }
   block_flush(a, ncol, s_sh, &ctl->ring[qp][0][(L + 1) % 3], &ctl->ring[qp][1][(L + 1) % 3]);
 }
+
+// Plain s–t queries by teams (team.hpp): each XCD's blocks visit a query of
+// their own, level after level with a barrier inside the XCD, until no query
+// is left. The visit is phase_kernel's (the same expansion, claims, frontier
+// counters and stop rule), and so are the answers and the counters. A level
+// of a long path costs one chain of dependent loads and a barrier instead of a
+// launch (a 4096^2 grid: 8 us a level with launches), and eight queries run
+// at a time.
+//
+// Query k of a machine uses the counters of parity k mod 4. Block 0 clears
+// those of query k + 2 when query k starts: all blocks have then left query
+// k - 2, whose counters they were (its last reader passed a barrier of query
+// k - 1), and no block appends to query k + 2 before two more barriers.
+template <typename OffT>
+__global__ __launch_bounds__(kBlock) void st_team_kernel(StTeamRun tr) {
+  __shared__ VisitParams<OffT> p;
+  __shared__ int32_t s_stage[kWavesPerBlock * kStageCap];
+  __shared__ int32_t s_hub[2][kWavesPerBlock * kHubStage];
+  __shared__ BlockShared s_sh;
+  __shared__ OffT s_root[4];
+  __shared__ unsigned long long s_now[8];  // the level's rings, the best candidate, the error word
+  __shared__ int s_num, s_size, s_q, s_ok;
+  static_assert(sizeof(Ring) == 3 * sizeof(unsigned long long), "a ring is three words");
+  static_assert(offsetof(VisitCtl, err) % sizeof(unsigned long long) == 0, "the error word is read with its neighbour");
+  const int machine = xcc_id();
+  TeamSync* ts = tr.sync + machine;
+  TeamBar* bar = tr.bar + machine;
+  StTeamCtl* ctl = tr.ctl + machine;
+  if (threadIdx.x == 0) {
+    uint32_t members = 0;
+    s_num = team_register(ts, tr.expected, &members);
+    s_size = (int)members;
+    if (s_num == 0) {
+      st_agent(&ctl->q[0], atomicAdd(tr.ticket, 1u));
+      __builtin_amdgcn_s_waitcnt(0);
+      st_agent(&ts->size.v, members);
+    } else if (s_num > 0) {
+      s_size = team_wait(&ts->size.v, 1u) ? (int)ld_agent(&ts->size.v) : 0;
+      if (!s_size) st_agent(tr.err, 1u);
+    }
+  }
+  constexpr int kWords = (int)(sizeof(VisitParams<OffT>) / sizeof(uint32_t));
+  static_assert(kWords <= kBlock, "one word per thread");
+  if (threadIdx.x < kWords)
+    reinterpret_cast<uint32_t*>(&p)[threadIdx.x] =
+        reinterpret_cast<const uint32_t*>(tr.params)[machine * kWords + threadIdx.x];
+  __syncthreads();
+  const int bid = __builtin_amdgcn_readfirstlane(s_num), nb = __builtin_amdgcn_readfirstlane(s_size);
+  if (bid < 0 || nb == 0) return;
+  const bool lead = bid == 0 && threadIdx.x == 0;
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int gwave = bid * kWavesPerBlock + w, nwaves = nb * kWavesPerBlock;
+  uint32_t bars = 0;
+  for (uint32_t k = 0;; ++k) {
+    const int qp = (int)(k & 3u);
+    if (threadIdx.x == 0) s_q = (int)ld_agent(&ctl->q[qp]);
+    __syncthreads();
+    const int q = __builtin_amdgcn_readfirstlane(s_q);
+    if (q >= tr.nq) return;
+    const int32_t src = p.qs[q], dst = p.qt[q];
+    const uint32_t epoch = tr.epoch0 + (uint32_t)q;
+    if (threadIdx.x < 4) s_root[threadIdx.x] = p.off[(threadIdx.x < 2 ? src : dst) + (int)(threadIdx.x & 1)];
+    __syncthreads();
+    const uint64_t ds = (uint64_t)(s_root[1] - s_root[0]), dt = (uint64_t)(s_root[3] - s_root[2]);
+    if (lead) {
+      st_agent(&ctl->q[(k + 1) & 3u], atomicAdd(tr.ticket, 1u));
+      const int far = (int)((k + 2) & 3u);
+      for (int c = 0; c < 2; ++c)
+        for (int r = 0; r < 3; ++r) zero_ring(&ctl->ring[far][c][r]);
+      ctl->best[far] = ~0ull;
+      p.sst[src] = st_word(epoch, 0, 0);
+      p.sst[dst] = st_word(epoch, 1, 0);
+    }
+    int steps = 0, td = 0, maxf = 1;
+    int64_t vis_v = 2, vis_e = (int64_t)(ds + dt), expv = 2, expe = (int64_t)(ds + dt);
+    for (int L = 0;; ++L) {
+      Ring cur[2] = {{0u, 0u, 0ull, ds}, {0u, 0u, 0ull, dt}};
+      int vw0 = 4, vw1 = 4;
+      if (L > 0) {
+        if (threadIdx.x < 8) {
+          const int i = (int)threadIdx.x;
+          const unsigned long long* word =
+              i < 6 ? reinterpret_cast<const unsigned long long*>(&ctl->ring[qp][i / 3][L % 3]) + i % 3
+              : i == 6 ? &ctl->best[qp]
+                       : reinterpret_cast<const unsigned long long*>(&ctl->v.err);
+          s_now[i] = ld_team(word);
+        }
+        __syncthreads();
+        auto now = [&](int i) { return (uint64_t)bcast64((int64_t)s_now[i], 0); };
+        const uint64_t best = now(6);
+        const uint32_t err = (uint32_t)now(7);
+        cur[0] = Ring{(uint32_t)now(0), 0u, now(1), now(2)};
+        cur[1] = Ring{(uint32_t)now(3), 0u, now(4), now(5)};
+        const uint32_t nf0 = ring_size(cur[0]), nf1 = ring_size(cur[1]);
+        const int64_t mf01 = (int64_t)(cur[0].mf + cur[1].mf);
+        vis_v += (int64_t)nf0 + (int64_t)nf1;
+        vis_e += mf01;
+        const bool met = best != ~0ull, runaway = steps > p.V + 2;
+        if (met || nf0 == 0 || nf1 == 0 || err || runaway) {
+          if (lead) {
+            VisitOut o;
+            o.status = (err || runaway) ? FC_CAPACITY_STATUS : 0;
+            o.levels = steps;
+            o.depth = met ? steps : 0;
+            o.dist = met ? (int32_t)(best >> 32) : -1;
+            o.meet = met ? (int32_t)(uint32_t)best : -1;
+            o.topdown = td;
+            o.bottomup = 0;
+            o.max_frontier = maxf;
+            o.visited_vertices = vis_v;
+            o.visited_edges = vis_e;
+            o.expanded_vertices = expv;
+            o.expanded_edges = expe;
+            o.err = (int32_t)err;
+            o.launches = 0;  // the one launch is the call's
+            p.out[q] = o;
+          }
+          break;
+        }
+        expv += (int64_t)nf0 + (int64_t)nf1;
+        expe += mf01;
+        const int32_t mx = (int32_t)(nf0 > nf1 ? nf0 : nf1);
+        maxf = mx > maxf ? mx : maxf;
+        vw0 = tr.vw_fixed > 0 ? tr.vw_fixed : degree_width(cur[0].n, cur[0].mf - (cur[0].hub & kHubEdgeMask));
+        vw1 = tr.vw_fixed > 0 ? tr.vw_fixed : degree_width(cur[1].n, cur[1].mf - (cur[1].hub & kHubEdgeMask));
+        if (lead) {
+          zero_ring(&ctl->ring[qp][0][(L + 2) % 3]);
+          zero_ring(&ctl->ring[qp][1][(L + 2) % 3]);
+        }
+      }
+      ++steps;
+      td += 2;
+      const int w0 = colour_split((double)cur[0].mf, (double)cur[1].mf, nwaves);
+      const int cw = gwave < w0 ? 0 : 1;
+      const int lw = cw ? gwave - w0 : gwave, nlw = cw ? nwaves - w0 : w0;
+      Appender<OffT> a;
+      a.p = &p;
+      a.c = cw;
+      a.nxt_par = (L & 1) ^ 1;
+      a.nxt = &ctl->ring[qp][cw][(L + 1) % 3];
+      a.nfbm = nullptr;
+      a.best_out = &ctl->best[qp];
+      a.bitmaps = false;
+      a.epoch = epoch;
+      a.root_own = cw ? dst : src;
+      a.root_other = cw ? src : dst;
+      a.buf = s_stage + w * kStageCap;
+      a.cnt = 0;
+      a.mf = 0;
+      a.best = ~0ull;
+      a.h.u = &s_hub[0][w * kHubStage];
+      a.h.d = &s_hub[1][w * kHubStage];
+      a.h.cnt = 0;
+      if (L == 0) {
+        td_root<true>(a, (int32_t*)nullptr, cw ? dst : src, s_root[2 * cw], s_root[2 * cw + 1], lw, nlw);
+      } else {
+        td_normal<true>(a, (int32_t*)nullptr, true, cw ? vw1 : vw0, L, L & 1, cw ? cur[1].n : cur[0].n, lw, nlw);
+        td_hubs<true>(a, (int32_t*)nullptr, true, L, L & 1, cw ? cur[1].hub : cur[0].hub, lw, nlw);
+      }
+      block_flush(a, 2, s_sh, &ctl->ring[qp][0][(L + 1) % 3], &ctl->ring[qp][1][(L + 1) % 3]);
+      if (!team_barrier(bar, (uint32_t)nb, bars, &s_ok)) {
+        if (threadIdx.x == 0) st_agent(tr.err, 1u);
+        return;
+      }
+    }
+  }
+}
+
+template <typename OffT>
+hipError_t launch_st_team(const StTeamRun& tr, int blocks, hipStream_t s) {
+  hipLaunchKernelGGL(st_team_kernel<OffT>, dim3(blocks), dim3(kBlock), 0, s, tr);
+  return hipGetLastError();
+}
+
+template <typename OffT>
+int st_team_occupancy() {
+  int nb = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, st_team_kernel<OffT>, kBlock, 0) != hipSuccess) return 0;
+  return nb;
+}
+
+template hipError_t launch_st_team<int32_t>(const StTeamRun&, int, hipStream_t);
+template hipError_t launch_st_team<int64_t>(const StTeamRun&, int, hipStream_t);
+template int st_team_occupancy<int32_t>();
+template int st_team_occupancy<int64_t>();
 
 template <typename OffT>
 hipError_t launch_phase(VisitCtl* ctl, int parity, int blocks, hipStream_t s) {

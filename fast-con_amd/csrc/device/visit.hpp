@@ -142,6 +142,30 @@ struct VisitCtl {
 static_assert(sizeof(VisitCtl) == 1024, "VisitCtl layout");
 static_assert(sizeof(VisitParams<int64_t>) <= 320 && sizeof(VisitParams<int32_t>) <= 320, "params fit the block");
 
+// A team's control block for plain s–t queries (st_team_kernel): its counters
+// are kept by query mod 4.
+struct StTeamCtl {
+  VisitCtl v;                   // the error bits only
+  Ring ring[4][2][3];           // [query][colour][level % 3]
+  unsigned long long best[4];   // (distance << 32) | meet vertex; ~0 = none
+  uint32_t q[4];                // the query
+};
+
+struct TeamSync;
+struct TeamBar;
+struct StTeamRun {
+  TeamSync* sync;       // per XCD, cleared before each launch
+  TeamBar* bar;         // per XCD, cleared before each launch
+  StTeamCtl* ctl;       // per XCD: zero, best ~0
+  uint32_t* ticket;     // next unclaimed query
+  uint32_t* err;        // a wait that was given up
+  const void* params;   // VisitParams of each machine
+  int32_t nq;
+  uint32_t epoch0;      // query q tags its words epoch0 + q
+  int32_t vw_fixed;
+  uint32_t expected;    // blocks per XCD
+};
+
 constexpr int kFeatures = 12;
 constexpr int kHidden = 32;
 constexpr int kActions = 9;  // sides {s, t, both} x {top-down, top-down width 64, bottom-up}

@@ -1,7 +1,8 @@
-"""The team engine of fc_stcon_batch (one launch per batch, a wave machine per
-XCD or half of one): distances against the host BFS at the edges of its wave
+"""The team engines (team.hpp). fc_stcon_batch in one launch, a wave machine per
+XCD or half of one: distances against the host BFS at the edges of its wave
 and machine counts, with every kind of step forced on small graphs, and the
-graphs it must leave to the launch engine."""
+graphs it must leave to the launch engine. Plain queries, one per XCD at a
+time: distances and every counter against the launch engine's."""
 import numpy as np
 import pytest
 
@@ -83,3 +84,29 @@ def test_directed_graphs_keep_the_launch_engine(fc, monkeypatch):
             b = g.stcon_batch(s, t, policy=pol, lanes=3)
             assert a.stats["launches"] > 1
             assert np.array_equal(a.dist, b.dist)
+
+
+@pytest.mark.parametrize("name", ["rmat9", "rmat13", "rmat12-sparse", "two-hubs-and-a-tail", "er4000", "grid60", "K300"])
+def test_plain_teams(fc, orc, monkeypatch, name):
+    hg = _graphs(fc)[name]()
+    rng = np.random.default_rng(21)
+    s = rng.integers(0, hg.V, 1500).astype(np.int32)
+    t = rng.integers(0, hg.V, 1500).astype(np.int32)
+    t[::97] = s[::97]
+    exp = oracle_pair_dists(orc, hg, s, t)
+    for off64, keep_ids in ((False, False), (True, False), (False, True)):
+        monkeypatch.setenv("FASTCON_PLAIN_TEAMS", "0")
+        with fc.Graph(hg, force64=off64, keep_ids=keep_ids) as g:
+            ref = {n: g.stcon_many(s[:n], t[:n]) for n in (1, 2, 9, 1500)}
+            one = [g.stcon(int(a), int(b)) for a, b in zip(s[1:6], t[1:6])]
+        monkeypatch.delenv("FASTCON_PLAIN_TEAMS")
+        with fc.Graph(hg, force64=off64, keep_ids=keep_ids) as g:
+            for _ in range(2):  # a second pass meets the first one's state words
+                for n, r in ref.items():
+                    x = g.stcon_many(s[:n], t[:n])
+                    assert np.array_equal(x.dist, exp[:n]) and np.array_equal(x.connected, r.connected)
+                    for k in ("levels", "depth", "visited_vertices", "visited_edges", "expanded_vertices",
+                              "expanded_edges", "topdown_levels", "max_frontier"):
+                        assert x.stats[k] == r.stats[k], (name, n, k)
+            for (c, d, m, _), a, b in zip(one, s[1:6], t[1:6]):
+                assert g.stcon(int(a), int(b))[:3] == (c, d, m)
