@@ -242,7 +242,7 @@ static fc_status st_teams_run(fc_graph* g, const int32_t* s, const int32_t* t, i
     set_param(prm.qt, (const int32_t*)(w->d_io + o_qt));
     set_param(prm.out, (VisitOut*)(w->d_io + o_out));
     std::memcpy(w->h_io + o_par + (size_t)k * sizeof(prm), &prm, sizeof(prm));
-    for (auto& b : ((StTeamCtl*)(w->h_io + o_ctl))[k].best) b = ~0ull;
+    for (auto& b : ((StTeamCtl*)(w->h_io + o_ctl))[k].best) b[0] = b[1] = ~0ull;
   };
   for (int k = 0; k < kXcds; ++k) {
     if (g->off64)

@@ -122,7 +122,7 @@ inline VisitCtl visit_init(const VisitParams<OffT>& prm, int mode, int32_t n, co
   st.dst = t[0];
   st.nsrc = st.ndst = -1;
   st.epoch = epoch0;
-  c.best[0] = c.best[1] = ~0ull;
+  for (auto& b : c.best) b[0] = b[1] = ~0ull;
   c.nq = n;
   c.mode = mode;
   c.vw_fixed = vw_fixed;

@@ -749,7 +749,7 @@ __global__ __launch_bounds__(kBlock) void phase_kernel(VisitCtl* ctl, int parity
   if (!start) {
     // see whether the query is finished
     const bool empty = counted && (nf0 == 0 || (st && nf1 == 0));
-    const unsigned long long best = h.best[qp];
+    const unsigned long long best = h.best[qp][(L + 1) & 1];  // the last level's
     const bool runaway = S.steps > p.V + 2;
     if ((st && best != ~0ull) || empty || h.err || runaway) {
       if (lead) {
@@ -831,7 +831,7 @@ __global__ __launch_bounds__(kBlock) void phase_kernel(VisitCtl* ctl, int parity
         for (int k = 0; k < 3; ++k) zero_ring(&ctl->ring[qp ^ 1][c][k]);
         zero_ring(&ctl->ring[qp][c][2]);
       }
-      ctl->best[qp ^ 1] = ~0ull;
+      ctl->best[qp ^ 1][0] = ctl->best[qp ^ 1][1] = ~0ull;
     }
   } else {
     const double mu = (double)p.E - (double)seen;
@@ -894,7 +894,7 @@ __global__ __launch_bounds__(kBlock) void phase_kernel(VisitCtl* ctl, int parity
   a.nxt_par = cur_par ^ 1;
   a.nxt = &ctl->ring[qp][cw][(L + 1) % 3];
   a.nfbm = p.fbm[cw][(L + 1) % 3];
-  a.best_out = &ctl->best[qp];
+  a.best_out = &ctl->best[qp][L & 1];
   a.bitmaps = !st;
   a.epoch = epoch;
   a.root_own = cw ? dst : src;
@@ -941,10 +941,9 @@ __global__ __launch_bounds__(kBlock) void st_team_kernel(StTeamRun tr) {
   __shared__ int32_t s_hub[2][kWavesPerBlock * kHubStage];
   __shared__ BlockShared s_sh;
   __shared__ OffT s_root[4];
-  __shared__ unsigned long long s_now[8];  // the level's rings, the best candidate, the error word
+  __shared__ unsigned long long s_now[7];  // the level's rings and the best candidate of the last level
   __shared__ int s_num, s_size, s_q, s_ok;
   static_assert(sizeof(Ring) == 3 * sizeof(unsigned long long), "a ring is three words");
-  static_assert(offsetof(VisitCtl, err) % sizeof(unsigned long long) == 0, "the error word is read with its neighbour");
   const int machine = xcc_id();
   TeamSync* ts = tr.sync + machine;
   TeamBar* bar = tr.bar + machine;
@@ -990,7 +989,7 @@ __global__ __launch_bounds__(kBlock) void st_team_kernel(StTeamRun tr) {
       const int far = (int)((k + 2) & 3u);
       for (int c = 0; c < 2; ++c)
         for (int r = 0; r < 3; ++r) zero_ring(&ctl->ring[far][c][r]);
-      ctl->best[far] = ~0ull;
+      ctl->best[far][0] = ctl->best[far][1] = ~0ull;
       p.sst[src] = st_word(epoch, 0, 0);
       p.sst[dst] = st_word(epoch, 1, 0);
     }
@@ -1000,27 +999,27 @@ __global__ __launch_bounds__(kBlock) void st_team_kernel(StTeamRun tr) {
       Ring cur[2] = {{0u, 0u, 0ull, ds}, {0u, 0u, 0ull, dt}};
       int vw0 = 4, vw1 = 4;
       if (L > 0) {
-        if (threadIdx.x < 8) {
+        if (threadIdx.x < 7) {
           const int i = (int)threadIdx.x;
-          const unsigned long long* word =
-              i < 6 ? reinterpret_cast<const unsigned long long*>(&ctl->ring[qp][i / 3][L % 3]) + i % 3
-              : i == 6 ? &ctl->best[qp]
-                       : reinterpret_cast<const unsigned long long*>(&ctl->v.err);
-          s_now[i] = ld_team(word);
+          s_now[i] = ld_team(i < 6 ? reinterpret_cast<const unsigned long long*>(&ctl->ring[qp][i / 3][L % 3]) + i % 3
+                                   : &ctl->best[qp][(L - 1) & 1]);
         }
         __syncthreads();
         auto now = [&](int i) { return (uint64_t)bcast64((int64_t)s_now[i], 0); };
         const uint64_t best = now(6);
-        const uint32_t err = (uint32_t)now(7);
         cur[0] = Ring{(uint32_t)now(0), 0u, now(1), now(2)};
         cur[1] = Ring{(uint32_t)now(3), 0u, now(4), now(5)};
         const uint32_t nf0 = ring_size(cur[0]), nf1 = ring_size(cur[1]);
         const int64_t mf01 = (int64_t)(cur[0].mf + cur[1].mf);
         vis_v += (int64_t)nf0 + (int64_t)nf1;
         vis_e += mf01;
+        // The stop decision rests on words that no block changes during the
+        // level (the error bits can: they only colour the result; a guard that
+        // trips drops entries, so the visit still ends).
         const bool met = best != ~0ull, runaway = steps > p.V + 2;
-        if (met || nf0 == 0 || nf1 == 0 || err || runaway) {
+        if (met || nf0 == 0 || nf1 == 0 || runaway) {
           if (lead) {
+            const uint32_t err = ld_team(&ctl->v.err);
             VisitOut o;
             o.status = (err || runaway) ? FC_CAPACITY_STATUS : 0;
             o.levels = steps;
@@ -1062,7 +1061,7 @@ __global__ __launch_bounds__(kBlock) void st_team_kernel(StTeamRun tr) {
       a.nxt_par = (L & 1) ^ 1;
       a.nxt = &ctl->ring[qp][cw][(L + 1) % 3];
       a.nfbm = nullptr;
-      a.best_out = &ctl->best[qp];
+      a.best_out = &ctl->best[qp][L & 1];
       a.bitmaps = false;
       a.epoch = epoch;
       a.root_own = cw ? dst : src;

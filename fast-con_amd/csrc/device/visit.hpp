@@ -129,14 +129,17 @@ struct VisitParams {
 struct VisitCtl {
   VisitState st[2];                  // by launch parity
   Ring ring[2][2][3];                // [query parity][colour][level % 3]
-  unsigned long long best[2];        // by query parity: (distance << 32) | meet vertex; ~0 = none
+  // by query parity and by the parity of the level that found it (a block that
+  // starts late must not read what this launch's first blocks propose):
+  // (distance << 32) | meet vertex; ~0 = none
+  unsigned long long best[2][2];
   uint32_t err;                      // bit 0: queue slot out of range, bit 1: bad vertex id read,
                                      // bit 2: an s–t claim did not settle
   int32_t nq;                        // number of queries
   int32_t mode;
   int32_t vw_fixed;                  // 0: width from frontier degree
   int32_t record_parents;
-  int32_t pad[31];
+  int32_t pad[27];
   alignas(16) unsigned char params[320];  // VisitParams<OffT> of the run
 };
 static_assert(sizeof(VisitCtl) == 1024, "VisitCtl layout");
@@ -147,7 +150,10 @@ static_assert(sizeof(VisitParams<int64_t>) <= 320 && sizeof(VisitParams<int32_t>
 struct StTeamCtl {
   VisitCtl v;                   // the error bits only
   Ring ring[4][2][3];           // [query][colour][level % 3]
-  unsigned long long best[4];   // (distance << 32) | meet vertex; ~0 = none
+  // (distance << 32) | meet vertex, ~0 = none, by the parity of the level that
+  // found it: a block that is already in the next level may propose there
+  // while another still reads this level's
+  unsigned long long best[4][2];
   uint32_t q[4];                // the query
 };
 
