@@ -122,7 +122,7 @@ struct StTeams {
   char* mem = nullptr;   // kXcds machines' workspaces
   size_t stride = 0;
   size_t o_q = 0, q1 = 0, o_hq = 0, hq1 = 0, o_hb = 0, hb1 = 0;  // pieces of one (state words first); x1: one array
-  int blocks = 0;
+  int blocks = 0, narrow_blocks = 0;
   uint32_t epoch_next = 1;
   char* d_io = nullptr;  // what a run uploads and reads back, and its pinned copy
   char* h_io = nullptr;
@@ -155,6 +155,7 @@ static fc_status st_teams_alloc(fc_graph* g) {
   w->o_hb = w->o_hq + 4 * w->hq1;
   w->stride = w->o_hb + 4 * w->hb1;
   const int occ = g->off64 ? st_team_occupancy<int64_t>() : st_team_occupancy<int32_t>();
+  const int nocc = g->off64 ? narrow_occupancy<int64_t>() : narrow_occupancy<int32_t>();
   // at most an eighth of the device's memory (a 4096^2 grid takes 3.2 GB)
   if (occ < 1 || g->cus % kXcds != 0 || kXcds * w->stride > prop.totalGlobalMem / 8) {
     w->off = true;
@@ -169,6 +170,7 @@ static fc_status st_teams_alloc(fc_graph* g) {
   // 1,024 queries at s22 took 18.1, 11.9, 10.1 and 9.3 ms with 1 to 4 blocks
   // per CU, 8 queries on a 4096^2 grid 32.9, 27.1 and 25.4 ms with 1, 2 and 4.
   w->blocks = std::min(occ, 4) * g->cus;
+  w->narrow_blocks = nocc > 0 ? g->cus : 0;
   // only the state words are read before they are written
   for (int k = 0; k < kXcds; ++k) FC_HIP(hipMemsetAsync(w->mem + (size_t)k * w->stride, 0, 8 * V, g->stream));
   return FC_OK;
@@ -183,14 +185,38 @@ static bool st_teams_take(const fc_graph* g, int32_t n) {
   return g->use_st_teams && (n > 1 || !g->hub_steps || g->E <= (1 << 23));
 }
 
-// Run n plain s–t queries by teams; results in g->h_out. *ran is false when
-// the teams are not available for this graph.
-static fc_status st_teams_run(fc_graph* g, const int32_t* s, const int32_t* t, int32_t n, double* ms, bool* ran) {
+// Levels (and parents) of a narrow BFS in caller ids, from the state words of
+// the machine that ran it (out->meet).
+__global__ void narrow_levels_kernel(const int32_t* __restrict__ perm, const int32_t* __restrict__ iperm,
+                                     const char* __restrict__ mem, size_t stride, const VisitOut* __restrict__ out,
+                                     uint32_t epoch, const int32_t* par, int32_t* __restrict__ lv_out,
+                                     int32_t* par_out, int64_t V) {  // par_out may be par (without perm)
+  const unsigned long long* sst =
+      reinterpret_cast<const unsigned long long*>(mem + (size_t)(out->meet & (kXcds - 1)) * stride);
+  const int64_t n = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < V; v += n) {
+    const int32_t k = perm ? perm[v] : (int32_t)v;
+    const unsigned long long w = sst[k];
+    const bool r = (uint32_t)(w >> 32) == epoch;
+    lv_out[v] = r ? (int32_t)((uint32_t)w & (uint32_t)kLevelMask) : -1;
+    if (par_out) {
+      const int32_t q = r ? par[k] : -1;
+      par_out[v] = iperm && (uint32_t)q < (uint32_t)V ? iperm[q] : q;
+    }
+  }
+}
+
+// Run n plain s–t queries by teams (narrow: as narrow visits), or with bfs one
+// BFS from s[0] as a narrow visit, whose levels (and, with par_out, parents)
+// go to lv_out; results in g->h_out. *ran is false when the teams are not
+// available for this graph.
+static fc_status st_teams_run(fc_graph* g, const int32_t* s, const int32_t* t, int32_t n, bool narrow, bool bfs,
+                              int32_t* lv_out, int32_t* par_out, double* ms, bool* ran) {
   *ran = false;
   fc_status st = st_teams_alloc(g);
   if (st != FC_OK) return st;
   StTeams* w = g->st_teams;
-  if (w->off) return FC_OK;
+  if (w->off || (narrow && !w->narrow_blocks)) return FC_OK;
   if ((uint64_t)w->epoch_next + (uint64_t)n >= 0xFFFFFFF0ull) {
     for (int k = 0; k < kXcds; ++k)
       FC_HIP(hipMemsetAsync(w->mem + (size_t)k * w->stride, 0, 8 * (size_t)g->V, g->stream));
@@ -225,7 +251,13 @@ static fc_status st_teams_run(fc_graph* g, const int32_t* s, const int32_t* t, i
   tr.nq = n;
   tr.epoch0 = w->epoch_next;
   tr.vw_fixed = g->vw_fixed;
-  tr.expected = (uint32_t)(w->blocks / kXcds);
+  if (narrow && tr.vw_fixed == 0) {  // published vertices: the graph's mean degree, rounded up to a power of two
+    tr.vw_fixed = 4;
+    while (tr.vw_fixed < 64 && (int64_t)tr.vw_fixed * g->V < g->E) tr.vw_fixed <<= 1;
+  }
+  const int blocks = narrow ? w->narrow_blocks : w->blocks;
+  tr.expected = (uint32_t)(blocks / kXcds);
+  tr.parents = par_out != nullptr;
   w->epoch_next += (uint32_t)n;
   auto machine = [&](auto prm, int k) {
     char* m = w->mem + (size_t)k * w->stride;
@@ -252,7 +284,18 @@ static fc_status st_teams_run(fc_graph* g, const int32_t* s, const int32_t* t, i
   }
   FC_HIP(hipMemcpyAsync(w->d_io, w->h_io, o_out, hipMemcpyHostToDevice, g->stream));
   FC_HIP(hipEventRecord(g->ev0, g->stream));
-  FC_HIP(g->off64 ? launch_st_team<int64_t>(tr, w->blocks, g->stream) : launch_st_team<int32_t>(tr, w->blocks, g->stream));
+  if (narrow)
+    FC_HIP(g->off64 ? launch_narrow<int64_t>(tr, bfs, blocks, g->stream)
+                    : launch_narrow<int32_t>(tr, bfs, blocks, g->stream));
+  else
+    FC_HIP(g->off64 ? launch_st_team<int64_t>(tr, blocks, g->stream) : launch_st_team<int32_t>(tr, blocks, g->stream));
+  if (bfs) {
+    const int lb = (int)std::min<int64_t>((g->V + 255) / 256, (int64_t)g->cus * 8);
+    hipLaunchKernelGGL(narrow_levels_kernel, dim3(lb), dim3(256), 0, g->stream, g->d_perm, g->d_iperm, w->mem,
+                       w->stride, (const VisitOut*)(w->d_io + o_out), tr.epoch0, g->d_parent, lv_out, par_out,
+                       (int64_t)g->V);
+    FC_HIP(hipGetLastError());
+  }
   FC_HIP(hipEventRecord(g->ev1, g->stream));
   FC_HIP(hipMemcpyAsync(w->h_io + o_err, w->d_io + o_err, bytes - o_err, hipMemcpyDeviceToHost, g->stream));
   FC_HIP(hipStreamSynchronize(g->stream));
@@ -279,8 +322,32 @@ fc_status run_visits(fc_graph* g, int mode, const int32_t* s, const int32_t* t, 
   if (st != FC_OK) return st;
   if (mode == kModePlainSt && !parents && st_teams_take(g, n)) {
     bool ran = false;
-    st = st_teams_run(g, s, t, n, ms, &ran);
-    if (st != FC_OK || ran) return st;
+    const bool narrow = g->narrow && g->narrow_st;
+    st = st_teams_run(g, s, t, n, narrow, false, nullptr, nullptr, ms, &ran);
+    if (st != FC_OK) return st;
+    if (ran && narrow) {
+      // the queries whose frontiers grew too wide run again, and the next
+      // calls on this graph do not try
+      std::vector<int32_t> idx, vs, vt;
+      for (int32_t i = 0; i < n; ++i)
+        if (g->h_out[i].status == kTooWide) {
+          idx.push_back(i);
+          vs.push_back(s[i]);
+          vt.push_back(t[i]);
+        }
+      if (!idx.empty()) {
+        g->narrow_st = false;
+        const std::vector<VisitOut> kept(g->h_out, g->h_out + n);
+        double more = 0.0;
+        st = st_teams_run(g, vs.data(), vt.data(), (int32_t)idx.size(), false, false, nullptr, nullptr, &more, &ran);
+        if (st != FC_OK) return st;
+        std::vector<VisitOut> again(g->h_out, g->h_out + idx.size());
+        std::copy(kept.begin(), kept.end(), g->h_out);
+        for (size_t k = 0; k < idx.size(); ++k) g->h_out[idx[k]] = again[k];
+        *ms += more;
+      }
+    }
+    if (ran) return FC_OK;
   }
   if (g->use_graphs) {
     st = ensure_graph(g);
@@ -476,6 +543,13 @@ static fc_status graph_create(const OffT* off, const int32_t* col, int64_t V, in
       d2 += d * d;
     }
     g->f_branch = (float)(std::log2(1.0 + (E > 0 ? d2 / (double)E : 0.0)) / 16.0);
+    // A vertex reached over an edge leads to at most five others on average:
+    // frontiers grow slowly or, on a grid, hardly. Measured (start engine
+    // against narrow visits, device time): 2048^2 grid (3.9), a BFS 30.4
+    // against 10.4 ms; a random graph of mean degree 3 (4.0), 50K vertices, a
+    // BFS 0.25 against 0.16 ms, 64 queries 0.32 against 0.29; of degree 8
+    // (9.0), 64 queries 0.15 against 0.18.
+    g->narrow = E > 0 && d2 / (double)E <= 6.0;
   }
 #define CK(call)                                            \
   do {                                                      \
@@ -690,18 +764,34 @@ extern "C" fc_status fc_bfs(fc_graph* g, int32_t src, int32_t* levels_out, int32
   const bool par = parents_out != nullptr;
   const int32_t none = -1;
   const int32_t dsrc = g->relabeled ? g->h_perm[(size_t)src] : src;
-  double ms = 0;
+  double ms = 0, tried = 0;
   g->levels_valid = g->parents_valid = false;
-  fc_status st = fcd::run_visits(g, fcd::kModeBfs, &dsrc, &none, 1, par, &ms);
-  if (st != FC_OK) return st;
+  const size_t bytes = sizeof(int32_t) * (size_t)g->V;
+  if (g->relabeled && !g->d_lv_out) FC_HIP(hipMalloc((void**)&g->d_lv_out, bytes));
+  if (g->relabeled && par && !g->d_par_out) FC_HIP(hipMalloc((void**)&g->d_par_out, bytes));
+  int32_t* const lv = g->relabeled ? g->d_lv_out : g->d_state;
+  int32_t* const pa = g->relabeled ? g->d_par_out : g->d_parent;
+  bool narrow = false;
+  fc_status st;
+  if (g->use_st_teams && g->narrow && g->narrow_bfs) {
+    if ((st = fcd::ensure_queries(g, 1)) != FC_OK) return st;
+    st = fcd::st_teams_run(g, &dsrc, &none, 1, true, true, lv, par ? pa : nullptr, &ms, &narrow);
+    if (st != FC_OK) return st;
+    if (narrow && g->h_out[0].status == fcd::kTooWide) {
+      narrow = g->narrow_bfs = false;
+      tried = ms;
+    }
+  }
+  if (!narrow) {
+    st = fcd::run_visits(g, fcd::kModeBfs, &dsrc, &none, 1, par, &ms);
+    if (st != FC_OK) return st;
+    ms += tried;
+  }
   const fcd::VisitOut o = g->h_out[0];
   st = check_out(o);
   if (st != FC_OK) return st;
-  if (g->relabeled) {
+  if (!narrow && g->relabeled) {
     // the results in caller ids are part of the BFS: timed with it
-    const size_t bytes = sizeof(int32_t) * (size_t)g->V;
-    if (!g->d_lv_out) FC_HIP(hipMalloc((void**)&g->d_lv_out, bytes));
-    if (par && !g->d_par_out) FC_HIP(hipMalloc((void**)&g->d_par_out, bytes));
     FC_HIP(hipEventRecord(g->ev0, g->stream));
     const int blocks = (int)std::min<int64_t>((g->V + 255) / 256, (int64_t)g->cus * 8);
     hipLaunchKernelGGL(unpermute_kernel, dim3(blocks), dim3(256), 0, g->stream, g->d_perm, g->d_iperm, g->d_visited,
@@ -720,10 +810,8 @@ extern "C" fc_status fc_bfs(fc_graph* g, int32_t src, int32_t* levels_out, int32
     stats->time_ms = ms;
     add_stats(o, stats);
   }
-  const int32_t* lv = g->relabeled ? g->d_lv_out : g->d_state;
-  const int32_t* pa = g->relabeled ? g->d_par_out : g->d_parent;
-  if (levels_out) FC_HIP(read_back(levels_out, lv, sizeof(int32_t) * (size_t)g->V, g));
-  if (parents_out) FC_HIP(read_back(parents_out, pa, sizeof(int32_t) * (size_t)g->V, g));
+  if (levels_out) FC_HIP(read_back(levels_out, lv, bytes, g));
+  if (parents_out) FC_HIP(read_back(parents_out, pa, bytes, g));
   return FC_OK;
 }
 

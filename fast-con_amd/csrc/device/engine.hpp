@@ -86,7 +86,9 @@ struct fc_graph {
   fcd::BatchWorkspace* batch = nullptr;
   fcd::TeamWorkspace* team = nullptr;
   fcd::StTeams* st_teams = nullptr;  // plain s–t queries by teams (allocated on first use)
-  bool use_st_teams = true;          // FASTCON_PLAIN_TEAMS=0: every query through the launches
+  bool use_st_teams = true;          // FASTCON_PLAIN_TEAMS=0: every visit through the launches
+  bool narrow = false;               // even degrees: visits are likely to stay narrow (narrow_kernel)
+  bool narrow_st = true, narrow_bfs = true;  // until one did not
 };
 
 namespace fcd {
@@ -135,6 +137,10 @@ template <typename OffT>
 hipError_t launch_st_team(const StTeamRun& tr, int blocks, hipStream_t s);
 template <typename OffT>
 int st_team_occupancy();
+template <typename OffT>
+hipError_t launch_narrow(const StTeamRun& tr, bool bfs, int blocks, hipStream_t s);
+template <typename OffT>
+int narrow_occupancy();
 
 void batch_free(BatchWorkspace* b);
 void team_free(TeamWorkspace* w);

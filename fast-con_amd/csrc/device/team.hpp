@@ -60,6 +60,13 @@ __device__ __forceinline__ T ld_team(const T* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// A store that other blocks of the XCD see with ld_team: to the L2 and no
+// further, in one piece.
+template <typename T>
+__device__ __forceinline__ void st_team(T* p, T v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
 // Register with the XCD's team (one thread). Returns this block's number, or
 // -1 when registration is closed. *members is set for number 0 only, which
 // has closed the registration and publishes the size itself (team_publish).

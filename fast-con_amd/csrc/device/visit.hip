@@ -346,9 +346,10 @@ __device__ __forceinline__ bool probe_done(Appender<OffT>& a, int32_t* parent, b
 
 // The width is a run-time value: a copy of the code per width had made the
 // kernel 48 KB of the 64 KB of instruction cache that two CUs share.
-template <bool TEAM, typename OffT>
+// push(claimed, u, first edge, degree) takes the claimed vertices (wave-collective).
+template <bool TEAM, typename OffT, typename Push>
 __device__ __forceinline__ void td_normal(Appender<OffT>& a, int32_t* parent, bool st, int vw, int lvl, int cur_par,
-                                          uint32_t n, int gwave, int nwaves) {
+                                          uint32_t n, int gwave, int nwaves, Push push) {
   const VisitParams<OffT>& p = *a.p;
   const int lane = lane_id();
   const int sh = 31 - __builtin_clz((uint32_t)vw);  // vw is a power of two in [4, 64]
@@ -381,8 +382,8 @@ __device__ __forceinline__ void td_normal(Appender<OffT>& a, int32_t* parent, bo
       int64_t d0, d1;
       const bool c0 = probe_done(a, parent, st, lvl, v, u0, a0, r0, d0);
       const bool c1 = probe_done(a, parent, st, lvl, v, u1, a1, r1, d1);
-      push_next(a, c0, u0, d0, a.bitmaps);
-      push_next(a, c1, u1, d1, a.bitmaps);
+      push(c0, u0, r0.ob, d0);
+      push(c1, u1, r1.ob, d1);
       b += 2 * vw;
     }
   }
@@ -397,9 +398,9 @@ __device__ __forceinline__ void td_normal(Appender<OffT>& a, int32_t* parent, bo
 // smaller chunks spread the passes over more waves.
 constexpr int kHubChunkMax = 256;
 
-template <bool TEAM, typename OffT>
+template <bool TEAM, typename OffT, typename Push>
 __device__ __forceinline__ void td_hubs(Appender<OffT>& a, int32_t* parent, bool st, int lvl, int cur_par,
-                                        uint64_t hubpk, int gwave, int nwaves) {
+                                        uint64_t hubpk, int gwave, int nwaves, Push push) {
   const VisitParams<OffT>& p = *a.p;
   uint32_t nh = (uint32_t)(hubpk >> kHubEdgeBits);
   if (nh > p.hcap) nh = p.hcap;
@@ -452,16 +453,16 @@ __device__ __forceinline__ void td_hubs(Appender<OffT>& a, int32_t* parent, bool
       probe_issue(a, st, lvl, u, ok, r);
       int64_t d;
       const bool cl = probe_done(a, parent, st, lvl, v, u, ok, r, d);
-      push_next(a, cl, u, d, a.bitmaps);
+      push(cl, u, r.ob, d);
     }
   }
 }
 
 // Level 0 of an s–t query: the root's adjacency [b, e) cut into 64-edge
 // chunks over the waves of the grid (one edge per lane), whatever its degree.
-template <bool TEAM, typename OffT>
+template <bool TEAM, typename OffT, typename Push>
 __device__ __forceinline__ void td_root(Appender<OffT>& a, int32_t* parent, int32_t r, OffT b, OffT e, int gwave,
-                                        int nwaves) {
+                                        int nwaves, Push push) {
   const VisitParams<OffT>& p = *a.p;
   for (OffT k = b + (OffT)gwave * kWave; k < e; k += (OffT)nwaves * kWave) {
     const OffT j = k + (OffT)lane_id();
@@ -471,7 +472,7 @@ __device__ __forceinline__ void td_root(Appender<OffT>& a, int32_t* parent, int3
     probe_issue(a, true, 0, u, act, pr);
     int64_t d;
     const bool cl = probe_done(a, parent, true, 0, r, u, act, pr, d);
-    push_next(a, cl, u, d, false);
+    push(cl, u, pr.ob, d);
   }
 }
 
@@ -906,16 +907,17 @@ __global__ __launch_bounds__(kBlock) void phase_kernel(VisitCtl* ctl, int parity
   a.h.u = &s_hub[0][(threadIdx.x >> 6) * kHubStage];
   a.h.d = &s_hub[1][(threadIdx.x >> 6) * kHubStage];
   a.h.cnt = 0;
+  auto push = [&](bool claimed, int32_t u, OffT, int64_t deg) { push_next(a, claimed, u, deg, a.bitmaps); };
   if (start) {
-    td_root<false>(a, parent, cw ? dst : src, s_root[2 * cw], s_root[2 * cw + 1], lw, nlw);
+    td_root<false>(a, parent, cw ? dst : src, s_root[2 * cw], s_root[2 * cw + 1], lw, nlw, push);
   } else if (strat == kTopDown) {
     // selects, not indexing: a local array indexed by a runtime value
     // would live in scratch memory
     const int vwc = cw ? vw1 : vw0;
     const uint32_t nc = cw ? cur[1].n : cur[0].n;
     const uint64_t hc = cw ? cur[1].hub : cur[0].hub;
-    td_normal<false>(a, parent, st, vwc, L, cur_par, nc, lw, nlw);
-    td_hubs<false>(a, parent, st, L, cur_par, hc, lw, nlw);
+    td_normal<false>(a, parent, st, vwc, L, cur_par, nc, lw, nlw, push);
+    td_hubs<false>(a, parent, st, L, cur_par, hc, lw, nlw, push);
   } else {
     bu_step(a, parent, L, p.fbm[cw][L % 3], lw, nlw);
   }
@@ -936,7 +938,9 @@ __global__ __launch_bounds__(kBlock) void phase_kernel(VisitCtl* ctl, int parity
 // k - 1), and no block appends to query k + 2 before two more barriers.
 template <typename OffT>
 __global__ __launch_bounds__(kBlock) void st_team_kernel(StTeamRun tr) {
-  __shared__ VisitParams<OffT> p;
+  // read with scalar loads (the launch does not write it)
+  typedef __attribute__((address_space(4))) const VisitParams<OffT>* params_ptr;
+  const VisitParams<OffT>& p = *(const VisitParams<OffT>*)((params_ptr)(uintptr_t)tr.params + xcc_id());
   __shared__ int32_t s_stage[kWavesPerBlock * kStageCap];
   __shared__ int32_t s_hub[2][kWavesPerBlock * kHubStage];
   __shared__ BlockShared s_sh;
@@ -961,11 +965,6 @@ __global__ __launch_bounds__(kBlock) void st_team_kernel(StTeamRun tr) {
       if (!s_size) st_agent(tr.err, 1u);
     }
   }
-  constexpr int kWords = (int)(sizeof(VisitParams<OffT>) / sizeof(uint32_t));
-  static_assert(kWords <= kBlock, "one word per thread");
-  if (threadIdx.x < kWords)
-    reinterpret_cast<uint32_t*>(&p)[threadIdx.x] =
-        reinterpret_cast<const uint32_t*>(tr.params)[machine * kWords + threadIdx.x];
   __syncthreads();
   const int bid = __builtin_amdgcn_readfirstlane(s_num), nb = __builtin_amdgcn_readfirstlane(s_size);
   if (bid < 0 || nb == 0) return;
@@ -1073,11 +1072,12 @@ __global__ __launch_bounds__(kBlock) void st_team_kernel(StTeamRun tr) {
       a.h.u = &s_hub[0][w * kHubStage];
       a.h.d = &s_hub[1][w * kHubStage];
       a.h.cnt = 0;
+      auto push = [&](bool claimed, int32_t u, OffT, int64_t deg) { push_next(a, claimed, u, deg, false); };
       if (L == 0) {
-        td_root<true>(a, (int32_t*)nullptr, cw ? dst : src, s_root[2 * cw], s_root[2 * cw + 1], lw, nlw);
+        td_root<true>(a, (int32_t*)nullptr, cw ? dst : src, s_root[2 * cw], s_root[2 * cw + 1], lw, nlw, push);
       } else {
-        td_normal<true>(a, (int32_t*)nullptr, true, cw ? vw1 : vw0, L, L & 1, cw ? cur[1].n : cur[0].n, lw, nlw);
-        td_hubs<true>(a, (int32_t*)nullptr, true, L, L & 1, cw ? cur[1].hub : cur[0].hub, lw, nlw);
+        td_normal<true>(a, (int32_t*)nullptr, true, cw ? vw1 : vw0, L, L & 1, cw ? cur[1].n : cur[0].n, lw, nlw, push);
+        td_hubs<true>(a, (int32_t*)nullptr, true, L, L & 1, cw ? cur[1].hub : cur[0].hub, lw, nlw, push);
       }
       block_flush(a, 2, s_sh, &ctl->ring[qp][0][(L + 1) % 3], &ctl->ring[qp][1][(L + 1) % 3]);
       if (!team_barrier(bar, (uint32_t)nb, bars, &s_ok)) {
@@ -1105,6 +1105,549 @@ template hipError_t launch_st_team<int32_t>(const StTeamRun&, int, hipStream_t);
 template hipError_t launch_st_team<int64_t>(const StTeamRun&, int, hipStream_t);
 template int st_team_occupancy<int32_t>();
 template int st_team_occupancy<int64_t>();
+
+// ---------------------------------------------------------------------------
+// Narrow visits: a query or BFS whose frontiers stay small over many levels
+// (grids, road networks, sparse random graphs), by one team per query.
+//
+// On such a visit a level's time is its chain of dependent memory round trips,
+// not its work: a frontier entry, its offsets, a column, the neighbour's state
+// word, the claiming atomic, the list reservation, the barrier. st_team_kernel
+// pays all of them (7.6 us a level on a 4096^2 grid), a launch per level 7.9.
+// Here
+//  * a block keeps the vertices it claims, up to kKeep of them, in its LDS,
+//    with their offsets, and its waves expand them at the next level. A CU
+//    takes about one scattered lane per clock, so the widest block sets the
+//    pace: one with much more than its part of the frontier publishes the
+//    rest in the frontier lists, from where all waves take their shares
+//    (2048^2 grid, BFS: 15.5 -> 14.4 ms);
+//  * between its arrival at the barrier and the barrier's end, when it would
+//    wait anyway, a wave loads the first columns of these vertices, the state
+//    words and offsets they lead to, and the line of the columns after that. A
+//    word that another wave changes meanwhile is settled by the claim, as
+//    every stale look is;
+//  * a level ends without an atomic: each block stores a word of its own with
+//    the counts of its claimed vertices, and one wave per block, which does
+//    nothing else, reads the words of all blocks until they carry the level's
+//    tag. The store is a plain one: an agent-scope store writes through the
+//    L2, and the level ended 1.3 us later (15.8 against 11.0 ms). From the
+//    sums every block takes the stop decision; the lists' counters and the
+//    best candidate are only read when a block has flagged them.
+// What is left of a level is the claiming atomic, two block-wide steps, a
+// store and the loads that see it: 2.7 us for 2,000 vertices. Measured
+// against one launch (BFS) or st_team_kernel: BFS of a 2048^2 grid 30.4 ->
+// 10.4 ms, eight queries on a 4096^2 grid 22.9 -> 13.3 ms, of 500^2 7.35 ->
+// 2.35 ms. A visit whose frontier reaches kNarrowMax vertices is given up
+// (kTooWide): the caller runs it on the engine that uses the whole GPU.
+// A BFS is a visit with one colour and no target. Levels, counters and answers
+// are those of the other engines.
+constexpr int kNarrowWaves = kNarrowThreads / kWave;
+constexpr int kSets = 2;                 // kept entries per lane group of four
+constexpr uint32_t kNarrowStage = 256;   // entries a wave stages for publication
+constexpr uint32_t kNarrowSpill = 64;    // and room for what the block gives up
+constexpr uint32_t kNarrowMax = 65535;
+
+// Colours, waves per block and colour that expand, and entries a block can
+// keep per colour.
+template <bool BFS>
+struct NarrowSplit {
+  static constexpr int kColours = BFS ? 1 : 2, kWorkers = (kNarrowWaves - 1) / kColours;
+  static constexpr uint32_t kKeep = 16u * kSets * kWorkers;
+  static_assert(kKeep <= kNarrowSpill * kWorkers, "kNarrowSpill");
+};
+
+template <typename OffT, bool BFS>
+struct NarrowKept {  // a block's kept vertices of one colour, by level parity
+  static constexpr uint32_t kKeep = NarrowSplit<BFS>::kKeep;
+  uint32_t n[2];  // may exceed kKeep: the rest was staged
+  int32_t v[2][kKeep];
+  int32_t d[2][kKeep];
+  OffT b[2][kKeep];
+};
+
+struct NarrowShared {
+  uint32_t cnt[2][kNarrowWaves];
+  uint32_t hcnt[2][kNarrowWaves];
+  unsigned long long hedges[2][kNarrowWaves];
+  uint32_t base[2];
+  unsigned long long hbase[2];
+  uint32_t claims[kNarrowWaves];
+  unsigned long long sums[2][kNarrowWaves];
+  // the level's end, from the service wave: narrow_word sums, and after a look
+  // per colour the lists' n and hub words and the best candidate
+  unsigned long long sum, now[5];
+  int look[2];                // by level parity: this block has something to look at
+};
+
+// Add the claimed vertices to the next frontier: kept by the block, staged for
+// publication, or staged as hubs (wave-collective).
+template <typename OffT, bool BFS>
+__device__ __forceinline__ void push_kept(Appender<OffT>& a, NarrowKept<OffT, BFS>& kp, int par, uint32_t& claims,
+                                          bool claimed, int32_t u, OffT b, int64_t deg) {
+  const VisitParams<OffT>& p = *a.p;
+  const bool hub = claimed && deg >= p.hub_threshold;
+  const bool norm = claimed && !hub;
+  const uint64_t m = ballot(norm);
+  claims += (uint32_t)__popcll(ballot(claimed));
+  if (m) {
+    uint32_t base = 0;
+    if (lane_id() == 0) base = atomicAdd(&kp.n[par], (uint32_t)__popcll(m));
+    const uint32_t at = (uint32_t)bcast((int32_t)base, 0) + lane_rank(m);
+    const bool over = norm && at >= kp.kKeep;
+    if (norm && !over) {
+      kp.v[par][at] = u;
+      kp.d[par][at] = (int32_t)deg;
+      kp.b[par][at] = b;
+    }
+    const uint64_t mo = ballot(over);
+    if (mo) {
+      const uint32_t k = (uint32_t)__popcll(mo);
+      if (a.cnt + k > kNarrowStage) wave_flush(a);
+      if (over) a.buf[a.cnt + lane_rank(mo)] = u;
+      a.cnt += k;
+    }
+  }
+  hub_push(a.h, hub, u, deg, (unsigned long long*)&a.nxt->hub, p.hq[a.c][a.nxt_par], p.hb[a.c][a.nxt_par], p.hcap,
+           &p.ctl->err);
+  if (claimed) a.mf += (uint64_t)deg;
+}
+
+// Block-collective publication of the staged entries, as block_flush (whose
+// sums and candidates travel elsewhere here).
+template <typename OffT>
+__device__ __forceinline__ void narrow_flush(Appender<OffT>& a, NarrowShared& sh, Ring* nxt0, Ring* nxt1) {
+  const int w = (int)(threadIdx.x >> 6), lane = lane_id(), own = a.c;
+  {
+    const unsigned long long hd =
+        wave_reduce_full_nz_u64<kWaveSum>((uint32_t)lane < a.h.cnt ? (unsigned long long)a.h.d[lane] : 0ull);
+    if (lane == 0) {
+      sh.cnt[own][w] = a.cnt;
+      sh.hcnt[own][w] = a.h.cnt;
+      sh.hedges[own][w] = hd;
+      sh.cnt[own ^ 1][w] = 0;
+      sh.hcnt[own ^ 1][w] = 0;
+      sh.hedges[own ^ 1][w] = 0;
+    }
+  }
+  __syncthreads();
+  if (lane == 0 && w < 4) {
+    const int c = w & 1;
+    Ring* nxt = c ? nxt1 : nxt0;
+    uint32_t tot = 0;
+    unsigned long long e = 0;
+    for (int i = 0; i < kNarrowWaves; ++i) {
+      uint32_t& k = w < 2 ? sh.cnt[c][i] : sh.hcnt[c][i];
+      const uint32_t ki = k;
+      k = tot;
+      tot += ki;
+      if (w >= 2) {
+        const unsigned long long ei = sh.hedges[c][i];
+        sh.hedges[c][i] = e;
+        e += ei;
+      }
+    }
+    if (w < 2)
+      sh.base[c] = tot ? atomicAdd(&nxt->n, tot) : 0u;
+    else
+      sh.hbase[c] =
+          tot ? atomicAdd((unsigned long long*)&nxt->hub, ((unsigned long long)tot << kHubEdgeBits) | e) : 0ull;
+  }
+  __syncthreads();
+  const uint32_t base = sh.base[own] + sh.cnt[own][w];
+  int32_t* q = a.p->q[own][a.nxt_par];
+  for (uint32_t i = (uint32_t)lane; i < a.cnt; i += kWave) {
+    if (base + i < a.p->qcap)
+      q[base + i] = a.buf[i];
+    else
+      atomicOr(&a.p->ctl->err, 1u);
+  }
+  if (a.h.cnt) {
+    const unsigned long long hb = sh.hbase[own];
+    hub_write(a.h, (uint32_t)(hb >> kHubEdgeBits) + sh.hcnt[own][w], (hb & kHubEdgeMask) + sh.hedges[own][w],
+              a.p->hq[own][a.nxt_par], a.p->hb[own][a.nxt_par], a.p->hcap, &a.p->ctl->err);
+  }
+}
+
+// A block's word at the end of a level: 16 bits of the level's tag, look, and
+// the block's claimed vertices of both colours (each at most 2^16 - 1, so that
+// the sums over 64 blocks fit their 23 bits).
+__device__ __forceinline__ unsigned long long narrow_word(uint32_t tag, bool look, uint32_t n0, uint32_t n1) {
+  const uint32_t m0 = n0 < 0xffffu ? n0 : 0xffffu, m1 = n1 < 0xffffu ? n1 : 0xffffu;
+  return ((unsigned long long)(tag & 0xffffu) << 48) | (look ? 1ull << 47 : 0ull) | ((unsigned long long)m1 << 23) | m0;
+}
+
+template <typename OffT, bool BFS>
+__global__ __launch_bounds__(kNarrowThreads) void narrow_kernel(StTeamRun tr) {
+  // read with scalar loads (the launch does not write it)
+  typedef __attribute__((address_space(4))) const VisitParams<OffT>* params_ptr;
+  const VisitParams<OffT>& p = *(const VisitParams<OffT>*)((params_ptr)(uintptr_t)tr.params + xcc_id());
+  using Split = NarrowSplit<BFS>;
+  constexpr int kColours = Split::kColours, kWorkers = Split::kWorkers;
+  __shared__ NarrowKept<OffT, BFS> s_kept[kColours];
+  __shared__ int32_t s_stage[kNarrowWaves * (kNarrowStage + kNarrowSpill)];
+  __shared__ int32_t s_hub[2][kNarrowWaves * kHubStage];
+  __shared__ NarrowShared sh;
+  __shared__ OffT s_root[4];
+  __shared__ int s_num, s_size, s_q, s_ok;
+  const int machine = xcc_id();
+  TeamSync* ts = tr.sync + machine;
+  TeamBar* bar = tr.bar + machine;
+  StTeamCtl* ctl = tr.ctl + machine;
+  if (threadIdx.x == 0) {
+    uint32_t members = 0;
+    s_num = team_register(ts, tr.expected, &members);
+    if (s_num >= kWave) s_num = -1;  // a wave reads a word of each block
+    members = members < kWave ? members : kWave;
+    s_size = (int)members;
+    if (s_num == 0) {
+      st_agent(&ctl->q[0], atomicAdd(tr.ticket, 1u));
+      __builtin_amdgcn_s_waitcnt(0);
+      st_agent(&ts->size.v, members);
+    } else if (s_num > 0) {
+      s_size = team_wait(&ts->size.v, 1u) ? (int)ld_agent(&ts->size.v) : 0;
+      if (!s_size) st_agent(tr.err, 1u);
+    }
+  }
+  __syncthreads();
+  const int bid = __builtin_amdgcn_readfirstlane(s_num), nb = __builtin_amdgcn_readfirstlane(s_size);
+  if (bid < 0 || nb == 0) return;
+  const bool lead = bid == 0 && threadIdx.x == 0;
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = lane_id();
+  // The last wave serves: it ends the levels. The others alternate between the
+  // colours (with two, one is left over).
+  const bool serve = w == kNarrowWaves - 1, work = w < kWorkers * kColours;
+  const int cw = BFS ? 0 : w & 1;
+  const int wi = w / kColours, lw = bid * kWorkers + wi, nlw = nb * kWorkers;
+  int32_t* const parent = BFS && tr.parents ? p.parent : nullptr;
+  NarrowKept<OffT, BFS>& kp = s_kept[cw];
+  // this lane's kept entries are ent(0), ent(1), ...: each wave takes 16 in turn
+  const int sub = lane & 3;
+  auto keep_limit = [](uint32_t part) {
+    const uint32_t k = part + part / 4 + 32;
+    return k < Split::kKeep ? k : Split::kKeep;
+  };
+  auto ent = [&](int i) { return (uint32_t)(16 * (i * kWorkers + wi) + (lane >> 2)); };
+  uint32_t bars = 0, tag = 0;
+  for (uint32_t k = 0;; ++k) {
+    const int qp = (int)(k & 3u);
+    if (threadIdx.x == 0) {
+      s_q = (int)ld_agent(&ctl->q[qp]);
+      sh.look[0] = sh.look[1] = 0;
+      for (int c = 0; c < kColours; ++c) s_kept[c].n[0] = s_kept[c].n[1] = 0;
+    }
+    __syncthreads();
+    const int q = __builtin_amdgcn_readfirstlane(s_q);
+    if (q >= tr.nq) return;
+    const int32_t src = p.qs[q], dst = BFS ? -1 : p.qt[q];
+    const uint32_t epoch = tr.epoch0 + (uint32_t)q;
+    if (threadIdx.x < 2 * kColours)
+      s_root[threadIdx.x] = p.off[(threadIdx.x < 2 ? src : dst) + (int)(threadIdx.x & 1)];
+    __syncthreads();
+    const uint64_t ds = (uint64_t)(s_root[1] - s_root[0]), dt = BFS ? 0ull : (uint64_t)(s_root[3] - s_root[2]);
+    if (lead) {
+      st_agent(&ctl->q[(k + 1) & 3u], atomicAdd(tr.ticket, 1u));
+      const int far = (int)((k + 2) & 3u);
+      for (int c = 0; c < 2; ++c)
+        for (int r = 0; r < 3; ++r) zero_ring(&ctl->ring[far][c][r]);
+      ctl->best[far][0] = ctl->best[far][1] = ~0ull;
+      ctl->sum[far][0] = ctl->sum[far][1] = 0ull;
+      p.sst[src] = st_word(epoch, 0, 0);
+      if (!BFS) p.sst[dst] = st_word(epoch, 1, 0);
+      if (parent) parent[src] = src;
+    }
+    Appender<OffT> a;
+    a.p = &p;
+    a.c = cw;
+    a.nfbm = nullptr;
+    a.bitmaps = false;
+    a.epoch = epoch;
+    a.root_own = cw ? dst : src;
+    a.root_other = BFS ? -1 : cw ? src : dst;
+    a.buf = s_stage + w * (kNarrowStage + kNarrowSpill);
+    a.cnt = 0;
+    a.mf = 0;
+    a.h.u = &s_hub[0][w * kHubStage];
+    a.h.d = &s_hub[1][w * kHubStage];
+    a.h.cnt = 0;
+    int steps = 0, maxf = 1, status = 0;
+    int64_t vis_v = kColours, expv = kColours;
+    uint64_t mf_done = 0;  // this lane's claimed degrees, but for the last level's
+    uint32_t nf0 = 1, nf1 = BFS ? 0u : 1u, kept = 0;
+    unsigned long long best = ~0ull;
+    bool look = false;
+    // the first columns of this lane's kept vertices, what they lead to, and
+    // the line of the columns after that
+    int32_t pu[kSets], pt[kSets];
+    unsigned long long pw[kSets];
+    OffT pb[kSets], pe[kSets];
+    auto fresh = [&](int32_t u, unsigned long long word) {
+      return u != a.root_own && u != a.root_other && (uint32_t)(word >> 32) != a.epoch;
+    };
+    for (int L = 0;; ++L) {
+      uint32_t n_pub = 0;
+      uint64_t h_pub = 0;
+      if (L > 0) {
+        if (look) {
+          auto now = [&](int i) { return (uint64_t)bcast64((int64_t)sh.now[i], 0); };
+          best = now(4);
+          n_pub = (uint32_t)now(2 * cw);
+          h_pub = now(2 * cw + 1);
+        }
+        vis_v += (int64_t)nf0 + (int64_t)nf1;
+        const bool met = !BFS && best != ~0ull;
+        if (steps > p.V + 2) status = FC_CAPACITY_STATUS;
+        if (!met && !status && (nf0 >= kNarrowMax || nf1 >= kNarrowMax)) status = kTooWide;
+        if (met || nf0 == 0 || (!BFS && nf1 == 0) || status) break;
+        expv += (int64_t)nf0 + (int64_t)nf1;
+        const int32_t mx = (int32_t)(nf0 > nf1 ? nf0 : nf1);
+        maxf = mx > maxf ? mx : maxf;
+        if (lead) {
+          zero_ring(&ctl->ring[qp][0][(L + 2) % 3]);
+          if (!BFS) zero_ring(&ctl->ring[qp][1][(L + 2) % 3]);
+        }
+      }
+      ++steps;
+      ++tag;
+      const int par = L & 1, npar = par ^ 1;
+      uint32_t claims = 0;
+      a.nxt_par = npar;
+      a.nxt = &ctl->ring[qp][cw][(L + 1) % 3];
+      a.best = ~0ull;
+      a.best_out = &ctl->best[qp][par];
+      mf_done += a.mf;
+      a.mf = 0;
+      auto push = [&](bool claimed, int32_t u, OffT b, int64_t deg) {
+        push_kept(a, kp, npar, claims, claimed, u, b, deg);
+      };
+      if (!work) {
+      } else if (L == 0) {
+        td_root<true>(a, parent, cw ? dst : src, s_root[2 * cw], s_root[2 * cw + 1], lw, nlw, push);
+      } else {
+        // kept vertices: their first four columns are here already
+        if (ent(0) - (uint32_t)(lane >> 2) < kept) {
+          Probe<OffT> r[kSets];
+          uint64_t more = 0;
+#pragma unroll
+          for (int i = 0; i < kSets; ++i) {
+            r[i].w = pw[i];
+            r[i].old = 0;
+            r[i].ob = pb[i];
+            r[i].oe = pe[i];
+            r[i].tried = pu[i] >= 0 && fresh(pu[i], pw[i]);
+            if (r[i].tried) r[i].old = atomicCAS(&p.sst[pu[i]], pw[i], st_word(a.epoch, a.c, L + 1));
+            more |= ballot(ent(i) < kept && kp.d[par][ent(i) < kept ? ent(i) : 0] > 4);
+          }
+#pragma unroll
+          for (int i = 0; i < kSets; ++i) {
+            const int32_t v = parent && ent(i) < kept ? kp.v[par][ent(i)] : 0;
+            int64_t d;
+            const bool cl = probe_done(a, parent, true, L, v, pu[i], pu[i] >= 0, r[i], d);
+            push(cl, pu[i], r[i].ob, d);
+            asm volatile("" ::"v"(pt[i]));  // nothing uses the value: the line is in the L2 now
+          }
+          // and the rest of longer lists
+          if (more) {
+#pragma unroll 1
+            for (int i = 0; i < kSets; ++i) {
+              const uint32_t e = ent(i);
+              const bool on = e < kept;
+              const OffT b = on ? kp.b[par][e] : (OffT)0;
+              const int32_t d = on ? kp.d[par][e] : 0, v = on ? kp.v[par][e] : 0;
+              for (int32_t j = 4 + sub; ballot(j < d); j += 4) {
+                const bool act = j < d;
+                const int32_t u = act ? p.col[b + (OffT)j] : 0;
+                Probe<OffT> pr = probe_look<true>(a, true, u, act);
+                probe_issue(a, true, L, u, act, pr);
+                int64_t dg;
+                const bool cl = probe_done(a, parent, true, L, v, u, act, pr, dg);
+                push(cl, u, pr.ob, dg);
+              }
+            }
+          }
+        }
+        // Published vertices go to the waves one by one while there are few
+        // (they and what they claim stay with their wave), from another wave
+        // on at each level.
+        if (n_pub) {
+          int vw = kWave;
+          while (vw > tr.vw_fixed && (uint64_t)n_pub * (uint64_t)vw > (uint64_t)nlw * kWave) vw >>= 1;
+          const int at = (int)(((uint32_t)lw + 29u * (uint32_t)L) % (uint32_t)nlw);
+          td_normal<true>(a, parent, true, vw, L, par, n_pub, at, nlw, push);
+        }
+        if (h_pub) td_hubs<true>(a, parent, true, L, par, h_pub, lw, nlw, push);
+      }
+      // end of the level: publish if a wave of this block has to
+      const bool cand = ballot(a.best != ~0ull) != 0;
+      if (cand) {
+        const unsigned long long b = wave_reduce_full_u64<kWaveMin>(a.best);
+        if (lane == 0) atomicMin(a.best_out, b);
+      }
+      if (lane == 0) {
+        sh.claims[w] = claims;
+        if (cand || a.cnt || a.h.cnt) sh.look[par] = 1;
+      }
+      __builtin_amdgcn_s_waitcnt(0);
+      __syncthreads();
+      kept = kp.n[npar];
+      // a block with much more than its part of the colour's frontier (as it
+      // was at this level) gives away all above that part
+      const uint32_t nf = cw ? nf1 : nf0, part = nf / (uint32_t)nb;
+      bool flag = __builtin_amdgcn_readfirstlane(sh.look[par]) != 0;
+      for (int c = 0; c < kColours; ++c) flag |= s_kept[c].n[npar] > keep_limit((c ? nf1 : nf0) / (uint32_t)nb);
+      flag = __builtin_amdgcn_readfirstlane((int)flag) != 0;
+      if (serve && lane < kColours) s_kept[lane].n[par] = 0;
+      if (kept > keep_limit(part)) {
+        const uint32_t end = kept < Split::kKeep ? kept : Split::kKeep, low = part < end ? part : end;
+        kept = low;
+        const uint32_t e = low + kNarrowSpill * (uint32_t)wi;
+        if (work && e < end) {
+          const uint32_t k = end - e < kNarrowSpill ? end - e : kNarrowSpill;
+          if ((uint32_t)lane < k) a.buf[a.cnt + (uint32_t)lane] = kp.v[npar][e + (uint32_t)lane];
+          a.cnt += k;
+        }
+      }
+      if (flag) {
+        narrow_flush(a, sh, &ctl->ring[qp][0][(L + 1) % 3], &ctl->ring[qp][1][(L + 1) % 3]);
+        a.cnt = 0;
+        a.h.cnt = 0;
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+      }
+      if (serve) {
+        __builtin_amdgcn_s_setprio(3);  // before its block's prefetches
+        // lanes 0..15: a wave's claims each, colour 1's in the upper half
+        const unsigned long long cl = lane < kNarrowWaves ? (unsigned long long)sh.claims[lane] : 0ull;
+        const unsigned long long both = (unsigned long long)bcast64(
+            (int64_t)row_reduce_u64<kWaveSum>(!BFS && (lane & 1) ? cl << 32 : cl), 15);
+        if (lane == 0) {
+          sh.look[npar] = 0;  // for the next level; this level's readers have passed
+          st_team(&ctl->word[tag & 1][bid], narrow_word(tag, flag, (uint32_t)both, (uint32_t)(both >> 32)));
+        }
+        const bool on = lane < nb;
+        const unsigned long long* const from = &ctl->word[tag & 1][on ? lane : 0];
+        unsigned long long x = ld_agent(from);
+        uint64_t t0 = 0;
+        bool ok = true;
+        for (uint32_t i = 1; ballot((uint32_t)(x >> 48) != (tag & 0xffffu)); ++i) {
+          if (i % 4096 == 0) {
+            if (!t0) t0 = wall_clock64();
+            if (wall_clock64() - t0 > kTeamWaitTicks) {
+              ok = false;
+              break;
+            }
+          }
+          x = ld_agent(from);
+        }
+        const bool any = ballot((x >> 47) & 1ull) != 0;
+        x = on ? x & ((1ull << 46) - 1) : 0ull;
+        const unsigned long long sum = (unsigned long long)wave_reduce_full_nz_u64<kWaveSum>(x);
+        if (any && ok && lane < 5)
+          sh.now[lane] = ld_team(lane < 4 ? reinterpret_cast<const unsigned long long*>(
+                                                &ctl->ring[qp][lane >> 1][(L + 1) % 3]) + (lane & 1)
+                                          : &ctl->best[qp][par]);
+        if (lane == 0) {
+          sh.sum = sum | (any ? 1ull << 47 : 0ull);
+          s_ok = ok;
+        }
+      } else {
+        // meanwhile the others load the next level's first columns and the
+        // state words they lead to
+#pragma unroll
+        for (int i = 0; i < kSets; ++i) {
+          const uint32_t e = ent(i);
+          pu[i] = e < kept && sub < kp.d[npar][e] ? p.col[kp.b[npar][e] + (OffT)sub] : -1;
+        }
+#pragma unroll
+        for (int i = 0; i < kSets; ++i) {
+          pw[i] = probe_look<true>(a, true, pu[i], pu[i] >= 0).w;
+          pb[i] = pe[i] = 0;
+          if (pu[i] >= 0) {
+            OffT o[2];  // in one load
+            __builtin_memcpy(o, p.off + pu[i], sizeof(o));
+            pb[i] = o[0];
+            pe[i] = o[1];
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < kSets; ++i) {
+          pt[i] = 0;
+          if (pu[i] >= 0 && fresh(pu[i], pw[i]) && pb[i] < pe[i]) pt[i] = p.col[pb[i]];
+        }
+      }
+      __syncthreads();
+      if (!__builtin_amdgcn_readfirstlane(s_ok)) {
+        if (threadIdx.x == 0) st_agent(tr.err, 1u);
+        return;
+      }
+      const unsigned long long g = (unsigned long long)bcast64((int64_t)sh.sum, 0);
+      nf0 = (uint32_t)g & 0x7fffffu;
+      nf1 = (uint32_t)(g >> 23) & 0x7fffffu;
+      look = (g >> 47) & 1ull;
+    }
+    // the degree sums of the claimed vertices, all and without the last level's
+    {
+      const unsigned long long all = (unsigned long long)wave_reduce_full_nz_u64<kWaveSum>(mf_done + a.mf);
+      const unsigned long long exp = (unsigned long long)wave_reduce_full_nz_u64<kWaveSum>(mf_done);
+      if (lane == 0) {
+        sh.sums[0][w] = all;
+        sh.sums[1][w] = exp;
+      }
+      __syncthreads();
+      if (threadIdx.x < 2) {
+        unsigned long long t = 0;
+        for (int i = 0; i < kNarrowWaves; ++i) t += sh.sums[threadIdx.x][i];
+        if (t) atomicAdd(&ctl->sum[qp][threadIdx.x], t);
+      }
+      if (!team_barrier(bar, (uint32_t)nb, bars, &s_ok)) {
+        if (threadIdx.x == 0) st_agent(tr.err, 1u);
+        return;
+      }
+    }
+    if (lead) {
+      const bool met = !BFS && best != ~0ull;
+      VisitOut o;
+      const uint32_t err = ld_team(&ctl->v.err);
+      o.status = status ? status : err ? FC_CAPACITY_STATUS : 0;
+      o.levels = steps;
+      o.depth = met ? steps : 0;
+      o.dist = met ? (int32_t)(best >> 32) : -1;
+      o.meet = BFS ? machine : met ? (int32_t)(uint32_t)best : -1;  // BFS: whose state words hold the levels
+      o.topdown = kColours * steps;
+      o.bottomup = 0;
+      o.max_frontier = maxf;
+      o.visited_vertices = vis_v;
+      o.visited_edges = (int64_t)(ds + dt + ld_team(&ctl->sum[qp][0]));
+      o.expanded_vertices = expv;
+      o.expanded_edges = (int64_t)(ds + dt + ld_team(&ctl->sum[qp][1]));
+      o.err = (int32_t)err;
+      o.launches = 0;  // the one launch is the call's
+      p.out[q] = o;
+    }
+  }
+}
+
+template <typename OffT>
+hipError_t launch_narrow(const StTeamRun& tr, bool bfs, int blocks, hipStream_t s) {
+  if (bfs)
+    hipLaunchKernelGGL((narrow_kernel<OffT, true>), dim3(blocks), dim3(kNarrowThreads), 0, s, tr);
+  else
+    hipLaunchKernelGGL((narrow_kernel<OffT, false>), dim3(blocks), dim3(kNarrowThreads), 0, s, tr);
+  return hipGetLastError();
+}
+
+template <typename OffT>
+int narrow_occupancy() {
+  int a = 0, b = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, narrow_kernel<OffT, true>, kNarrowThreads, 0) != hipSuccess ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, narrow_kernel<OffT, false>, kNarrowThreads, 0) != hipSuccess)
+    return 0;
+  return a < b ? a : b;
+}
+
+template hipError_t launch_narrow<int32_t>(const StTeamRun&, bool, int, hipStream_t);
+template hipError_t launch_narrow<int64_t>(const StTeamRun&, bool, int, hipStream_t);
+template int narrow_occupancy<int32_t>();
+template int narrow_occupancy<int64_t>();
 
 template <typename OffT>
 hipError_t launch_phase(VisitCtl* ctl, int parity, int blocks, hipStream_t s) {

@@ -155,7 +155,13 @@ struct StTeamCtl {
   // while another still reads this level's
   unsigned long long best[4][2];
   uint32_t q[4];                // the query
+  // narrow visits only:
+  unsigned long long sum[4][2]; // degrees of the claimed vertices: all, without the last level's
+  unsigned long long pad[12];
+  alignas(128) unsigned long long word[2][kWave];  // by level parity: a block's narrow_word
 };
+constexpr int kNarrowThreads = 1024;
+constexpr int32_t kTooWide = 100;  // VisitOut::status: the frontier outgrew a narrow visit
 
 struct TeamSync;
 struct TeamBar;
@@ -168,8 +174,9 @@ struct StTeamRun {
   const void* params;   // VisitParams of each machine
   int32_t nq;
   uint32_t epoch0;      // query q tags its words epoch0 + q
-  int32_t vw_fixed;
+  int32_t vw_fixed;     // st_team_kernel: 0: from the frontier's degrees; narrow visits: of the published vertices
   uint32_t expected;    // blocks per XCD
+  int32_t parents;      // narrow BFS: record parents
 };
 
 constexpr int kFeatures = 12;

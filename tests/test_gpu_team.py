@@ -110,3 +110,57 @@ def test_plain_teams(fc, orc, monkeypatch, name):
                         assert x.stats[k] == r.stats[k], (name, n, k)
             for (c, d, m, _), a, b in zip(one, s[1:6], t[1:6]):
                 assert g.stcon(int(a), int(b))[:3] == (c, d, m)
+
+
+def _narrow_graphs(fc):
+    def edges(V, e):
+        u, v = np.concatenate([e, e[:, ::-1]]).T
+        order = np.lexsort((v, u))
+        off = np.concatenate([[0], np.cumsum(np.bincount(u, minlength=V))])
+        return fc.HostGraph(off, v[order].astype(np.int32))
+
+    def tree():  # binary: twice as wide at each level, beyond a narrow visit's 65,534 vertices
+        k = np.arange(1, 1 << 18)
+        return edges(1 << 18, np.stack([(k - 1) // 2, k], 1))
+
+    def ladder():  # 16 rungs wide, one list of 300 that its block publishes
+        k = np.arange(3000 * 16).reshape(3000, 16)
+        e = [np.stack([k[:-1].ravel(), k[1:].ravel()], 1), np.stack([k[:, :-1].ravel(), k[:, 1:].ravel()], 1)]
+        e.append(np.stack([np.full(300, k[1500, 0]), 3000 * 16 + np.arange(300)], 1))
+        return edges(3000 * 16 + 300, np.concatenate(e))
+
+    return {"path": lambda: fc.gen_grid(1, 3000, 0.0, 1), "grid7x900": lambda: fc.gen_grid(7, 900, 0.05, 2),
+            "grid500": lambda: fc.gen_grid(500, 500, 0.02, 3), "er-degree-3": lambda: fc.gen_er(100000, 3.0, 4),
+            "tree": tree, "ladder": ladder}
+
+
+@pytest.mark.parametrize("name", ["path", "grid7x900", "grid500", "er-degree-3", "tree", "ladder"])
+def test_narrow_visits(fc, orc, monkeypatch, name):
+    hg = _narrow_graphs(fc)[name]()
+    rng = np.random.default_rng(31)
+    s = np.concatenate([[0], rng.integers(0, hg.V, 39)]).astype(np.int32)
+    t = rng.integers(0, hg.V, 40).astype(np.int32)
+    t[::13] = s[::13]
+    exp = oracle_pair_dists(orc, hg, s, t)
+    keys = ("levels", "visited_vertices", "visited_edges", "expanded_vertices", "expanded_edges", "max_frontier")
+    for off64, keep_ids in ((False, False), (True, False), (False, True)):
+        monkeypatch.setenv("FASTCON_PLAIN_TEAMS", "0")
+        with fc.Graph(hg, force64=off64, keep_ids=keep_ids) as g:
+            ref = [g.bfs(int(r), parents=True) for r in s[:3]]
+            st = {n: g.stcon_many(s[:n], t[:n]) for n in (1, 2, 40)}
+        monkeypatch.delenv("FASTCON_PLAIN_TEAMS")
+        with fc.Graph(hg, force64=off64, keep_ids=keep_ids) as g:
+            for r, (lv, _, stats) in zip(s, ref):  # the root 0 is the tree's: too wide from there
+                for parents in (True, False):
+                    x = g.bfs(int(r), parents=parents)
+                    assert np.array_equal(x[0], lv)
+                    for k in keys:
+                        assert x[2][k] == stats[k], (name, k)
+                    if parents:
+                        assert orc.validate_bfs_tree(hg.offsets, hg.columns, int(r), x[0], x[1]) == 0
+                        assert np.array_equal(x[1] < 0, lv < 0)
+            for n, r in st.items():
+                x = g.stcon_many(s[:n], t[:n])
+                assert np.array_equal(x.dist, exp[:n]) and np.array_equal(x.connected, r.connected)
+                for k in keys + ("depth", "topdown_levels"):
+                    assert x.stats[k] == r.stats[k], (name, n, k)
