@@ -1576,7 +1576,7 @@ __device__ __forceinline__ bool batch_phase(const BatchParams<OffT>& p, const Ba
       wave_add_slot(p.red, bid, kRActV, red[kRActV]);
       wave_add_slot(p.red, bid, kRActE, red[kRActE]);
       red[kRActV] = red[kRActE] = 0;
-      if (!team_barrier(bar, (uint32_t)nb, bars, &lds.sh.last)) return false;
+      if (!team_barrier(bar, bid, nb, bars, &lds.sh.last)) return false;
     }
       [[fallthrough]];
     case kBCommit: {
@@ -1924,7 +1924,7 @@ __global__ __launch_bounds__(kBlock, 4) void batch_team_kernel(TeamRun tr) {
         __builtin_amdgcn_wave_barrier();
       }
       __builtin_amdgcn_s_waitcnt(0);
-      if (lane == 0) st_agent(&ts->size.v, (uint32_t)s_size);
+      if (lane == 0) st_team(&ts->size.v, (uint32_t)s_size);
     }
   } else if (threadIdx.x == 0) {
     s_size = team_wait(&ts->size.v, 1u) ? (int)ld_agent(&ts->size.v) : 0;
@@ -1954,19 +1954,31 @@ __global__ __launch_bounds__(kBlock, 4) void batch_team_kernel(TeamRun tr) {
       return;
     }
     if (phase == kBExpand) phase = kBCommit;
-    const bool last = batch_vote(p, bid, nb, lds.sh);
-    if (last) {
-      if (threadIdx.x < kWave) {
-        batch_finish<true, LEARN>(p, lc, phase, lds);
-        __builtin_amdgcn_s_waitcnt(0);
-        if (threadIdx.x == 0) st_agent(&tr.gen[machine].v, round);
+    // The end of the phase: block 0 waits for all and decides, the others
+    // wait for what it decided.
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    ++bars;
+    if (threadIdx.x < kWave) {
+      if (threadIdx.x == 0) team_arrive(&tr.bar[machine], bid, bars);
+      bool ok;
+      if (bid == 0) {
+        ok = team_all(&tr.bar[machine], nb, bars);
+        if (ok) {
+          batch_finish<true, LEARN>(p, lc, phase, lds);
+          __builtin_amdgcn_s_waitcnt(0);
+          if (threadIdx.x == 0) st_team(&tr.gen[machine].v, round);
+        }
+      } else {
+        ok = team_wait(&tr.gen[machine].v, round);
       }
-    } else if (threadIdx.x == 0) {
-      s_size = team_wait(&tr.gen[machine].v, round);
-      if (!s_size) st_agent(tr.err, 1u);
+      if (threadIdx.x == 0) {
+        s_size = ok;
+        if (!ok) st_agent(tr.err, 1u);
+      }
     }
     __syncthreads();
-    if (!last && !__builtin_amdgcn_readfirstlane(s_size)) return;
+    if (!__builtin_amdgcn_readfirstlane(s_size)) return;
   }
   if (bid == 0 && threadIdx.x < kCtlHotWords) tr.out[(size_t)machine * kTeamOutWords + threadIdx.x] = lds.ctl[threadIdx.x];
 }

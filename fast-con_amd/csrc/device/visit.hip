@@ -957,9 +957,9 @@ __global__ __launch_bounds__(kBlock) void st_team_kernel(StTeamRun tr) {
     s_num = team_register(ts, tr.expected, &members);
     s_size = (int)members;
     if (s_num == 0) {
-      st_agent(&ctl->q[0], atomicAdd(tr.ticket, 1u));
+      st_team(&ctl->q[0], atomicAdd(tr.ticket, 1u));
       __builtin_amdgcn_s_waitcnt(0);
-      st_agent(&ts->size.v, members);
+      st_team(&ts->size.v, members);
     } else if (s_num > 0) {
       s_size = team_wait(&ts->size.v, 1u) ? (int)ld_agent(&ts->size.v) : 0;
       if (!s_size) st_agent(tr.err, 1u);
@@ -984,7 +984,7 @@ __global__ __launch_bounds__(kBlock) void st_team_kernel(StTeamRun tr) {
     __syncthreads();
     const uint64_t ds = (uint64_t)(s_root[1] - s_root[0]), dt = (uint64_t)(s_root[3] - s_root[2]);
     if (lead) {
-      st_agent(&ctl->q[(k + 1) & 3u], atomicAdd(tr.ticket, 1u));
+      st_team(&ctl->q[(k + 1) & 3u], atomicAdd(tr.ticket, 1u));
       const int far = (int)((k + 2) & 3u);
       for (int c = 0; c < 2; ++c)
         for (int r = 0; r < 3; ++r) zero_ring(&ctl->ring[far][c][r]);
@@ -1080,7 +1080,7 @@ __global__ __launch_bounds__(kBlock) void st_team_kernel(StTeamRun tr) {
         td_hubs<true>(a, (int32_t*)nullptr, true, L, L & 1, cw ? cur[1].hub : cur[0].hub, lw, nlw, push);
       }
       block_flush(a, 2, s_sh, &ctl->ring[qp][0][(L + 1) % 3], &ctl->ring[qp][1][(L + 1) % 3]);
-      if (!team_barrier(bar, (uint32_t)nb, bars, &s_ok)) {
+      if (!team_barrier(bar, bid, nb, bars, &s_ok)) {
         if (threadIdx.x == 0) st_agent(tr.err, 1u);
         return;
       }
@@ -1300,9 +1300,9 @@ __global__ __launch_bounds__(kNarrowThreads) void narrow_kernel(StTeamRun tr) {
     members = members < kWave ? members : kWave;
     s_size = (int)members;
     if (s_num == 0) {
-      st_agent(&ctl->q[0], atomicAdd(tr.ticket, 1u));
+      st_team(&ctl->q[0], atomicAdd(tr.ticket, 1u));
       __builtin_amdgcn_s_waitcnt(0);
-      st_agent(&ts->size.v, members);
+      st_team(&ts->size.v, members);
     } else if (s_num > 0) {
       s_size = team_wait(&ts->size.v, 1u) ? (int)ld_agent(&ts->size.v) : 0;
       if (!s_size) st_agent(tr.err, 1u);
@@ -1345,7 +1345,7 @@ __global__ __launch_bounds__(kNarrowThreads) void narrow_kernel(StTeamRun tr) {
     __syncthreads();
     const uint64_t ds = (uint64_t)(s_root[1] - s_root[0]), dt = BFS ? 0ull : (uint64_t)(s_root[3] - s_root[2]);
     if (lead) {
-      st_agent(&ctl->q[(k + 1) & 3u], atomicAdd(tr.ticket, 1u));
+      st_team(&ctl->q[(k + 1) & 3u], atomicAdd(tr.ticket, 1u));
       const int far = (int)((k + 2) & 3u);
       for (int c = 0; c < 2; ++c)
         for (int r = 0; r < 3; ++r) zero_ring(&ctl->ring[far][c][r]);
@@ -1598,7 +1598,7 @@ __global__ __launch_bounds__(kNarrowThreads) void narrow_kernel(StTeamRun tr) {
         for (int i = 0; i < kNarrowWaves; ++i) t += sh.sums[threadIdx.x][i];
         if (t) atomicAdd(&ctl->sum[qp][threadIdx.x], t);
       }
-      if (!team_barrier(bar, (uint32_t)nb, bars, &s_ok)) {
+      if (!team_barrier(bar, bid, nb, bars, &s_ok)) {
         if (threadIdx.x == 0) st_agent(tr.err, 1u);
         return;
       }
