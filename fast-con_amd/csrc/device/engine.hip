@@ -97,8 +97,9 @@ static VisitParams<OffT> make_params(fc_graph* g) {
 }
 
 static hipError_t launch_raw(fc_graph* g, int parity) {
-  if (g->off64) return launch_phase<int64_t>(g->d_ctl, parity, g->blocks, g->stream);
-  return launch_phase<int32_t>(g->d_ctl, parity, g->blocks, g->stream);
+  const bool wide = g->E >= kWideEdges;
+  if (g->off64) return launch_phase<int64_t>(g->d_ctl, parity, g->blocks, wide, g->stream);
+  return launch_phase<int32_t>(g->d_ctl, parity, g->blocks, wide, g->stream);
 }
 
 static fc_status ensure_graph(fc_graph* g) {

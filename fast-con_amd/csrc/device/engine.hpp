@@ -107,7 +107,7 @@ fc_status run_visits(fc_graph* g, int mode, const int32_t* s, const int32_t* t, 
 // One launch of the visit kernel on the control block ctl (which carries the
 // launch parameters); launches alternate parity 0, 1, 0, ...
 template <typename OffT>
-hipError_t launch_phase(VisitCtl* ctl, int parity, int blocks, hipStream_t s);
+hipError_t launch_phase(VisitCtl* ctl, int parity, int blocks, bool wide, hipStream_t s);
 
 // Control block for a run of n queries: s–t queries start directly in their
 // level phase (query i has epoch epoch0 + i), a BFS starts with its reset.

@@ -151,19 +151,20 @@ __device__ __forceinline__ void push_next(Appender<OffT>& a, bool claimed, int32
 // same time: wave 0 colour 0's normal list (with its degree sum and best
 // meeting candidate), wave 1 colour 1's, waves 2 and 3 the two hub lists;
 // after a second barrier every wave writes its entries.
+template <int W>  // waves of the block
 struct BlockShared {
-  uint32_t cnt[2][kWavesPerBlock];
-  unsigned long long mf[2][kWavesPerBlock];
-  unsigned long long best[2][kWavesPerBlock];
-  uint32_t hcnt[2][kWavesPerBlock];
-  unsigned long long hedges[2][kWavesPerBlock];
+  uint32_t cnt[2][W];
+  unsigned long long mf[2][W];
+  unsigned long long best[2][W];
+  uint32_t hcnt[2][W];
+  unsigned long long hedges[2][W];
   uint32_t base[2];
   unsigned long long hbase[2];
 };
-static_assert(kWavesPerBlock >= 4, "one publishing wave per list");
 
-template <typename OffT>
-__device__ __forceinline__ void block_flush(Appender<OffT>& a, int ncol, BlockShared& sh, Ring* nxt0, Ring* nxt1) {
+template <int W, typename OffT>
+__device__ __forceinline__ void block_flush(Appender<OffT>& a, int ncol, BlockShared<W>& sh, Ring* nxt0, Ring* nxt1) {
+  static_assert(W >= 4, "one publishing wave per list");
   const int w = (int)(threadIdx.x >> 6);
   const int lane = lane_id();
   const int own = a.c;  // this wave staged entries of its own colour only
@@ -192,7 +193,7 @@ __device__ __forceinline__ void block_flush(Appender<OffT>& a, int ncol, BlockSh
     if (w < 2) {
       uint32_t tot = 0;
       unsigned long long mft = 0, bt = ~0ull;
-      for (int i = 0; i < kWavesPerBlock; ++i) {
+      for (int i = 0; i < W; ++i) {
         const uint32_t k = sh.cnt[pc][i];
         sh.cnt[pc][i] = tot;
         tot += k;
@@ -205,7 +206,7 @@ __device__ __forceinline__ void block_flush(Appender<OffT>& a, int ncol, BlockSh
     } else {
       uint32_t k = 0;
       unsigned long long e = 0;
-      for (int i = 0; i < kWavesPerBlock; ++i) {
+      for (int i = 0; i < W; ++i) {
         const uint32_t ki = sh.hcnt[pc][i];
         const unsigned long long ei = sh.hedges[pc][i];
         sh.hcnt[pc][i] = k;
@@ -653,8 +654,8 @@ __device__ __forceinline__ int colour_split(double e0, double e1, int nwaves) {
 // the levels and parents), and block 0 seeds the root.
 template <typename OffT>
 __device__ void bfs_reset(const VisitParams<OffT>& p, const VisitState& S, VisitState* nxt, int32_t* parent) {
-  const int64_t gtid = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  const int64_t nthr = (int64_t)gridDim.x * kBlock;
+  const int64_t gtid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t nthr = (int64_t)gridDim.x * blockDim.x;
   const uint32_t nwords = (((uint32_t)p.V + 63u) >> 6) * 2u;
   const int32_t src = S.src;
   if (!p.lazy_state) {
@@ -704,12 +705,13 @@ __device__ void bfs_reset(const VisitParams<OffT>& p, const VisitState& S, Visit
   *nxt = n;
 }
 
-template <typename OffT>
-__global__ __launch_bounds__(kBlock) void phase_kernel(VisitCtl* ctl, int parity) {
+// W: waves of a block (W or kWideWaves)
+template <typename OffT, int W>
+__global__ __launch_bounds__(W * kWave) void phase_kernel(VisitCtl* ctl, int parity) {
   __shared__ VisitCtl h;
-  __shared__ int32_t s_stage[kWavesPerBlock * kStageCap];
-  __shared__ int32_t s_hub[2][kWavesPerBlock * kHubStage];
-  __shared__ BlockShared s_sh;
+  __shared__ int32_t s_stage[W * kStageCap];
+  __shared__ int32_t s_hub[2][W * kHubStage];
+  __shared__ BlockShared<W> s_sh;
   __shared__ OffT s_root[4];
   static_assert(sizeof(VisitCtl) == kWave * sizeof(uint4), "one 16-byte load per lane");
   if (threadIdx.x < kWave)
@@ -789,10 +791,10 @@ __global__ __launch_bounds__(kBlock) void phase_kernel(VisitCtl* ctl, int parity
     }
   }
 
-  const int64_t gtid = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  const int64_t nthr = (int64_t)gridDim.x * kBlock;
-  const int gwave = (int)(blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6));
-  const int nwaves = (int)(gridDim.x * kWavesPerBlock);
+  const int64_t gtid = (int64_t)blockIdx.x * (W * kWave) + threadIdx.x;
+  const int64_t nthr = (int64_t)gridDim.x * (W * kWave);
+  const int gwave = (int)(blockIdx.x * W + (threadIdx.x >> 6));
+  const int nwaves = (int)(gridDim.x * W);
   int strat = kTopDown;
   int vw0 = 4, vw1 = 4;
   if (start) {
@@ -943,7 +945,7 @@ __global__ __launch_bounds__(kBlock) void st_team_kernel(StTeamRun tr) {
   const VisitParams<OffT>& p = *(const VisitParams<OffT>*)((params_ptr)(uintptr_t)tr.params + xcc_id());
   __shared__ int32_t s_stage[kWavesPerBlock * kStageCap];
   __shared__ int32_t s_hub[2][kWavesPerBlock * kHubStage];
-  __shared__ BlockShared s_sh;
+  __shared__ BlockShared<kWavesPerBlock> s_sh;
   __shared__ OffT s_root[4];
   __shared__ unsigned long long s_now[7];  // the level's rings and the best candidate of the last level
   __shared__ int s_num, s_size, s_q, s_ok;
@@ -1650,20 +1652,27 @@ template int narrow_occupancy<int32_t>();
 template int narrow_occupancy<int64_t>();
 
 template <typename OffT>
-hipError_t launch_phase(VisitCtl* ctl, int parity, int blocks, hipStream_t s) {
-  hipLaunchKernelGGL(phase_kernel<OffT>, dim3(blocks), dim3(kBlock), 0, s, ctl, parity);
+hipError_t launch_phase(VisitCtl* ctl, int parity, int blocks, bool wide, hipStream_t s) {
+  if (wide)
+    hipLaunchKernelGGL((phase_kernel<OffT, kWideWaves>), dim3((blocks * kWavesPerBlock + kWideWaves - 1) / kWideWaves),
+                       dim3(kWideWaves * kWave), 0, s, ctl, parity);
+  else
+    hipLaunchKernelGGL((phase_kernel<OffT, kWavesPerBlock>), dim3(blocks), dim3(kBlock), 0, s, ctl, parity);
   return hipGetLastError();
 }
 
 template <typename OffT>
 int phase_occupancy() {
-  int nb = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, phase_kernel<OffT>, kBlock, 0) != hipSuccess) return 0;
-  return nb;
+  int nb = 0, wide = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, phase_kernel<OffT, kWavesPerBlock>, kBlock, 0) != hipSuccess ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&wide, phase_kernel<OffT, kWideWaves>, kWideWaves * kWave, 0) !=
+          hipSuccess)
+    return 0;
+  return wide < 1 ? 0 : nb;
 }
 
-template hipError_t launch_phase<int32_t>(VisitCtl*, int, int, hipStream_t);
-template hipError_t launch_phase<int64_t>(VisitCtl*, int, int, hipStream_t);
+template hipError_t launch_phase<int32_t>(VisitCtl*, int, int, bool, hipStream_t);
+template hipError_t launch_phase<int64_t>(VisitCtl*, int, int, bool, hipStream_t);
 template int phase_occupancy<int32_t>();
 template int phase_occupancy<int64_t>();
 
