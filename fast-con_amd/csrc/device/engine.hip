@@ -93,6 +93,7 @@ static VisitParams<OffT> make_params(fc_graph* g) {
   set_param(p.out, g->d_out);
   p.lazy_state = g->relabeled ? 1 : 0;
   p.v_active = (int32_t)g->v_active;
+  set_param(p.head, g->d_head);
   return p;
 }
 
@@ -448,6 +449,18 @@ __device__ __forceinline__ unsigned long long edge_hash(uint32_t a, uint32_t b) 
   return z ^ (z >> 31);
 }
 
+// Each vertex's first two columns side by side (VisitParams::head).
+template <typename OffT>
+__global__ __launch_bounds__(256) void head_kernel(const OffT* __restrict__ off, const int32_t* __restrict__ col,
+                                                   int64_t V, unsigned long long* __restrict__ head) {
+  const int64_t n = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < V; v += n) {
+    const OffT b = off[v], d = off[v + 1] - b;
+    const uint32_t u0 = d > 0 ? (uint32_t)col[b] : 0xffffffffu, u1 = d > 1 ? (uint32_t)col[b + 1] : 0xffffffffu;
+    head[v] = ((unsigned long long)u1 << 32) | u0;
+  }
+}
+
 template <typename OffT>
 __global__ __launch_bounds__(256) void symmetry_kernel(const OffT* __restrict__ off, const int32_t* __restrict__ col,
                                                        int64_t V, int64_t E, unsigned long long* __restrict__ out) {
@@ -646,6 +659,14 @@ static fc_status graph_create(const OffT* off, const int32_t* col, int64_t V, in
   CK(hipMalloc((void**)&g->d_mlp, 2 * sizeof(float) * fcd::kMlpParams));
   CK(hipMemsetAsync(g->d_mlp, 0, 2 * sizeof(float) * fcd::kMlpParams, g->stream));
   CK(hipHostMalloc((void**)&g->h_phase, 4 * sizeof(int32_t), hipHostMallocDefault));
+  if (hipMalloc((void**)&g->d_head, sizeof(unsigned long long) * (size_t)std::max<int64_t>(V, 1)) == hipSuccess) {
+    hipLaunchKernelGGL(fcd::head_kernel<OffT>, dim3(g->cus * 8), dim3(256), 0, g->stream, (const OffT*)g->d_off, g->d_col, V,
+                       g->d_head);
+    CK(hipGetLastError());
+  } else {
+    (void)hipGetLastError();  // a bottom-up level does without
+    g->d_head = nullptr;
+  }
   // the sum lands in the parameters' buffer, which is still unused
   hipLaunchKernelGGL(fcd::symmetry_kernel<OffT>, dim3(g->cus * 8), dim3(256), 0, g->stream, (const OffT*)g->d_off,
                      g->d_col, V, E, (unsigned long long*)g->d_mlp);
@@ -699,6 +720,7 @@ extern "C" fc_status fc_graph_destroy(fc_graph* g) {
   (void)hipFree(g->d_mlp);
   (void)hipFree(g->d_ws);
   (void)hipFree(g->d_col);
+  (void)hipFree(g->d_head);
   (void)hipFree(g->d_off);
   (void)hipFree(g->d_perm);
   (void)hipFree(g->d_iperm);

@@ -26,6 +26,7 @@ struct fc_graph {
   bool off64 = false;
   void* d_off = nullptr;
   int32_t* d_col = nullptr;
+  unsigned long long* d_head = nullptr;  // VisitParams::head
   int cus = 0;
   int blocks = 0;               // cooperative grid of the visit kernel
   int32_t hub_threshold = 4096;

@@ -130,6 +130,8 @@ struct VisitParams {
   int32_t lazy_state;       // BFS leaves unreached state/parent unwritten (renumbered graphs:
                             // the un-permutation takes reached-ness from the visited bitmap)
   int32_t v_active;         // vertices [0, v_active) have degree > 0 (the rest are isolated)
+  FC_GLOBAL const unsigned long long* head;  // each vertex's first two columns (the second in the upper half), -1
+                                             // where there is none; null: not kept
 };
 
 // Control block: 1 KB, loaded whole by every block at the start of a launch

@@ -324,3 +324,24 @@ def test_plain_counters_equal_oracle_work(fc, orc):
                     assert st["expanded_vertices"] <= vx and st["expanded_edges"] <= ex, f"{name} pair {i}"
         say(f"{name}: counters checked on {conn_seen} connected and {unconn_seen} unconnected pairs")
         assert conn_seen > 0
+
+
+@pytest.mark.parametrize("name", ["degrees", "degrees-unsorted", "wide"])
+def test_bfs_bottom_up_heads(fc, orc, name):
+    rng = np.random.default_rng(41)
+    if name == "wide":  # at least 2^22 edges: wide launch blocks
+        hg = fc.gen_er(540000, 8.0, 6)
+        assert hg.E >= 1 << 22
+    else:  # degrees around the heads' two, the first round's eight and a lane's 128, and isolated vertices
+        deg = np.tile([0, 1, 2, 3, 7, 8, 9, 10, 11, 127, 128, 129, 130, 300], 80)
+        u = np.repeat(np.arange(len(deg)), deg)
+        e = np.stack([u, rng.integers(0, len(deg), len(u))], 1)
+        e = e[deg[e[:, 1]] > 0]
+        e = np.unique(np.concatenate([e, e[:, ::-1]]), axis=0)
+        off = np.concatenate([[0], np.cumsum(np.bincount(e[:, 0], minlength=len(deg)))])
+        hg = fc.HostGraph(off, e[:, 1].astype(np.int32))
+    kinds = [{}, {"force64": True}] if name != "degrees-unsorted" else [{"keep_order": True}, {"keep_ids": True}]
+    for kind in kinds:
+        with fc.Graph(hg, **kind) as g:
+            _bfs_check(fc, orc, name, hg, g, hg.sample_roots(3, 5))
+            assert g.bfs(int(hg.sample_roots(1, 5)[0]))[2]["bottomup_levels"] > 0
