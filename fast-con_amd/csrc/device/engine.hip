@@ -49,16 +49,13 @@ fc_status ensure_queries(fc_graph* g, int32_t n) {
   // are rewritten by every run, so the graph stays valid
   (void)hipFree(g->d_qs);
   (void)hipFree(g->d_qt);
-  (void)hipFree(g->d_out);
   if (g->h_out) (void)hipHostFree(g->h_out);
   g->d_qs = g->d_qt = nullptr;
-  g->d_out = nullptr;
   g->h_out = nullptr;
   g->q_cap = 0;
   const int32_t cap = std::max<int32_t>(n, 1024);
   FC_HIP(hipMalloc((void**)&g->d_qs, sizeof(int32_t) * (size_t)cap));
   FC_HIP(hipMalloc((void**)&g->d_qt, sizeof(int32_t) * (size_t)cap));
-  FC_HIP(hipMalloc((void**)&g->d_out, sizeof(VisitOut) * (size_t)cap));
   FC_HIP(hipHostMalloc((void**)&g->h_out, sizeof(VisitOut) * (size_t)cap, hipHostMallocDefault));
   g->q_cap = cap;
   return FC_OK;
@@ -90,7 +87,7 @@ static VisitParams<OffT> make_params(fc_graph* g) {
   set_param(p.ctl, g->d_ctl);
   set_param(p.qs, g->d_qs);
   set_param(p.qt, g->d_qt);
-  set_param(p.out, g->d_out);
+  set_param(p.out, g->h_out);
   p.lazy_state = g->relabeled ? 1 : 0;
   p.v_active = (int32_t)g->v_active;
   set_param(p.head, g->d_head);
@@ -179,13 +176,12 @@ static fc_status st_teams_alloc(fc_graph* g) {
 }
 
 // Whether n queries go to the teams: several always (eight are visited at a
-// time: R-MAT s22, 16 queries, 0.42 -> 0.22 ms, two 41 -> 35 us); a single one
-// when one XCD expands its levels as fast as a launch of the whole GPU does
-// (s16, 1.8M edges: 20 us both ways, and 58 against 107 us with the host's
-// share), which is not expected of a skewed graph of more than 2^23 edges.
-static bool st_teams_take(const fc_graph* g, int32_t n) {
-  return g->use_st_teams && (n > 1 || !g->hub_steps || g->E <= (1 << 23));
-}
+// time: R-MAT s22, 16 queries, 0.42 -> 0.23 ms); a single one where its
+// frontiers are likely to stay narrow (random graph of 50K vertices and degree
+// 3, 53 against 68 us a call, 100^2 grid 160 against 341), since a few wide
+// levels take the whole GPU no longer (s16 47 us against 53, the random graph
+// with degree 8 45 against 49).
+static bool st_teams_take(const fc_graph* g, int32_t n) { return g->use_st_teams && (n > 1 || g->narrow); }
 
 // Levels (and parents) of a narrow BFS in caller ids, from the state words of
 // the machine that ran it (out->meet).
@@ -208,12 +204,57 @@ __global__ void narrow_levels_kernel(const int32_t* __restrict__ perm, const int
   }
 }
 
+// What a launch by teams starts from, written by one small launch before it: a
+// block per machine clears the machine's words and writes its parameters (those
+// of machine 0, its workspace moved by the stride). As an upload from pinned
+// memory, 40 KB, it took 10 us of a query's 58.
+constexpr int kStartThreads = 256;
+template <typename Params>
+struct TeamStart {
+  Params prm;
+  int32_t s[kStartPairs], t[kStartPairs];
+};
+template <typename T>
+__device__ __forceinline__ void clear_words(T* p) {
+  static_assert(sizeof(T) % sizeof(uint4) == 0, "16 bytes a store");
+  for (uint32_t i = threadIdx.x; i < sizeof(T) / sizeof(uint4); i += kStartThreads)
+    reinterpret_cast<uint4*>(p)[i] = make_uint4(0, 0, 0, 0);
+}
+template <typename Params>
+__global__ __launch_bounds__(kStartThreads) void team_start_kernel(const TeamStart<Params> v, StTeamRun tr, size_t stride,
+                                                                   int32_t* qs, int32_t* qt, int n) {
+  const int k = (int)blockIdx.x;
+  clear_words(tr.sync + k);
+  clear_words(tr.bar + k);
+  clear_words(tr.ctl + k);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (auto& b : tr.ctl[k].best) b[0] = b[1] = ~0ull;
+    if (k == 0) *tr.ticket = 0;
+    Params p = v.prm;
+    const size_t by = (size_t)k * stride;
+    set_param(p.sst, (unsigned long long*)((char*)p.sst + by));
+    for (int c = 0; c < 2; ++c)
+      for (int r = 0; r < 2; ++r) {
+        set_param(p.q[c][r], (int32_t*)((char*)p.q[c][r] + by));
+        set_param(p.hq[c][r], (int32_t*)((char*)p.hq[c][r] + by));
+        set_param(p.hb[c][r], (int64_t*)((char*)p.hb[c][r] + by));
+      }
+    set_param(p.ctl, &tr.ctl[k].v);
+    ((Params*)tr.params)[k] = p;
+  }
+  if (k == 0 && (int)threadIdx.x < n) {
+    qs[threadIdx.x] = v.s[threadIdx.x];
+    qt[threadIdx.x] = v.t[threadIdx.x];
+  }
+}
+
 // Run n plain s–t queries by teams (narrow: as narrow visits), or with bfs one
 // BFS from s[0] as a narrow visit, whose levels (and, with par_out, parents)
 // go to lv_out; results in g->h_out. *ran is false when the teams are not
 // available for this graph.
 static fc_status st_teams_run(fc_graph* g, const int32_t* s, const int32_t* t, int32_t n, bool narrow, bool bfs,
-                              int32_t* lv_out, int32_t* par_out, double* ms, bool* ran) {
+                              int32_t* lv_out, int32_t* par_out, double* ms, bool* ran, const VisitTail& after = {}) {
   *ran = false;
   fc_status st = st_teams_alloc(g);
   if (st != FC_OK) return st;
@@ -239,16 +280,13 @@ static fc_status st_teams_run(fc_graph* g, const int32_t* s, const int32_t* t, i
     FC_HIP(hipHostMalloc((void**)&w->h_io, cap, hipHostMallocDefault));
     w->io_bytes = cap;
   }
-  std::memset(w->h_io, 0, o_qs);
-  std::memset(w->h_io + o_err, 0, o_out - o_err);
-  std::memcpy(w->h_io + o_qs, s, 4 * (size_t)n);
-  std::memcpy(w->h_io + o_qt, t, 4 * (size_t)n);
+  *(uint32_t*)(w->h_io + o_err) = 0;
   StTeamRun tr;
   tr.sync = (TeamSync*)w->d_io;
   tr.bar = (TeamBar*)(w->d_io + o_bar);
   tr.ctl = (StTeamCtl*)(w->d_io + o_ctl);
   tr.ticket = (uint32_t*)(w->d_io + o_tick);
-  tr.err = (uint32_t*)(w->d_io + o_err);
+  tr.err = (uint32_t*)(w->h_io + o_err);
   tr.params = w->d_io + o_par;
   tr.nq = n;
   tr.epoch0 = w->epoch_next;
@@ -261,30 +299,35 @@ static fc_status st_teams_run(fc_graph* g, const int32_t* s, const int32_t* t, i
   tr.expected = (uint32_t)(blocks / kXcds);
   tr.parents = par_out != nullptr;
   w->epoch_next += (uint32_t)n;
-  auto machine = [&](auto prm, int k) {
-    char* m = w->mem + (size_t)k * w->stride;
-    set_param(prm.sst, (unsigned long long*)m);
+  const int few = n <= kStartPairs ? n : 0;
+  if (!few) {
+    std::memcpy(w->h_io + o_qs, s, 4 * (size_t)n);
+    std::memcpy(w->h_io + o_qt, t, 4 * (size_t)n);
+    FC_HIP(hipMemcpyAsync(w->d_io + o_qs, w->h_io + o_qs, o_err - o_qs, hipMemcpyHostToDevice, g->stream));
+  }
+  auto start = [&](auto prm) {
+    TeamStart<decltype(prm)> v;
     for (int c = 0; c < 2; ++c)
       for (int r = 0; r < 2; ++r) {
-        const size_t i = (size_t)(2 * c + r);
-        set_param(prm.q[c][r], (int32_t*)(m + w->o_q + i * w->q1));
-        set_param(prm.hq[c][r], (int32_t*)(m + w->o_hq + i * w->hq1));
-        set_param(prm.hb[c][r], (int64_t*)(m + w->o_hb + i * w->hb1));
+        const size_t k = (size_t)(2 * c + r);
+        set_param(prm.q[c][r], (int32_t*)(w->mem + w->o_q + k * w->q1));
+        set_param(prm.hq[c][r], (int32_t*)(w->mem + w->o_hq + k * w->hq1));
+        set_param(prm.hb[c][r], (int64_t*)(w->mem + w->o_hb + k * w->hb1));
       }
-    set_param(prm.ctl, &tr.ctl[k].v);
+    set_param(prm.sst, (unsigned long long*)w->mem);
     set_param(prm.qs, (const int32_t*)(w->d_io + o_qs));
     set_param(prm.qt, (const int32_t*)(w->d_io + o_qt));
-    set_param(prm.out, (VisitOut*)(w->d_io + o_out));
-    std::memcpy(w->h_io + o_par + (size_t)k * sizeof(prm), &prm, sizeof(prm));
-    for (auto& b : ((StTeamCtl*)(w->h_io + o_ctl))[k].best) b[0] = b[1] = ~0ull;
+    set_param(prm.out, (VisitOut*)((bfs ? w->d_io : w->h_io) + o_out));  // a BFS's is read on the device too
+    v.prm = prm;
+    for (int i = 0; i < kStartPairs; ++i) {
+      v.s[i] = i < few ? s[i] : 0;
+      v.t[i] = i < few ? t[i] : 0;
+    }
+    hipLaunchKernelGGL(team_start_kernel<decltype(prm)>, dim3(kXcds), dim3(kStartThreads), 0, g->stream, v, tr, w->stride,
+                       (int32_t*)(w->d_io + o_qs), (int32_t*)(w->d_io + o_qt), few);
+    return hipGetLastError();
   };
-  for (int k = 0; k < kXcds; ++k) {
-    if (g->off64)
-      machine(make_params<int64_t>(g), k);
-    else
-      machine(make_params<int32_t>(g), k);
-  }
-  FC_HIP(hipMemcpyAsync(w->d_io, w->h_io, o_out, hipMemcpyHostToDevice, g->stream));
+  FC_HIP(g->off64 ? start(make_params<int64_t>(g)) : start(make_params<int32_t>(g)));
   FC_HIP(hipEventRecord(g->ev0, g->stream));
   if (narrow)
     FC_HIP(g->off64 ? launch_narrow<int64_t>(tr, bfs, blocks, g->stream)
@@ -299,12 +342,15 @@ static fc_status st_teams_run(fc_graph* g, const int32_t* s, const int32_t* t, i
     FC_HIP(hipGetLastError());
   }
   FC_HIP(hipEventRecord(g->ev1, g->stream));
-  FC_HIP(hipMemcpyAsync(w->h_io + o_err, w->d_io + o_err, bytes - o_err, hipMemcpyDeviceToHost, g->stream));
+  if (bfs) {
+    FC_HIP(hipMemcpyAsync(w->h_io + o_out, w->d_io + o_out, sizeof(VisitOut), hipMemcpyDeviceToHost, g->stream));
+    if (after) FC_HIP(after());
+  }
   FC_HIP(hipStreamSynchronize(g->stream));
   float fms = 0.f;
   FC_HIP(hipEventElapsedTime(&fms, g->ev0, g->ev1));
   *ms = fms;
-  if (*(const uint32_t*)(w->h_io + o_err)) {
+  if (*(const volatile uint32_t*)(w->h_io + o_err)) {
     // queues and counters are in an unknown state: the next run takes new ones
     st_teams_free(w);
     g->st_teams = nullptr;
@@ -316,8 +362,25 @@ static fc_status st_teams_run(fc_graph* g, const int32_t* s, const int32_t* t, i
   return FC_OK;
 }
 
+// A run's control block and, of a few queries, their ends, as kernel arguments:
+// one launch instead of three copies from pageable memory and the wait for
+// them (25 us before the first level).
+struct VisitStart {
+  VisitCtl ctl;
+  int32_t s[kStartPairs], t[kStartPairs];
+};
+__global__ __launch_bounds__(kWave) void visit_start_kernel(const VisitStart v, VisitCtl* ctl, int32_t* qs,
+                                                            int32_t* qt, int n) {
+  const int i = (int)threadIdx.x;
+  reinterpret_cast<uint4*>(ctl)[i] = reinterpret_cast<const uint4*>(&v.ctl)[i];
+  if (i < n) {
+    qs[i] = v.s[i];
+    qt[i] = v.t[i];
+  }
+}
+
 fc_status run_visits(fc_graph* g, int mode, const int32_t* s, const int32_t* t, int32_t n, bool parents,
-                     double* ms) {
+                     double* ms, const VisitTail& tail, const VisitTail& after) {
   *ms = 0.0;
   if (n <= 0) return FC_OK;
   fc_status st = ensure_queries(g, n);
@@ -366,14 +429,27 @@ fc_status run_visits(fc_graph* g, int mode, const int32_t* s, const int32_t* t, 
     epoch0 = g->epoch_next;
     g->epoch_next += (uint32_t)n;
   }
-  FC_HIP(hipMemcpyAsync(g->d_qs, s, sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice, g->stream));
-  FC_HIP(hipMemcpyAsync(g->d_qt, t, sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice, g->stream));
-  const VisitCtl init = g->off64 ? visit_init(make_params<int64_t>(g), mode, n, s, t, epoch0, g->vw_fixed, parents)
-                                 : visit_init(make_params<int32_t>(g), mode, n, s, t, epoch0, g->vw_fixed, parents);
-  FC_HIP(hipMemcpyAsync(g->d_ctl, &init, sizeof(init), hipMemcpyHostToDevice, g->stream));
-  // The async copies above read pageable host memory: finish them before the
-  // caller's arrays can go away, and before timing starts.
-  FC_HIP(hipStreamSynchronize(g->stream));
+  VisitStart init;
+  init.ctl = g->off64 ? visit_init(make_params<int64_t>(g), mode, n, s, t, epoch0, g->vw_fixed, parents)
+                      : visit_init(make_params<int32_t>(g), mode, n, s, t, epoch0, g->vw_fixed, parents);
+  const int few = n <= kStartPairs ? n : 0;
+  for (int i = 0; i < kStartPairs; ++i) {
+    init.s[i] = i < few ? s[i] : 0;
+    init.t[i] = i < few ? t[i] : 0;
+  }
+  if (!few) {
+    FC_HIP(hipMemcpyAsync(g->d_qs, s, sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice, g->stream));
+    FC_HIP(hipMemcpyAsync(g->d_qt, t, sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice, g->stream));
+    // pageable host memory: finish the copies before the caller's arrays can
+    // go away, and before timing starts
+    FC_HIP(hipStreamSynchronize(g->stream));
+  }
+  hipLaunchKernelGGL(visit_start_kernel, dim3(1), dim3(kWave), 0, g->stream, init, g->d_ctl, g->d_qs, g->d_qt, few);
+  FC_HIP(hipGetLastError());
+  // the launches write a query's result here when it is finished
+  constexpr int32_t kRunning = INT32_MIN;
+  volatile VisitOut* const out = g->h_out;
+  for (int32_t i = 0; i < n; ++i) out[i].status = kRunning;
 
   // Launch budget: the running estimate of working launches per query, plus
   // the launch that notices the last query's end. A single BFS needs no
@@ -388,6 +464,7 @@ fc_status run_visits(fc_graph* g, int mode, const int32_t* s, const int32_t* t, 
   const double est = g->est_launches[mode];
   int64_t expected = (int64_t)std::ceil((double)n * est) + 1;
   int64_t launched = 0;
+  int32_t qi = 0;  // queries finished
   FC_HIP(hipEventRecord(g->ev0, g->stream));
   for (int round = 0;; ++round) {
     int64_t want = expected - launched;
@@ -410,13 +487,12 @@ fc_status run_visits(fc_graph* g, int mode, const int32_t* s, const int32_t* t, 
       for (int64_t i = 0; i < ng; ++i) FC_HIP(hipGraphLaunch(g->gexec, g->stream));
       launched += ng * kGraphLaunches;
     }
+    if (tail) FC_HIP(tail());
     FC_HIP(hipEventRecord(g->ev1, g->stream));
-    // the state the next launch would read
-    FC_HIP(hipMemcpyAsync(g->h_phase, &g->d_ctl->st[launched & 1], 2 * sizeof(int32_t), hipMemcpyDeviceToHost,
-                          g->stream));
+    if (after) FC_HIP(after());
     FC_HIP(hipStreamSynchronize(g->stream));
-    const int32_t phase = g->h_phase[0], qi = g->h_phase[1];
-    if (phase == kPhaseIdle) break;
+    while (qi < n && out[qi].status != kRunning) ++qi;
+    if (qi == n) break;
     // Every query stops within V+2 levels (device guard), so this bound is
     // never reached by a working visit.
     if (launched > (int64_t)n * (g->V + 4) + 64)
@@ -430,8 +506,6 @@ fc_status run_visits(fc_graph* g, int mode, const int32_t* s, const int32_t* t, 
   float fms = 0.f;
   FC_HIP(hipEventElapsedTime(&fms, g->ev0, g->ev1));
   *ms = fms;
-  FC_HIP(hipMemcpyAsync(g->h_out, g->d_out, sizeof(VisitOut) * (size_t)n, hipMemcpyDeviceToHost, g->stream));
-  FC_HIP(hipStreamSynchronize(g->stream));
   double wl = 0;
   for (int32_t i = 0; i < n; ++i) wl += g->h_out[i].launches;
   g->est_launches[mode] = 0.5 * g->est_launches[mode] + 0.5 * (wl / n);
@@ -716,7 +790,7 @@ extern "C" fc_status fc_graph_destroy(fc_graph* g) {
   if (g->h_phase) (void)hipHostFree(g->h_phase);
   (void)hipFree(g->d_qs);
   (void)hipFree(g->d_qt);
-  (void)hipFree(g->d_out);
+  if (g->h_stage) (void)hipHostFree(g->h_stage);
   (void)hipFree(g->d_mlp);
   (void)hipFree(g->d_ws);
   (void)hipFree(g->d_col);
@@ -794,11 +868,31 @@ extern "C" fc_status fc_bfs(fc_graph* g, int32_t src, int32_t* levels_out, int32
   if (g->relabeled && par && !g->d_par_out) FC_HIP(hipMalloc((void**)&g->d_par_out, bytes));
   int32_t* const lv = g->relabeled ? g->d_lv_out : g->d_state;
   int32_t* const pa = g->relabeled ? g->d_par_out : g->d_parent;
+  // small results come back behind the visit, through pinned memory
+  const int results = (levels_out ? 1 : 0) + (par ? 1 : 0);
+  const bool staged = results > 0 && bytes * (size_t)results <= fcd::kStageBytes;
+  if (staged && !g->h_stage) FC_HIP(hipHostMalloc((void**)&g->h_stage, fcd::kStageBytes, hipHostMallocDefault));
+  fcd::VisitTail tail, after;
+  if (g->relabeled)  // the results in caller ids are part of the BFS: timed with it
+    tail = [&]() {
+      const int blocks = (int)std::min<int64_t>((g->V + 255) / 256, (int64_t)g->cus * 8);
+      hipLaunchKernelGGL(unpermute_kernel, dim3(blocks), dim3(256), 0, g->stream, g->d_perm, g->d_iperm, g->d_visited,
+                         g->d_state, par ? g->d_parent : nullptr, g->d_lv_out, g->d_par_out, (int64_t)g->V);
+      return hipGetLastError();
+    };
+  if (staged)
+    after = [&]() {
+      hipError_t e = hipSuccess;
+      if (levels_out) e = hipMemcpyAsync(g->h_stage, lv, bytes, hipMemcpyDeviceToHost, g->stream);
+      if (par && e == hipSuccess)
+        e = hipMemcpyAsync(g->h_stage + (levels_out ? bytes : 0), pa, bytes, hipMemcpyDeviceToHost, g->stream);
+      return e;
+    };
   bool narrow = false;
   fc_status st;
   if (g->use_st_teams && g->narrow && g->narrow_bfs) {
     if ((st = fcd::ensure_queries(g, 1)) != FC_OK) return st;
-    st = fcd::st_teams_run(g, &dsrc, &none, 1, true, true, lv, par ? pa : nullptr, &ms, &narrow);
+    st = fcd::st_teams_run(g, &dsrc, &none, 1, true, true, lv, par ? pa : nullptr, &ms, &narrow, after);
     if (st != FC_OK) return st;
     if (narrow && g->h_out[0].status == fcd::kTooWide) {
       narrow = g->narrow_bfs = false;
@@ -806,32 +900,24 @@ extern "C" fc_status fc_bfs(fc_graph* g, int32_t src, int32_t* levels_out, int32
     }
   }
   if (!narrow) {
-    st = fcd::run_visits(g, fcd::kModeBfs, &dsrc, &none, 1, par, &ms);
+    st = fcd::run_visits(g, fcd::kModeBfs, &dsrc, &none, 1, par, &ms, tail, after);
     if (st != FC_OK) return st;
     ms += tried;
   }
   const fcd::VisitOut o = g->h_out[0];
   st = check_out(o);
   if (st != FC_OK) return st;
-  if (!narrow && g->relabeled) {
-    // the results in caller ids are part of the BFS: timed with it
-    FC_HIP(hipEventRecord(g->ev0, g->stream));
-    const int blocks = (int)std::min<int64_t>((g->V + 255) / 256, (int64_t)g->cus * 8);
-    hipLaunchKernelGGL(unpermute_kernel, dim3(blocks), dim3(256), 0, g->stream, g->d_perm, g->d_iperm, g->d_visited,
-                       g->d_state, par ? g->d_parent : nullptr, g->d_lv_out, g->d_par_out, (int64_t)g->V);
-    FC_HIP(hipGetLastError());
-    FC_HIP(hipEventRecord(g->ev1, g->stream));
-    FC_HIP(hipEventSynchronize(g->ev1));
-    float fms = 0.f;
-    FC_HIP(hipEventElapsedTime(&fms, g->ev0, g->ev1));
-    ms += fms;
-  }
   g->levels_valid = true;
   g->parents_valid = par;
   if (stats) {
     std::memset(stats, 0, sizeof(*stats));
     stats->time_ms = ms;
     add_stats(o, stats);
+  }
+  if (staged) {
+    if (levels_out) std::memcpy(levels_out, g->h_stage, bytes);
+    if (parents_out) std::memcpy(parents_out, g->h_stage + (levels_out ? bytes : 0), bytes);
+    return FC_OK;
   }
   if (levels_out) FC_HIP(read_back(levels_out, lv, bytes, g));
   if (parents_out) FC_HIP(read_back(parents_out, pa, bytes, g));

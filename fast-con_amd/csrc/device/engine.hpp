@@ -2,6 +2,7 @@
 // stream, and all per-query workspace, allocated once at creation.
 #pragma once
 
+#include <functional>
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -54,10 +55,10 @@ struct fc_graph {
   // host copy of the results; capacity q_cap.
   int32_t* d_qs = nullptr;
   int32_t* d_qt = nullptr;
-  fcd::VisitOut* d_out = nullptr;
-  fcd::VisitOut* h_out = nullptr;
+  fcd::VisitOut* h_out = nullptr;   // pinned; the visits' launches write it
+  char* h_stage = nullptr;          // pinned: small read-backs (kStageBytes)
   int32_t q_cap = 0;
-  int32_t* h_phase = nullptr;       // pinned: phase + qi read back between batches
+  int32_t* h_phase = nullptr;       // pinned: small words read back
   // Captured hipGraph of kGraphLaunches identical phase launches.
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
@@ -101,9 +102,14 @@ fc_status hip_fail(hipError_t e, const char* what);
 fc_status ensure_queries(fc_graph* g, int32_t n);
 
 // Run n visits through the phase machine (s[i], t[i]; t = -1 for BFS) and
-// leave their results in g->h_out[0..n). *ms receives the device time.
+// leave their results in g->h_out[0..n). *ms receives the device time. tail:
+// work to queue behind the visits, part of that time (and queued again if they
+// needed more launches than expected); after: read-backs behind that.
+typedef std::function<hipError_t()> VisitTail;
 fc_status run_visits(fc_graph* g, int mode, const int32_t* s, const int32_t* t, int32_t n, bool parents,
-                     double* ms);
+                     double* ms, const VisitTail& tail = {}, const VisitTail& after = {});
+constexpr size_t kStageBytes = 1u << 20;
+constexpr int kStartPairs = 32;
 
 // One launch of the visit kernel on the control block ctl (which carries the
 // launch parameters); launches alternate parity 0, 1, 0, ...

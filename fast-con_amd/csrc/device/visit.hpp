@@ -97,7 +97,7 @@ static_assert(sizeof(VisitState) == 128, "VisitState layout");
 
 // Host code stores a device pointer into such a field with an explicit cast.
 template <typename F, typename T>
-inline void set_param(F& field, T* v) {
+__host__ __device__ inline void set_param(F& field, T* v) {
   field = (F)v;
 }
 

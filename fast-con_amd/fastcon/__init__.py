@@ -474,10 +474,18 @@ class Graph:
 
     @staticmethod
     def _rows(feats: np.ndarray, cost: np.ndarray):
+        feats, cost = np.asarray(feats), np.asarray(cost)
+        if len(cost) < len(feats):
+            raise IndexError("a cost for every row")
+        cost = cost[: len(feats)]
+        if len(feats) and (feats.shape[1:] != (SCHED_FEATURES,) or cost.shape[1:] != (SCHED_ACTIONS,)):
+            raise ValueError("rows of %d features and %d costs" % (SCHED_FEATURES, SCHED_ACTIONS))
         rows = (TraceRow * len(feats))()
-        for i in range(len(feats)):
-            rows[i].features[:] = [float(x) for x in feats[i]]
-            rows[i].cost_us[:] = [float(x) for x in cost[i]]
+        if len(feats):
+            table = np.frombuffer(rows, dtype=np.dtype(TraceRow))
+            with np.errstate(over="ignore"):
+                table["features"] = feats
+                table["cost_us"] = cost
         return rows
 
     def sched_train(self, feats: np.ndarray, cost: np.ndarray, epochs: int = 2000, lr: float = 3e-3,
