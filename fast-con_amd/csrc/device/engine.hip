@@ -95,7 +95,7 @@ static VisitParams<OffT> make_params(fc_graph* g) {
 }
 
 static hipError_t launch_raw(fc_graph* g, int parity) {
-  const bool wide = g->E >= kWideEdges;
+  const bool wide = g->E >= kWideEdges && !g->narrow;
   if (g->off64) return launch_phase<int64_t>(g->d_ctl, parity, g->blocks, wide, g->stream);
   return launch_phase<int32_t>(g->d_ctl, parity, g->blocks, wide, g->stream);
 }

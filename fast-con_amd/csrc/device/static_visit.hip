@@ -144,7 +144,7 @@ fc_status static_pass(DeviceSlot& slot, const VisitParams<int32_t>& p, int32_t n
   for (int round = 0;; ++round) {
     int64_t want = std::min<int64_t>(std::max<int64_t>(expected - launched, 1), kPollLaunches);
     for (int64_t i = 0; i < want; ++i, ++launched) {
-      hipError_t e = launch_phase<int32_t>(p.ctl, (int)(launched & 1), slot.blocks, p.E >= kWideEdges, nullptr);
+      hipError_t e = launch_phase<int32_t>(p.ctl, (int)(launched & 1), slot.blocks, false, nullptr);
       if (e != hipSuccess) return hip_fail(e, "phase kernel launch");
     }
     int32_t word[2] = {0, 0};
