@@ -1144,10 +1144,9 @@ template int st_team_occupancy<int64_t>();
 //    rest in the frontier lists, from where all waves take their shares
 //    (2048^2 grid, BFS: 15.5 -> 14.4 ms);
 //  * between its arrival at the barrier and the barrier's end, when it would
-//    wait anyway, a wave loads the first columns of these vertices, the state
-//    words and offsets they lead to, and the line of the columns after that. A
-//    word that another wave changes meanwhile is settled by the claim, as
-//    every stale look is;
+//    wait anyway, a wave loads the first columns of these vertices and the
+//    state words and offsets they lead to. A word that another wave changes
+//    meanwhile is settled by the claim, as every stale look is;
 //  * a level ends without an atomic: each block stores a word of its own with
 //    the counts of its claimed vertices, and one wave per block, which does
 //    nothing else, reads the words of all blocks until they carry the level's
@@ -1156,15 +1155,16 @@ template int st_team_occupancy<int64_t>();
 //    sums every block takes the stop decision; the lists' counters and the
 //    best candidate are only read when a block has flagged them.
 // What is left of a level is the claiming atomic, two block-wide steps, a
-// store and the loads that see it: 2.7 us for 2,000 vertices. Measured
-// against one launch (BFS) or st_team_kernel: BFS of a 2048^2 grid 30.4 ->
-// 10.4 ms, eight queries on a 4096^2 grid 22.9 -> 13.3 ms, of 500^2 7.35 ->
-// 2.35 ms. A visit whose frontier reaches kNarrowMax vertices is given up
+// store and the loads that see it: 2.5 us for 2,000 vertices. Measured
+// against one launch a level (BFS) or st_team_kernel: BFS of a 2048^2 grid 30.4
+// -> 9.7 ms, of 500^2 7.35 -> 2.22 ms, eight queries on a 4096^2 grid 22.9 ->
+// 12.3 ms. (Loading a line of the columns after the next as well cost the
+// queries 5%; two kept entries per lane group, which a query's half of the
+// waves needs on grids of 4096^2, cost a BFS 5%.) A visit whose frontier reaches kNarrowMax vertices is given up
 // (kTooWide): the caller runs it on the engine that uses the whole GPU.
 // A BFS is a visit with one colour and no target. Levels, counters and answers
 // are those of the other engines.
 constexpr int kNarrowWaves = kNarrowThreads / kWave;
-constexpr int kSets = 2;                 // kept entries per lane group of four
 constexpr uint32_t kNarrowStage = 256;   // entries a wave stages for publication
 constexpr uint32_t kNarrowSpill = 64;    // and room for what the block gives up
 constexpr uint32_t kNarrowMax = 65535;
@@ -1174,6 +1174,7 @@ constexpr uint32_t kNarrowMax = 65535;
 template <bool BFS>
 struct NarrowSplit {
   static constexpr int kColours = BFS ? 1 : 2, kWorkers = (kNarrowWaves - 1) / kColours;
+  static constexpr int kSets = BFS ? 1 : 2;  // kept entries per lane group of four
   static constexpr uint32_t kKeep = 16u * kSets * kWorkers;
   static_assert(kKeep <= kNarrowSpill * kWorkers, "kNarrowSpill");
 };
@@ -1304,7 +1305,7 @@ __global__ __launch_bounds__(kNarrowThreads) void narrow_kernel(StTeamRun tr) {
   typedef __attribute__((address_space(4))) const VisitParams<OffT>* params_ptr;
   const VisitParams<OffT>& p = *(const VisitParams<OffT>*)((params_ptr)(uintptr_t)tr.params + xcc_id());
   using Split = NarrowSplit<BFS>;
-  constexpr int kColours = Split::kColours, kWorkers = Split::kWorkers;
+  constexpr int kColours = Split::kColours, kWorkers = Split::kWorkers, kSets = Split::kSets;
   __shared__ NarrowKept<OffT, BFS> s_kept[kColours];
   __shared__ int32_t s_stage[kNarrowWaves * (kNarrowStage + kNarrowSpill)];
   __shared__ int32_t s_hub[2][kNarrowWaves * kHubStage];
@@ -1397,9 +1398,8 @@ __global__ __launch_bounds__(kNarrowThreads) void narrow_kernel(StTeamRun tr) {
     uint32_t nf0 = 1, nf1 = BFS ? 0u : 1u, kept = 0;
     unsigned long long best = ~0ull;
     bool look = false;
-    // the first columns of this lane's kept vertices, what they lead to, and
-    // the line of the columns after that
-    int32_t pu[kSets], pt[kSets];
+    // the first columns of this lane's kept vertices and what they lead to
+    int32_t pu[kSets];
     unsigned long long pw[kSets];
     OffT pb[kSets], pe[kSets];
     auto fresh = [&](int32_t u, unsigned long long word) {
@@ -1465,7 +1465,6 @@ __global__ __launch_bounds__(kNarrowThreads) void narrow_kernel(StTeamRun tr) {
             int64_t d;
             const bool cl = probe_done(a, parent, true, L, v, pu[i], pu[i] >= 0, r[i], d);
             push(cl, pu[i], r[i].ob, d);
-            asm volatile("" ::"v"(pt[i]));  // nothing uses the value: the line is in the L2 now
           }
           // and the rest of longer lists
           if (more) {
@@ -1589,11 +1588,6 @@ __global__ __launch_bounds__(kNarrowThreads) void narrow_kernel(StTeamRun tr) {
             pb[i] = o[0];
             pe[i] = o[1];
           }
-        }
-#pragma unroll
-        for (int i = 0; i < kSets; ++i) {
-          pt[i] = 0;
-          if (pu[i] >= 0 && fresh(pu[i], pw[i]) && pb[i] < pe[i]) pt[i] = p.col[pb[i]];
         }
       }
       __syncthreads();
