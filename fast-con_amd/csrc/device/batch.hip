@@ -20,10 +20,10 @@
 // one launch: every XCD's blocks form one or two wave machines that step from
 // phase to phase with a barrier inside the XCD (team.hpp). batch_kernel is one
 // launch per phase over all blocks, for traces, directed graphs, graphs whose
-// machines' workspaces would not fit and callers that ask for lanes. In both
-// the last block to finish a phase decides the next one.
+// machines' workspaces would not fit and callers that ask for lanes. There
+// the last block to finish a phase decides the next one, in a team block 0.
 // Measured (R-MAT s22, 1,024 queries; s24, 16,384 of uneven reach): launches
-// on three lanes 2.06 and 83 ms, teams 0.22 and 8.8 ms: no launch between two
+// on three lanes 2.06 and 77 ms, teams 0.21 and 9.0 ms: no launch between two
 // phases, every wave's state in the L2 of its XCD, narrower waves when there
 // are too few, and hub steps in place of most level-2 expansions.
 // Only the masks a wave touched are cleared afterwards (dirty bitmap), so a

@@ -750,9 +750,10 @@ static fc_status graph_create(const OffT* off, const int32_t* col, int64_t V, in
 
   int occ = sizeof(OffT) == 8 ? fcd::phase_occupancy<int64_t>() : fcd::phase_occupancy<int32_t>();
   if (occ < 1) return bail(fail(FC_ERR_NOGPU, "phase kernel has no occupancy on this device (missing gfx950 code?)"));
-  // 4 resident blocks per CU measured best for BFS and plain s–t at s22
-  // (2: 345, 3: 384, 4: 401, 6: 392, 8: 348 GTEPS): more blocks add
+  // 16 waves per CU, in blocks of four, measured best for BFS and plain s–t at
+  // s22 (8: 345, 12: 384, 16: 401, 24: 392, 32: 348 GTEPS): more blocks add
   // contention on the launch's shared counters more than they hide latency.
+  // Wide graphs run the same waves in larger blocks (kWideWaves).
   int per_cu = std::min(occ, 4);
   const char* bpc = std::getenv("FASTCON_BLOCKS_PER_CU");
   if (bpc && std::atoi(bpc) > 0) per_cu = std::min(occ, std::atoi(bpc));

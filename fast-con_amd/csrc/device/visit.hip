@@ -1,12 +1,20 @@
-// Visit engine for BFS and s–t connectivity on gfx950: one kernel launch per
-// level, driven by a device-side phase machine in VisitCtl.
+// Visit engines for BFS and s–t connectivity on gfx950. Three kernels run the
+// same expansion and claims:
+//  * phase_kernel: one launch per level over the whole GPU, driven by a
+//    device-side phase machine in VisitCtl (BFS of wide frontiers, single
+//    queries, path output);
+//  * st_team_kernel: one launch for a list of plain queries, eight at a time,
+//    one per XCD (team.hpp);
+//  * narrow_kernel: one launch for a BFS or queries whose frontiers stay
+//    narrow over many levels, by one team each.
 //
-// Why launches and not a persistent kernel: on MI355X a grid-wide software
+// Why launches where the whole GPU works on a level: a grid-wide software
 // barrier with the agent-scope release/acquire that cross-XCD visibility
 // needs costs 16-35 us, a cooperative launch ~20 us, while a back-to-back
 // ordinary launch costs ~2.4 us (1.6 us inside a hipGraph) and its boundary
-// already orders every block's writes. So each launch does one level with
-// all blocks. This replaces the reference's host-driven level loop with a
+// already orders every block's writes. Inside one XCD a barrier costs 0.6 us,
+// which is what the other two build on. The launch per level replaces the
+// reference's host-driven level loop with a
 // 16-byte readback per level (BFS-4K/src/device/BFS_WorkEfficient.cu:81-118)
 // and ST-CON's ~12 host round trips per level (st-conn/make_stcon.c:968-1187).
 //

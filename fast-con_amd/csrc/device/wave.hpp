@@ -5,8 +5,9 @@
 // and its warp-aggregated frontier reservation (BFS-4K/src/device/Util/GlobalWrite.cu:13-46).
 // On CDNA a wave has 64 lanes, so ballots are 64-bit and ranks come from
 // v_mbcnt_lo/hi. The reference's software grid barrier
-// (BFS-4K/src/device/Util/GlobalSync.cu:5-36) has no counterpart: levels are
-// separated by kernel launches (see visit.hip).
+// (BFS-4K/src/device/Util/GlobalSync.cu:5-36) has no counterpart over the whole
+// GPU, whose levels are separate launches (visit.hip); inside one XCD team.hpp
+// has barriers.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -204,7 +204,7 @@ fc_status fc_bfs(fc_graph* g, int32_t src, int32_t* levels_out, int32_t* parents
 fc_status fc_graph_levels(fc_graph* g, int32_t* levels_out);
 fc_status fc_graph_parents(fc_graph* g, int32_t* parents_out);
 
-/* Plain s–t connectivity: one query per launch, two colours, one atomicCAS
+/* Plain s–t connectivity: a visit per query, two colours, one atomicCAS
  * per vertex, both frontiers expanded each iteration, stop when they meet
  * (ST-CON make_stcon, st-conn/make_stcon.c:730-1497, and the BFS_4K_DS
  * visit, BFS_4K_DS/src/device/WorkEfficientKernel/BFS_WE_Kernels1.cu:25-89).
