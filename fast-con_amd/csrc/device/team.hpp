@@ -62,9 +62,11 @@ __device__ __forceinline__ T ld_team(const T* p) {
 }
 
 // A store that other blocks of the XCD see with ld_team: to the L2 and no
-// further, in one piece.
+// further, in one piece. The compiler keeps it behind the accesses before it;
+// that those are out is the caller's wait.
 template <typename T>
 __device__ __forceinline__ void st_team(T* p, T v) {
+  asm volatile("" ::: "memory");
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
