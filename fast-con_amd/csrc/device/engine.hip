@@ -90,6 +90,7 @@ static VisitParams<OffT> make_params(fc_graph* g) {
   set_param(p.out, g->h_out);
   p.lazy_state = g->relabeled ? 1 : 0;
   p.v_active = (int32_t)g->v_active;
+  p.bottom_up = g->symmetric ? 1 : 0;
   set_param(p.head, g->d_head);
   return p;
 }

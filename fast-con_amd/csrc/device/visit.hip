@@ -871,7 +871,8 @@ __global__ __launch_bounds__(W * kWave) void phase_kernel(VisitCtl* ctl, int par
     int bu = S.bu_mode;
     if (!st) {
       if (!bu) {
-        if ((double)cur[0].mf > mu / kAlpha) bu = 1;
+        // (a list holds a vertex's parents only where edges go both ways)
+        if (p.bottom_up && (double)cur[0].mf > mu / kAlpha) bu = 1;
       } else if ((double)nf0 * kBeta < (double)p.V) {
         bu = 0;
       }

@@ -132,6 +132,7 @@ struct VisitParams {
   int32_t lazy_state;       // BFS leaves unreached state/parent unwritten (renumbered graphs:
                             // the un-permutation takes reached-ness from the visited bitmap)
   int32_t v_active;         // vertices [0, v_active) have degree > 0 (the rest are isolated)
+  int32_t bottom_up;        // BFS may go bottom-up: every edge is stored in both directions
   FC_GLOBAL const unsigned long long* head;  // each vertex's first two columns (the second in the upper half), -1
                                              // where there is none; null: not kept
 };

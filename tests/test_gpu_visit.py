@@ -345,3 +345,21 @@ def test_bfs_bottom_up_heads(fc, orc, name):
         with fc.Graph(hg, **kind) as g:
             _bfs_check(fc, orc, name, hg, g, hg.sample_roots(3, 5))
             assert g.bfs(int(hg.sample_roots(1, 5)[0]))[2]["bottomup_levels"] > 0
+
+
+@pytest.mark.parametrize("degree", [2, 16])
+def test_bfs_directed(fc, orc, degree):
+    rng = np.random.default_rng(43)
+    V = 20000
+    u = np.repeat(np.arange(V), degree)
+    e = np.unique(np.stack([u, rng.integers(0, V, len(u))], 1), axis=0)
+    off = np.concatenate([[0], np.cumsum(np.bincount(e[:, 0], minlength=V))])
+    hg = fc.HostGraph(off, e[:, 1].astype(np.int32), directed=True)
+    with fc.Graph(hg) as g:
+        for r in (0, 77, 4095):  # (the tree validator's edge rules are for undirected graphs)
+            _bfs_check(fc, orc, f"directed-{degree}", hg, g, [r], parents=False)
+            lv, pa, _ = g.bfs(r, parents=True)
+            v = np.flatnonzero((lv >= 0) & (np.arange(V) != r))
+            assert pa[r] == r and np.array_equal(pa < 0, lv < 0)
+            assert np.array_equal(lv[pa[v]], lv[v] - 1)
+            assert np.isin(pa[v].astype(np.int64) * V + v, e[:, 0] * V + e[:, 1]).all()
