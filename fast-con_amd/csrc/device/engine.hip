@@ -589,7 +589,7 @@ static fc_status graph_create(const OffT* off, const int32_t* col, int64_t V, in
   const bool ht_set = ht && std::atoi(ht) > 0;
   g->hub_threshold = ht_set ? std::atoi(ht) : 256;
   const char* vwf = std::getenv("FASTCON_VW");
-  if (vwf && std::atoi(vwf) > 0) g->vw_fixed = std::atoi(vwf);
+  if (vwf) g->vw_fixed = fcd::visit_width(std::atoi(vwf));
   // Direct launches instead of replayed hipGraphs, for profiler runs: under
   // rocprofv3's kernel trace a hipGraphLaunch of the visit's graph ended in
   // a host segmentation fault inside the runtime, while direct launches of
@@ -769,6 +769,9 @@ static fc_status graph_create(const OffT* off, const int32_t* col, int64_t V, in
   *out = g;
   return FC_OK;
 }
+
+// For tests on hosts without a GPU.
+extern "C" int32_t fcd_visit_width(int32_t asked) { return fcd::visit_width(asked); }
 
 extern "C" fc_status fc_graph_create_csr32(const int32_t* off, const int32_t* col, int32_t V, int64_t E,
                                            uint32_t flags, fc_graph** out) {

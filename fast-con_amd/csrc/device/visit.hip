@@ -354,14 +354,16 @@ __device__ __forceinline__ bool probe_done(Appender<OffT>& a, int32_t* parent, b
 }
 
 // The width is a run-time value: a copy of the code per width had made the
-// kernel 48 KB of the 64 KB of instruction cache that two CUs share.
+// kernel 48 KB of the 64 KB of instruction cache that two CUs share. It is a
+// power of two in [4, 64] (visit_width, degree_width): with another one lanes
+// would skip edges, and above 64 the loop over the frontier would not advance.
 // push(claimed, u, first edge, degree) takes the claimed vertices (wave-collective).
 template <bool TEAM, typename OffT, typename Push>
 __device__ __forceinline__ void td_normal(Appender<OffT>& a, int32_t* parent, bool st, int vw, int lvl, int cur_par,
                                           uint32_t n, int gwave, int nwaves, Push push) {
   const VisitParams<OffT>& p = *a.p;
   const int lane = lane_id();
-  const int sh = 31 - __builtin_clz((uint32_t)vw);  // vw is a power of two in [4, 64]
+  const int sh = 31 - __builtin_clz((uint32_t)vw);
   const int grp = lane >> sh, sub = lane & (vw - 1);
   const uint32_t G = (uint32_t)kWave >> sh;
   const int32_t* q = p.q[a.c][cur_par];

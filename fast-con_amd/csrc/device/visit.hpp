@@ -21,6 +21,14 @@ constexpr int kWavesPerBlock = kBlock / kWave;
 // per level, 30.4 ms against 38.6 with 16.
 constexpr int kWideWaves = 16;
 constexpr int64_t kWideEdges = 1ll << 22;
+// The fixed width of top-down levels that a caller asked for (0: none). The
+// kernels split a wave's lanes into groups of that many with shifts and masks,
+// so that only the powers of two from 4 to 64 are widths; every other positive
+// value means a whole wave.
+constexpr int visit_width(int asked) {
+  if (asked <= 0) return 0;
+  return asked == 4 || asked == 8 || asked == 16 || asked == 32 ? asked : kWave;
+}
 constexpr int32_t kColorBit = 1 << 30;        // colour of an s–t state word (0 = s side, 1 = t side)
 constexpr int32_t kLevelMask = kColorBit - 1;
 constexpr uint64_t kHubEdgeBits = 40;         // hub counter: (entries << 40) | edges

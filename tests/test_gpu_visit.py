@@ -363,3 +363,20 @@ def test_bfs_directed(fc, orc, degree):
             assert pa[r] == r and np.array_equal(pa < 0, lv < 0)
             assert np.array_equal(lv[pa[v]], lv[v] - 1)
             assert np.isin(pa[v].astype(np.int64) * V + v, e[:, 0] * V + e[:, 1]).all()
+
+
+@pytest.mark.parametrize("vw", ["1", "6", "12", "48", "128"])
+def test_widths_that_are_no_powers_of_two(fc, orc, monkeypatch, vw):
+    """FASTCON_VW changes speed only: other values than 4 to 64's powers of
+    two run at 64 lanes a vertex."""
+    monkeypatch.setenv("FASTCON_VW", vw)
+    hg = fc.gen_rmat(10, 8, seed=23)
+    rng = np.random.default_rng(24)
+    s = rng.integers(0, hg.V, 40).astype(np.int32)
+    t = rng.integers(0, hg.V, 40).astype(np.int32)
+    exp = np.array([orc.stcon(hg.offsets, hg.columns, int(a), int(b))[1] for a, b in zip(s, t)], np.int32)
+    with fc.Graph(hg) as g:
+        for r in s[:4]:
+            assert np.array_equal(g.bfs(int(r))[0], orc.bfs(hg.offsets, hg.columns, int(r))[0])
+        assert np.array_equal(g.stcon_many(s, t).dist, exp)
+        assert [g.stcon(int(a), int(b))[1] for a, b in zip(s, t)] == list(exp)

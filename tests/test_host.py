@@ -308,3 +308,20 @@ def test_generators_match_golden_fixtures(fc):
     assert rmat22["E"] == 128302336  # the benchmark graph
     g = fc.gen_grid(64, 64, 0.0, 3)
     assert g.E == 4 * 64 * 63  # no deletions: every undirected edge in both directions
+
+
+def test_visit_width_covers_every_edge(fc):
+    """A fixed width (FASTCON_VW) as the kernels use it: lanes lane & (w - 1)
+    of a group walk a list in steps of 2 w, two edges each, and 64 >> log2(w)
+    groups share a wave. Every edge once, at least one group, whatever was
+    asked for; 4 to 64 are kept and the rest means 64."""
+    width = fc.lib().fcd_visit_width
+    assert width(0) == 0 and width(-7) == 0
+    for asked in range(1, 301):
+        w = width(asked)
+        assert w == (asked if asked in (4, 8, 16, 32, 64) else 64)
+        assert 64 >> (w.bit_length() - 1) >= 1
+        lanes = {lane & (w - 1) for lane in range(w)}
+        for n in (1, 3, 63, 64, 65, 200):
+            seen = sorted(e for sub in lanes for b in range(sub, n, 2 * w) for e in (b, b + w) if e < n)
+            assert seen == list(range(n)), (asked, w, n)
