@@ -70,20 +70,29 @@ __device__ __forceinline__ void st_team(T* p, T v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
+// The number of the block that counted k on the registration word of a team
+// for which `expected` blocks were planned, or -1: closed, or full. What a
+// team's blocks own (tables, state words) is laid out for `expected` of them,
+// and no placement of a launch's blocks on the XCDs may put more to work.
+__host__ __device__ constexpr uint32_t team_full(uint32_t expected) { return expected < kTeamMax ? expected : kTeamMax; }
+__host__ __device__ constexpr int team_admit(uint32_t k, uint32_t expected) {
+  return (k & kTeamClosed) || k >= team_full(expected) ? -1 : (int)k;
+}
+
 // Register with the XCD's team (one thread). Returns this block's number, or
 // -1 when registration is closed. *members is set for number 0 only, which
 // has closed the registration and publishes the size itself (team_publish).
 __device__ __forceinline__ int team_register(TeamSync* ts, uint32_t expected, uint32_t* members) {
   const uint32_t k = __hip_atomic_fetch_add(&ts->reg.v, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  if ((k & kTeamClosed) || k >= kTeamMax) return -1;
-  if (k == 0) {
+  const int number = team_admit(k, expected);
+  if (number == 0) {
     const uint64_t t0 = wall_clock64();
     while (ld_agent(&ts->reg.v) < expected && wall_clock64() - t0 < kTeamJoinTicks) __builtin_amdgcn_s_sleep(1);
     const uint32_t n =
         __hip_atomic_fetch_or(&ts->reg.v, kTeamClosed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & ~kTeamClosed;
-    *members = n < kTeamMax ? n : kTeamMax;
+    *members = n < team_full(expected) ? n : team_full(expected);
   }
-  return (int)k;
+  return number;
 }
 
 // Wait until the counter *p has reached v (one thread; a difference, so that

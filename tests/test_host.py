@@ -325,3 +325,16 @@ def test_visit_width_covers_every_edge(fc):
         for n in (1, 3, 63, 64, 65, 200):
             seen = sorted(e for sub in lanes for b in range(sub, n, 2 * w) for e in (b, b + w) if e < n)
             assert seen == list(range(n)), (asked, w, n)
+
+
+def test_teams_admit_the_planned_blocks_only(fc):
+    """Blocks of a launch are numbered as they reach their XCD's registration
+    word, wherever the hardware puts them. 128 blocks of a device that shows
+    one XCD of 32 compute units, for which 16 a team were planned, and 192
+    blocks that all land on one of eight XCDs: the numbers stay below what a
+    team's tables have room for."""
+    admit = fc.lib().fcd_team_admit
+    for blocks, expected in ((128, 16), (192, 24), (1024, 128), (2048, 256), (256, 32), (1, 1)):
+        numbers = [admit(k, expected) for k in range(blocks)]
+        assert [n for n in numbers if n >= 0] == list(range(min(blocks, expected, 128)))
+    assert admit(0x80000000 - (1 << 32), 16) == -1  # closed
