@@ -2577,17 +2577,24 @@ static fc_status team_alloc(fc_graph* g) {
     w->off = true;
     return FC_OK;
   }
-  if (hipMalloc((void**)&w->mem, (size_t)(kXcds * teams) * stride) != hipSuccess) {
+  char* mem = nullptr;
+  if (hipMalloc((void**)&mem, (size_t)(kXcds * teams) * stride) != hipSuccess) {
     (void)hipGetLastError();
-    w->mem = nullptr;
     w->off = true;
     return FC_OK;
   }
+  // The memory is the machines' once it is cleared (every wave leaves its
+  // records, masks and marks zero and relies on finding them so).
+  const hipError_t e = hipMemsetAsync(mem, 0, (size_t)(kXcds * teams) * stride, g->stream);
+  if (e != hipSuccess) {
+    (void)hipFree(mem);
+    return hip_fail(e, "clearing the machines' workspaces");
+  }
+  w->mem = mem;
   w->stride = stride;
   w->layout = l;
   w->teams = teams;
   w->blocks = blocks;
-  FC_HIP(hipMemsetAsync(w->mem, 0, (size_t)(kXcds * teams) * stride, g->stream));
   return FC_OK;
 }
 

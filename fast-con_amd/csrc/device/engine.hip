@@ -161,18 +161,26 @@ static fc_status st_teams_alloc(fc_graph* g) {
     w->off = true;
     return FC_OK;
   }
-  if (hipMalloc((void**)&w->mem, kXcds * w->stride) != hipSuccess) {
+  char* mem = nullptr;
+  if (hipMalloc((void**)&mem, kXcds * w->stride) != hipSuccess) {
     (void)hipGetLastError();
-    w->mem = nullptr;
     w->off = true;
     return FC_OK;
   }
+  // Only the state words are read before they are written. The memory is the
+  // teams' once they are cleared: a call that fails here leaves none behind.
+  for (int k = 0; k < kXcds; ++k) {
+    const hipError_t e = hipMemsetAsync(mem + (size_t)k * w->stride, 0, 8 * V, g->stream);
+    if (e != hipSuccess) {
+      (void)hipFree(mem);
+      return hip_fail(e, "clearing the teams' state words");
+    }
+  }
+  w->mem = mem;
   // 1,024 queries at s22 took 18.1, 11.9, 10.1 and 9.3 ms with 1 to 4 blocks
   // per CU, 8 queries on a 4096^2 grid 32.9, 27.1 and 25.4 ms with 1, 2 and 4.
   w->blocks = std::min(occ, 4) * g->cus;
   w->narrow_blocks = nocc > 0 ? g->cus : 0;
-  // only the state words are read before they are written
-  for (int k = 0; k < kXcds; ++k) FC_HIP(hipMemsetAsync(w->mem + (size_t)k * w->stride, 0, 8 * V, g->stream));
   return FC_OK;
 }
 
