@@ -2152,7 +2152,7 @@ static fc_status batch_alloc_lane(fc_graph* g, BatchWorkspace** out, bool own_st
   BatchWorkspace* b = new BatchWorkspace();
   const BatchLayout l = batch_layout(g->V, g->hcap);
   b->bytes = l.bytes;
-  hipError_t e = hipMalloc((void**)&b->mem, b->bytes);
+  hipError_t e = dev_malloc((void**)&b->mem, b->bytes);
   if (e != hipSuccess) {
     delete b;
     return hip_fail(e, "batch workspace allocation");
@@ -2236,9 +2236,9 @@ static fc_status batch_queries(fc_graph* g, BatchWorkspace* b, int32_t n) {
   b->qs = b->qt = b->dist = b->h_dist = nullptr;
   b->qcap = 0;
   const int32_t cap = std::max<int32_t>(n, 4096);
-  FC_HIP(hipMalloc((void**)&b->qs, sizeof(int32_t) * (size_t)cap));
-  FC_HIP(hipMalloc((void**)&b->qt, sizeof(int32_t) * (size_t)cap));
-  FC_HIP(hipMalloc((void**)&b->dist, sizeof(int32_t) * (size_t)cap));
+  FC_HIP(dev_malloc((void**)&b->qs, sizeof(int32_t) * (size_t)cap));
+  FC_HIP(dev_malloc((void**)&b->qt, sizeof(int32_t) * (size_t)cap));
+  FC_HIP(dev_malloc((void**)&b->dist, sizeof(int32_t) * (size_t)cap));
   FC_HIP(hipHostMalloc((void**)&b->h_dist, sizeof(int32_t) * (size_t)cap, hipHostMallocDefault));
   b->qcap = cap;
   return FC_OK;
@@ -2537,9 +2537,8 @@ constexpr uint64_t kTeamBothMaxEdges = 1u << 16;
 constexpr uint64_t kTeamBridgeMinEdges = 1u << 14;
 constexpr uint64_t kTeamHubMinEdges = 1u << 15;
 constexpr int kTeamTile = 256;  // hub chunk when the caller gives none
-// The machines' workspaces take at most this share of the device's memory
-// (16 machines at R-MAT s24: 22 GB); larger graphs run the launch engine.
-constexpr size_t kTeamMemShare = 8;
+// Graphs whose machines' workspaces are more than team_budget allows (16
+// machines at R-MAT s24 take 22 GB) run the launch engine.
 
 struct TeamWorkspace {
   char* mem = nullptr;
@@ -2570,7 +2569,7 @@ static fc_status team_alloc(fc_graph* g) {
   const int occ = g->off64 ? team_occupancy<int64_t>() : team_occupancy<int32_t>();
   const int blocks = std::min(occ, 4) * g->cus;
   const BatchLayout l = batch_layout(g->V, g->hcap, blocks / kXcds);
-  const size_t stride = l.bytes, budget = prop.totalGlobalMem / kTeamMemShare;
+  const size_t stride = l.bytes, budget = team_budget(prop.totalGlobalMem);
   int teams = kMaxTeams;
   while (teams > 0 && (size_t)(kXcds * teams) * stride > budget) --teams;
   if (teams < 1 || occ < 1 || g->V > kTeamMaxV || g->cus % kXcds != 0 || !g->symmetric) {
@@ -2636,7 +2635,7 @@ static fc_status team_run(fc_graph* g, const int32_t* s, const int32_t* t, int32
     w->d_io = w->h_io = nullptr;
     w->io_bytes = 0;
     const size_t cap = std::max<size_t>(bytes, 1u << 17);
-    FC_HIP(hipMalloc((void**)&w->d_io, cap));
+    FC_HIP(dev_malloc((void**)&w->d_io, cap));
     FC_HIP(hipHostMalloc((void**)&w->h_io, cap, hipHostMallocDefault));
     w->io_bytes = cap;
   }
@@ -2816,16 +2815,28 @@ extern "C" fc_status fc_stcon_batch(fc_graph* g, const int32_t* s, const int32_t
   float ms = 0;
   BatchCtl c;
   int64_t launches = 0;
-  const int32_t* got = nullptr;
   fc_status st;
+  auto answer = [&](const int32_t* got) {
+    for (int32_t i = 0; i < n; ++i) {
+      const int32_t d = got[i];
+      if (dist) dist[i] = d;
+      if (connected) connected[i] = d >= 0 ? 1 : 0;
+    }
+  };
   // The team engine takes every batch whose lanes the caller leaves open: a
   // number of lanes asks for that many launch-driven machines.
   bool ran = false;
   if (o.lanes == 0) {
+    const fcd::TeamUse use(g);  // the distances are read in the workspace
     const int ttile = tile ? tile : fcd::kTeamTile;
+    const int32_t* got = nullptr;
     st = fcd::team_run(g, s, t, n, o.policy, vw, ttile, o.learn_margin, &ms, &c, &got, &ran);
     if (st != FC_OK) return st;
-    if (ran) tile = ttile, launches = 1;
+    if (ran) {
+      answer(got);
+      tile = ttile;
+      launches = 1;
+    }
   }
   if (!ran) {
     st = fcd::batch_alloc(g);
@@ -2842,12 +2853,7 @@ extern "C" fc_status fc_stcon_batch(fc_graph* g, const int32_t* s, const int32_t
     if (tile == 0) tile = 256;
     st = fcd::batch_run(g, s, t, n, o.policy, vw, tile, o.use_graph != 0, &ms, &c, &launches, o.learn_margin, lanes);
     if (st != FC_OK) return st;
-    got = b->h_dist;
-  }
-  for (int32_t i = 0; i < n; ++i) {
-    const int32_t d = got[i];
-    if (dist) dist[i] = d;
-    if (connected) connected[i] = d >= 0 ? 1 : 0;
+    answer(b->h_dist);
   }
   if (stats) {
     stats->time_ms = ms;
@@ -2893,7 +2899,7 @@ extern "C" fc_status fc_sched_trace(fc_graph* g, const int32_t* s, const int32_t
   g->levels_valid = g->parents_valid = false;
   fcd::BatchWorkspace* b = g->batch;
   if ((st = fcd::batch_queries(g, b, n)) != FC_OK) return st;
-  if (!b->snap && hipMalloc((void**)&b->snap, b->bytes) != hipSuccess) {
+  if (!b->snap && fcd::dev_malloc((void**)&b->snap, b->bytes) != hipSuccess) {
     b->snap = nullptr;
     return fc::fail(FC_ERR_NOMEM, "fc_sched_trace: no room for the workspace copy (%zu bytes)", b->bytes);
   }

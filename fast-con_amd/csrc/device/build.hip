@@ -392,7 +392,7 @@ struct BuildMem {
   template <typename T>
   hipError_t alloc(T** p, int64_t n) {
     *p = nullptr;
-    hipError_t e = hipMalloc((void**)p, sizeof(T) * (size_t)std::max<int64_t>(n, 1));
+    hipError_t e = dev_malloc((void**)p, sizeof(T) * (size_t)std::max<int64_t>(n, 1));
     if (e == hipSuccess) bufs.push_back(*p);
     return e;
   }

@@ -20,6 +20,8 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
+#include <thread>
 #include <vector>
 
 using fc::fail;
@@ -43,6 +45,62 @@ fc_status hip_fail(hipError_t e, const char* what) {
               "%s: %s", what, hipGetErrorString(e));
 }
 
+// Every graph of the process, for dev_malloc. Never destroyed: graphs may be
+// freed by the caller's own static destructors.
+struct Graphs {
+  std::mutex mu;
+  std::vector<fc_graph*> all;
+};
+static Graphs& graphs() {
+  static Graphs* g = new Graphs();
+  return *g;
+}
+static void graphs_remove(fc_graph* g) {
+  std::lock_guard<std::mutex> lock(graphs().mu);
+  auto& a = graphs().all;
+  a.erase(std::remove(a.begin(), a.end(), g), a.end());
+}
+
+TeamUse::TeamUse(fc_graph* g_) : g(g_) {
+  for (;;) {
+    int n = g->team_use.load();
+    if (n >= 0 && g->team_use.compare_exchange_weak(n, n + 1)) return;
+    if (n < 0) std::this_thread::yield();  // for as long as a few frees take
+  }
+}
+
+hipError_t dev_malloc(void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipErrorOutOfMemory) return e;
+  (void)hipGetLastError();
+  int device = 0;
+  (void)hipGetDevice(&device);
+  bool freed = false;
+  {
+    std::lock_guard<std::mutex> lock(graphs().mu);
+    for (fc_graph* g : graphs().all) {
+      int idle = 0;
+      if (g->device != device || !g->team_use.compare_exchange_strong(idle, -1)) continue;
+      freed |= g->team || g->st_teams;
+      team_free(g->team);
+      st_teams_free(g->st_teams);
+      g->team = nullptr;
+      g->st_teams = nullptr;
+      g->team_use.store(0);
+    }
+  }
+  return freed ? hipMalloc(p, bytes) : e;
+}
+
+size_t team_budget(size_t total) {
+  size_t free = 0, all = 0;
+  if (hipMemGetInfo(&free, &all) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  return std::min(total / 8, free / 4);
+}
+
 fc_status ensure_queries(fc_graph* g, int32_t n) {
   if (n <= g->q_cap) return FC_OK;
   // the captured launches take only the control block, whose parameters
@@ -54,8 +112,8 @@ fc_status ensure_queries(fc_graph* g, int32_t n) {
   g->h_out = nullptr;
   g->q_cap = 0;
   const int32_t cap = std::max<int32_t>(n, 1024);
-  FC_HIP(hipMalloc((void**)&g->d_qs, sizeof(int32_t) * (size_t)cap));
-  FC_HIP(hipMalloc((void**)&g->d_qt, sizeof(int32_t) * (size_t)cap));
+  FC_HIP(dev_malloc((void**)&g->d_qs, sizeof(int32_t) * (size_t)cap));
+  FC_HIP(dev_malloc((void**)&g->d_qt, sizeof(int32_t) * (size_t)cap));
   FC_HIP(hipHostMalloc((void**)&g->h_out, sizeof(VisitOut) * (size_t)cap, hipHostMallocDefault));
   g->q_cap = cap;
   return FC_OK;
@@ -156,8 +214,8 @@ static fc_status st_teams_alloc(fc_graph* g) {
   w->stride = w->o_hb + 4 * w->hb1;
   const int occ = g->off64 ? st_team_occupancy<int64_t>() : st_team_occupancy<int32_t>();
   const int nocc = g->off64 ? narrow_occupancy<int64_t>() : narrow_occupancy<int32_t>();
-  // at most an eighth of the device's memory (a 4096^2 grid takes 3.2 GB)
-  if (occ < 1 || g->cus % kXcds != 0 || kXcds * w->stride > prop.totalGlobalMem / 8) {
+  // (a 4096^2 grid takes 3.2 GB)
+  if (occ < 1 || g->cus % kXcds != 0 || kXcds * w->stride > team_budget(prop.totalGlobalMem)) {
     w->off = true;
     return FC_OK;
   }
@@ -265,6 +323,7 @@ __global__ __launch_bounds__(kStartThreads) void team_start_kernel(const TeamSta
 static fc_status st_teams_run(fc_graph* g, const int32_t* s, const int32_t* t, int32_t n, bool narrow, bool bfs,
                               int32_t* lv_out, int32_t* par_out, double* ms, bool* ran, const VisitTail& after = {}) {
   *ran = false;
+  const TeamUse use(g);
   fc_status st = st_teams_alloc(g);
   if (st != FC_OK) return st;
   StTeams* w = g->st_teams;
@@ -285,7 +344,7 @@ static fc_status st_teams_run(fc_graph* g, const int32_t* s, const int32_t* t, i
     w->d_io = w->h_io = nullptr;
     w->io_bytes = 0;
     const size_t cap = std::max<size_t>(bytes, 1u << 17);
-    FC_HIP(hipMalloc((void**)&w->d_io, cap));
+    FC_HIP(dev_malloc((void**)&w->d_io, cap));
     FC_HIP(hipHostMalloc((void**)&w->h_io, cap, hipHostMallocDefault));
     w->io_bytes = cap;
   }
@@ -660,8 +719,8 @@ static fc_status graph_create(const OffT* off, const int32_t* col, int64_t V, in
   CK(hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking));
   CK(hipEventCreate(&g->ev0));
   CK(hipEventCreate(&g->ev1));
-  CK(hipMalloc(&g->d_off, sizeof(OffT) * (size_t)(V + 1)));
-  CK(hipMalloc((void**)&g->d_col, sizeof(int32_t) * (size_t)std::max<int64_t>(E, 1)));
+  CK(fcd::dev_malloc(&g->d_off, sizeof(OffT) * (size_t)(V + 1)));
+  CK(fcd::dev_malloc((void**)&g->d_col, sizeof(int32_t) * (size_t)std::max<int64_t>(E, 1)));
   if (!(flags & FC_GRAPH_KEEP_IDS)) {
     g->relabeled = true;
     g->h_perm.resize((size_t)V);
@@ -674,8 +733,8 @@ static fc_status graph_create(const OffT* off, const int32_t* col, int64_t V, in
     else
       fc::relabel32((const int32_t*)off, col, V, (flags & FC_GRAPH_KEEP_ORDER) != 0, g->h_perm.data(),
                     g->h_iperm.data(), (int32_t*)noff.data(), ncol.data());
-    CK(hipMalloc((void**)&g->d_perm, sizeof(int32_t) * (size_t)V));
-    CK(hipMalloc((void**)&g->d_iperm, sizeof(int32_t) * (size_t)V));
+    CK(fcd::dev_malloc((void**)&g->d_perm, sizeof(int32_t) * (size_t)V));
+    CK(fcd::dev_malloc((void**)&g->d_iperm, sizeof(int32_t) * (size_t)V));
     CK(hipMemcpyAsync(g->d_perm, g->h_perm.data(), sizeof(int32_t) * (size_t)V, hipMemcpyHostToDevice, g->stream));
     CK(hipMemcpyAsync(g->d_iperm, g->h_iperm.data(), sizeof(int32_t) * (size_t)V, hipMemcpyHostToDevice, g->stream));
     CK(hipMemcpyAsync(g->d_off, noff.data(), sizeof(OffT) * (size_t)(V + 1), hipMemcpyHostToDevice, g->stream));
@@ -723,7 +782,7 @@ static fc_status graph_create(const OffT* off, const int32_t* col, int64_t V, in
   size_t off_hb = off_hq + 4 * al(sizeof(int32_t) * (size_t)g->hcap);
   size_t off_ctl = off_hb + 4 * al(sizeof(int64_t) * (size_t)g->hcap);
   g->ws_bytes = off_ctl + al(sizeof(fcd::VisitCtl));
-  CK(hipMalloc((void**)&g->d_ws, g->ws_bytes));
+  CK(fcd::dev_malloc((void**)&g->d_ws, g->ws_bytes));
   CK(hipMemsetAsync(g->d_ws, 0, g->ws_bytes, g->stream));
   g->d_state = (int32_t*)(g->d_ws + off_state);
   g->d_sst = (unsigned long long*)(g->d_ws + off_sst);
@@ -739,10 +798,10 @@ static fc_status graph_create(const OffT* off, const int32_t* col, int64_t V, in
   }
   g->d_ctl = (fcd::VisitCtl*)(g->d_ws + off_ctl);
   // canonical parameters, then the copy in the batch kernel's layout
-  CK(hipMalloc((void**)&g->d_mlp, 2 * sizeof(float) * fcd::kMlpParams));
+  CK(fcd::dev_malloc((void**)&g->d_mlp, 2 * sizeof(float) * fcd::kMlpParams));
   CK(hipMemsetAsync(g->d_mlp, 0, 2 * sizeof(float) * fcd::kMlpParams, g->stream));
   CK(hipHostMalloc((void**)&g->h_phase, 4 * sizeof(int32_t), hipHostMallocDefault));
-  if (hipMalloc((void**)&g->d_head, sizeof(unsigned long long) * (size_t)std::max<int64_t>(V, 1)) == hipSuccess) {
+  if (fcd::dev_malloc((void**)&g->d_head, sizeof(unsigned long long) * (size_t)std::max<int64_t>(V, 1)) == hipSuccess) {
     hipLaunchKernelGGL(fcd::head_kernel<OffT>, dim3(g->cus * 8), dim3(256), 0, g->stream, (const OffT*)g->d_off, g->d_col, V,
                        g->d_head);
     CK(hipGetLastError());
@@ -774,6 +833,10 @@ static fc_status graph_create(const OffT* off, const int32_t* col, int64_t V, in
   CK(hipStreamSynchronize(g->stream));
   g->symmetric = g->h_phase[0] == 0 && g->h_phase[1] == 0;
 #undef CK
+  {
+    std::lock_guard<std::mutex> lock(fcd::graphs().mu);
+    fcd::graphs().all.push_back(g);
+  }
   *out = g;
   return FC_OK;
 }
@@ -794,6 +857,7 @@ extern "C" fc_status fc_graph_create_csr64(const int64_t* off, const int32_t* co
 
 extern "C" fc_status fc_graph_destroy(fc_graph* g) {
   if (!g) return FC_OK;
+  fcd::graphs_remove(g);
   if (g->stream) (void)hipStreamSynchronize(g->stream);
   fcd::batch_free(g->batch);
   fcd::team_free(g->team);
@@ -878,8 +942,8 @@ extern "C" fc_status fc_bfs(fc_graph* g, int32_t src, int32_t* levels_out, int32
   double ms = 0, tried = 0;
   g->levels_valid = g->parents_valid = false;
   const size_t bytes = sizeof(int32_t) * (size_t)g->V;
-  if (g->relabeled && !g->d_lv_out) FC_HIP(hipMalloc((void**)&g->d_lv_out, bytes));
-  if (g->relabeled && par && !g->d_par_out) FC_HIP(hipMalloc((void**)&g->d_par_out, bytes));
+  if (g->relabeled && !g->d_lv_out) FC_HIP(fcd::dev_malloc((void**)&g->d_lv_out, bytes));
+  if (g->relabeled && par && !g->d_par_out) FC_HIP(fcd::dev_malloc((void**)&g->d_par_out, bytes));
   int32_t* const lv = g->relabeled ? g->d_lv_out : g->d_state;
   int32_t* const pa = g->relabeled ? g->d_par_out : g->d_parent;
   // small results come back behind the visit, through pinned memory

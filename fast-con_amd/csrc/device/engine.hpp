@@ -2,6 +2,7 @@
 // stream, and all per-query workspace, allocated once at creation.
 #pragma once
 
+#include <atomic>
 #include <functional>
 #include <hip/hip_runtime.h>
 
@@ -91,6 +92,7 @@ struct fc_graph {
   bool use_st_teams = true;          // FASTCON_PLAIN_TEAMS=0: every visit through the launches
   bool narrow = false;               // even degrees: visits are likely to stay narrow (narrow_kernel)
   bool narrow_st = true, narrow_bfs = true;  // until one did not
+  std::atomic<int> team_use{0};      // calls that use the two workspaces above; -1: they are being given back
 };
 
 namespace fcd {
@@ -99,6 +101,23 @@ constexpr int kGraphLaunches = 16;
 constexpr int64_t kPollLaunches = 4096;  // launches queued between two host polls of the phase word
 
 fc_status hip_fail(hipError_t e, const char* what);
+
+// Device memory. The teams' workspaces (team, st_teams) are the one part of a
+// graph that it can do without: when memory runs out, those of every graph on
+// the device whose teams are not at work are given back and the allocation is
+// tried again. Their owners allocate them anew when they next fit.
+hipError_t dev_malloc(void** p, size_t bytes);
+// What a graph's next teams may take: an eighth of the device's memory, and no
+// more than a quarter of what is free.
+size_t team_budget(size_t total);
+// Held while a call uses its graph's team workspaces.
+struct TeamUse {
+  fc_graph* g;
+  explicit TeamUse(fc_graph* g_);
+  ~TeamUse() { g->team_use.fetch_sub(1); }
+  TeamUse(const TeamUse&) = delete;
+  TeamUse& operator=(const TeamUse&) = delete;
+};
 fc_status ensure_queries(fc_graph* g, int32_t n);
 
 // Run n visits through the phase machine (s[i], t[i]; t = -1 for BFS) and

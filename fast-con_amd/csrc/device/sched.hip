@@ -313,7 +313,7 @@ struct MlpBuffers {
         sum += weight[r];
       }
       if (!(sum > 0.0)) return fc::fail(FC_ERR_INVALID, "scheduler row weights sum to zero");
-      if (hipMalloc((void**)&wr, sizeof(float) * (size_t)n) != hipSuccess)
+      if (fcd::dev_malloc((void**)&wr, sizeof(float) * (size_t)n) != hipSuccess)
         return fc::fail(FC_ERR_NOMEM, "scheduler buffers: device allocation failed");
       FC_HIP(hipMemcpyAsync(wr, weight, sizeof(float) * (size_t)n, hipMemcpyHostToDevice, s));
     } else {
@@ -323,7 +323,7 @@ struct MlpBuffers {
     return FC_OK;
   }
   fc_status alloc(int n, bool train) {
-    auto A = [](float** p, size_t cnt) { return hipMalloc((void**)p, sizeof(float) * (cnt ? cnt : 1)); };
+    auto A = [](float** p, size_t cnt) { return fcd::dev_malloc((void**)p, sizeof(float) * (cnt ? cnt : 1)); };
     const size_t N = (size_t)n, P = padded_rows(n);
     if (A(&X, N * kFeatures) != hipSuccess || A(&XT, P * kFeatures) != hipSuccess || A(&T, N * kActions) != hipSuccess ||
         A(&Y, N * kActions) != hipSuccess || A(&H1, P * kHidden) != hipSuccess || A(&H2, P * kHidden) != hipSuccess ||

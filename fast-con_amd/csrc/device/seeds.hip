@@ -280,7 +280,7 @@ static fc_status seeds_run(fc_graph* g, const std::vector<int32_t>& seeds, int32
   const int K = (int)seeds.size();
   char* mem = nullptr;
   const size_t cbytes = sizeof(uint32_t) * (size_t)kMaxSeeds * kSeedWords;
-  FC_HIP(hipMalloc((void**)&mem, cbytes + 256 + sizeof(int32_t) * kMaxSeeds));
+  FC_HIP(dev_malloc((void**)&mem, cbytes + 256 + sizeof(int32_t) * kMaxSeeds));
   struct Free {
     char* m;
     ~Free() { (void)hipFree(m); }

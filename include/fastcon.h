@@ -33,6 +33,14 @@
  * Threading: one fc_graph per host thread; each fc_graph owns one HIP stream
  * (default priority) and its own device workspace. Calls are synchronous from
  * the caller's point of view.
+ *
+ * Memory: the CSR and about 50 bytes per vertex at creation. Calls that run
+ * inside one launch (fc_stcon_batch, fc_stcon_many, fc_stcon and fc_bfs on
+ * graphs of even degrees) add workspaces on first use, 24 bytes per vertex and
+ * machine for eight visit machines and 85 for eight or sixteen batch machines.
+ * Each of the two takes at most an eighth of the device's memory and a quarter
+ * of what is free (calls that do not fit run launch by launch), and both are
+ * given back when an allocation of this library, on any graph, finds no room.
  */
 #ifndef FASTCON_H
 #define FASTCON_H
@@ -331,8 +339,7 @@ typedef struct fc_batch_stats {
  * mask per vertex and side). Verdicts and distances equal fc_stcon's.
  * With lanes = 0 a batch runs in one launch when every edge of the graph is
  * stored in both directions (checked at creation), V < 2^28, and the machines'
- * workspaces (about 85 bytes per vertex each) take at most an eighth of the
- * device's memory; otherwise it runs three launch-driven machines. There the
+ * workspaces (about 85 bytes per vertex each) fit (see Memory above); otherwise it runs three launch-driven machines. There the
  * heuristic and learned schedules also run hub steps on skewed graphs: meets
  * at the 512 vertices of the highest degree, with the same exact distances. */
 fc_status fc_stcon_batch(fc_graph* g, const int32_t* s, const int32_t* t, int32_t n,

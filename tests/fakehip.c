@@ -113,22 +113,31 @@ hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void* f, i
   return hipSuccess;
 }
 static int handle;
-#define OK { return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned f) { (void)f; *s = (hipStream_t)&handle; return hipSuccess; }
 hipError_t hipEventCreate(hipEvent_t* e) { *e = (hipEvent_t)&handle; return hipSuccess; }
 hipError_t hipEventElapsedTime(float* ms, hipEvent_t a, hipEvent_t b) { (void)a; (void)b; *ms = 1.f; return hipSuccess; }
-hipError_t hipStreamDestroy(hipStream_t s) { (void)s; OK }
-hipError_t hipStreamSynchronize(hipStream_t s) { (void)s; OK }
-hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned f) { (void)s; (void)e; (void)f; OK }
-hipError_t hipEventDestroy(hipEvent_t e) { (void)e; OK }
-hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) { (void)e; (void)s; OK }
-hipError_t hipEventSynchronize(hipEvent_t e) { (void)e; OK }
-hipError_t hipGetLastError(void) OK
+hipError_t hipStreamDestroy(hipStream_t s) { (void)s; return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t s) { (void)s; return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned f) { (void)s; (void)e; (void)f; return hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t e) { (void)e; return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) { (void)e; (void)s; return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t e) { (void)e; return hipSuccess; }
+hipError_t hipGetLastError(void) { return hipSuccess; }
 const char* hipGetErrorString(hipError_t e) { (void)e; return "fake"; }
 hipError_t hipLaunchKernel(const void* f, dim3 g, dim3 b, void** a, size_t m, hipStream_t s) {
-  (void)f; (void)g; (void)b; (void)a; (void)m; (void)s; OK
+  (void)f; (void)g; (void)b; (void)a; (void)m; (void)s; return hipSuccess;
 }
-hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t m, hipStream_t s) { (void)g; (void)b; (void)m; (void)s; OK }
+hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t m, hipStream_t s) { (void)g; (void)b; (void)m; (void)s; return hipSuccess; }
 hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* m, hipStream_t* s) {
-  (void)g; (void)b; (void)m; (void)s; OK
+  (void)g; (void)b; (void)m; (void)s; return hipSuccess;
 }
+hipError_t hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode m) { (void)s; (void)m; return hipSuccess; }
+hipError_t hipStreamEndCapture(hipStream_t s, hipGraph_t* g) { (void)s; *g = (hipGraph_t)&handle; return hipSuccess; }
+hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t g, hipGraphNode_t* n, char* l, size_t k) {
+  (void)g; (void)n; (void)l; (void)k;
+  *e = (hipGraphExec_t)&handle;
+  return hipSuccess;
+}
+hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t s) { (void)e; (void)s; return hipSuccess; }
+hipError_t hipGraphDestroy(hipGraph_t g) { (void)g; return hipSuccess; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t e) { (void)e; return hipSuccess; }

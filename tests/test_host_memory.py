@@ -66,3 +66,48 @@ def test_a_failed_clear_leaves_no_workspace_behind(run):
     assert raises(lambda: g.stcon_batch(s, t)) == fc.ERR_HIP
     assert hip.fake_used() == held
     """)
+
+
+def test_team_workspaces_make_room(run):
+    """Allocations that fit without the teams' workspaces succeed beside them,
+    on the same graph and on another, and the workspaces come back later."""
+    run("""
+    hg = fc.gen_er(100000, 12.0, 1)
+    g = fc.Graph(hg)
+    held = hip.fake_used()
+    g.stcon_many(s, t)
+    teams = hip.fake_used() - held
+    assert teams >= 8 * 24 * hg.V
+    other = fc.Graph(hg)  # its size, for the limit
+    size = hip.fake_used() - held - teams
+    other.close()
+    assert size < teams
+    hip.fake_limit(held + teams + size // 2)
+    other = fc.Graph(hg)  # needs what the first graph's teams hold
+    assert hip.fake_used() == held + size
+    hip.fake_limit(held + size + 64 * teams)
+    g.stcon_many(s, t)
+    assert hip.fake_used() == held + size + teams
+    other.close()
+    hip.fake_limit(hip.fake_used() + 1000)
+    status = raises(lambda: g.sched_trace(s, t))  # a wave machine of its own and its copy (launches do nothing here)
+    assert status == fc.ERR_CAPACITY, status
+    assert hip.fake_used() > held
+    """)
+
+
+def test_team_workspaces_leave_room(run):
+    """At most a quarter of what is free."""
+    run("""
+    hg = fc.gen_er(3000, 12.0, 1)
+    g = fc.Graph(hg)
+    held = hip.fake_used()
+    g.stcon_many(s, t)
+    teams = hip.fake_used() - held
+    g.close()
+    hip.fake_limit(held + 4 * (teams - (1 << 17)) - 4096)  # (what a run uploads and reads back takes 2^17)
+    g = fc.Graph(hg)
+    status = raises(lambda: g.stcon_many(s, t))  # by launches, which do nothing here
+    assert status == fc.ERR_CAPACITY, status
+    assert hip.fake_used() == held, (hip.fake_used(), held, teams)
+    """)
