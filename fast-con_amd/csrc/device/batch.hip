@@ -2540,6 +2540,38 @@ constexpr int kTeamTile = 256;  // hub chunk when the caller gives none
 // Graphs whose machines' workspaces are more than team_budget allows (16
 // machines at R-MAT s24 take 22 GB) run the launch engine.
 
+// Whether a batch of n queries under the plain schedule runs in one launch.
+// Its waves hold 64 queries and it has no step that spares the wide
+// expansions, so a batch of few waves works on few XCDs and its widest steps
+// take up to eight times as long as on the whole GPU: more than launches cost
+// once they are wide. Measured, us, one launch against launches on three
+// lanes: R-MAT s22, 64 queries, 2,270 and 770, one query 155 and 193; s20, 4,
+// 64 and 256 queries 183 / 207, 1,271 / 459, 1,629 / 1,439; s18, 64 and 1,024:
+// 737 / 353, 1,435 / 2,791; random graph of 2M vertices and degree 8, 16, 64
+// and 256: 254 / 274, 542 / 496, 836 / 1,449; 1000^2 grid, 16, 64 and 192: 18.5
+// / 19.4, 38.9 / 26.2, 40.4 / 54.7 ms; 128^3 mesh, 4 and 64: 5.6 / 3.7, 38.1 /
+// 10.3 ms.
+//  * Random and skewed graphs: the queries per wave at which both take the
+//    same time follow E^0.6 branch^0.25, a fit over R-MAT s14 to s24 and random
+//    graphs of 300K to 4M vertices, to within a quarter either way. With more
+//    waves more XCDs share the work.
+//  * Equal degrees of at most 8, a mesh of about branch / 2 dimensions: a ball's surface has about
+//    V^(1 - 2 / branch) vertices, over most of a wave's steps.
+//  * Four waves or more pay wherever no hub makes the steps long (the random
+//    graph above; that mesh with 1,024 queries: 137 and 133 ms, 64^3 11 and 29).
+constexpr double kPlainTeamWork = 8e5;
+constexpr double kPlainTeamMesh = 8e4;
+static bool plain_teams(const fc_graph* g, int32_t n) {
+  const double queries = (double)std::min(n, 64);
+  const int waves = (n + 63) / 64;
+  if (!g->skewed && waves >= 4) return true;
+  if (g->regular && g->branch <= 8.0)
+    return queries * g->branch * std::pow((double)g->V, 1.0 - 2.0 / std::max(g->branch, 2.0)) <=
+           kPlainTeamMesh * (double)std::min(waves, kXcds);
+  return queries * std::pow((double)g->E, 0.6) * std::pow(g->branch, 0.25) <=
+         kPlainTeamWork * (1.5 * (double)std::min(waves, kXcds) - 0.5);
+}
+
 struct TeamWorkspace {
   char* mem = nullptr;
   BatchLayout layout;
@@ -2605,6 +2637,7 @@ static fc_status team_run(fc_graph* g, const int32_t* s, const int32_t* t, int32
   *ran = false;
   const char* env = std::getenv("FASTCON_BATCH_TEAMS");
   if ((env && std::atoi(env) == 0 && env[0]) || std::getenv("FASTCON_BATCH_LOG")) return FC_OK;
+  if (policy == FC_POLICY_PLAIN && !(env && std::atoi(env) > 0) && !plain_teams(g, n)) return FC_OK;
   fc_status st = team_alloc(g);
   if (st != FC_OK) return st;
   TeamWorkspace* w = g->team;
@@ -2842,7 +2875,11 @@ extern "C" fc_status fc_stcon_batch(fc_graph* g, const int32_t* s, const int32_t
     st = fcd::batch_alloc(g);
     if (st != FC_OK) return st;
     fcd::BatchWorkspace* b = g->batch;
-    if (vw == 0 && tile == 0) {
+    // A plain batch that its width keeps off the teams takes the width by degree
+    // and chunks of 256 edges, which no pair the tuner tries beats by more than
+    // the runs differ, without the tuner's 24 runs.
+    const bool untuned = o.lanes == 0 && o.policy == FC_POLICY_PLAIN && g->symmetric;
+    if (vw == 0 && tile == 0 && (b->tuned_vw >= 0 || !untuned)) {
       if (b->tuned_vw < 0) {
         st = fcd::batch_autotune(g, s, t, n, o.policy, lanes);
         if (st != FC_OK) return st;

@@ -694,18 +694,24 @@ static fc_status graph_create(const OffT* off, const int32_t* col, int64_t V, in
   };
   {
     double d2 = 0.0;
+    int64_t active = 0;
     for (int64_t v = 0; v < V; ++v) {
       const double d = (double)((int64_t)off[v + 1] - (int64_t)off[v]);
       d2 += d * d;
+      active += d > 0.0;
     }
-    g->f_branch = (float)(std::log2(1.0 + (E > 0 ? d2 / (double)E : 0.0)) / 16.0);
+    g->branch = E > 0 ? d2 / (double)E : 0.0;
+    const double mean = active > 0 ? (double)E / (double)active : 0.0;
+    g->regular = E > 0 && g->branch < mean + 0.5;
+    g->skewed = g->branch > 4.0 * mean;
+    g->f_branch = (float)(std::log2(1.0 + g->branch) / 16.0);
     // A vertex reached over an edge leads to at most five others on average:
     // frontiers grow slowly or, on a grid, hardly. Measured (start engine
     // against narrow visits, device time): 2048^2 grid (3.9), a BFS 30.4
     // against 10.4 ms; a random graph of mean degree 3 (4.0), 50K vertices, a
     // BFS 0.25 against 0.16 ms, 64 queries 0.32 against 0.29; of degree 8
     // (9.0), 64 queries 0.15 against 0.18.
-    g->narrow = E > 0 && d2 / (double)E <= 6.0;
+    g->narrow = E > 0 && g->branch <= 6.0;
   }
 #define CK(call)                                            \
   do {                                                      \

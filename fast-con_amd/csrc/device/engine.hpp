@@ -34,7 +34,10 @@ struct fc_graph {
   int32_t hub_threshold = 4096;
   bool symmetric = false;       // every edge is stored in both directions (checked by hash sums)
   bool hub_steps = false;       // the top vertices are on enough edges for hub steps
-  float f_branch = 0.f;         // scheduler feature: log2(1 + sum d^2 / sum d) / 16
+  double branch = 0.0;          // sum d^2 / sum d: the mean degree of a vertex reached over an edge
+  bool regular = false;         // degrees hardly differ: a grid, a mesh
+  bool skewed = false;          // branch is several mean degrees: hubs
+  float f_branch = 0.f;         // scheduler feature: log2(1 + branch) / 16
   uint32_t hcap = 1;
   uint32_t qcap = 1;
 

@@ -338,10 +338,12 @@ typedef struct fc_batch_stats {
 /* Batched s–t: queries are run as bit-parallel waves of up to 64 (one uint64
  * mask per vertex and side). Verdicts and distances equal fc_stcon's.
  * With lanes = 0 a batch runs in one launch when every edge of the graph is
- * stored in both directions (checked at creation), V < 2^28, and the machines'
- * workspaces (about 85 bytes per vertex each) fit (see Memory above); otherwise it runs three launch-driven machines. There the
- * heuristic and learned schedules also run hub steps on skewed graphs: meets
- * at the 512 vertices of the highest degree, with the same exact distances. */
+ * stored in both directions (checked at creation), V < 2^28, the machines'
+ * workspaces fit (see Memory above), and, under the plain schedule, its waves
+ * are narrow or many enough; otherwise it runs three launch-driven machines.
+ * In one launch the heuristic and learned schedules also run hub steps on
+ * skewed graphs: meets at the 512 vertices of the highest degree, with the
+ * same exact distances. */
 fc_status fc_stcon_batch(fc_graph* g, const int32_t* s, const int32_t* t, int32_t n,
                          int32_t* connected, int32_t* dist, const fc_batch_opts* opts,
                          fc_batch_stats* stats);

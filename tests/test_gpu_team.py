@@ -164,3 +164,39 @@ def test_narrow_visits(fc, orc, monkeypatch, name):
                 assert np.array_equal(x.dist, exp[:n]) and np.array_equal(x.connected, r.connected)
                 for k in keys + ("depth", "topdown_levels"):
                     assert x.stats[k] == r.stats[k], (name, n, k)
+
+
+def _mesh(fc, n):  # n x n x n
+    k = np.arange(n ** 3).reshape(n, n, n)
+    e = [np.stack([a.ravel(), b.ravel()], 1)
+         for a, b in ((k[:-1], k[1:]), (k[:, :-1], k[:, 1:]), (k[:, :, :-1], k[:, :, 1:]))]
+    e = np.concatenate(e)
+    u, v = np.concatenate([e, e[:, ::-1]]).T
+    order = np.lexsort((v, u))
+    off = np.concatenate([[0], np.cumsum(np.bincount(u, minlength=n ** 3))])
+    return fc.HostGraph(off, v[order].astype(np.int32))
+
+
+@pytest.mark.parametrize("name,one_launch,launches", [
+    ("rmat16", (1, 8, 1024), (64,)), ("er100k", (1, 64, 256), ()), ("er1m", (8, 256), (64, 128)),
+    ("grid300", (1, 64), ()), ("mesh48", (1, 256), (64,))])
+def test_plain_batches_by_width(fc, orc, name, one_launch, launches):
+    """The plain schedule's waves of 64 run in one launch where they are narrow
+    or many, else by launches: the same distances and counters on both."""
+    hg = {"rmat16": lambda: fc.gen_rmat(16, 16, seed=9), "er100k": lambda: fc.gen_er(100000, 8.0, 9),
+          "er1m": lambda: fc.gen_er(1000000, 16.0, 9), "grid300": lambda: fc.gen_grid(300, 300, 0.02, 9),
+          "mesh48": lambda: _mesh(fc, 48)}[name]()
+    rng = np.random.default_rng(51)
+    s = rng.integers(0, hg.V, 1024).astype(np.int32)
+    t = rng.integers(0, hg.V, 1024).astype(np.int32)
+    exp = oracle_pair_dists(orc, hg, s[:16], t[:16])
+    with fc.Graph(hg) as g:
+        for n in one_launch + launches:
+            r = g.stcon_batch(s[:n], t[:n], policy=fc.POLICY_PLAIN)
+            assert (r.stats["launches"] == 1) == (n in one_launch), n
+            k = min(n, 16)
+            assert np.array_equal(r.dist[:k], exp[:k])
+            ref = g.stcon_batch(s[:n], t[:n], policy=fc.POLICY_PLAIN, lanes=1, tile=256)
+            assert np.array_equal(r.dist, ref.dist)
+            for key in ("waves", "levels", "active_vertices", "active_edges", "touched_vertices"):
+                assert r.stats[key] == ref.stats[key], (n, key)
