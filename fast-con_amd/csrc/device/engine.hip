@@ -242,6 +242,18 @@ static fc_status st_teams_alloc(fc_graph* g) {
   return FC_OK;
 }
 
+// A query that reaches a level of more than this many edges per query of its
+// call is given up and run again by launches: an XCD takes about as long for
+// such a level (3.4 G claims/s) as the launches for all of the call's queries.
+// Unbounded, a few hub expansions held up whole calls: R-MAT s24, 3, 6, 16 and
+// 64 queries 0.78, 0.68, 1.53 and 2.44 ms, given up at 2^17 0.18, 0.25, 0.63
+// and 1.49, by launches alone 0.21, 0.34, 0.93 and 3.01; s22, 64 queries 2.21,
+// 0.95 and 2.16; two queries between two random graphs of 1M vertices, which
+// they exhaust, 2.49, 1.05 and 1.07. At 2^16 and 2^18 within 5% of that. Where
+// more than half of a call's eight or more queries are given up (64 such
+// queries: 38 ms, unbounded 23), the graph's next calls are not bounded.
+constexpr int64_t kTeamLevelEdges = 1 << 17;
+
 // Whether n queries go to the teams: several always (eight are visited at a
 // time: R-MAT s22, 16 queries, 0.42 -> 0.23 ms); a single one where its
 // frontiers are likely to stay narrow (random graph of 50K vertices and degree
@@ -366,6 +378,7 @@ static fc_status st_teams_run(fc_graph* g, const int32_t* s, const int32_t* t, i
   const int blocks = narrow ? w->narrow_blocks : w->blocks;
   tr.expected = (uint32_t)(blocks / kXcds);
   tr.parents = par_out != nullptr;
+  tr.max_edges = n >= kXcds && !g->st_limit ? INT64_MAX : (int64_t)n * kTeamLevelEdges;
   w->epoch_next += (uint32_t)n;
   const int few = n <= kStartPairs ? n : 0;
   if (!few) {
@@ -447,6 +460,36 @@ __global__ __launch_bounds__(kWave) void visit_start_kernel(const VisitStart v, 
   }
 }
 
+// Run the queries among s, t whose visit was given up (kTooWide) again and put
+// their results in place; *found: whether there were any.
+template <typename Run>
+static fc_status redo_wide(fc_graph* g, const int32_t* s, const int32_t* t, int32_t n, double* ms, bool* found, Run run) {
+  std::vector<int32_t> idx, vs, vt;
+  for (int32_t i = 0; i < n; ++i)
+    if (g->h_out[i].status == kTooWide) {
+      idx.push_back(i);
+      vs.push_back(s[i]);
+      vt.push_back(t[i]);
+    }
+  *found = !idx.empty();
+  if (idx.empty()) return FC_OK;
+  const std::vector<VisitOut> kept(g->h_out, g->h_out + n);
+  double more = 0.0;
+  const fc_status st = run(vs.data(), vt.data(), (int32_t)idx.size(), &more);
+  if (st != FC_OK) return st;
+  const std::vector<VisitOut> again(g->h_out, g->h_out + idx.size());
+  std::copy(kept.begin(), kept.end(), g->h_out);
+  for (size_t k = 0; k < idx.size(); ++k) {
+    g->h_out[idx[k]] = again[k];
+    g->h_out[idx[k]].launches += kept[(size_t)idx[k]].launches;  // the first call's one
+  }
+  *ms += more;
+  return FC_OK;
+}
+
+static fc_status run_launches(fc_graph* g, int mode, const int32_t* s, const int32_t* t, int32_t n, bool parents,
+                              double* ms, const VisitTail& tail, const VisitTail& after);
+
 fc_status run_visits(fc_graph* g, int mode, const int32_t* s, const int32_t* t, int32_t n, bool parents,
                      double* ms, const VisitTail& tail, const VisitTail& after) {
   *ms = 0.0;
@@ -454,34 +497,29 @@ fc_status run_visits(fc_graph* g, int mode, const int32_t* s, const int32_t* t, 
   fc_status st = ensure_queries(g, n);
   if (st != FC_OK) return st;
   if (mode == kModePlainSt && !parents && st_teams_take(g, n)) {
-    bool ran = false;
+    bool ran = false, found = false;
     const bool narrow = g->narrow && g->narrow_st;
     st = st_teams_run(g, s, t, n, narrow, false, nullptr, nullptr, ms, &ran);
     if (st != FC_OK) return st;
     if (ran && narrow) {
-      // the queries whose frontiers grew too wide run again, and the next
-      // calls on this graph do not try
-      std::vector<int32_t> idx, vs, vt;
-      for (int32_t i = 0; i < n; ++i)
-        if (g->h_out[i].status == kTooWide) {
-          idx.push_back(i);
-          vs.push_back(s[i]);
-          vt.push_back(t[i]);
-        }
-      if (!idx.empty()) {
-        g->narrow_st = false;
-        const std::vector<VisitOut> kept(g->h_out, g->h_out + n);
-        double more = 0.0;
-        st = st_teams_run(g, vs.data(), vt.data(), (int32_t)idx.size(), false, false, nullptr, nullptr, &more, &ran);
-        if (st != FC_OK) return st;
-        std::vector<VisitOut> again(g->h_out, g->h_out + idx.size());
-        std::copy(kept.begin(), kept.end(), g->h_out);
-        for (size_t k = 0; k < idx.size(); ++k) g->h_out[idx[k]] = again[k];
-        *ms += more;
-      }
+      st = redo_wide(g, s, t, n, ms, &found, [&](const int32_t* vs, const int32_t* vt, int32_t k, double* more) {
+        return st_teams_run(g, vs, vt, k, false, false, nullptr, nullptr, more, &ran);
+      });
+      if (st != FC_OK) return st;
+      if (found) g->narrow_st = false;  // the next calls on this graph do not try
     }
-    if (ran) return FC_OK;
+    if (ran)
+      return redo_wide(g, s, t, n, ms, &found, [&](const int32_t* vs, const int32_t* vt, int32_t k, double* more) {
+        if (n >= kXcds && k > n / 2) g->st_limit = false;
+        return run_launches(g, mode, vs, vt, k, false, more, {}, {});
+      });
   }
+  return run_launches(g, mode, s, t, n, parents, ms, tail, after);
+}
+
+static fc_status run_launches(fc_graph* g, int mode, const int32_t* s, const int32_t* t, int32_t n, bool parents,
+                              double* ms, const VisitTail& tail, const VisitTail& after) {
+  fc_status st = FC_OK;
   if (g->use_graphs) {
     st = ensure_graph(g);
     if (st != FC_OK) return st;

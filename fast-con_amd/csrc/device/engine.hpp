@@ -95,6 +95,7 @@ struct fc_graph {
   bool use_st_teams = true;          // FASTCON_PLAIN_TEAMS=0: every visit through the launches
   bool narrow = false;               // even degrees: visits are likely to stay narrow (narrow_kernel)
   bool narrow_st = true, narrow_bfs = true;  // until one did not
+  bool st_limit = true;              // wide levels are left to the whole GPU (kTeamLevelEdges), until most queries had one
   std::atomic<int> team_use{0};      // calls that use the two workspaces above; -1: they are being given back
 };
 

@@ -965,6 +965,9 @@ __global__ __launch_bounds__(W * kWave) void phase_kernel(VisitCtl* ctl, int par
 // launch (a 4096^2 grid: 8 us a level with launches), and eight queries run
 // at a time.
 //
+// A query with a level of more than max_edges edges is given up (kTooWide): the
+// caller runs it again by launches, on the whole GPU.
+//
 // Query k of a machine uses the counters of parity k mod 4. Block 0 clears
 // those of query k + 2 when query k starts: all blocks have then left query
 // k - 2, whose counters they were (its last reader passed a barrier of query
@@ -1027,6 +1030,7 @@ __global__ __launch_bounds__(kBlock) void st_team_kernel(StTeamRun tr) {
     }
     int steps = 0, td = 0, maxf = 1;
     int64_t vis_v = 2, vis_e = (int64_t)(ds + dt), expv = 2, expe = (int64_t)(ds + dt);
+    bool wide = (int64_t)(ds + dt) > tr.max_edges;  // then the roots are not expanded, and level 1 ends the query
     for (int L = 0;; ++L) {
       Ring cur[2] = {{0u, 0u, 0ull, ds}, {0u, 0u, 0ull, dt}};
       int vw0 = 4, vw1 = 4;
@@ -1049,11 +1053,13 @@ __global__ __launch_bounds__(kBlock) void st_team_kernel(StTeamRun tr) {
         // level (the error bits can: they only colour the result; a guard that
         // trips drops entries, so the visit still ends).
         const bool met = best != ~0ull, runaway = steps > p.V + 2;
-        if (met || nf0 == 0 || nf1 == 0 || runaway) {
+        const bool empty = nf0 == 0 || nf1 == 0;
+        wide |= !met && !empty && mf01 > tr.max_edges;
+        if (met || empty || wide || runaway) {
           if (lead) {
             const uint32_t err = ld_team(&ctl->v.err);
             VisitOut o;
-            o.status = (err || runaway) ? FC_CAPACITY_STATUS : 0;
+            o.status = (err || runaway) ? FC_CAPACITY_STATUS : wide ? kTooWide : 0;
             o.levels = steps;
             o.depth = met ? steps : 0;
             o.dist = met ? (int32_t)(best >> 32) : -1;
@@ -1107,7 +1113,7 @@ __global__ __launch_bounds__(kBlock) void st_team_kernel(StTeamRun tr) {
       a.h.cnt = 0;
       auto push = [&](bool claimed, int32_t u, OffT, int64_t deg) { push_next(a, claimed, u, deg, false); };
       if (L == 0) {
-        td_root<true>(a, (int32_t*)nullptr, cw ? dst : src, s_root[2 * cw], s_root[2 * cw + 1], lw, nlw, push);
+        if (!wide) td_root<true>(a, (int32_t*)nullptr, cw ? dst : src, s_root[2 * cw], s_root[2 * cw + 1], lw, nlw, push);
       } else {
         td_normal<true>(a, (int32_t*)nullptr, true, cw ? vw1 : vw0, L, L & 1, cw ? cur[1].n : cur[0].n, lw, nlw, push);
         td_hubs<true>(a, (int32_t*)nullptr, true, L, L & 1, cw ? cur[1].hub : cur[0].hub, lw, nlw, push);

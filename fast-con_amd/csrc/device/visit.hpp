@@ -182,7 +182,7 @@ struct StTeamCtl {
   alignas(128) unsigned long long word[2][kWave];  // by level parity: a block's narrow_word
 };
 constexpr int kNarrowThreads = 1024;
-constexpr int32_t kTooWide = 100;  // VisitOut::status: the frontier outgrew a narrow visit
+constexpr int32_t kTooWide = 100;  // VisitOut::status: the frontier outgrew a narrow visit, or a level a team
 
 struct TeamSync;
 struct TeamBar;
@@ -198,6 +198,7 @@ struct StTeamRun {
   int32_t vw_fixed;     // st_team_kernel: 0: from the frontier's degrees; narrow visits: of the published vertices
   uint32_t expected;    // blocks per XCD
   int32_t parents;      // narrow BFS: record parents
+  int64_t max_edges;    // st_team_kernel: a query with a level of more edges is given up (kTooWide)
 };
 
 constexpr int kFeatures = 12;

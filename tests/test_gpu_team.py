@@ -200,3 +200,49 @@ def test_plain_batches_by_width(fc, orc, name, one_launch, launches):
             assert np.array_equal(r.dist, ref.dist)
             for key in ("waves", "levels", "active_vertices", "active_edges", "touched_vertices"):
                 assert r.stats[key] == ref.stats[key], (n, key)
+
+
+@pytest.mark.parametrize("name", ["rmat19", "star", "two"])
+def test_wide_levels_go_to_the_whole_gpu(fc, orc, monkeypatch, name):
+    """Queries that a team gives up at a wide level (rmat19), at the root
+    (star: 400,000 edges at level 0) or all of them (two: unconnected, and
+    more than half of a call) come back with the launches' answers and
+    counters, and so do the others of the call."""
+    def star():
+        k = np.arange(1, 400001)
+        off = np.concatenate([[0, 400000], 400000 + np.arange(1, 400001)])
+        return fc.HostGraph(off, np.concatenate([k, np.zeros(400000)]).astype(np.int32))
+
+    def two():
+        h = fc.gen_er(200000, 16.0, 5)
+        return fc.HostGraph(np.concatenate([h.offsets, h.offsets[1:] + h.E]), np.concatenate([h.columns, h.columns + h.V]))
+
+    hg = {"rmat19": lambda: fc.gen_rmat(19, 16, seed=61), "star": star, "two": two}[name]()
+    rng = np.random.default_rng(62)
+    s = rng.integers(0, hg.V // 2, 40).astype(np.int32)
+    t = rng.integers(hg.V // 2, hg.V, 40).astype(np.int32)
+    if name == "star":
+        s[1::2] = 0
+    keys = ("levels", "depth", "visited_vertices", "visited_edges", "expanded_vertices", "expanded_edges",
+            "topdown_levels", "max_frontier")
+    monkeypatch.setenv("FASTCON_PLAIN_TEAMS", "0")
+    with fc.Graph(hg) as g:
+        if name == "rmat19":  # the heaviest of many first
+            s, t = rng.integers(0, hg.V, (2, 300)).astype(np.int32)
+            work = [g.stcon(int(a), int(b))[3]["expanded_edges"] for a, b in zip(s, t)]
+            top = np.argsort(work)[::-1][:40]
+            assert work[top[0]] > 1 << 19
+            s, t = s[top], t[top]
+        ref = {n: g.stcon_many(s[:n], t[:n]) for n in (1, 2, 3, 9, 40)}
+    monkeypatch.delenv("FASTCON_PLAIN_TEAMS")
+    assert np.array_equal(ref[9].dist, oracle_pair_dists(orc, hg, s[:9], t[:9]))
+    launches = {}
+    with fc.Graph(hg) as g:
+        for _ in range(2):
+            for n, r in ref.items():
+                x = g.stcon_many(s[:n], t[:n])
+                launches[n] = x.stats["launches"]
+                assert np.array_equal(x.dist, r.dist) and np.array_equal(x.connected, r.connected), n
+                for k in keys:
+                    assert x.stats[k] == r.stats[k], (n, k)
+    assert max(launches[2], launches[3]) > 1  # some were given up
