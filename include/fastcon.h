@@ -32,7 +32,10 @@
  *
  * Threading: one fc_graph per host thread; each fc_graph owns one HIP stream
  * (default priority) and its own device workspace. Calls are synchronous from
- * the caller's point of view.
+ * the caller's point of view. A call that runs inside one launch (below) holds
+ * the GPU's compute units until it ends: a short call of another thread waits
+ * for it. FASTCON_BATCH_TEAMS=0 and FASTCON_PLAIN_TEAMS=0 run such calls
+ * launch by launch, slower, with other threads' launches between theirs.
  *
  * Memory: the CSR and about 50 bytes per vertex at creation. Calls that run
  * inside one launch (fc_stcon_batch, fc_stcon_many, fc_stcon and fc_bfs on

@@ -246,3 +246,32 @@ def test_wide_levels_go_to_the_whole_gpu(fc, orc, monkeypatch, name):
                 for k in keys:
                     assert x.stats[k] == r.stats[k], (n, k)
     assert max(launches[2], launches[3]) > 1  # some were given up
+
+
+def test_two_callers_at_a_time(fc, orc):
+    """One graph per thread is a supported use: one-launch calls that find the
+    GPU taken, or a part of it, and launches between them, answer as they do
+    alone."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    def work(hg, seed):
+        rng = np.random.default_rng(seed)
+        s, t = rng.integers(0, hg.V, (2, 300)).astype(np.int32)
+        return hg, s, t, oracle_pair_dists(orc, hg, s, t, workers=4), orc.bfs(hg.offsets, hg.columns, int(s[0]))[0]
+
+    def call(w):
+        hg, s, t, exp, lv = w
+        with fc.Graph(hg) as g:
+            for k in range(12):
+                n = (300, 40, 9, 2)[k % 4]
+                assert np.array_equal(g.stcon_batch(s[:n], t[:n]).dist, exp[:n])
+                assert np.array_equal(g.stcon_many(s[:n], t[:n]).dist, exp[:n])
+                assert np.array_equal(g.stcon_batch(s[:n], t[:n], policy=fc.POLICY_PLAIN, lanes=2, tile=256).dist, exp[:n])
+                assert np.array_equal(g.bfs(int(s[0]))[0], lv)
+                assert g.stcon(int(s[k]), int(t[k]))[1] == exp[k]
+        return True
+
+    graphs = [work(fc.gen_rmat(14, 16, seed=71), 1), work(fc.gen_grid(150, 150, 0.02, 72), 2)]
+    for pair in ((graphs[0], graphs[1]), (graphs[0], graphs[0]), (graphs[1], graphs[1])):
+        with ThreadPoolExecutor(2) as ex:
+            assert all(ex.map(call, pair))
