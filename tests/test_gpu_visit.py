@@ -380,3 +380,30 @@ def test_widths_that_are_no_powers_of_two(fc, orc, monkeypatch, vw):
             assert np.array_equal(g.bfs(int(r))[0], orc.bfs(hg.offsets, hg.columns, int(r))[0])
         assert np.array_equal(g.stcon_many(s, t).dist, exp)
         assert [g.stcon(int(a), int(b))[1] for a, b in zip(s, t)] == list(exp)
+
+
+def test_repeated_edges_keep_a_graph_undirected(fc, orc):
+    """An undirected graph some of whose lists repeat a neighbour that the
+    other end lists once: still bottom-up levels and one-launch batches; with
+    one direction of one edge left out, neither."""
+    h = fc.gen_rmat(13, 16, seed=81)
+    src = np.repeat(np.arange(h.V), h.degree())
+    e = np.stack([src, h.columns], 1)
+    rng = np.random.default_rng(82)
+    for whole in (True, False):
+        x = np.concatenate([e, e[rng.integers(0, len(e), 500)], np.repeat(e[:3], 70, axis=0)])
+        if not whole:
+            gone = e[rng.integers(len(e))]
+            x = x[(x != gone).any(axis=1)]
+        x = x[np.lexsort((x[:, 1], x[:, 0]))]
+        hg = fc.HostGraph(np.concatenate([[0], np.cumsum(np.bincount(x[:, 0], minlength=h.V))]), x[:, 1].astype(np.int32))
+        r = int(np.argmax(hg.degree()))
+        with fc.Graph(hg) as g:
+            lv, _, st = g.bfs(r)
+            assert np.array_equal(lv, orc.bfs(hg.offsets, hg.columns, r)[0])
+            assert (st["bottomup_levels"] > 0) == whole
+            s, t = rng.integers(0, h.V, (2, 200)).astype(np.int32)
+            b = g.stcon_batch(s, t)
+            assert (b.stats["launches"] == 1) == whole
+            if whole:
+                assert np.array_equal(b.dist, [orc.stcon(hg.offsets, hg.columns, int(i), int(j))[1] for i, j in zip(s, t)])
