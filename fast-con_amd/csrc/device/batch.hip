@@ -1394,7 +1394,6 @@ __device__ __forceinline__ int batch_finalize(const BatchParams<OffT>& p, BatchC
       const unsigned long long hit = r.v[kROdd] & act;
       fd = FinDist{hit, 0ull, 0ull, ctl->lvl[0] + ctl->lvl[1]};
       ctl->act = act & ~hit;
-      ctl->hub_steps++;
       return batch_next(ctl, true);
     }
     case kBClearF: {

@@ -88,7 +88,6 @@ struct BatchCtl {
   int32_t bridge_lv;       // (lvl[0] + 1) << 16 | (lvl[1] + 1) of this wave's last bridge step (0: none)
   int32_t bridges;         // bridge steps (whole batch)
   int32_t hub_lv;          // as bridge_lv, of the last hub step
-  int32_t hub_steps;       // hub steps (whole batch)
   unsigned long long hub_min_e;   // a hub step runs when the frontiers have at least this many live edges
   int64_t bridged;         // queries answered by bridge steps (whole batch)
   uint32_t ticket;

@@ -275,3 +275,21 @@ def test_two_callers_at_a_time(fc, orc):
     for pair in ((graphs[0], graphs[1]), (graphs[0], graphs[0]), (graphs[1], graphs[1])):
         with ThreadPoolExecutor(2) as ex:
             assert all(ex.map(call, pair))
+
+
+def test_hub_steps_answer_queries(fc, orc, monkeypatch):
+    """A hub step answers, before the bridge step of the same levels, the
+    queries whose balls meet at a top vertex: fewer are left to the bridges,
+    and the distances are the same."""
+    hg = fc.gen_rmat(13, 16, seed=91)
+    s, t = np.random.default_rng(92).integers(0, hg.V, (2, 512)).astype(np.int32)
+    exp = oracle_pair_dists(orc, hg, s, t)
+    monkeypatch.setenv("FASTCON_BRIDGE_MIN_EDGES", "1")
+    got = {}
+    with fc.Graph(hg) as g:
+        for least in ("1", str(1 << 56)):
+            monkeypatch.setenv("FASTCON_HUB_MIN_EDGES", least)
+            r = g.stcon_batch(s, t)
+            assert r.stats["launches"] == 1 and np.array_equal(r.dist, exp)
+            got[least] = r.stats
+    assert got["1"]["bridged"] < got[str(1 << 56)]["bridged"]
