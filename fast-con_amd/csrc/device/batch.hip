@@ -271,7 +271,7 @@ __device__ __forceinline__ void appends_block_flush(const BatchParams<OffT>& p, 
 // a load and an update so that a lane's loads for several edges are in
 // flight together. The update ORs the new bits into u's N word with an
 // atomic that returns nothing and, when the loaded N word was zero, marks
-// u's group of 32 vertices with a plain byte store (every writer stores the
+// u's group of eight vertices with a plain byte store (every writer stores the
 // same value, so the race is benign). Every vertex whose N word becomes
 // non-zero is in a marked group: the first atomic on it is issued by a lane
 // whose earlier load saw zero.

@@ -9,10 +9,12 @@
 // fc_stcon replaces make_stcon's single-GPU path (st-conn/make_stcon.c:730-1497).
 //
 // Queries run through the device-side phase machine of visit.hip: the host
-// writes the query list and an initial control block, then replays a
-// captured hipGraph of identical phase launches (or launches them directly
-// when only a few are needed), reading back the 8-byte phase word between
-// batches to know whether every query has finished.
+// starts it with one small launch that writes the control block, then replays
+// a captured hipGraph of identical phase launches (or launches them directly
+// when only a few are needed). The launches write a query's result to pinned
+// memory when it is finished, where the host looks between batches of
+// launches. Lists of plain queries, and visits that stay narrow, run inside
+// one launch instead (st_teams_run).
 #include "engine.hpp"
 #include "team.hpp"
 

@@ -55,8 +55,8 @@ struct fc_graph {
   int64_t* d_hb[2][2] = {};
   fcd::VisitCtl* d_ctl = nullptr;
 
-  // Query lists and results of the phase machine (device), with a pinned
-  // host copy of the results; capacity q_cap.
+  // Query lists of the phase machine (device) and its results (pinned host
+  // memory); capacity q_cap.
   int32_t* d_qs = nullptr;
   int32_t* d_qt = nullptr;
   fcd::VisitOut* h_out = nullptr;   // pinned; the visits' launches write it
@@ -102,7 +102,7 @@ struct fc_graph {
 namespace fcd {
 
 constexpr int kGraphLaunches = 16;
-constexpr int64_t kPollLaunches = 4096;  // launches queued between two host polls of the phase word
+constexpr int64_t kPollLaunches = 4096;  // launches queued between two looks of the host at the results
 
 fc_status hip_fail(hipError_t e, const char* what);
 
