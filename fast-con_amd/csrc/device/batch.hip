@@ -638,6 +638,12 @@ __device__ __forceinline__ void bottom_up(const BatchParams<OffT>& p, const Batc
   const int nxt[2] = {uni<TEAM>(rc->cur[0]) ^ 1, uni<TEAM>(rc->cur[1]) ^ 1};
   const unsigned long long* FS = p.F[0][uni<TEAM>(rc->cur[0])];
   const unsigned long long* FT = p.F[1][uni<TEAM>(rc->cur[1])];
+  // The first expanded side's masks, and whether there is a second: one branch
+  // a round, so that its four loads stay in flight together. R-MAT s16 by
+  // launches (heuristic schedule, 256 queries) takes 3.07 ms; with a branch per
+  // load and side it took 4.87, with code for each set of sides 4.36.
+  const unsigned long long* F0 = DS ? FS : FT;
+  const bool two = DS && DT;
   const int lane = lane_id();
   const int64_t nthr = (int64_t)nwaves * kWave;
   // isolated vertices (the tail of a degree-ordered numbering) gain no bit
@@ -659,21 +665,26 @@ __device__ __forceinline__ void bottom_up(const BatchParams<OffT>& p, const Batc
     }
     if (b < e) {
       red[kRActV] += 1;
+      const unsigned long long need0 = DS ? needS : needT;
+      unsigned long long acc0 = 0, acc1 = 0;
       for (OffT j = b; j < e; j += 4) {
         int32_t c[4];
-        c[0] = p.col[j];
-        c[1] = j + 1 < e ? p.col[j + 1] : -1;
-        c[2] = j + 2 < e ? p.col[j + 2] : -1;
-        c[3] = j + 3 < e ? p.col[j + 3] : -1;
+        unsigned long long m[4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          if (c[k] < 0) continue;
-          if (DS) accS |= ldw<TEAM>(FS + c[k]);
-          if (DT) accT |= ldw<TEAM>(FT + c[k]);
+        for (int k = 0; k < 4; ++k) c[k] = p.col[j + k < e ? j + k : e - 1];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) m[k] = ldw<TEAM>(F0 + c[k]);
+        acc0 |= m[0] | m[1] | m[2] | m[3];
+        if (two) {
+#pragma unroll
+          for (int k = 0; k < 4; ++k) m[k] = ldw<TEAM>(FT + c[k]);
+          acc1 |= m[0] | m[1] | m[2] | m[3];
         }
         red[kRActE] += (unsigned long long)((j + 4 <= e) ? 4 : (e - j));
-        if ((accS & needS) == needS && (accT & needT) == needT) break;
+        if ((acc0 & need0) == need0 && (!two || (acc1 & needT) == needT)) break;
       }
+      accS = DS ? acc0 : 0ull;
+      accT = DS ? acc1 : acc0;
     }
     const unsigned long long nS = accS & needS, nT = accT & needT;
     int64_t deg = 0;
