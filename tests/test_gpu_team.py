@@ -293,3 +293,62 @@ def test_hub_steps_answer_queries(fc, orc, monkeypatch):
             assert r.stats["launches"] == 1 and np.array_equal(r.dist, exp)
             got[least] = r.stats
     assert got["1"]["bridged"] < got[str(1 << 56)]["bridged"]
+
+
+def _directed(fc, V, degree, seed):
+    rng = np.random.default_rng(seed)
+    e = np.unique(np.stack([np.repeat(np.arange(V), degree), rng.integers(0, V, V * degree)], 1), axis=0)
+    off = np.concatenate([[0], np.cumsum(np.bincount(e[:, 0], minlength=V))])
+    return fc.HostGraph(off, e[:, 1].astype(np.int32), directed=True)
+
+
+@pytest.mark.parametrize("degree", [2, 8])
+def test_plain_visits_of_directed_graphs(fc, orc, monkeypatch, degree):
+    """Queries and BFS inside one launch on directed graphs (degree 2: narrow
+    visits, 8: eight queries at a time) as by launches."""
+    hg = _directed(fc, 30000, degree, 101)
+    s, t = np.random.default_rng(102).integers(0, hg.V, (2, 300)).astype(np.int32)
+    keys = ("levels", "depth", "visited_vertices", "visited_edges", "expanded_vertices", "expanded_edges", "max_frontier")
+    monkeypatch.setenv("FASTCON_PLAIN_TEAMS", "0")
+    with fc.Graph(hg) as g:
+        ref = {n: g.stcon_many(s[:n], t[:n]) for n in (1, 2, 9, 300)}
+        lv = g.bfs(int(s[0]))[0]
+    monkeypatch.delenv("FASTCON_PLAIN_TEAMS")
+    assert np.array_equal(lv, orc.bfs(hg.offsets, hg.columns, int(s[0]))[0])
+    for off64, keep_ids in ((False, False), (True, False), (False, True)):
+        with fc.Graph(hg, force64=off64, keep_ids=keep_ids) as g:
+            for n, r in ref.items():
+                x = g.stcon_many(s[:n], t[:n])
+                assert np.array_equal(x.dist, r.dist) and np.array_equal(x.connected, r.connected)
+                for k in keys:
+                    assert x.stats[k] == r.stats[k], (n, k)
+            assert np.array_equal(g.bfs(int(s[0]))[0], lv)
+
+
+def test_plain_batches_of_directed_graphs(fc):
+    """The plain schedule on a directed graph against a host visit by its
+    rules: both balls grow along the edges at each step, and the first meet
+    sets the distance."""
+    hg = _directed(fc, 2000, 3, 103)
+    out = [set(hg.columns[hg.offsets[v]:hg.offsets[v + 1]].tolist()) for v in range(hg.V)]
+
+    def visit(a, b):
+        if a == b:
+            return 0
+        ball, front = [{a}, {b}], [{a}, {b}]
+        for step in range(hg.V):
+            new = [set().union(*(out[v] for v in front[x])) - ball[x] for x in (0, 1)]
+            if new[0] & ball[1] or new[1] & ball[0]:
+                return 2 * step + 1
+            if new[0] & new[1]:
+                return 2 * step + 2
+            if not new[0] or not new[1]:
+                return -1
+            ball, front = [ball[x] | new[x] for x in (0, 1)], new
+
+    s, t = np.random.default_rng(104).integers(0, hg.V, (2, 200)).astype(np.int32)
+    t[::50] = s[::50]
+    exp = [visit(int(a), int(b)) for a, b in zip(s, t)]
+    with fc.Graph(hg) as g:
+        r = g.stcon_batch(s, t, policy=fc.POLICY_PLAIN)
+        assert r.stats["launches"] > 1 and list(r.dist) == exp
