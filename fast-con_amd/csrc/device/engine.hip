@@ -893,6 +893,7 @@ static fc_status graph_create(const OffT* off, const int32_t* col, int64_t V, in
 
 // For tests on hosts without a GPU.
 extern "C" int32_t fcd_visit_width(int32_t asked) { return fcd::visit_width(asked); }
+extern "C" int32_t fcd_query_set(int32_t q) { return fcd::query_set(q); }
 extern "C" int32_t fcd_team_admit(uint32_t k, uint32_t expected) { return fcd::team_admit(k, expected); }
 
 extern "C" fc_status fc_graph_create_csr32(const int32_t* off, const int32_t* col, int32_t V, int64_t E,

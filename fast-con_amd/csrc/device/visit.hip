@@ -766,7 +766,7 @@ __global__ __launch_bounds__(W * kWave) void phase_kernel(VisitCtl* ctl, int par
   // (Scalars only below: a local copy of the state, or arrays indexed by the
   // colour, would be put in scratch memory.)
   int q = S.qi, L = S.lvl;
-  int qp = q & 1;
+  int qp = query_set(q);
   int32_t src = S.src, dst = S.dst;
   uint32_t epoch = S.epoch;
   bool start = st && L == 0;  // s–t: this launch expands the roots of query q
@@ -812,7 +812,7 @@ __global__ __launch_bounds__(W * kWave) void phase_kernel(VisitCtl* ctl, int par
       }
       // the next s–t query starts in this launch
       ++q;
-      qp = q & 1;
+      qp = query_set(q);
       src = S.nsrc;
       dst = S.ndst;
       epoch = S.epoch + 1;
@@ -860,11 +860,12 @@ __global__ __launch_bounds__(W * kWave) void phase_kernel(VisitCtl* ctl, int par
       }
       // the next query's counters (this query's level-1 ring was cleared when
       // the previous query started), and this query's level-2 ring
+      const int nq = query_set(q + 1);
       for (int c = 0; c < 2; ++c) {
-        for (int k = 0; k < 3; ++k) zero_ring(&ctl->ring[qp ^ 1][c][k]);
+        for (int k = 0; k < 3; ++k) zero_ring(&ctl->ring[nq][c][k]);
         zero_ring(&ctl->ring[qp][c][2]);
       }
-      ctl->best[qp ^ 1][0] = ctl->best[qp ^ 1][1] = ~0ull;
+      ctl->best[nq][0] = ctl->best[nq][1] = ~0ull;
     }
   } else {
     const double mu = (double)p.E - (double)seen;

@@ -86,12 +86,10 @@ struct VisitState {
   int32_t steps, td, bu, maxf;
   int32_t launches;
   int32_t bu_mode;          // BFS: direction-optimising switch state
-  int32_t pad[2];
   uint64_t seen_edges;      // sum of degrees of the vertices labelled before this level
   int64_t visited_v, visited_e, expv, expe;
-  int64_t pad2[3];
 };
-static_assert(sizeof(VisitState) == 128, "VisitState layout");
+static_assert(sizeof(VisitState) == 96, "VisitState layout");
 
 // Pointers into device memory. In the device pass they carry the global
 // address space: the kernel reads them from its LDS copy of the control
@@ -145,22 +143,30 @@ struct VisitParams {
                                              // where there is none; null: not kept
 };
 
+constexpr int kQuerySets = 3;
+#if defined(__HIPCC__)
+__host__ __device__
+#endif
+constexpr int query_set(int q) { return (int)((uint32_t)q % (uint32_t)kQuerySets); }
 // Control block: 1 KB, loaded whole by every block at the start of a launch
 // (one 16-byte load per lane of one wave).
 struct VisitCtl {
   VisitState st[2];                  // by launch parity
-  Ring ring[2][2][3];                // [query parity][colour][level % 3]
-  // by query parity and by the parity of the level that found it (a block that
-  // starts late must not read what this launch's first blocks propose):
+  // Counters, by query mod kQuerySets. A launch may notice the end of query q
+  // and start q + 1: its first blocks clear the counters of q + 2 while a block
+  // that starts late still reads those of q, so that three sets are needed.
+  Ring ring[kQuerySets][2][3];       // [query][colour][level % 3]
+  // by query and by the parity of the level that found it (a block that starts
+  // late must not read what this launch's first blocks propose):
   // (distance << 32) | meet vertex; ~0 = none
-  unsigned long long best[2][2];
+  unsigned long long best[kQuerySets][2];
   uint32_t err;                      // bit 0: queue slot out of range, bit 1: bad vertex id read,
                                      // bit 2: an s–t claim did not settle
   int32_t nq;                        // number of queries
   int32_t mode;
   int32_t vw_fixed;                  // 0: width from frontier degree
   int32_t record_parents;
-  int32_t pad[27];
+  int32_t pad[3];
   alignas(16) unsigned char params[320];  // VisitParams<OffT> of the run
 };
 static_assert(sizeof(VisitCtl) == 1024, "VisitCtl layout");

@@ -407,3 +407,24 @@ def test_repeated_edges_keep_a_graph_undirected(fc, orc):
             assert (b.stats["launches"] == 1) == whole
             if whole:
                 assert np.array_equal(b.dist, [orc.stcon(hg.offsets, hg.columns, int(i), int(j))[1] for i, j in zip(s, t)])
+
+
+@pytest.mark.parametrize("name", ["er", "rmat"])
+def test_lists_by_launches(fc, orc, monkeypatch, name):
+    """Long lists of short queries by launches: hundreds of launches that end
+    one query and start the next. Every answer, and the counters of the
+    one-launch engine."""
+    hg = fc.gen_er(100000, 3.0, 4) if name == "er" else fc.gen_rmat(12, 8, seed=95)
+    rng = np.random.default_rng(96)
+    s, t = rng.integers(0, hg.V, (2, 600)).astype(np.int32)
+    with fc.Graph(hg) as g:
+        ref = g.stcon_many(s, t)
+    exp = [orc.stcon(hg.offsets, hg.columns, int(a), int(b))[1] for a, b in zip(s, t)]
+    assert list(ref.dist) == exp
+    monkeypatch.setenv("FASTCON_PLAIN_TEAMS", "0")
+    with fc.Graph(hg) as g:
+        for _ in range(6):
+            r = g.stcon_many(s, t)
+            assert list(r.dist) == exp
+            for k in ("levels", "depth", "visited_vertices", "visited_edges", "expanded_vertices", "expanded_edges"):
+                assert r.stats[k] == ref.stats[k], k

@@ -338,3 +338,12 @@ def test_teams_admit_the_planned_blocks_only(fc):
         numbers = [admit(k, expected) for k in range(blocks)]
         assert [n for n in numbers if n >= 0] == list(range(min(blocks, expected, 128)))
     assert admit(0x80000000 - (1 << 32), 16) == -1  # closed
+
+
+def test_query_counters_outlive_their_last_reader(fc):
+    """The launch that starts query q writes the counters of q (its level-1
+    frontier) and clears those of q + 1, while blocks of it that start late
+    still read the end of q - 1 from theirs."""
+    s = fc.lib().fcd_query_set
+    for q in list(range(1, 50)) + [2 ** 31 - 2]:
+        assert len({s(q - 1), s(q), s(q + 1)}) == 3, q
