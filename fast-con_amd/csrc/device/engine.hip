@@ -156,7 +156,7 @@ static VisitParams<OffT> make_params(fc_graph* g) {
 }
 
 static hipError_t launch_raw(fc_graph* g, int parity) {
-  const bool wide = g->E >= kWideEdges && !g->narrow;
+  const bool wide = g->E >= kWideEdges && !g->narrow && !(g->regular && g->surface < kWideSurface);
   if (g->off64) return launch_phase<int64_t>(g->d_ctl, parity, g->blocks, wide, g->stream);
   return launch_phase<int32_t>(g->d_ctl, parity, g->blocks, wide, g->stream);
 }
@@ -748,6 +748,9 @@ static fc_status graph_create(const OffT* off, const int32_t* col, int64_t V, in
     const double mean = active > 0 ? (double)E / (double)active : 0.0;
     g->regular = E > 0 && g->branch < mean + 0.5;
     g->skewed = g->branch > 4.0 * mean;
+    // a mesh of D dimensions, with 2 D neighbours or 3^D - 1
+    const double dims = std::max(1.0, g->branch < 7.0 ? g->branch / 2.0 : std::log(1.0 + g->branch) / std::log(3.0));
+    if (g->regular) g->surface = g->branch * std::pow((double)active, 1.0 - 1.0 / dims);
     g->f_branch = (float)(std::log2(1.0 + g->branch) / 16.0);
     // A vertex reached over an edge leads to at most five others on average:
     // frontiers grow slowly or, on a grid, hardly. Measured (start engine

@@ -36,6 +36,7 @@ struct fc_graph {
   bool hub_steps = false;       // the top vertices are on enough edges for hub steps
   double branch = 0.0;          // sum d^2 / sum d: the mean degree of a vertex reached over an edge
   bool regular = false;         // degrees hardly differ: a grid, a mesh
+  double surface = 0.0;         // regular: edges on the surface of a ball half the graph wide, as expected
   bool skewed = false;          // branch is several mean degrees: hubs
   float f_branch = 0.f;         // scheduler feature: log2(1 + branch) / 16
   uint32_t hcap = 1;
