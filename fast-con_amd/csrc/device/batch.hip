@@ -2565,21 +2565,22 @@ constexpr int kTeamTile = 256;  // hub chunk when the caller gives none
 //    same time follow E^0.6 branch^0.25, a fit over R-MAT s14 to s24 and random
 //    graphs of 300K to 4M vertices, to within a quarter either way. With more
 //    waves more XCDs share the work.
-//  * Equal degrees of at most 8, a mesh of about branch / 2 dimensions: a ball's surface has about
-//    V^(1 - 2 / branch) vertices, over most of a wave's steps.
+//  * Equal degrees: a mesh, where the balls' surfaces (fc_graph::surface) stay
+//    wide over most of a wave's steps. 100^3 vertices with 26 neighbours, 8, 64, 256 and 1,024
+//    queries: 4.5 / 2.1, 26 / 7.0, 34 / 19, 75 / 66 ms; 1000^2 with 8: 7.2 /
+//    9.8, 25 / 17, 30 / 39, 66 / 123.
 //  * Four waves or more pay wherever no hub makes the steps long (the random
-//    graph above; that mesh with 1,024 queries: 137 and 133 ms, 64^3 11 and 29).
+//    graph above).
 constexpr double kPlainTeamWork = 8e5;
-constexpr double kPlainTeamMesh = 8e4;
+constexpr double kPlainTeamMesh = 1.2e5;
 static bool plain_teams(const fc_graph* g, int32_t n) {
   const double queries = (double)std::min(n, 64);
   const int waves = (n + 63) / 64;
+  const double w = (double)std::min(waves, kXcds);
+  if (g->regular)
+    return std::min(queries * g->surface, (double)g->E) <= kPlainTeamMesh * (waves < 4 ? w : 0.5 * w * w);
   if (!g->skewed && waves >= 4) return true;
-  if (g->regular && g->branch <= 8.0)
-    return queries * g->branch * std::pow((double)g->V, 1.0 - 2.0 / std::max(g->branch, 2.0)) <=
-           kPlainTeamMesh * (double)std::min(waves, kXcds);
-  return queries * std::pow((double)g->E, 0.6) * std::pow(g->branch, 0.25) <=
-         kPlainTeamWork * (1.5 * (double)std::min(waves, kXcds) - 0.5);
+  return queries * std::pow((double)g->E, 0.6) * std::pow(g->branch, 0.25) <= kPlainTeamWork * (1.5 * w - 0.5);
 }
 
 struct TeamWorkspace {
@@ -2885,9 +2886,11 @@ extern "C" fc_status fc_stcon_batch(fc_graph* g, const int32_t* s, const int32_t
     st = fcd::batch_alloc(g);
     if (st != FC_OK) return st;
     fcd::BatchWorkspace* b = g->batch;
-    // A plain batch that its width keeps off the teams takes the width by degree
-    // and chunks of 256 edges, which no pair the tuner tries beats by more than
-    // the runs differ, without the tuner's 24 runs.
+    // A plain batch that its width keeps off the teams runs without the tuner's
+    // 24 runs: with chunks of 256 edges and the width by degree no pair is
+    // faster by more than the runs differ, but on meshes of many neighbours, 8
+    // lanes a vertex (100^3 with 26, 64 queries: 5.0 ms, by degree 7.3; R-MAT
+    // s22 0.52 and 0.50).
     const bool untuned = o.lanes == 0 && o.policy == FC_POLICY_PLAIN && g->symmetric;
     if (vw == 0 && tile == 0 && (b->tuned_vw >= 0 || !untuned)) {
       if (b->tuned_vw < 0) {
@@ -2897,6 +2900,7 @@ extern "C" fc_status fc_stcon_batch(fc_graph* g, const int32_t* s, const int32_t
       vw = b->tuned_vw;
       tile = b->tuned_tile;
     }
+    if (untuned && vw == 0 && g->regular && g->branch > 8.0) vw = 8;
     if (tile == 0) tile = 256;
     st = fcd::batch_run(g, s, t, n, o.policy, vw, tile, o.use_graph != 0, &ms, &c, &launches, o.learn_margin, lanes);
     if (st != FC_OK) return st;
