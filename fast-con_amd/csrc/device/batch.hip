@@ -2870,14 +2870,22 @@ extern "C" fc_status fc_stcon_batch(fc_graph* g, const int32_t* s, const int32_t
   // The team engine takes every batch whose lanes the caller leaves open: a
   // number of lanes asks for that many launch-driven machines.
   bool ran = false;
+  // The width where the caller gives none: by the frontier's degrees (0), but
+  // 8 on meshes of many neighbours, whose lists overlap. 100^3 with 26, by
+  // degree (32 lanes) and at 8: heuristic schedule, 64 and 256 queries, 7.4 / 5.3
+  // and 22.5 / 15.1 ms, plain by launches, 64 queries, 7.3 / 5.0; at 16
+  // neighbours (random) and at 10 (a ring) within 6% either way.
+  const int mesh_vw = g->regular && g->branch > 16.0 ? 8 : 0;
   if (o.lanes == 0) {
     const fcd::TeamUse use(g);  // the distances are read in the workspace
     const int ttile = tile ? tile : fcd::kTeamTile;
     const int32_t* got = nullptr;
-    st = fcd::team_run(g, s, t, n, o.policy, vw, ttile, o.learn_margin, &ms, &c, &got, &ran);
+    const int tvw = vw ? vw : mesh_vw;
+    st = fcd::team_run(g, s, t, n, o.policy, tvw, ttile, o.learn_margin, &ms, &c, &got, &ran);
     if (st != FC_OK) return st;
     if (ran) {
       answer(got);
+      vw = tvw;
       tile = ttile;
       launches = 1;
     }
@@ -2887,10 +2895,8 @@ extern "C" fc_status fc_stcon_batch(fc_graph* g, const int32_t* s, const int32_t
     if (st != FC_OK) return st;
     fcd::BatchWorkspace* b = g->batch;
     // A plain batch that its width keeps off the teams runs without the tuner's
-    // 24 runs: with chunks of 256 edges and the width by degree no pair is
-    // faster by more than the runs differ, but on meshes of many neighbours, 8
-    // lanes a vertex (100^3 with 26, 64 queries: 5.0 ms, by degree 7.3; R-MAT
-    // s22 0.52 and 0.50).
+    // 24 runs: no pair of its is faster than this width and chunks of 256 edges
+    // by more than the runs differ.
     const bool untuned = o.lanes == 0 && o.policy == FC_POLICY_PLAIN && g->symmetric;
     if (vw == 0 && tile == 0 && (b->tuned_vw >= 0 || !untuned)) {
       if (b->tuned_vw < 0) {
@@ -2900,7 +2906,7 @@ extern "C" fc_status fc_stcon_batch(fc_graph* g, const int32_t* s, const int32_t
       vw = b->tuned_vw;
       tile = b->tuned_tile;
     }
-    if (untuned && vw == 0 && g->regular && g->branch > 8.0) vw = 8;
+    if (untuned && vw == 0) vw = mesh_vw;
     if (tile == 0) tile = 256;
     st = fcd::batch_run(g, s, t, n, o.policy, vw, tile, o.use_graph != 0, &ms, &c, &launches, o.learn_margin, lanes);
     if (st != FC_OK) return st;
