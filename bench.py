@@ -172,12 +172,13 @@ def main():
         log(f"batched (learned, margin {g.learn_margin}): {l_ms:.3f} ms/step, {learned['qps']:.0f} q/s, "
             f"{learned['vs_headline']:.3f}x the {policy_name} schedule")
 
-    # Roofline of the batch's phases. The headline's one launch mixes all of
-    # them, and its hub steps leave out most of the work that the algorithmic
-    # bytes charge, so the fraction is taken where a launch is one phase: the
-    # same queries on one launch-driven machine (lanes=1), timed with HIP
-    # events on its stream over the timed steps (device time / launches). The
-    # algorithmic bytes per launch are those of that run.
+    # Roofline of the headline's kernel: the HBM bytes that counters measured
+    # for a batch (FETCH_SIZE and WRITE_SIZE runs, scaled by a copy kernel of
+    # known size, kept in profiles/) over its time, when this run is the
+    # workload they were measured on. The bytes that the algorithm charges say
+    # nothing here: hub steps leave out most of them. They are taken where a
+    # launch is one phase, on the same queries by one launch-driven machine
+    # (lanes=1), and reported beside it.
     one = []
     for _ in range(args.steps):
         r1 = g.stcon_batch(s, t, policy=policy, vw=stats["vw"], tile=stats["tile"],
@@ -187,32 +188,31 @@ def main():
     one_ms = float(np.mean([x["time_ms"] for x in one]))
     one_launches = float(np.mean([x["launches"] for x in one]))
     one_bytes = float(np.mean([batch_bytes(x, V, g.offsets64) for x in one]))
-    avg_launch_us = one_ms * 1e3 / one_launches
-    achieved = one_bytes / one_launches / (avg_launch_us * 1e-6) / 1e9
-    log(f"batched, one lane: {one_ms:.3f} ms/step, {one_launches:.0f} launches, {avg_launch_us:.2f} us per launch, "
-        f"{achieved:.0f} GB/s algorithmic")
-    # Measured HBM traffic (FETCH_SIZE and WRITE_SIZE counter runs, scaled by
-    # a copy kernel of known size) is kept per step in profiles/; it applies
-    # when this run is the workload it was measured on.
-    traffic, traffic_src = None, None
+    one_gbs = one_bytes / (one_ms * 1e-3) / 1e9
+    log(f"batched, one lane: {one_ms:.3f} ms/step, {one_launches:.0f} launches, "
+        f"{one_ms * 1e3 / one_launches:.2f} us per launch, {one_gbs:.0f} GB/s algorithmic")
+    traffic, one_traffic, traffic_src = None, None, None
     pmc_path = os.path.join(ROOT, "profiles", "batch_kernel_rmat_s22_pmc.json")
     if os.path.exists(pmc_path):
         pmc = json.load(open(pmc_path))
         m = pmc.get("match", {})
         if (m.get("scale"), m.get("edgefactor"), m.get("pairs"), m.get("policy"), m.get("seed")) == \
                 (args.scale, args.edgefactor, args.pairs, policy_name, args.seed):
-            traffic = int(pmc["traffic_bytes_per_step"] / one_launches)
             traffic_src = pmc_path[len(ROOT) + 1:]
-    launches = int(stats["launches"])
-    roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic, "traffic_source": traffic_src,
-                "kernel": "fcd::batch_kernel<int>", "bytes_per_launch": int(one_bytes / one_launches),
-                "avg_launch_us": round(avg_launch_us, 2), "launches_per_step": round(one_launches, 1),
-                "measured_on": "one launch-driven machine (same queries)",
-                "headline_kernel": "fcd::batch_kernel<int>" if args.lanes else "fcd::batch_team_kernel<int>",
-                "headline_lanes": args.lanes, "headline_launches_per_step": launches,
-                "headline_working_launches_per_step": int(stats["phases"]),
-                "headline_algorithmic_gbs": round(batch_bytes(stats, V, g.offsets64) / (ms_step / 1e3) / 1e9, 1)}
+            one_traffic = int(pmc["traffic_bytes_per_step"])
+            if not args.lanes:
+                traffic = int(pmc["team"]["traffic_bytes_per_step"])
+    achieved = traffic / (ms_step * 1e-3) / 1e9 if traffic else None
+    roofline = {"bound": "hbm", "achieved": round(achieved, 1) if achieved else None, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                "frac": round(achieved / HBM_PEAK_GBS, 4) if achieved else None, "traffic": traffic,
+                "traffic_source": traffic_src,
+                "kernel": "fcd::batch_kernel<int>" if args.lanes else "fcd::batch_team_kernel<int>",
+                "measured_on": "the headline's batches: measured HBM bytes per batch over its time",
+                "lanes": args.lanes, "launches_per_step": int(stats["launches"]), "phases_per_step": int(stats["phases"]),
+                "one_launch_driven_machine": {
+                    "kernel": "fcd::batch_kernel<int>", "ms": round(one_ms, 4), "launches": round(one_launches, 1),
+                    "avg_launch_us": round(one_ms * 1e3 / one_launches, 2), "algorithmic_gbs": round(one_gbs, 1),
+                    "algorithmic_frac": round(one_gbs / HBM_PEAK_GBS, 4), "traffic": one_traffic}}
 
     # ---- plain visits of the same pairs ----
     plain = None
@@ -227,7 +227,7 @@ def main():
         pbytes = 8 * pst["expanded_edges"] + 20 * pst["expanded_vertices"] + 4 * V * nq
         plain = {"qps": round(plain_qps, 1), "ms": round(p_ms, 3), "speedup_batched": round(qps / plain_qps, 2),
                  "roofline": {"kernel": "fcd::st_team_kernel<int> (eight queries at a time, one launch)",
-                              "achieved": round(pbytes / (p_ms / 1e3) / 1e9, 1), "unit": "GB/s",
+                              "measured_on": "algorithmic bytes", "achieved": round(pbytes / (p_ms / 1e3) / 1e9, 1), "unit": "GB/s",
                               "frac": round(pbytes / (p_ms / 1e3) / 1e9 / HBM_PEAK_GBS, 4)}}
         log(f"plain: {p_ms:.1f} ms = {plain_qps:.0f} q/s; batched speedup {qps / plain_qps:.2f}x")
 
@@ -266,6 +266,9 @@ def main():
                "roofline": {"bound": "hbm", "achieved": round(bw, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                             "frac": round(bw / HBM_PEAK_GBS, 4), "kernel": "fcd::phase_kernel<int> (BFS)",
                             "bytes_per_bfs": int(b_bfs / len(bfs_roots)), "traffic_per_bfs": b_traffic,
+                            "traffic_gbs": round(b_traffic / (ms_tot / len(bfs_roots) * 1e-3) / 1e9, 1) if b_traffic else None,
+                            "measured_on": "algorithmic bytes (every edge of a reached vertex); traffic is what "
+                                           "counters measured, less because bottom-up levels stop at a parent",
                             "traffic_source": b_src}}
         log(f"bfs: {gteps:.1f} GTEPS over {len(bfs_roots)} roots, {ms_tot / len(bfs_roots):.3f} ms avg, "
             f"{bw:.0f} GB/s algorithmic = {bw / HBM_PEAK_GBS:.1%} of HBM peak")
