@@ -1858,7 +1858,13 @@ __device__ __forceinline__ void batch_finish(const BatchParams<OffT>& p, const B
       float f[12];
 #pragma unroll
       for (int k = 0; k < 12; ++k) f[k] = lc->feat[k];
-      a = mlp_pick_wave_t(s_mlp, f, a, 1e-3f * (float)lc->learn_margin_milli);
+      const int picked = mlp_pick_wave_t(s_mlp, f, a, 1e-3f * (float)lc->learn_margin_milli);
+      // A team goes bottom-up only where the heuristic does. The network knows
+      // the costs of launches over the whole GPU, where a scan of all vertices
+      // takes tens of us; a team's takes milliseconds (at margin 0, 64 queries
+      // on a random graph of 2M vertices and degree 8: 11.1 ms, 0.39 so; three
+      // lanes 0.44).
+      if (!TEAM || picked / 3 != 2 || a / 3 == 2) a = picked;
     }
     if (threadIdx.x == 0) {
       if (pause) {

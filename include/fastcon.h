@@ -311,7 +311,8 @@ typedef struct fc_batch_opts {
   int32_t words;         /* 64-bit query words per vertex: 1 (64 queries per wave) or 0 (the
                             same); other values are FC_ERR_UNSUPPORTED */
   float   learn_margin;  /* learned policy: the network overrides the heuristic's action only
-                            when it predicts a log-cost lower by at least this; < 0 = 1.0, the
+                            when it predicts a log-cost lower by at least this (in one launch its
+                            bottom-up steps only where the heuristic takes one); < 0 = 1.0, the
                             margin chosen on validation graphs for the shipped parameters (at
                             which the network follows the heuristic on held-out graphs) */
   int32_t lanes;         /* 0 (default): one launch per batch, with a wave machine on each XCD of the

@@ -352,3 +352,20 @@ def test_plain_batches_of_directed_graphs(fc):
     with fc.Graph(hg) as g:
         r = g.stcon_batch(s, t, policy=fc.POLICY_PLAIN)
         assert r.stats["launches"] > 1 and list(r.dist) == exp
+
+
+def test_learned_bottom_up_steps_of_teams(fc, orc):
+    """At margin 0 the network proposes bottom-up steps wherever they are cheap
+    for the whole GPU. A team takes them only where the heuristic would: on a
+    sparse random graph nowhere, so the work stays near the heuristic's."""
+    hg = fc.gen_er(100000, 8.0, 105)
+    s, t = np.random.default_rng(106).integers(0, hg.V, (2, 64)).astype(np.int32)
+    exp = oracle_pair_dists(orc, hg, s, t)
+    with fc.Graph(hg) as g:
+        assert fc.load_default_sched_params(g)
+        h = g.stcon_batch(s, t)
+        for margin in (0.0, 0.25, 1.0):
+            r = g.stcon_batch(s, t, policy=fc.POLICY_LEARNED, learn_margin=margin)
+            assert r.stats["launches"] == 1 and np.array_equal(r.dist, exp)
+            # a step scans at most its frontier, a bottom-up step every vertex
+            assert r.stats["active_vertices"] < h.stats["active_vertices"] + hg.V // 2
